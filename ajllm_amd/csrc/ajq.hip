@@ -43,6 +43,7 @@ int check_launch(const char* what) {
 }
 
 constexpr int kMaxGemvM = 16;
+constexpr int kQuantizeW8RowMaxK = 16384;  // rows that quantize_w8_row_kernel holds in registers
 
 // ---- scratch of the entry point that allocates nothing (ajq_w4a16_gemm_noalloc): the per-row,
 // per-group activation sums of the W4 tile kernels.  Every GPU the library runs on holds its own
@@ -196,28 +197,59 @@ const char* ajq_status_string(int status) {
   }
 }
 
-int ajq_quantize_w8(const float* W, int N, int K, int8_t* q, uint16_t* scales, void* stream) {
-  if (!W || !q || !scales) return fail(AJQ_ERR_NULL, "ajq_quantize_w8: null pointer argument");
+static int quantize_w8(const char* name, const float* W, int N, int K, int8_t* q, uint16_t* scales, uint32_t* wq, hipStream_t st) {
+  if (!W || !q || !scales) return fail(AJQ_ERR_NULL, "%s: null pointer argument", name);
   if (N < 1 || K < 4 || K % 4 != 0)
-    return fail(AJQ_ERR_SHAPE, "ajq_quantize_w8: need N >= 1 and K a positive multiple of 4 (got N=%d, K=%d)", N, K);
-  if (!aligned16(W) || (reinterpret_cast<uintptr_t>(q) & 3u))
-    return fail(AJQ_ERR_ALIGN, "ajq_quantize_w8: W must be 16-byte and q 4-byte aligned");
-  hipLaunchKernelGGL(quantize_w8_kernel, dim3(N), dim3(256), 0, (hipStream_t)stream, W, K, q, scales);
-  return check_launch("ajq_quantize_w8");
+    return fail(AJQ_ERR_SHAPE, "%s: need N >= 1 and K a positive multiple of 4 (got N=%d, K=%d)", name, N, K);
+  if (!aligned16(W) || (reinterpret_cast<uintptr_t>(q) & 3u) || (reinterpret_cast<uintptr_t>(wq) & 3u))
+    return fail(AJQ_ERR_ALIGN, "%s: W must be 16-byte, q and wq 4-byte aligned", name);
+  if (K > kQuantizeW8RowMaxK) {
+    if (wq) return fail(AJQ_ERR_UNSUPPORTED, "%s: K=%d is above %d (quantize and repack one after the other)", name, K, kQuantizeW8RowMaxK);
+    hipLaunchKernelGGL(quantize_w8_kernel, dim3(N), dim3(256), 0, st, W, K, q, scales);
+    return check_launch(name);
+  }
+  const int K128 = (K + kGroup - 1) / kGroup * kGroup;
+  const long long blocks = 128LL * (((N + kTileN - 1) / kTileN + 7) / 8);  // whole tiles of 16 rows, dealt to the 8 XCDs
+  if (blocks > 0x7FFFFFFFLL) return fail(AJQ_ERR_SHAPE, "%s: too many rows", name);
+  auto kernel = K128 <= 1024 ? quantize_w8_row_kernel<1> : K128 <= 2048 ? quantize_w8_row_kernel<2> : K128 <= 4096 ? quantize_w8_row_kernel<4>
+                : K128 <= 8192 ? quantize_w8_row_kernel<8> : quantize_w8_row_kernel<16>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, W, N, K, K128, reinterpret_cast<uint32_t*>(q), scales, wq);
+  return check_launch(name);
+}
+
+int ajq_quantize_w8(const float* W, int N, int K, int8_t* q, uint16_t* scales, void* stream) {
+  return quantize_w8("ajq_quantize_w8", W, N, K, q, scales, nullptr, (hipStream_t)stream);
+}
+
+int ajq_quantize_pack_w8(const float* W, int N, int K, int8_t* q, uint16_t* scales, uint32_t* wq, void* stream) {
+  if (!wq) return fail(AJQ_ERR_NULL, "ajq_quantize_pack_w8: null pointer argument");
+  return quantize_w8("ajq_quantize_pack_w8", W, N, K, q, scales, wq, (hipStream_t)stream);
+}
+
+static int quantize_w4(const char* name, const float* W, int N, int K, int32_t* qweight, uint16_t* scales, uint8_t* zeros,
+                       uint32_t* wq, uint32_t* meta, hipStream_t st) {
+  if (!W || !qweight || !scales || !zeros) return fail(AJQ_ERR_NULL, "%s: null pointer argument", name);
+  if (N < 1 || K < kGroup || K % kGroup != 0)
+    return fail(AJQ_ERR_SHAPE, "%s: need N >= 1 and K a positive multiple of 128 (got N=%d, K=%d)", name, N, K);
+  if (!aligned16(W) || !aligned16(wq)) return fail(AJQ_ERR_ALIGN, "%s: W and wq must be 16-byte aligned", name);
+  const int G = K / kGroup;
+  const long long tiles = (N + kTileN - 1) / kTileN;
+  const long long blocks = tiles * ((G + kQuantizeGroups - 1) / kQuantizeGroups);
+  if (blocks > 0x7FFFFFFFLL) return fail(AJQ_ERR_SHAPE, "%s: too many groups", name);
+  hipLaunchKernelGGL(quantize_w4_kernel, dim3((unsigned)blocks), dim3(256), 0, st, W, N, G, reinterpret_cast<uint32_t*>(qweight),
+                     scales, zeros, reinterpret_cast<u32x4_t*>(wq), meta);
+  return check_launch(name);
 }
 
 int ajq_quantize_w4_g128(const float* W, int N, int K, int32_t* qweight, uint16_t* scales, uint8_t* zeros,
                          void* stream) {
-  if (!W || !qweight || !scales || !zeros) return fail(AJQ_ERR_NULL, "ajq_quantize_w4_g128: null pointer argument");
-  if (N < 1 || K < kGroup || K % kGroup != 0)
-    return fail(AJQ_ERR_SHAPE, "ajq_quantize_w4_g128: need N >= 1 and K a positive multiple of 128 (got N=%d, K=%d)", N, K);
-  if (!aligned16(W)) return fail(AJQ_ERR_ALIGN, "ajq_quantize_w4_g128: W must be 16-byte aligned");
-  const long long groups = (long long)N * (K / kGroup);
-  const long long blocks = (groups + 15) / 16;
-  if (blocks > 0x7FFFFFFFLL) return fail(AJQ_ERR_SHAPE, "ajq_quantize_w4_g128: too many groups");
-  hipLaunchKernelGGL(quantize_w4_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, W, groups,
-                     qweight, scales, zeros);
-  return check_launch("ajq_quantize_w4_g128");
+  return quantize_w4("ajq_quantize_w4_g128", W, N, K, qweight, scales, zeros, nullptr, nullptr, (hipStream_t)stream);
+}
+
+int ajq_quantize_pack_w4_g128(const float* W, int N, int K, int32_t* qweight, uint16_t* scales, uint8_t* zeros, uint32_t* wq,
+                              uint32_t* meta, void* stream) {
+  if (!wq || !meta) return fail(AJQ_ERR_NULL, "ajq_quantize_pack_w4_g128: null pointer argument");
+  return quantize_w4("ajq_quantize_pack_w4_g128", W, N, K, qweight, scales, zeros, wq, meta, (hipStream_t)stream);
 }
 
 static int check_repack(const char* name, const void* a, const void* b, int N, int K, int kmul) {

@@ -23,6 +23,7 @@ SCHEMES = ("w4a16_g128", "w8a16")
 GROUP = 128
 TILE_N = 16
 GEMV_MAX_M = 16
+QUANTIZE_PACK_MAX_K = 16384   # longest row quantize_pack_w8 holds in registers
 
 
 def _stream() -> int:
@@ -140,6 +141,44 @@ def unrepack_w8(wq: torch.Tensor) -> torch.Tensor:
     return q
 
 
+def quantize_pack_w8(weight: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """:func:`quantize_w8` and :func:`repack_w8` of its codes in one pass: (q, scales, wq)."""
+    _require_cuda(weight)
+    if weight.dim() != 2:
+        raise ValueError("weight must be [N, K]")
+    w = weight.detach().to(torch.float32).contiguous()
+    n, k = w.shape
+    q = torch.empty((n, k), dtype=torch.int8, device=w.device)
+    scales = torch.empty((n,), dtype=torch.float16, device=w.device)
+    wq = torch.empty(((n + TILE_N - 1) // TILE_N, (k + GROUP - 1) // GROUP * 2, 64, 4), dtype=torch.int32, device=w.device)
+    with torch.cuda.device(w.device):
+        status = _lib.load().ajq_quantize_pack_w8(w.data_ptr(), n, k, q.data_ptr(), scales.data_ptr(), wq.data_ptr(), _stream())
+    _lib.check(status, "quantize_pack_w8")
+    return q, scales, wq
+
+
+def quantize_pack_w4(weight: torch.Tensor) -> tuple[torch.Tensor, ...]:
+    """:func:`quantize_w4_g128` and :func:`repack_w4` of its tensors in one pass: (qweight, scales, zeros, wq, meta)."""
+    _require_cuda(weight)
+    if weight.dim() != 2:
+        raise ValueError("weight must be [N, K]")
+    w = weight.detach().to(torch.float32).contiguous()
+    n, k = w.shape
+    if k % GROUP != 0:
+        raise ValueError(f"K={k} must be a multiple of {GROUP} for w4a16_g128")
+    tiles, groups = (n + TILE_N - 1) // TILE_N, k // GROUP
+    qweight = torch.empty((n, k // 8), dtype=torch.int32, device=w.device)
+    scales = torch.empty((n, groups), dtype=torch.float16, device=w.device)
+    zeros = torch.empty((n, groups), dtype=torch.uint8, device=w.device)
+    wq = torch.empty((tiles, groups, 64, 4), dtype=torch.int32, device=w.device)
+    meta = torch.empty((tiles, groups, TILE_N), dtype=torch.int32, device=w.device)
+    with torch.cuda.device(w.device):
+        status = _lib.load().ajq_quantize_pack_w4_g128(w.data_ptr(), n, k, qweight.data_ptr(), scales.data_ptr(), zeros.data_ptr(),
+                                                       wq.data_ptr(), meta.data_ptr(), _stream())
+    _lib.check(status, "quantize_pack_w4")
+    return qweight, scales, zeros, wq, meta
+
+
 # --------------------------------------------------------------------------- matmul
 def _prep_x(x: torch.Tensor, k: int) -> torch.Tensor:
     _require_cuda(x)
@@ -236,12 +275,16 @@ class QuantLinear(nn.Module):
         """Quantize an fp32 ``[out, in]`` weight that already lives on the GPU."""
         out_features, in_features = weight.shape
         self = cls(in_features, out_features, scheme)
-        if scheme == "w8a16":
+        if scheme == "w8a16" and (in_features > QUANTIZE_PACK_MAX_K or in_features % 4 != 0):
             self.qweight, self.scales = quantize_w8(weight)
             self.zeros = torch.empty(0, dtype=torch.uint8, device=weight.device)
+            self.prepare()
+        elif scheme == "w8a16":
+            self.qweight, self.scales, self.wq = quantize_pack_w8(weight)
+            self.zeros = torch.empty(0, dtype=torch.uint8, device=weight.device)
+            self.meta = _pad_rows(self.scales, self.wq.shape[0] * TILE_N)
         else:
-            self.qweight, self.scales, self.zeros = quantize_w4_g128(weight)
-        self.prepare()
+            self.qweight, self.scales, self.zeros, self.wq, self.meta = quantize_pack_w4(weight)
         return self
 
     @classmethod

@@ -89,6 +89,12 @@ int ajq_quantize_w8(const float* W, int N, int K, int8_t* q, uint16_t* scales, v
  * zeros uint8 [N, K/128].  K % 128 == 0. */
 int ajq_quantize_w4_g128(const float* W, int N, int K, int32_t* qweight, uint16_t* scales,
                          uint8_t* zeros, void* stream);
+/* The same with the kernel-private tensors of ajq_repack_* (rows and, for W8, columns padded with zero codes) written in the
+ * same pass: wq [N16/16, K128/64, 64, 4] for W8 (K <= 16384; K128 = K rounded up to 128, N16 = N to 16), wq
+ * [N16/16, K/128, 64, 4] and meta [N16/16, K/128, 16] for W4. */
+int ajq_quantize_pack_w8(const float* W, int N, int K, int8_t* q, uint16_t* scales, uint32_t* wq, void* stream);
+int ajq_quantize_pack_w4_g128(const float* W, int N, int K, int32_t* qweight, uint16_t* scales, uint8_t* zeros, uint32_t* wq,
+                              uint32_t* meta, void* stream);
 
 /* canonical -> kernel-private layout and back.  N % 16 == 0; K % 128 == 0 for W4,
  * K % 64 == 0 for W8 (the W8 matmuls below additionally need K % 128 == 0). */

@@ -113,3 +113,43 @@ def test_repack_w8_round_trip(cuda, n, k):
     q2 = unrepack_w8(wq)
     assert torch.equal(q2[:n], q)
     assert int(q2[n:].abs().sum()) == 0
+
+
+def _odd_values(n: int, k: int) -> torch.Tensor:
+    """Rows and groups whose quotients leave the ordinary range: infinities, NaN, huge offsets, overflowing scales, denormals."""
+    g = torch.Generator().manual_seed(n + k)
+    w = torch.randn(n, k, generator=g)
+    values = (float("inf"), float("-inf"), float("nan"), 3e38, -3e38, 2e6, 1e-40, 2.0 ** 100)
+    for i in range(min(n, 3 * len(values))):
+        w[i, (37 * i) % k] = values[i % len(values)]
+    if n > 2:
+        w[-1] = 1e38 + 1e31 * w[-1]
+        w[-2] *= 1e-42
+    return w
+
+
+@pytest.mark.parametrize("odd", [False, True])
+@pytest.mark.parametrize("n,k", [(1, 128), (16, 512), (33, 1152), (24, 8320), (1000, 2048), (5, 16512)])
+def test_quantize_and_pack_in_one_pass(cuda, n, k, odd):
+    """The layer's tensors against the quantizer's statement and the repack kernels: row and column remainders, rows that are too
+    long for the registers, one and several runs of groups per workgroup; bit for bit."""
+    from ajllm_amd import QuantLinear, repack_w4, repack_w8
+    from ajllm_amd.quant import _pad_rows
+
+    w = _odd_values(n, k) if odd else make_weight(n, k, 11)
+    layer = QuantLinear.from_weight(w.to(cuda), "w4a16_g128")
+    with np.errstate(all="ignore"):
+        q, s, z = qspec.quantize_w4_g128(w.numpy())
+    if not odd:   # (the statement leaves the codes of quotients that are no number open)
+        assert np.array_equal(layer.qweight.cpu().numpy(), qspec.pack_int4(q)) and np.array_equal(layer.zeros.cpu().numpy(), z)
+    assert np.array_equal(layer.scales.cpu().numpy().view(np.uint16), s.view(np.uint16)) or odd
+    wq, meta = repack_w4(layer.qweight, layer.scales, layer.zeros)
+    assert torch.equal(layer.wq, wq) and torch.equal(layer.meta, meta)
+    for cols in (k, k - 4):   # W8 columns need no grid
+        layer = QuantLinear.from_weight(w[:, :cols].contiguous().to(cuda), "w8a16")
+        with np.errstate(all="ignore"):
+            q, s = qspec.quantize_w8(w[:, :cols].numpy())
+        if not odd:
+            assert np.array_equal(layer.qweight.cpu().numpy(), q) and np.array_equal(layer.scales.cpu().numpy().view(np.uint16), s.view(np.uint16))
+        assert torch.equal(layer.wq, repack_w8(layer.qweight))
+        assert torch.equal(layer.meta.view(torch.int16), _pad_rows(layer.scales, layer.wq.shape[0] * 16).view(torch.int16))
