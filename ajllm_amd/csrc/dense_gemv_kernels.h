@@ -13,8 +13,8 @@
 //   dense_out_streams_kernel  product whose epilogue mixes it into several residual streams and forms what the next sublayer reads
 //
 // A 16 x 16 output tile (16 weight rows, 16 batch columns) belongs to a wave, or to kWaves waves that split K and meet in
-// LDS.  Lane l = 16 g + r loads 16 bytes of weight row r at k = 32 step + 8 g: four lanes cover 64 contiguous bytes of a
-// row, two steps a cache line.
+// LDS.  The small products' lane l = 16 g + r loads 16 bytes of weight row r at k = 32 step + 8 g (`tile_steps`); the large
+// ones stream whole lines (`stream_rows`).
 #pragma once
 #include "dense_kernels.h"
 #include "latent_attention.h"
@@ -59,14 +59,6 @@ __device__ __forceinline__ void tile_steps(const uint16_t* __restrict__ wrow, in
   }
 }
 
-// the K range of one of kWaves waves, in pairs of steps (a cache line of a weight row stays with one wave)
-__device__ __forceinline__ void wave_steps(int K, int wave, int waves, int& begin, int& end) {
-  const int steps = (K + 31) >> 5;
-  const int per = ((steps + waves - 1) / waves + 1) & ~1;
-  begin = min(steps, wave * per);
-  end = min(steps, begin + per);
-}
-
 // sum of the waves' tiles; tile (n, t) is valid in wave n BT + t
 template <int kWaves, int RT, int BT>
 __device__ __forceinline__ void meet(f32x4_t (&acc)[RT][BT], float* red, int wave, int lane) {
@@ -92,6 +84,135 @@ __device__ __forceinline__ void meet(f32x4_t (&acc)[RT][BT], float* red, int wav
   }
 }
 
+// acc[n][t] += W[rows of tile n, :] x_t for RT tiles of ROWS (16 or 8) consecutive rows of a row-major W [.., K], K split over
+// kWaves waves in blocks of 128 columns.  `w`: the first row; `x(t, step)`: the B fragment of batch tile t at 32 step (batch
+// column r, k = 32 step + 8 g ..), finite or zero past K; `between` runs while the first blocks travel.  `lds`:
+// stream_lds() bytes; the tiles' sums of all waves are complete in wave n BT + t (as `meet` leaves them).
+//
+// Bound: HBM.  What costs is how a row-major matrix is asked for: the product's own operand layout wants 64 bytes of each of 16
+// rows per instruction, half a line everywhere, and streams at 4.4 TB/s; four rows of 256 bytes per instruction stream at 5.9
+// (4096 x 18432, 8 sequences: 38.3 -> 25.7 us; 35424 x 4096: 63.0 -> 46.3; 2048 x 8192: 13.9 -> 7.9 with tiles of 8 rows on
+// twice as many CUs).  The block then takes the operand layout on its way through wave-private LDS (no barrier; chunk c of row
+// r lies in slot c ^ r, so that both the rows' writes and the operand reads meet all banks), while the next one travels.
+constexpr int kStreamBlock = 128;
+constexpr int stream_lds(int waves, int rows, int rt, int bt, int uq) {
+  return waves * uq * rt * rows * 256 > rt * bt * waves * 1024 ? waves * uq * rt * rows * 256 : rt * bt * waves * 1024;
+}
+template <int kWaves, int ROWS, int RT, int BT, int UQ, typename Between, typename XFn>
+__device__ __forceinline__ void stream_rows(const uint16_t* __restrict__ w, int K, int wave, int lane, unsigned char* lds,
+                                            f32x4_t (&acc)[RT][BT], Between&& between, XFn&& x) {
+  static_assert(ROWS == 16 || ROWS == 8, "tiles of 16 or 8 rows");
+  constexpr int kLoads = ROWS / 4;  // instructions of 1 KiB per tile and block
+  const int r = lane & 15, g = lane >> 4, rr = ROWS == 16 ? r : r & 7;
+  const int full = K / kStreamBlock, per = (full + kWaves - 1) / kWaves;
+  const int begin = min(full, wave * per), count = min(full, begin + per) - begin;
+  unsigned char* mine = lds + wave * (UQ * RT * ROWS * 256);
+  // row 4 j + lane / 16 of a tile, chunk (lane % 16) ^ row
+  uint32_t at[kLoads];
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) at[j] = (uint32_t)(4 * j + g) * (2u * K) + 16u * (r ^ (4 * j + g));
+  const unsigned char* base = reinterpret_cast<const unsigned char*>(w);
+  const size_t tile = (size_t)ROWS * 2 * K;
+  u32x4_t wr[2][UQ][RT][kLoads], xr[2][UQ][BT][4];
+  auto load_w = [&](int buf, int q) {
+#pragma unroll
+    for (int i = 0; i < UQ; ++i)
+#pragma unroll
+      for (int n = 0; n < RT; ++n)
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j)
+          wr[buf][i][n][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(base + n * tile + (size_t)(q + i) * 256 + at[j]));
+  };
+  auto load_x = [&](int buf, int q) {
+#pragma unroll
+    for (int i = 0; i < UQ; ++i)
+#pragma unroll
+      for (int t = 0; t < BT; ++t)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) xr[buf][i][t][s] = x(t, 4 * (q + i) + s);
+  };
+  auto put = [&](int i, int n, int j, const u32x4_t& v) {
+    *reinterpret_cast<u32x4_t*>(mine + ((i * RT + n) * kLoads + j) * 1024 + lane * 16) = v;
+  };
+  auto operand = [&](int i, int n, int s) {
+    return *reinterpret_cast<const u32x4_t*>(mine + (i * RT + n) * kLoads * 1024 + rr * 256 + ((4 * s + g) ^ rr) * 16);
+  };
+  auto use = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < UQ; ++i)
+#pragma unroll
+      for (int n = 0; n < RT; ++n)
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) put(i, n, j, wr[buf][i][n][j]);
+#pragma unroll
+    for (int i = 0; i < UQ; ++i)
+#pragma unroll
+      for (int n = 0; n < RT; ++n)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const u32x4_t f = operand(i, n, s);
+#pragma unroll
+          for (int t = 0; t < BT; ++t) acc[n][t] = mfma16(f, xr[buf][i][t][s], acc[n][t]);
+        }
+  };
+  if (count >= UQ) load_w(0, begin);
+  between();
+  int s = begin, left = count;
+  if (left >= UQ) {
+    load_x(0, s);
+    for (; left >= 3 * UQ; left -= 2 * UQ, s += 2 * UQ) {
+      load_w(1, s + UQ);
+      load_x(1, s + UQ);
+      __builtin_amdgcn_sched_barrier(0);
+      use(0);
+      load_w(0, s + 2 * UQ);
+      load_x(0, s + 2 * UQ);
+      __builtin_amdgcn_sched_barrier(0);
+      use(1);
+    }
+    if (left >= 2 * UQ) {
+      load_w(1, s + UQ);
+      load_x(1, s + UQ);
+      __builtin_amdgcn_sched_barrier(0);
+      use(0);
+      use(1);
+      left -= 2 * UQ;
+      s += 2 * UQ;
+    } else {
+      use(0);
+      left -= UQ;
+      s += UQ;
+    }
+  }
+  // a block at a time: what UQ leaves over, and (in the last wave) the columns of a block that K cuts short, zero past it
+  const bool cut = wave == kWaves - 1 && K % kStreamBlock != 0;
+  for (; left > 0 || (left == 0 && cut); --left) {
+    const bool partial = left == 0;
+    const int q = partial ? full : s++;
+    const u32x4_t zero = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int n = 0; n < RT; ++n)
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        u32x4_t v = zero;
+        if (!partial || kStreamBlock * q + 8 * (r ^ (4 * j + g)) < K)
+          v = *reinterpret_cast<const u32x4_t*>(base + n * tile + (size_t)q * 256 + at[j]);
+        put(0, n, j, v);
+      }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int t = 0; t < BT; ++t) {
+        u32x4_t v = zero;
+        if (!partial || kStreamBlock * q + 32 * k + 8 * g < K) v = x(t, 4 * q + k);
+#pragma unroll
+        for (int n = 0; n < RT; ++n) acc[n][t] = mfma16(operand(0, n, k), v, acc[n][t]);
+      }
+  }
+  __syncthreads();
+  meet<kWaves, RT, BT>(acc, reinterpret_cast<float*>(lds), wave, lane);
+}
+
 struct DenseIn {
   const float* x;           // [B, Dp] residual rows (norm prologue)
   const uint16_t* n1;       // or [B, Dp] bf16 rows already normed by gain 1 / gain 2
@@ -111,18 +232,16 @@ struct DenseIn {
 template <int kWaves, bool kNorm, int RT, int BT>
 __global__ __launch_bounds__(64 * kWaves) void dense_in_kernel(DenseIn a) {
   extern __shared__ __attribute__((aligned(16))) uint16_t normed[];
-  __shared__ __attribute__((aligned(16))) float red[kWaves > 1 ? RT * BT * kWaves * 256 : 4];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[stream_lds(kWaves, 16, RT, BT, 1)];
   __shared__ float stat[kWaves];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int b0 = blockIdx.y * kGemvBatch * BT, nb = min(kGemvBatch * BT, a.batch - b0);
   const int groups1 = (a.tiles1 + RT - 1) / RT;
   const bool second = (int)blockIdx.x >= groups1;
   const int tiles = second ? a.tiles2 : a.tiles1;
   // the last workgroup of an odd matrix overlaps its neighbour: the same rows give the same values twice
   const int tile0 = max(0, min(RT * (second ? (int)blockIdx.x - groups1 : (int)blockIdx.x), tiles - RT));
-  const uint16_t* wrow = (second ? a.w2 : a.w1) + (size_t)(16 * tile0 + r) * a.Dp;
-  int begin, end;
-  wave_steps(a.Dp, wave, kWaves, begin, end);
+  const uint16_t* wrow = (second ? a.w2 : a.w1) + (size_t)(16 * tile0) * a.Dp;
   f32x4_t acc[RT][BT] = {};
   if constexpr (kNorm) {
     const float* gain = second ? a.gain2 : a.gain1;
@@ -138,64 +257,63 @@ __global__ __launch_bounds__(64 * kWaves) void dense_in_kernel(DenseIn a) {
       for (int w = 1; w < kWaves; ++w) s += stat[w];
       return s;
     };
-    for (int b = 0; b < nb; ++b) {
-      const float* x = a.x + (size_t)(b0 + b) * a.Dp;
-      float4 keep[kKeep];
-      float sum = 0.f;
-#pragma unroll
-      for (int j = 0; j < kKeep; ++j) {
-        const int i = 4 * (threadIdx.x + kThreads * j);
-        keep[j] = i < a.Dp ? load4(x + i) : float4{0.f, 0.f, 0.f, 0.f};
-        sum += (keep[j].x + keep[j].y) + (keep[j].z + keep[j].w);
-      }
-      for (int i = 4 * (threadIdx.x + kThreads * kKeep); i < a.Dp; i += 4 * kThreads) {
-        const float4 v = load4(x + i);
-        sum += (v.x + v.y) + (v.z + v.w);
-      }
-      const float mean = a.center ? block_sum(sum) / (float)a.D : 0.f;
-      float ss = 0.f;
-      auto square = [&](int i, const float4& v) {
-        const float p = v.x - mean, q = v.y - mean, s = v.z - mean, t = v.w - mean;
-        if (i + 3 < a.D) {
-          ss += (p * p + q * q) + (s * s + t * t);
-        } else {
-          if (i < a.D) ss += p * p;
-          if (i + 1 < a.D) ss += q * q;
-          if (i + 2 < a.D) ss += s * s;
+    auto norm = [&]() {
+      for (int b = 0; b < nb; ++b) {
+        const float* x = a.x + (size_t)(b0 + b) * a.Dp;
+        float4 keep[kKeep];
+        float sum = 0.f;
+  #pragma unroll
+        for (int j = 0; j < kKeep; ++j) {
+          const int i = 4 * (threadIdx.x + kThreads * j);
+          keep[j] = i < a.Dp ? load4(x + i) : float4{0.f, 0.f, 0.f, 0.f};
+          sum += (keep[j].x + keep[j].y) + (keep[j].z + keep[j].w);
         }
-      };
-#pragma unroll
-      for (int j = 0; j < kKeep; ++j) square(4 * (threadIdx.x + kThreads * j), keep[j]);
-      for (int i = 4 * (threadIdx.x + kThreads * kKeep); i < a.Dp; i += 4 * kThreads) square(i, load4(x + i));
-      const Divisor by(sqrtf(block_sum(ss) / (float)a.D + a.eps));
-      auto put = [&](int i, const float4& v) {
-        const float4 w = load4(gain + i);
-        store4(normed + b * stride + i, float4{by.divide(v.x - mean) * w.x, by.divide(v.y - mean) * w.y,
-                                               by.divide(v.z - mean) * w.z, by.divide(v.w - mean) * w.w});
-      };
-#pragma unroll
-      for (int j = 0; j < kKeep; ++j) {
-        const int i = 4 * (threadIdx.x + kThreads * j);
-        if (i < a.Dp) put(i, keep[j]);
+        for (int i = 4 * (threadIdx.x + kThreads * kKeep); i < a.Dp; i += 4 * kThreads) {
+          const float4 v = load4(x + i);
+          sum += (v.x + v.y) + (v.z + v.w);
+        }
+        const float mean = a.center ? block_sum(sum) / (float)a.D : 0.f;
+        float ss = 0.f;
+        auto square = [&](int i, const float4& v) {
+          const float p = v.x - mean, q = v.y - mean, s = v.z - mean, t = v.w - mean;
+          if (i + 3 < a.D) {
+            ss += (p * p + q * q) + (s * s + t * t);
+          } else {
+            if (i < a.D) ss += p * p;
+            if (i + 1 < a.D) ss += q * q;
+            if (i + 2 < a.D) ss += s * s;
+          }
+        };
+  #pragma unroll
+        for (int j = 0; j < kKeep; ++j) square(4 * (threadIdx.x + kThreads * j), keep[j]);
+        for (int i = 4 * (threadIdx.x + kThreads * kKeep); i < a.Dp; i += 4 * kThreads) square(i, load4(x + i));
+        const Divisor by(sqrtf(block_sum(ss) / (float)a.D + a.eps));
+        auto put = [&](int i, const float4& v) {
+          const float4 w = load4(gain + i);
+          store4(normed + b * stride + i, float4{by.divide(v.x - mean) * w.x, by.divide(v.y - mean) * w.y,
+                                                 by.divide(v.z - mean) * w.z, by.divide(v.w - mean) * w.w});
+        };
+  #pragma unroll
+        for (int j = 0; j < kKeep; ++j) {
+          const int i = 4 * (threadIdx.x + kThreads * j);
+          if (i < a.Dp) put(i, keep[j]);
+        }
+        for (int i = 4 * (threadIdx.x + kThreads * kKeep); i < a.Dp; i += 4 * kThreads) put(i, load4(x + i));
       }
-      for (int i = 4 * (threadIdx.x + kThreads * kKeep); i < a.Dp; i += 4 * kThreads) put(i, load4(x + i));
-    }
-    __syncthreads();
-    tile_steps<RT, BT>(wrow, a.Dp, begin, end, g, acc, [&](int t, int s) {
-      const int row = 16 * t + r;
-      return row < nb ? *reinterpret_cast<const u32x4_t*>(normed + row * stride + 8 * g + 32 * s) : u32x4_t{0u, 0u, 0u, 0u};
+      __syncthreads();
+    };
+    stream_rows<kWaves, 16, RT, BT, 1>(wrow, a.Dp, wave, lane, lds, acc, norm, [&](int t, int s) {
+      return *reinterpret_cast<const u32x4_t*>(normed + min(16 * t + r, nb - 1) * stride + 8 * g + 32 * s);
     });
   } else {
     const uint16_t* xr = (second ? a.n2 : a.n1) + (size_t)b0 * a.Dp + 8 * g;
-    tile_steps<RT, BT>(wrow, a.Dp, begin, end, g, acc, [&](int t, int s) {
-      const int row = 16 * t + r;
-      return row < nb ? *reinterpret_cast<const u32x4_t*>(xr + (size_t)row * a.Dp + 32 * s) : u32x4_t{0u, 0u, 0u, 0u};
+    stream_rows<kWaves, 16, RT, BT, 1>(wrow, a.Dp, wave, lane, lds, acc, [] {}, [&](int t, int s) {
+      return *reinterpret_cast<const u32x4_t*>(xr + (size_t)min(16 * t + r, nb - 1) * a.Dp + 32 * s);
     });
   }
-  meet<kWaves, RT, BT>(acc, red, wave, lane);
 #pragma unroll
   for (int i = 0; i < RT * BT; ++i) {
-    if (kWaves > 1 && wave != i) continue;
+    if (wave != i) continue;
     const f32x4_t& sum = acc[i / BT][i % BT];
     const int row = 16 * (i % BT) + r, tile = tile0 + i / BT;
     if (!second) {
@@ -224,45 +342,38 @@ struct DenseOut {
   const float* step;        // [Dp] or null, added too
   int batch, K, Dp;
 };
-template <int kWaves, int RT, int BT>
+// ROWS, kWaves: tiles of 16 rows on four waves, or of 8 on eight (few tiles); UQ as in stream_rows.
+template <int kWaves, int ROWS, int RT, int BT, int UQ>
 __global__ __launch_bounds__(64 * kWaves) void dense_out_kernel(DenseOut a) {
-  __shared__ __attribute__((aligned(16))) float red[kWaves > 1 ? RT * BT * kWaves * 256 : 4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[stream_lds(kWaves, ROWS, RT, BT, UQ)];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int b0 = blockIdx.y * kGemvBatch * BT, nb = min(kGemvBatch * BT, a.batch - b0);
-  const int first = blockIdx.x * RT * 16;  // (RT divides the row tiles: x is updated in place)
-  const uint16_t* wrow = a.w + (size_t)(first + r) * a.K;
+  const int first = blockIdx.x * RT * ROWS;  // (RT divides the row tiles: x is updated in place)
   const uint16_t* xr = a.in + (size_t)b0 * a.K + 8 * g;
-  int begin, end;
-  wave_steps(a.K, wave, kWaves, begin, end);
-  // what the product of tile i = (row tile, batch tile) is added to, requested ahead of it by the wave that will write it
-  auto place = [&](int i) { return (size_t)(b0 + min(16 * (i % BT) + r, nb - 1)) * a.Dp + first + 16 * (i / BT) + 4 * g; };
-  float4 old[kWaves > 1 ? 1 : RT * BT];
-#pragma unroll
-  for (int i = 0; i < RT * BT; ++i) {
-    if (kWaves > 1 && wave != i) continue;
-    float4 v = load4(a.x + place(i));
+  // what the product of tile wave = (row tile, batch tile) is added to, requested ahead of it by the wave that will write it
+  const bool writes = wave < RT * BT && 4 * g < ROWS;
+  const int row = 16 * (wave % BT) + r, column = first + ROWS * (wave / BT) + 4 * g;
+  const size_t place = (size_t)(b0 + min(row, nb - 1)) * a.Dp + column;
+  float4 v = float4{0.f, 0.f, 0.f, 0.f};
+  if (writes) {
+    v = load4(a.x + place);
     if (a.again) {
-      const float4 e = load4(a.again + place(i));
+      const float4 e = load4(a.again + place);
       v.x += e.x; v.y += e.y; v.z += e.z; v.w += e.w;
     }
     if (a.step) {
-      const float4 e = load4(a.step + first + 16 * (i / BT) + 4 * g);
+      const float4 e = load4(a.step + column);
       v.x += e.x; v.y += e.y; v.z += e.z; v.w += e.w;
     }
-    old[kWaves > 1 ? 0 : i] = v;
   }
   f32x4_t acc[RT][BT] = {};
-  tile_steps<RT, BT>(wrow, a.K, begin, end, g, acc, [&](int t, int s) {
-    const int row = 16 * t + r;
-    return row < nb ? *reinterpret_cast<const u32x4_t*>(xr + (size_t)row * a.K + 32 * s) : u32x4_t{0u, 0u, 0u, 0u};
+  stream_rows<kWaves, ROWS, RT, BT, UQ>(a.w + (size_t)first * a.K, a.K, wave, lane, lds, acc, [] {}, [&](int t, int s) {
+    return *reinterpret_cast<const u32x4_t*>(xr + (size_t)min(16 * t + r, nb - 1) * a.K + 32 * s);
   });
-  meet<kWaves, RT, BT>(acc, red, wave, lane);
 #pragma unroll
   for (int i = 0; i < RT * BT; ++i) {
-    if ((kWaves > 1 && wave != i) || 16 * (i % BT) + r >= nb) continue;
-    const float4 v = old[kWaves > 1 ? 0 : i];
     const f32x4_t& sum = acc[i / BT][i % BT];
-    store4(a.x + place(i), float4{v.x + sum[0], v.y + sum[1], v.z + sum[2], v.w + sum[3]});
+    if (wave == i && writes && row < nb) store4(a.x + place, float4{v.x + sum[0], v.y + sum[1], v.z + sum[2], v.w + sum[3]});
   }
 }
 
@@ -277,41 +388,31 @@ struct DenseOutStreams {
   float* u;                 // [B, Dp], what the next reader gets
   int batch, K, Dp, streams;
 };
-template <int kWaves, int RT, int BT, int MAXS>
+template <int kWaves, int ROWS, int RT, int BT, int UQ, int MAXS>
 __global__ __launch_bounds__(64 * kWaves) void dense_out_streams_kernel(DenseOutStreams a) {
-  __shared__ __attribute__((aligned(16))) float red[kWaves > 1 ? RT * BT * kWaves * 256 : 4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[stream_lds(kWaves, ROWS, RT, BT, UQ)];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int b0 = blockIdx.y * kGemvBatch * BT, nb = min(kGemvBatch * BT, a.batch - b0);
-  const int first = blockIdx.x * RT * 16;
-  const uint16_t* wrow = a.w + (size_t)(first + r) * a.K;
+  const int first = blockIdx.x * RT * ROWS;
   const uint16_t* xr = a.in + (size_t)b0 * a.K + 8 * g;
-  int begin, end;
-  wave_steps(a.K, wave, kWaves, begin, end);
-  // the streams at this lane's place of tile i = (row tile, batch tile); with several waves each writes one tile and
-  // requests its streams ahead of the product
-  auto fetch = [&](int i, float4 (&v)[MAXS]) {
-    const float* x = a.x + (size_t)(b0 + min(16 * (i % BT) + r, nb - 1)) * a.streams * a.Dp + first + 16 * (i / BT) + 4 * g;
-#pragma unroll
-    for (int s = 0; s < MAXS; ++s)
-      if (s < a.streams) v[s] = load4(x + (size_t)s * a.Dp);
-  };
+  // the streams at this lane's place of tile wave = (row tile, batch tile), requested ahead of the product
+  const bool writes = wave < RT * BT && 4 * g < ROWS;
+  const int row = 16 * (wave % BT) + r, column = first + ROWS * (wave / BT) + 4 * g;
+  float* x = a.x + (size_t)(b0 + min(row, nb - 1)) * a.streams * a.Dp + column;
   float4 v[MAXS];
-  if (kWaves > 1 && wave < RT * BT) fetch(wave, v);
+#pragma unroll
+  for (int s = 0; s < MAXS; ++s)
+    if (writes && s < a.streams) v[s] = load4(x + (size_t)s * a.Dp);
   f32x4_t acc[RT][BT] = {};
-  tile_steps<RT, BT>(wrow, a.K, begin, end, g, acc, [&](int t, int s) {
-    const int row = 16 * t + r;
-    return row < nb ? *reinterpret_cast<const u32x4_t*>(xr + (size_t)row * a.K + 32 * s) : u32x4_t{0u, 0u, 0u, 0u};
+  stream_rows<kWaves, ROWS, RT, BT, UQ>(a.w + (size_t)first * a.K, a.K, wave, lane, lds, acc, [] {}, [&](int t, int s) {
+    return *reinterpret_cast<const u32x4_t*>(xr + (size_t)min(16 * t + r, nb - 1) * a.K + 32 * s);
   });
-  meet<kWaves, RT, BT>(acc, red, wave, lane);
 #pragma unroll
   for (int i = 0; i < RT * BT; ++i) {
-    const int row = 16 * (i % BT) + r, column = first + 16 * (i / BT) + 4 * g;
-    if ((kWaves > 1 && wave != i) || row >= nb) continue;
-    if (kWaves == 1) fetch(i, v);
+    if (wave != i || !writes || row >= nb) continue;
     const f32x4_t& sum = acc[i / BT][i % BT];
     const float4 f = load4(a.scale + column);
     mix_streams<MAXS>(v, a.streams, a.out, a.mix, float4{sum[0] * f.x, sum[1] * f.y, sum[2] * f.z, sum[3] * f.w});
-    float* x = a.x + (size_t)(b0 + row) * a.streams * a.Dp + column;
 #pragma unroll
     for (int s = 0; s < MAXS; ++s)
       if (s < a.streams) store4(x + (size_t)s * a.Dp, v[s]);

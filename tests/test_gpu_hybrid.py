@@ -747,3 +747,27 @@ def test_checkpoint_trace_and_command_line(cuda, tmp_path, capsys):
                     "--max-new-tokens", "12"]) == 0
     new = [int(t) for t in capsys.readouterr().out.strip().splitlines()[-1].split(",")]
     assert len(new) == 12 and float(_margins(cfg, weights, prompt, new).max()) < 1e-3
+
+
+@pytest.mark.parametrize("batch", [1, 16, 17])
+@pytest.mark.parametrize("k,width", [(128, 2064), (136, 2048), (1544, 8192), (6152, 2064), (8192, 48)])
+def test_streamed_products(cuda, batch, k, width):
+    """dense_out and dense_in where a wavefront has none, one, two, three and more blocks of 128 columns, with and without a block cut
+    short, on tiles of 8 and 16 rows, one and two row tiles; against 64 bits, 32-bit sums of k products."""
+    g = torch.Generator().manual_seed(k + width + batch)
+    a, w, x = _bf(g, batch, k), _bf(g, width, k, std=k ** -0.5), torch.randn((batch, width), generator=g)
+    da, dw, dx = a.to(cuda), w.to(cuda), x.to(cuda)
+    lib, want = _lib.load_dense(), a.double() @ w.double().T
+    _ok(lib.ajqd_dense_out(_p(da), _p(dw), _p(dx), None, None, batch, k, width, _st()))
+    assert _rel(dx, x.double() + want) < 2e-6
+    y = torch.full((batch, width), 9.0, device=cuda)
+    rows = torch.randn((batch, k), generator=g)
+    gain = torch.randn(k, generator=g)
+    dr, dg = rows.to(cuda), gain.to(cuda)
+    args = dict(w1=_p(dw), y1=_p(y), batch=batch, true_width=k, width=k, tiles1=width // 16, tiles2=0, gated_ld=0, act=0, center=0, pairs=0, eps=1e-3)
+    _ok(lib.ajqd_dense_in(ctypes.byref(_lib.DenseInArgs(n1=_p(da), **args)), _st()))
+    assert _rel(y, want) < 2e-6
+    if batch == 1:
+        _ok(lib.ajqd_dense_in(ctypes.byref(_lib.DenseInArgs(x=_p(dr), gain1=_p(dg), **args)), _st()))
+        normed = O.centered_rms_norm(rows, gain - 1, 1e-3).bfloat16()
+        assert _rel(y, normed.double() @ w.double().T) < 1e-3   # (a norm rounded the other way moves an operand by 2^-8)
