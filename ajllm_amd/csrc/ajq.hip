@@ -15,6 +15,7 @@
 #include "gemm_split_kernels.h"
 #include "gemm_wide_kernels.h"
 #include "gemm128_kernels.h"
+#include "gemm_mid_kernels.h"
 #include "skinny_kernels.h"
 #include "skinny_resident_kernels.h"
 #include "decode_kernels.h"
@@ -167,7 +168,7 @@ int launch_gemm128(const uint16_t* x, int M, int K, const uint32_t* wq, const ui
   const int tiles = ((M + kG1BM - 1) / kG1BM) * ((N + kG1BN - 1) / kG1BN);
   hipLaunchKernelGGL(kernel, dim3(tiles), dim3(128 * AJQ_G1_WN), lds, stream, x, M, K,
                      reinterpret_cast<const u32x4_t*>(wq), meta, scales8,
-                     reinterpret_cast<const u32x4_t*>(gs3), N, y, out_f32);
+                     reinterpret_cast<const u32x4_t*>(gs3), N, y, out_f32, 1);
   return AJQ_OK;
 }
 
@@ -999,6 +1000,89 @@ MatmulKernel pick_matmul_kernel(int M, int N, int K, bool w4) {
   return us_small < us_big ? kTiles128 : kTiles256;
 }
 
+// ---- routes that cut K into parts and add the parts' sums in a second launch: shapes whose output is too small to fill the chip
+// and whose K is long.  They need a workspace, so only ajq_*_matmul takes them.
+//  * kRouteMid (gemm_mid_kernels.h): 17 .. 48 rows, int8 up to 64, K other than the resident form's 2048 and 4096, from 16 (int4:
+//    20) million weights on; up to 32 rows only K > 8192.  Below that the streaming kernel's one launch is the faster (3840 x 4816,
+//    32 rows, int8: 10.6 against 11.1 us; 8192 x 8192, 20 rows: 18.6 / 20.6; int4 at 64 rows, K = 14336: 21.0 / 20.1, 11008: 18.3 / 18.7);
+//  * kRouteTiles (gemm128_kernels.h): where the estimate says so by a clear margin.  A k-block of a 128 x 128 tile takes 0.76 us
+//    (int8) / 0.80 (int4) whether 32 or 256 workgroups run, so 256 / tiles parts of K cost that much less: K = 14336, N = 4096, int8 /
+//    int4: 256 rows 65 -> 39 / 54 -> 42 us, 512 rows 91 -> 64 / 97 -> 70; K = 5632, N = 2048, 384 rows, int8 30 -> 19.  The other side
+//    of the estimate: the streaming kernel at 420 (int8) / 440 TFLOP/s up to 128 rows and 470 above, whole 128- and 256-row tiles
+//    by rounds.  K = 2048 and 4096 stay with the resident form up to 256 rows (int4: 512: 27.3 us against 30.2), int4 below 160
+//    rows with the streaming kernel (K = 14336, 128 rows: 27.2 against 28.7), and small matrices below 320 (2048 x 7168, 256 rows, int8:
+//    18.4 against 18.2 at best).
+enum SplitKind { kRouteWhole, kRouteMid, kRouteTiles };
+struct SplitRoute {
+  SplitKind kind = kRouteWhole;
+  int S = 1, mb = 0;
+  size_t sums = 0, bytes = 0;   // int4 tiles: bytes of group sums ahead of the parts; all of the workspace
+};
+size_t group_sum_bytes(int M, int K) { return (size_t)(K / kGroup) * M * 16; }
+SplitRoute pick_split(int M, int N, int K, bool w4) {
+  SplitRoute r;
+  const int G = K / kGroup;
+  const double weights = (double)N * K;
+  if (M <= kMaxGemvM || (long long)M * K * 2 >= (1LL << 32)) return r;
+  if (M <= 64) {
+    if (K == 2048 || K == 4096 || weights < (w4 ? 20e6 : 16e6) || (M <= 32 && K <= 8192) || (M > 48 && (w4 || weights < 24e6))) return r;
+    if (skinny_split_applies(M, N, K)) return r;  // a lent buffer: the streaming kernel's own split, one launch
+    r.mb = M <= 32 ? 2 : M <= 48 ? 3 : 4;
+    const int blocks = (N + kMidColumns - 1) / kMidColumns;
+    r.S = std::max(1, std::min(std::min(256 / blocks, 16), G / kMidTeams));
+    r.kind = kRouteMid;
+    r.bytes = r.S > 1 ? (size_t)r.S * M * N * 4 : 0;
+    return r;
+  }
+  if ((w4 && M < 160) || ((K == 2048 || K == 4096) && M <= (w4 ? 512 : 256)) || (weights < 16e6 && (w4 || M < 320))) return r;
+  const long long tm = (M + 127) / 128, tn = (N + 127) / 128, tiles = tm * tn;
+  const int S = (int)std::min(std::min(256 / tiles, 16LL), (long long)(G / 4));
+  if (S < 2) return r;
+  const double split = (G + S - 1) / S * (w4 ? 0.80 : 0.76) + (w4 ? 9.7 : 7.7) + 8.0 * S * M * N / 13e6;
+  const double flops = 2.0 * M * N * K;
+  const double stream = M <= 128 ? flops / (w4 ? 440e6 : 420e6) + 3.0 : flops / 470e6 + 2.0;
+  const double small_ = (double)((tiles + 255) / 256) * G * 0.78 + 6.0;
+  double other = std::min(stream, small_);
+  if (M >= kGemm256MinM)
+    other = std::min(other, (double)(((M + 255) / 256 * tn + 255) / 256) * G * (w4 ? 1.45 : 1.15) + 5.0);
+  if (split >= 0.88 * other) return r;
+  r.kind = kRouteTiles;
+  r.S = S;
+  r.sums = w4 ? (group_sum_bytes(M, K) + 255) / 256 * 256 : 0;
+  r.bytes = r.sums + (size_t)S * M * N * 4;
+  return r;
+}
+
+template <bool kW4>
+int launch_split(const SplitRoute& r, const uint16_t* x, int M, int K, const uint32_t* wq, const uint32_t* meta, const uint16_t* scales8,
+                 int N, void* y, int out_f32, void* workspace, hipStream_t stream) {
+  float* parts = reinterpret_cast<float*>(static_cast<char*>(workspace) + r.sums);
+  if (r.kind == kRouteMid) {
+    auto kernel = r.mb == 2 ? dequant_gemm_mid_kernel<kW4, 2> : r.mb == 3 ? dequant_gemm_mid_kernel<kW4, 3> : dequant_gemm_mid_kernel<kW4, 4>;
+    if (int s = allow_big_lds(kernel, mid_lds_bytes(r.mb))) return s;
+    const int units = (N + kMidColumns - 1) / kMidColumns * r.S;
+    hipLaunchKernelGGL(kernel, dim3(8 * ((units + 7) / 8)), dim3(64 * kMidWaves * kMidTeams), mid_lds_bytes(r.mb), stream, x, M, K,
+                       reinterpret_cast<const u32x4_t*>(wq), meta, scales8, N, r.S, y, out_f32, parts);
+  } else {
+    if (kW4) {
+      const long long teams = (long long)M * ((K / kGroup + 3) / 4);
+      hipLaunchKernelGGL(group_sum3_kernel, dim3((unsigned)((teams + 15) / 16)), dim3(256), 0, stream, x, M, K,
+                         reinterpret_cast<u32x4_t*>(workspace));
+    }
+    auto kernel = dequant_gemm128_kernel<kW4, 4, false, true>;
+    constexpr size_t lds = kW4 ? kG1LdsBytesW4 : kG1LdsBytesW8;
+    if (int s = allow_big_lds(kernel, lds)) return s;
+    const int units = (N + kG1BN - 1) / kG1BN * r.S, tm = (M + kG1BM - 1) / kG1BM;
+    hipLaunchKernelGGL(kernel, dim3(8 * ((units + 7) / 8) * tm), dim3(512), lds, stream, x, M, K, reinterpret_cast<const u32x4_t*>(wq),
+                       meta, scales8, reinterpret_cast<const u32x4_t*>(workspace), N, parts, 1, r.S);
+  }
+  if (r.S > 1) {
+    const long long size = (long long)M * N;
+    hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)((size / 8 + 255) / 256)), dim3(256), 0, stream, parts, size, r.S, y, out_f32);
+  }
+  return AJQ_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1210,6 +1294,37 @@ int ajq_w4a16_gemm(const uint16_t* x, int M, int K, const uint32_t* wq, const ui
                      K, reinterpret_cast<u32x4_t*>(workspace));
   if (int s = launch_gemm128<true>(x, M, K, wq, meta, nullptr, workspace, N, y, out_f32, (hipStream_t)stream)) return s;
   return check_launch("ajq_w4a16_gemm");
+}
+
+size_t ajq_matmul_scratch_bytes(int M, int N, int K, int w4) {
+  if (M < 1 || N < kTileN || N % kTileN || K < kGroup || K % kGroup) return 0;
+  const SplitRoute r = pick_split(M, N, K, w4 != 0);
+  return r.kind != kRouteWhole ? r.bytes : w4 ? ajq_w4a16_gemm_workspace_bytes_for(M, N, K) : 0;
+}
+
+// the split route for these arguments, where the workspace holds it
+static SplitRoute split_route(int M, int N, int K, bool w4, const void* workspace, size_t bytes) {
+  SplitRoute r = pick_split(M, N, K, w4);
+  if (r.bytes > 0 && (!workspace || bytes < r.bytes || !aligned16(workspace))) r.kind = kRouteWhole;
+  return r;
+}
+
+int ajq_w4a16_matmul(const uint16_t* x, int M, int K, const uint32_t* wq, const uint32_t* meta, int N, void* y, int out_dtype,
+                     void* workspace, size_t workspace_bytes, void* stream) {
+  if (int s = check_matmul_args("ajq_w4a16_matmul", x, M, K, wq, meta, N, y, out_dtype, kGroup)) return s;
+  const SplitRoute r = split_route(M, N, K, true, workspace, workspace_bytes);
+  if (r.kind == kRouteWhole) return ajq_w4a16_gemm(x, M, K, wq, meta, N, y, out_dtype, workspace, workspace_bytes, stream);
+  if (int s = launch_split<true>(r, x, M, K, wq, meta, nullptr, N, y, out_dtype == AJQ_OUT_F32, workspace, (hipStream_t)stream)) return s;
+  return check_launch("ajq_w4a16_matmul");
+}
+
+int ajq_w8a16_matmul(const uint16_t* x, int M, int K, const uint32_t* wq, const uint16_t* scales, int N, void* y, int out_dtype,
+                     void* workspace, size_t workspace_bytes, void* stream) {
+  if (int s = check_matmul_args("ajq_w8a16_matmul", x, M, K, wq, scales, N, y, out_dtype, kGroup)) return s;
+  const SplitRoute r = split_route(M, N, K, false, workspace, workspace_bytes);
+  if (r.kind == kRouteWhole || (reinterpret_cast<uintptr_t>(scales) & 7u)) return ajq_w8a16_gemm(x, M, K, wq, scales, N, y, out_dtype, stream);
+  if (int s = launch_split<false>(r, x, M, K, wq, nullptr, scales, N, y, out_dtype == AJQ_OUT_F32, workspace, (hipStream_t)stream)) return s;
+  return check_launch("ajq_w8a16_matmul");
 }
 
 size_t ajq_noalloc_scratch_bytes(void) { return kScratchBytes; }

@@ -35,13 +35,15 @@ constexpr size_t kG1LdsBytesW8 = kG1WBase + kG1Ring * kG1W8Slot;       // 144 Ki
 // kGate (kWN = 4 only): w1 | w3 weights of a SwiGLU feed-forward, output bf16( silu(a) * u ),
 // [M, N / 2]; the workgroup's four 32-column blocks alternate between the two halves as in
 // the 256 x 128 kernels, here one block per wave, so the pairs meet in an fp32 staging tile.
-template <bool kW4, int kWN, bool kGate = false>
+// kSplit: K is cut into S parts of whole groups, a workgroup computes one part of a tile and leaves fp32 sums in
+// y = [S][M][N], which gemm_split_reduce_kernel adds in order; any M >= 1 (rows past the last repeat it and are not stored).
+template <bool kW4, int kWN, bool kGate = false, bool kSplit = false>
 __global__ __launch_bounds__(128 * kWN) void dequant_gemm128_kernel(
     const uint16_t* __restrict__ x, int M, int K, const u32x4_t* __restrict__ wq,
     const uint32_t* __restrict__ meta,     // W4: private meta; W8: unused
     const uint16_t* __restrict__ scales8,  // W8: fp16 [N]; W4: unused
     const u32x4_t* __restrict__ gs3,       // W4: [K/128][M] group-sum pieces; W8: unused
-    int N, void* __restrict__ y, int out_f32) {
+    int N, void* __restrict__ y, int out_f32, int S) {
   constexpr int MT = 2;
   constexpr int kSteps = kW4 ? 9 : 8;  // MFMA k-steps per 128-k block
   constexpr int kWaves = 2 * kWN;
@@ -61,11 +63,20 @@ __global__ __launch_bounds__(128 * kWN) void dequant_gemm128_kernel(
 
   // column-major walk over output tiles: consecutive workgroups share a column block of W
   const int tiles_m = (M + kG1BM - 1) / kG1BM;
-  const int tile_m = blockIdx.x % tiles_m, tile_n = blockIdx.x / tiles_m;
+  int tile_m = blockIdx.x % tiles_m, tile_n = blockIdx.x / tiles_m, split = 0;
+  if (kSplit) {  // the row tiles of one (column block, part of K) meet the same weights: consecutive slots of one XCD
+    const int unit = (int)(blockIdx.x & 7) + 8 * ((int)(blockIdx.x >> 3) / tiles_m);
+    tile_m = (int)(blockIdx.x >> 3) % tiles_m;
+    tile_n = unit / S;
+    split = unit % S;
+    if (tile_n >= (N + kG1BN - 1) / kG1BN) return;  // padding of the last round
+  }
   static_assert(!kGate || kWN == 4, "the gate epilogue pairs the blocks of waves 2 j and 2 j + 1");
-  const int m0 = min(tile_m * kG1BM, M - kG1BM);  // M >= 128: the last row tile is shifted up
+  // the last row tile is shifted up to end at row M; with fewer than 128 rows (kSplit) row M - 1 is repeated
+  const int m0 = kSplit ? max(0, min(tile_m * kG1BM, M - kG1BM)) : min(tile_m * kG1BM, M - kG1BM);
   const int n0 = tile_n * (kGate ? kG1BN / 2 : kG1BN);  // kGate: first of the workgroup's 64 columns of each half
   const int G = K >> 7;
+  const int kb0 = kSplit ? (int)((long long)G * split / S) : 0, kb1 = kSplit ? (int)((long long)G * (split + 1) / S) : G;
   const int ntiles16 = N / kTileN;
 
   // ---- global -> LDS.  Activations: wave w fills kLoadRows rows (128 / waves) with wave-wide
@@ -76,8 +87,9 @@ __global__ __launch_bounds__(128 * kWN) void dequant_gemm128_kernel(
   uint32_t a_voff[4];
 #pragma unroll
   for (int v = 0; v < 4; ++v)
-    a_voff[v] = (uint32_t)row_in * (uint32_t)K * 2u + (uint32_t)((slot16 ^ (4 * v + row_in)) * 16);
-  const char* a_base = reinterpret_cast<const char*>(x) + (size_t)(m0 + kLoadRows * wave) * K * 2;
+    a_voff[v] = (kSplit ? (uint32_t)min(m0 + kLoadRows * wave + 4 * v + row_in, M - 1) : (uint32_t)row_in) * (uint32_t)K * 2u +
+                (uint32_t)((slot16 ^ (4 * v + row_in)) * 16);
+  const char* a_base = reinterpret_cast<const char*>(x) + (kSplit ? (size_t)0 : (size_t)(m0 + kLoadRows * wave) * K * 2);
   const int nt16_0 = n0 / kTileN;
   // the workgroup's T-th private 16-column tile (T = 0 .. 7) in the weight tensor; tiles past the
   // matrix repeat the last one (their columns are never stored)
@@ -93,7 +105,8 @@ __global__ __launch_bounds__(128 * kWN) void dequant_gemm128_kernel(
       (uint32_t)((col_tile((wave & 1) * 4 + (lane >> 4)) * G * 16 + (lane & 15)) * 4);
   auto issue_load = [&](int j, int kb, int ring) {
     if (j < kALoads) {
-      const char* src = a_base + (size_t)kb * 256 + (size_t)j * 4 * K * 2;
+      static_assert(!kSplit || kLoadRows == 16, "a request per four of the wave's rows");
+      const char* src = a_base + (size_t)kb * 256 + (kSplit ? (size_t)0 : (size_t)j * 4 * K * 2);
       dma16(src, a_voff[j & 3], (uint32_t)(ring * kG1TileBytes + wave * (kLoadRows * 256) + j * 1024));
     } else if (j < kALoads + kBLoads) {
       const int T = wave * kBLoads + (j - kALoads);
@@ -105,7 +118,8 @@ __global__ __launch_bounds__(128 * kWN) void dequant_gemm128_kernel(
       dma16(tile, lane16, (uint32_t)(kG1WBase + ring * kWSlot + T * 1024));
     } else if (j == kALoads + kBLoads) {
       const int e = wave & 1;  // group-sum pieces of 64 rows
-      dma16(gs3 + (size_t)kb * M + m0 + 64 * e, lane16, (uint32_t)(kG1SideBase + ring * kG1SideSlot + e * 1024));
+      const uint32_t at = kSplit ? (uint32_t)min(m0 + 64 * e + lane, M - 1) * 16u : lane16;
+      dma16(gs3 + (size_t)kb * M + (kSplit ? 0 : m0 + 64 * e), at, (uint32_t)(kG1SideBase + ring * kG1SideSlot + e * 1024));
     } else {
       const int e = wave & 1;  // meta words, 4 tiles per load
       dma4(meta + (size_t)kb * 16, meta_voff, (uint32_t)(kG1MetaBase + ring * kG1MetaSlot + e * 256));
@@ -133,19 +147,19 @@ __global__ __launch_bounds__(128 * kWN) void dequant_gemm128_kernel(
 
   // blocks 0 and 1 are requested up front; block 0 has landed when at most one block's loads are out
 #pragma unroll
-  for (int j = 0; j < kLoads; ++j) issue_load(j, 0, 0);
+  for (int j = 0; j < kLoads; ++j) issue_load(j, kb0, 0);
 #pragma unroll
-  for (int j = 0; j < kLoads; ++j) issue_load(j, min(1, G - 1), 1);
+  for (int j = 0; j < kLoads; ++j) issue_load(j, min(kb0 + 1, kb1 - 1), 1);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
   __syncthreads();
 
   const W4Consts w4c = w4_consts();
 
   int ring = 0;  // slot of the current block
-  for (int kb = 0; kb < G; ++kb) {
+  for (int kb = kb0; kb < kb1; ++kb) {
     // Loads are issued unconditionally (past the end the last block is simply fetched again): a
     // branch between the MFMAs would cut the loop body into separately scheduled pieces.
-    const int kb_load = min(kb + 2, G - 1);
+    const int kb_load = min(kb + 2, kb1 - 1);
     const int ring_load = ring == 0 ? 2 : ring - 1;  // (ring + 2) % 3: the slot read one block ago
 
     u32x4_t raw[TB][kW4 ? 2 : 4];
@@ -303,7 +317,7 @@ __global__ __launch_bounds__(128 * kWN) void dequant_gemm128_kernel(
     }
     return;
   }
-  if (!out_f32) {
+  if (!kSplit && !out_f32) {
 #pragma unroll
     for (int t = 0; t < TB; ++t)
 #pragma unroll
@@ -336,9 +350,34 @@ __global__ __launch_bounds__(128 * kWN) void dequant_gemm128_kernel(
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = m0 + wm * kWaveRows + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * kh;
-        reinterpret_cast<float*>(y)[(size_t)m * N + n] = acc[i][t][r] * cs[t];
+        if (kSplit) {
+          if (m < M) reinterpret_cast<float*>(y)[((size_t)split * M + m) * N + n] = acc[i][t][r] * cs[t];
+        } else {
+          reinterpret_cast<float*>(y)[(size_t)m * N + n] = acc[i][t][r] * cs[t];
+        }
       }
     }
+  }
+}
+
+// y = the S parts' sums, added in order.  A thread makes eight columns of a row; bound by the partial sums' way through the caches
+// (S = 4, 256 x 4096: 3.5 us with its launch).
+__global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float* __restrict__ partial, long long size, int S,
+                                                                void* __restrict__ y, int out_f32) {
+  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (8 * idx >= size) return;
+  const f32x4_t* p = reinterpret_cast<const f32x4_t*>(partial) + 2 * idx;
+  f32x4_t a = p[0], b = p[1];
+#pragma unroll 4
+  for (int s = 1; s < S; ++s) {
+    a += p[(size_t)s * (size / 4)];
+    b += p[(size_t)s * (size / 4) + 1];
+  }
+  if (out_f32) {
+    reinterpret_cast<f32x4_t*>(y)[2 * idx] = a;
+    reinterpret_cast<f32x4_t*>(y)[2 * idx + 1] = b;
+  } else {
+    reinterpret_cast<u32x4_t*>(y)[idx] = u32x4_t{pack2_bf16(a[0], a[1]), pack2_bf16(a[2], a[3]), pack2_bf16(b[0], b[1]), pack2_bf16(b[2], b[3])};
   }
 }
 

@@ -216,11 +216,11 @@ def w4a16_matmul(
                 x.data_ptr(), m, k, wq.data_ptr(), meta.data_ptr(), n16, y.data_ptr(), flag, _stream()
             )
         else:
-            nbytes = lib.ajq_w4a16_gemm_workspace_bytes_for(m, n16, k)  # 0 unless the 128 x 128 tile kernel runs
-            workspace = torch.empty((max(nbytes, 16),), dtype=torch.uint8, device=x.device)
-            status = lib.ajq_w4a16_gemm(
+            nbytes = lib.ajq_matmul_scratch_bytes(m, n16, k, 1)
+            workspace = torch.empty((nbytes,), dtype=torch.uint8, device=x.device) if nbytes else None
+            status = lib.ajq_w4a16_matmul(
                 x.data_ptr(), m, k, wq.data_ptr(), meta.data_ptr(), n16, y.data_ptr(), flag,
-                workspace.data_ptr(), nbytes, _stream(),
+                workspace.data_ptr() if nbytes else None, nbytes, _stream(),
             )
     _lib.check(status, "w4a16_matmul")
     return y
@@ -241,9 +241,14 @@ def w8a16_matmul(
         return y
     lib = _lib.load()
     use_gemv = (m <= GEMV_MAX_M) if kernel == "auto" else (kernel == "gemv")
-    fn = lib.ajq_w8a16_gemv if use_gemv else lib.ajq_w8a16_gemm
     with torch.cuda.device(x.device):
-        status = fn(x.data_ptr(), m, k, wq.data_ptr(), scales.data_ptr(), n16, y.data_ptr(), flag, _stream())
+        if use_gemv:
+            status = lib.ajq_w8a16_gemv(x.data_ptr(), m, k, wq.data_ptr(), scales.data_ptr(), n16, y.data_ptr(), flag, _stream())
+        else:
+            nbytes = lib.ajq_matmul_scratch_bytes(m, n16, k, 0)
+            workspace = torch.empty((nbytes,), dtype=torch.uint8, device=x.device) if nbytes else None
+            status = lib.ajq_w8a16_matmul(x.data_ptr(), m, k, wq.data_ptr(), scales.data_ptr(), n16, y.data_ptr(), flag,
+                                          workspace.data_ptr() if nbytes else None, nbytes, _stream())
     _lib.check(status, "w8a16_matmul")
     return y
 

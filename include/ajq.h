@@ -243,6 +243,15 @@ int ajq_w8a16_gemm(const uint16_t* x, int M, int K, const uint32_t* wq, const ui
 size_t ajq_matmul_workspace_bytes(void);
 int ajq_matmul_workspace_set(void* workspace, size_t bytes);
 
+/* Any M on the fastest route, some of which cut K into parts whose sums lie in a workspace:
+ * ajq_matmul_scratch_bytes says how many bytes (0: none; w4: 1 for W4, 0 for W8).  With a smaller workspace (or none) the call
+ * runs as ajq_*_gemm does. */
+size_t ajq_matmul_scratch_bytes(int M, int N, int K, int w4);
+int ajq_w4a16_matmul(const uint16_t* x, int M, int K, const uint32_t* wq, const uint32_t* meta, int N, void* y, int out_dtype,
+                     void* workspace, size_t workspace_bytes, void* stream);
+int ajq_w8a16_matmul(const uint16_t* x, int M, int K, const uint32_t* wq, const uint16_t* scales, int N, void* y, int out_dtype,
+                     void* workspace, size_t workspace_bytes, void* stream);
+
 /* ajq_w4a16_gemm for callers that cannot allocate device memory or pass a workspace (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the group sums live in
  * a 16 MiB array inside the library's code object, one copy per GPU, held until the process ends

@@ -624,3 +624,40 @@ def test_gemv_residual_then_rowscale_against_the_oracle(cuda, scheme, m, k1, d, 
     assert lib.ajq_gemv_epilogue_supported(256, 2048) == 0 and lib.ajq_gemv_epilogue_supported(9, 5632) == 1
     assert row_fn(xt.data_ptr(), ssq.data_ptr(), 6, eps, m, d, wq2.data_ptr(), meta2.data_ptr(), n2, y.data_ptr(),
                   _lib.AJQ_OUT_F32, 0, st) != 0
+
+
+# (M, N, K) of the routes that cut K: every row-block height at its edges, a last column block cut short, parts of unequal length, one
+# part only; the tiles' shifted and short last row tile; and shapes beside the rules' lines
+_SPLIT_SHAPES = [(17, 2064, 14336), (32, 4096, 8320), (33, 4112, 5632), (48, 16016, 1408), (49, 8208, 3072), (64, 3088, 8192), (37, 33008, 640),
+                 (65, 4112, 8192), (128, 2576, 11008), (129, 4096, 5632), (200, 4112, 8320), (333, 2064, 5760), (384, 4096, 6144), (700, 2048, 8192)]
+
+
+@pytest.mark.parametrize("m,n,k", _SPLIT_SHAPES)
+@pytest.mark.parametrize("scheme", ["w4", "w8"])
+def test_matmul_split_into_parts_of_k(cuda, scheme, m, n, k):
+    """The fastest route (with the workspace it asks for) and the route without one, against the oracle's weight in fp64 and, to the
+    bit, against themselves on other contents of the workspace."""
+    from ajllm_amd import _lib
+
+    lib = _lib.load()
+    w_hat, wq, meta = _quantized(scheme, n, k, 900 + n + k, cuda)
+    x = make_activations(m, k, 3 * m + n, True).to(cuda)
+    want = x.double() @ w_hat.to(cuda).double().t()
+    nbytes = lib.ajq_matmul_scratch_bytes(m, n, k, int(scheme == "w4"))
+    fn = lib.ajq_w4a16_matmul if scheme == "w4" else lib.ajq_w8a16_matmul
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(size, fill, dtype):
+        y = torch.full((m, n), 7.0, dtype=dtype, device=cuda)
+        ws = torch.full((size + 256,), fill, dtype=torch.uint8, device=cuda)
+        _lib.check(fn(x.data_ptr(), m, k, wq.data_ptr(), meta.data_ptr(), n, y.data_ptr(),
+                      _lib.AJQ_OUT_F32 if dtype == torch.float32 else _lib.AJQ_OUT_BF16, ws.data_ptr() if size else None, size, stream), "matmul")
+        assert (ws[size:] == fill).all()
+        return y
+
+    y32 = run(nbytes, 0xFF, torch.float32)
+    for y in (y32, run(max(0, lib.ajq_w4a16_gemm_workspace_bytes_for(m, n, k)) if scheme == "w4" else 0, 0, torch.float32)):
+        max_abs, rel_fro = errors(y.double().cpu(), want.cpu())
+        assert max_abs <= 2e-3 and rel_fro <= 1e-5, (max_abs, rel_fro)
+    assert torch.equal(run(nbytes, 0x3C, torch.float32), y32)
+    assert torch.equal(run(nbytes, 0, torch.bfloat16), y32.to(torch.bfloat16))
