@@ -30,6 +30,11 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+# (handle of the current stream of a device, without the object around it that costs as much as the call it is for)
+_raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(torch._C, "_cuda_getCurrentRawStream") else (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 def _require_cuda(*tensors: torch.Tensor) -> None:
     for t in tensors:
         if not t.is_cuda:
@@ -180,21 +185,43 @@ def quantize_pack_w4(weight: torch.Tensor) -> tuple[torch.Tensor, ...]:
 
 
 # --------------------------------------------------------------------------- matmul
-def _prep_x(x: torch.Tensor, k: int) -> torch.Tensor:
-    _require_cuda(x)
+_OUT_FLAGS = {torch.bfloat16: _lib.AJQ_OUT_BF16, torch.float32: _lib.AJQ_OUT_F32}
+
+
+def _matmul(w4: bool, x: torch.Tensor, k: int, wq: torch.Tensor, aux: torch.Tensor, out_dtype: torch.dtype, kernel: str) -> torch.Tensor:
+    """One product through the C ABI.  A decode step makes one of these per projection and token: as little Python as the
+    checks need (5 us of 15 per call with device and stream objects made anew, 9 all told without)."""
+    if not x.is_cuda:
+        _require_cuda(x)
     if x.dim() != 2 or x.shape[1] != k:
         raise ValueError(f"x must be [M, {k}], got {tuple(x.shape)}")
-    if x.dtype != torch.bfloat16:
+    if x.dtype is not torch.bfloat16:
         raise ValueError("activations must be bfloat16")
-    return x.contiguous()
-
-
-def _out(m: int, n: int, out_dtype: torch.dtype, device: torch.device) -> tuple[torch.Tensor, int]:
-    if out_dtype == torch.bfloat16:
-        return torch.empty((m, n), dtype=torch.bfloat16, device=device), _lib.AJQ_OUT_BF16
-    if out_dtype == torch.float32:
-        return torch.empty((m, n), dtype=torch.float32, device=device), _lib.AJQ_OUT_F32
-    raise ValueError("out_dtype must be torch.bfloat16 or torch.float32")
+    flag = _OUT_FLAGS.get(out_dtype)
+    if flag is None:
+        raise ValueError("out_dtype must be torch.bfloat16 or torch.float32")
+    if not x.is_contiguous():
+        x = x.contiguous()
+    m, n16, index = x.shape[0], wq.shape[0] * TILE_N, x.device.index
+    if index != torch.cuda.current_device():
+        with torch.cuda.device(index):
+            return _matmul(w4, x, k, wq, aux, out_dtype, kernel)
+    y = x.new_empty((m, n16), dtype=out_dtype)
+    if m == 0:
+        return y
+    lib = _lib.load()
+    if (m <= GEMV_MAX_M) if kernel == "auto" else (kernel == "gemv"):
+        fn = lib.ajq_w4a16_gemv if w4 else lib.ajq_w8a16_gemv
+        status = fn(x.data_ptr(), m, k, wq.data_ptr(), aux.data_ptr(), n16, y.data_ptr(), flag, _raw_stream(index))
+    else:
+        nbytes = lib.ajq_matmul_scratch_bytes(m, n16, k, w4)
+        workspace = x.new_empty((nbytes,), dtype=torch.uint8) if nbytes else None
+        fn = lib.ajq_w4a16_matmul if w4 else lib.ajq_w8a16_matmul
+        status = fn(x.data_ptr(), m, k, wq.data_ptr(), aux.data_ptr(), n16, y.data_ptr(), flag,
+                    workspace.data_ptr() if nbytes else None, nbytes, _raw_stream(index))
+    if status:
+        _lib.check(status, "w4a16_matmul" if w4 else "w8a16_matmul")
+    return y
 
 
 def w4a16_matmul(
@@ -202,28 +229,7 @@ def w4a16_matmul(
     kernel: str = "auto",
 ) -> torch.Tensor:
     """y[M, N16] = x[M, K] @ W_hat^T for private W4 tensors.  ``kernel``: auto | gemv | gemm."""
-    n16, k = wq.shape[0] * TILE_N, wq.shape[1] * GROUP
-    x = _prep_x(x, k)
-    m = x.shape[0]
-    y, flag = _out(m, n16, out_dtype, x.device)
-    if m == 0:
-        return y
-    lib = _lib.load()
-    use_gemv = (m <= GEMV_MAX_M) if kernel == "auto" else (kernel == "gemv")
-    with torch.cuda.device(x.device):
-        if use_gemv:
-            status = lib.ajq_w4a16_gemv(
-                x.data_ptr(), m, k, wq.data_ptr(), meta.data_ptr(), n16, y.data_ptr(), flag, _stream()
-            )
-        else:
-            nbytes = lib.ajq_matmul_scratch_bytes(m, n16, k, 1)
-            workspace = torch.empty((nbytes,), dtype=torch.uint8, device=x.device) if nbytes else None
-            status = lib.ajq_w4a16_matmul(
-                x.data_ptr(), m, k, wq.data_ptr(), meta.data_ptr(), n16, y.data_ptr(), flag,
-                workspace.data_ptr() if nbytes else None, nbytes, _stream(),
-            )
-    _lib.check(status, "w4a16_matmul")
-    return y
+    return _matmul(True, x, wq.shape[1] * GROUP, wq, meta, out_dtype, kernel)
 
 
 def w8a16_matmul(
@@ -231,26 +237,11 @@ def w8a16_matmul(
     kernel: str = "auto",
 ) -> torch.Tensor:
     """y[M, N16] = x[M, K] @ W_hat^T for private W8 tensors; ``scales`` fp16 [N16]."""
-    n16, k = wq.shape[0] * TILE_N, wq.shape[1] * 64
-    x = _prep_x(x, k)
-    if scales.numel() != n16:
-        raise ValueError(f"scales must have {n16} entries (rows padded to a multiple of 16)")
-    m = x.shape[0]
-    y, flag = _out(m, n16, out_dtype, x.device)
-    if m == 0:
-        return y
-    lib = _lib.load()
-    use_gemv = (m <= GEMV_MAX_M) if kernel == "auto" else (kernel == "gemv")
-    with torch.cuda.device(x.device):
-        if use_gemv:
-            status = lib.ajq_w8a16_gemv(x.data_ptr(), m, k, wq.data_ptr(), scales.data_ptr(), n16, y.data_ptr(), flag, _stream())
-        else:
-            nbytes = lib.ajq_matmul_scratch_bytes(m, n16, k, 0)
-            workspace = torch.empty((nbytes,), dtype=torch.uint8, device=x.device) if nbytes else None
-            status = lib.ajq_w8a16_matmul(x.data_ptr(), m, k, wq.data_ptr(), scales.data_ptr(), n16, y.data_ptr(), flag,
-                                          workspace.data_ptr() if nbytes else None, nbytes, _stream())
-    _lib.check(status, "w8a16_matmul")
-    return y
+    if not x.is_cuda:
+        _require_cuda(x)
+    if scales.numel() != wq.shape[0] * TILE_N:
+        raise ValueError(f"scales must have {wq.shape[0] * TILE_N} entries (rows padded to a multiple of 16)")
+    return _matmul(False, x, wq.shape[1] * 64, wq, scales, out_dtype, kernel)
 
 
 # --------------------------------------------------------------------------- the layer
@@ -362,25 +353,24 @@ class QuantLinear(nn.Module):
             self.prepare()
 
     def forward(self, inputs: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.Tensor:
-        if self.wq is None:
+        buffers, k, want = self._buffers, self.in_features, out_dtype or inputs.dtype
+        wq = buffers["wq"]
+        if wq is None:
             raise RuntimeError("QuantLinear has no weights: build it with from_linear()/from_weight()")
         lead = inputs.shape[:-1]
-        x = inputs.reshape(-1, self.in_features)
-        want = out_dtype or inputs.dtype
-        if x.dtype != torch.bfloat16:
+        x = inputs if inputs.dim() == 2 and inputs.shape[1] == k else inputs.reshape(-1, k)
+        if x.dtype is not torch.bfloat16:
             x = x.to(torch.bfloat16)
-        if self.padded_in_features != self.in_features:  # W8 with in_features off the kernels' 128-column grid
-            x = torch.nn.functional.pad(x, (0, self.padded_in_features - self.in_features))
-        kernel_out = torch.float32 if want == torch.float32 else torch.bfloat16
-        if self.scheme == "w8a16":
-            y = w8a16_matmul(x, self.wq, self.meta, kernel_out)
-        else:
-            y = w4a16_matmul(x, self.wq, self.meta, kernel_out)
+        w4 = self.scheme != "w8a16"
+        if k % GROUP != 0:  # W8 with in_features off the kernels' 128-column grid
+            x = torch.nn.functional.pad(x, (0, self.padded_in_features - k))
+        kernel_out = torch.float32 if want is torch.float32 else torch.bfloat16
+        y = _matmul(w4, x, self.padded_in_features if k % GROUP else k, wq, buffers["meta"], kernel_out, "auto")
         if y.shape[1] != self.out_features:
             y = y[:, : self.out_features]
-        if y.dtype != want:
+        if kernel_out is not want:
             y = y.to(want)
-        return y.reshape(*lead, self.out_features)
+        return y if len(lead) == 1 and lead[0] == y.shape[0] else y.reshape(*lead, self.out_features)
 
     def extra_repr(self) -> str:
         return f"in_features={self.in_features}, out_features={self.out_features}, scheme={self.scheme}"

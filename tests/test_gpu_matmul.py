@@ -661,3 +661,18 @@ def test_matmul_split_into_parts_of_k(cuda, scheme, m, n, k):
         assert max_abs <= 2e-3 and rel_fro <= 1e-5, (max_abs, rel_fro)
     assert torch.equal(run(nbytes, 0x3C, torch.float32), y32)
     assert torch.equal(run(nbytes, 0, torch.bfloat16), y32.to(torch.bfloat16))
+
+
+def test_quant_linear_refuses_what_does_not_fit(cuda):
+    """Rows of another width are refused, also where their elements would make whole rows; empty inputs and any leading sizes are taken."""
+    from ajllm_amd import QuantLinear
+
+    layer = QuantLinear.from_weight(make_weight(48, 256, 5).to(cuda), "w4a16_g128")
+    for shape in ((2, 512), (4, 128), (2, 3, 512)):
+        with pytest.raises(RuntimeError):
+            layer(torch.zeros(shape, dtype=torch.bfloat16, device=cuda))
+    x = torch.randn(6, 256, device=cuda)
+    want = layer(x.bfloat16())
+    assert torch.equal(layer(x.bfloat16().view(2, 3, 256)), want.view(2, 3, 48)) and torch.equal(layer(x[0].bfloat16()), want[0])
+    assert torch.equal(layer(x).bfloat16(), want) and layer(x).dtype == torch.float32 and layer(x[:0]).shape == (0, 48)
+    assert torch.equal(layer(x.bfloat16().repeat(1, 2)[:, :256]), want)   # rows that are not contiguous
