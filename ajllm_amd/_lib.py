@@ -175,7 +175,7 @@ class DenseInArgs(ctypes.Structure):
 
     _fields_ = ([(n, c_void_p) for n in ("x", "n1", "n2", "gain1", "gain2", "w1", "w2", "y1", "gated")]
                 + [(n, c_int) for n in ("batch", "true_width", "width", "tiles1", "tiles2", "gated_ld", "act", "center", "pairs")]
-                + [("eps", c_float)])
+                + [("eps", c_float), ("sums", c_void_p), ("parts", c_int)])
 
 
 class KeyValueSplitArgs(ctypes.Structure):
@@ -225,6 +225,8 @@ DENSE_SIGNATURES: dict[str, tuple] = {
     "ajqd_latent_expand": (c_int, [_P, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _I, _P]),
     "ajqd_embed_streams": (c_int, [_P, _I, _P, _I, _P, _P, _P, _I, _I, _I, _P]),
     "ajqd_streams_norm": (c_int, [_P, _P, _P, _P, _P, _P, _P, _F, _P, _P, _I, _I, _I, _I, _I, _P]),
+    "ajqd_dense_out_streams_scaled": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
+    "ajqd_dense_out_parts": (c_int, [_I, _I]),
     "ajqd_dense_out_streams": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "ajqd_activation": (c_int, [_P, _P, _L, _I, _I, _P]),
     "ajqd_key_value_split": (c_int, [ctypes.POINTER(KeyValueSplitArgs), _I, _I, _P]),

@@ -319,12 +319,14 @@ int ajqd_dense_in(const ajqd_dense_in_args* a, void* stream) {
     return fail(AJQ_ERR_SHAPE, "ajqd_dense_in: unsupported shape (batch=%d width=%d/%d tiles=%d+%d)", a->batch, a->true_width,
                 a->width, a->tiles1, a->tiles2);
   if (a->act < 0 || a->act > AJQD_ACT_SQUARED_RELU) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_dense_in: unknown activation");
+  if (a->sums && (a->x || a->center || a->parts < 1)) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_dense_in: sums of squares go with scaled rows of an RMS norm");
   if (a->x && a->batch > 4) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_dense_in: the norm prologue takes at most 4 rows");
   DenseIn d;
   d.x = a->x; d.n1 = (const uint16_t*)a->n1; d.n2 = (const uint16_t*)a->n2; d.gain1 = a->gain1; d.gain2 = a->gain2;
   d.w1 = (const uint16_t*)a->w1; d.w2 = (const uint16_t*)a->w2; d.y1 = a->y1; d.gated = (uint16_t*)a->gated;
   d.batch = a->batch; d.D = a->true_width; d.Dp = a->width; d.tiles1 = a->tiles1; d.tiles2 = a->tiles2;
   d.gated_ld = a->gated_ld; d.act = a->act; d.center = a->center; d.pairs = a->pairs; d.eps = a->eps;
+  d.sums = a->sums; d.parts = a->parts;
   // more than 16 sequences: two batch tiles and (from two tiles of rows on) two row tiles per workgroup
   const bool wide = a->batch > kGemvBatch;
   const int block = wide ? 2 * kGemvBatch : kGemvBatch;
@@ -497,17 +499,16 @@ int ajqd_streams_norm(float* x, const float* delta, const float* scale, const fl
   return check_launch("ajqd_streams_norm");
 }
 
-int ajqd_dense_out_streams(const void* in, const void* w, float* x, const float* scale, const float* out, const float* mix,
-                           const float* next, float* u, int streams, int batch, int k, int width, void* stream) {
-  if (!in || !w || !x || !scale || !out || !mix || !u) return fail(AJQ_ERR_NULL, "ajqd_dense_out_streams: null pointer argument");
-  if (int e = check_streams(streams, "ajqd_dense_out_streams")) return e;
+static int dense_out_streams(const char* name, DenseOutStreams d, void* stream) {
+  const int batch = d.batch, k = d.K, width = d.Dp, streams = d.streams;
+  if (!d.in || !d.w || !d.x || !d.scale || !d.out || !d.mix) return fail(AJQ_ERR_NULL, "%s: null pointer argument", name);
+  if (int e = check_streams(streams, name)) return e;
   if (batch < 1 || k < 8 || k % 8 || width < 16 || width % 16)
-    return fail(AJQ_ERR_SHAPE, "ajqd_dense_out_streams: unsupported shape (batch=%d k=%d width=%d)", batch, k, width);
-  DenseOutStreams d{(const uint16_t*)in, (const uint16_t*)w, x, scale, out, mix, next, u, batch, k, width, streams};
+    return fail(AJQ_ERR_SHAPE, "%s: unsupported shape (batch=%d k=%d width=%d)", name, batch, k, width);
   const OutCut c = out_cut(batch, width);
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, c.grid, dim3(c.threads), 0, (hipStream_t)stream, d);
-    return check_launch("ajqd_dense_out_streams");
+    return check_launch(name);
   };
   auto pick = [&](auto room) {
     constexpr int M = decltype(room)::value;
@@ -520,6 +521,23 @@ int ajqd_dense_out_streams(const void* in, const void* w, float* x, const float*
     case 4: return pick(std::integral_constant<int, 4>{});
     default: return pick(std::integral_constant<int, kMaxStreams>{});
   }
+}
+
+int ajqd_dense_out_streams(const void* in, const void* w, float* x, const float* scale, const float* out, const float* mix,
+                           const float* next, float* u, int streams, int batch, int k, int width, void* stream) {
+  if (!u) return fail(AJQ_ERR_NULL, "ajqd_dense_out_streams: null pointer argument");
+  return dense_out_streams("ajqd_dense_out_streams", DenseOutStreams{(const uint16_t*)in, (const uint16_t*)w, x, scale, out, mix, next, u, nullptr,
+                                                                     nullptr, nullptr, batch, k, width, streams}, stream);
+}
+
+int ajqd_dense_out_parts(int batch, int width) { return batch < 1 || width < 16 || width % 16 ? 0 : width / out_cut(batch, width).rows; }
+
+int ajqd_dense_out_streams_scaled(const void* in, const void* w, float* x, const float* scale, const float* out, const float* mix,
+                                  const float* next, const float* gain, void* scaled, float* sums, int streams, int batch, int k, int width,
+                                  void* stream) {
+  if (!gain || !scaled || !sums) return fail(AJQ_ERR_NULL, "ajqd_dense_out_streams_scaled: null pointer argument");
+  return dense_out_streams("ajqd_dense_out_streams_scaled", DenseOutStreams{(const uint16_t*)in, (const uint16_t*)w, x, scale, out, mix, next, nullptr,
+                                                                            gain, (uint16_t*)scaled, sums, batch, k, width, streams}, stream);
 }
 
 int ajqd_activation(const void* y, void* out, int64_t count, int act, int dtype, void* stream) {

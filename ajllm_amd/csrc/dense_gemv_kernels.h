@@ -225,6 +225,8 @@ struct DenseIn {
   uint16_t* gated;          // [B, gated_ld], column 8 * tile + j (pairs) or 16 * tile + j
   int batch, D, Dp, tiles1, tiles2, gated_ld, act, center, pairs;
   float eps;
+  const float* sums;        // or null: n1 / n2 are rows times gain, not normed yet; [B, parts] holds their rows' sums of squares in parts,
+  int parts;                // and the norm's factor goes to the outputs
 };
 
 // kNorm: the norm is formed here, for the rows of one batch block (dynamic LDS: rows x (Dp + 8) bf16).
@@ -233,7 +235,7 @@ template <int kWaves, bool kNorm, int RT, int BT>
 __global__ __launch_bounds__(64 * kWaves) void dense_in_kernel(DenseIn a) {
   extern __shared__ __attribute__((aligned(16))) uint16_t normed[];
   __shared__ __attribute__((aligned(16))) unsigned char lds[stream_lds(kWaves, 16, RT, BT, 1)];
-  __shared__ float stat[kWaves];
+  __shared__ float stat[kNorm ? kWaves : kGemvBatch * BT];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int b0 = blockIdx.y * kGemvBatch * BT, nb = min(kGemvBatch * BT, a.batch - b0);
   const int groups1 = (a.tiles1 + RT - 1) / RT;
@@ -307,15 +309,28 @@ __global__ __launch_bounds__(64 * kWaves) void dense_in_kernel(DenseIn a) {
     });
   } else {
     const uint16_t* xr = (second ? a.n2 : a.n1) + (size_t)b0 * a.Dp + 8 * g;
-    stream_rows<kWaves, 16, RT, BT, 1>(wrow, a.Dp, wave, lane, lds, acc, [] {}, [&](int t, int s) {
+    // the rows' factors while the first weights travel: 16 lanes per row add its parts
+    auto factors = [&]() {
+      if (!a.sums) return;
+      for (int row = threadIdx.x >> 4; row < nb; row += 4 * kWaves) {
+        const float* part = a.sums + (size_t)(b0 + row) * a.parts;
+        float ss = 0.f;
+#pragma unroll 8
+        for (int i = r; i < a.parts; i += 16) ss += part[i];
+        ss = team_sum16(ss);
+        if (r == 0) stat[row] = 1.0f / sqrtf(ss / (float)a.D + a.eps);
+      }
+    };
+    stream_rows<kWaves, 16, RT, BT, 1>(wrow, a.Dp, wave, lane, lds, acc, factors, [&](int t, int s) {
       return *reinterpret_cast<const u32x4_t*>(xr + (size_t)min(16 * t + r, nb - 1) * a.Dp + 32 * s);
     });
   }
 #pragma unroll
   for (int i = 0; i < RT * BT; ++i) {
     if (wave != i) continue;
-    const f32x4_t& sum = acc[i / BT][i % BT];
+    f32x4_t sum = acc[i / BT][i % BT];
     const int row = 16 * (i % BT) + r, tile = tile0 + i / BT;
+    if (!kNorm && a.sums) sum *= stat[min(row, nb - 1)];
     if (!second) {
       if (row < nb) store4(a.y1 + (size_t)(b0 + row) * (16 * a.tiles1) + 16 * tile + 4 * g, float4{sum[0], sum[1], sum[2], sum[3]});
       continue;
@@ -385,7 +400,10 @@ struct DenseOutStreams {
   const float* out;         // [S]
   const float* mix;         // [S, S]
   const float* next;        // [S], weights of the next reader; null: the plain sum
-  float* u;                 // [B, Dp], what the next reader gets
+  float* u;                 // [B, Dp], what the next reader gets, or null and
+  const float* gain;        // [Dp] its norm's gain,
+  uint16_t* scaled;         // [B, Dp] bf16, what it gets times the gain,
+  float* sums;              // [B, Dp / ROWS] its sums of squares per tile
   int batch, K, Dp, streams;
 };
 template <int kWaves, int ROWS, int RT, int BT, int UQ, int MAXS>
@@ -416,7 +434,18 @@ __global__ __launch_bounds__(64 * kWaves) void dense_out_streams_kernel(DenseOut
 #pragma unroll
     for (int s = 0; s < MAXS; ++s)
       if (s < a.streams) store4(x + (size_t)s * a.Dp, v[s]);
-    store4(a.u + (size_t)(b0 + row) * a.Dp + column, read_streams<MAXS>(v, a.streams, a.next));
+    const float4 read = read_streams<MAXS>(v, a.streams, a.next);
+    if (a.u) {
+      store4(a.u + (size_t)(b0 + row) * a.Dp + column, read);
+      continue;
+    }
+    const float4 k = load4(a.gain + column);
+    store4(a.scaled + (size_t)(b0 + row) * a.Dp + column, float4{read.x * k.x, read.y * k.y, read.z * k.z, read.w * k.w});
+    // (the lanes of a row are 16 apart, and all of them here)
+    float ss = (read.x * read.x + read.y * read.y) + (read.z * read.z + read.w * read.w);
+    ss += __shfl_xor(ss, 16);
+    if (ROWS == 16) ss += __shfl_xor(ss, 32);
+    if (g == 0) a.sums[(size_t)(b0 + row) * (a.Dp / ROWS) + column / ROWS] = ss;
   }
 }
 

@@ -227,8 +227,10 @@ class DenseLM(nn.Module):
         _matvec(self._head, 1, normed, normed.shape[1], 0, y, y.shape[1], 0, rows)
         return y
 
-    def _dense_in(self, x, n1, n2, gain1, gain2, eps, center, w1, w2, y1, gated, gated_ld, act, pairs: bool = True) -> None:
-        """``y1 = norm1(x) w1^T`` and the activated ``norm2(x) w2^T`` of one decode step in one launch; either matrix may be None."""
+    def _dense_in(self, x, n1, n2, gain1, gain2, eps, center, w1, w2, y1, gated, gated_ld, act, pairs: bool = True,
+                  sums: torch.Tensor | None = None) -> None:
+        """``y1 = norm1(x) w1^T`` and the activated ``norm2(x) w2^T`` of one decode step in one launch; either matrix may be None.
+        With ``sums`` (their rows' sums of squares in parts) n1 / n2 are rows times gain, and the norm's factor goes to the outputs."""
         rows, w = next(t for t in (x, n1, n2) if t is not None), w1 if w1 is not None else w2
         batch = rows.shape[0]
         args = _lib.DenseInArgs(
@@ -236,5 +238,5 @@ class DenseLM(nn.Module):
             gated=gated, batch=batch, true_width=self.d_model, width=w.shape[1],
             tiles1=w1.shape[0] // 16 if w1 is not None else 0,
             tiles2=w2.shape[0] // 16 if w2 is not None else 0, gated_ld=gated_ld, act=act, center=center,
-            pairs=int(pairs), eps=eps)
+            pairs=int(pairs), eps=eps, sums=_ptr(sums), parts=sums.shape[1] if sums is not None else 0)
         _lib.check_dense(_lib.load_dense().ajqd_dense_in(ctypes.byref(args), _stream()), "dense_in")

@@ -439,29 +439,35 @@ class HybridLM(DenseLM):
         return self._recur(x, raw, low, y, w, cache.states[run], y.shape[0], 1, 0, cache.position)
 
     def _token_fused(self, token_ids: torch.Tensor, cache: RingCache) -> torch.Tensor:
-        """The bf16 step: a product in front of a sublayer (with the norm where that is free), what the sublayer is, a product
-        behind it that updates the streams and leaves the next sublayer's input."""
+        """The bf16 step: a product in front of a sublayer, what the sublayer is, a product behind it that updates the streams and
+        leaves the next sublayer's input times its norm's gain, with the sums of squares its norm needs (only the first sublayer's
+        norm is formed on its own)."""
         lib, st, dev = _lib.load_dense(), _stream(), self._embed.device
         batch, dp = token_ids.shape[0], self._embed.shape[1]
         order = self._sublayers()
         x, u = self._start(token_ids, order[0][2], True)
+        n, sums, parts = None, None, lib.ajqd_dense_out_parts(batch, dp)
+        if batch > NORM_PROLOGUE_ROWS:
+            n, u = _add_norms(u, None, None, None, order[0][2].gain, None, order[0][2].eps, 0, self.d_model, torch.bfloat16)[0], None
         for k, (run, w, sub) in enumerate(order):
             ff = isinstance(w, PackedFeedForward)
             y = torch.empty((batch, w.w_in.shape[0]), dtype=torch.bfloat16 if ff else torch.float32, device=dev)
-            rows, n = (u, None) if batch <= NORM_PROLOGUE_ROWS else (None, _add_norms(u, None, None, None, sub.gain, None, sub.eps, 0, self.d_model,
-                                                                                     torch.bfloat16)[0])
             if ff:
-                self._dense_in(rows, None, n, None, sub.gain, sub.eps, 0, None, w.w_in, None, _ptr(y), w.width, w.act, pairs=False)
+                self._dense_in(u, None, n, None, sub.gain, sub.eps, 0, None, w.w_in, None, _ptr(y), w.width, w.act, pairs=False, sums=sums)
                 mixed = y
             else:
-                self._dense_in(rows, n, None, sub.gain, None, sub.eps, 0, w.w_in, None, y, None, 0, 0)
+                self._dense_in(u, n, None, sub.gain, None, sub.eps, 0, w.w_in, None, y, None, 0, 0, sums=sums)
                 mixed = (self._attend_fused if isinstance(w, PackedAttention) else self._scan_fused)(y, w, cache, run)
-            following = order[k + 1][2].reads if k + 1 < len(order) else None
-            u = torch.empty_like(u)
-            _lib.check_dense(lib.ajqd_dense_out_streams(
-                _ptr(mixed), _ptr(w.w_out), _ptr(x), _ptr(sub.scale), _ptr(sub.writes), _ptr(sub.mix), _ptr(following), _ptr(u), self.streams,
-                batch, mixed.shape[1], dp, st), "dense_out_streams")
-        return u
+            args = (_ptr(mixed), _ptr(w.w_out), _ptr(x), _ptr(sub.scale), _ptr(sub.writes), _ptr(sub.mix))
+            if k + 1 == len(order):
+                u = torch.empty((batch, dp), dtype=torch.float32, device=dev)
+                _lib.check_dense(lib.ajqd_dense_out_streams(*args, None, _ptr(u), self.streams, batch, mixed.shape[1], dp, st), "dense_out_streams")
+                return u
+            following = order[k + 1][2]
+            u = None
+            n, sums = torch.empty((batch, dp), dtype=torch.bfloat16, device=dev), torch.empty((batch, parts), dtype=torch.float32, device=dev)
+            _lib.check_dense(lib.ajqd_dense_out_streams_scaled(*args, _ptr(following.reads), _ptr(following.gain), _ptr(n), _ptr(sums), self.streams,
+                                                               batch, mixed.shape[1], dp, st), "dense_out_streams_scaled")
 
     def _attend_fused(self, y: torch.Tensor, w: PackedAttention, cache: RingCache, run: int) -> torch.Tensor:
         lib, st, ring, batch = _lib.load_dense(), _stream(), cache.rings[run], y.shape[0]

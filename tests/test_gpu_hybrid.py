@@ -771,3 +771,32 @@ def test_streamed_products(cuda, batch, k, width):
         _ok(lib.ajqd_dense_in(ctypes.byref(_lib.DenseInArgs(x=_p(dr), gain1=_p(dg), **args)), _st()))
         normed = O.centered_rms_norm(rows, gain - 1, 1e-3).bfloat16()
         assert _rel(y, normed.double() @ w.double().T) < 1e-3   # (a norm rounded the other way moves an operand by 2^-8)
+
+
+@pytest.mark.parametrize("batch", [1, 5, 16, 17, 33])
+@pytest.mark.parametrize("width,streams", [(48, 1), (2048, 2), (2064, 3)])
+def test_norm_carried_to_the_outputs(cuda, batch, width, streams):
+    """dense_out_streams_scaled and the dense_in behind it against the norm as a launch of its own: the scaled rows are the rounding of
+    u gain, the sums are u's, and the two products agree as far as one rounding of an operand each (2^-9 a value, independent) lets them."""
+    g, k, n = torch.Generator().manual_seed(width + batch), 264, 96
+    a, w, w2 = _bf(g, batch, k), _bf(g, width, k, std=k ** -0.5), _bf(g, n, width, std=width ** -0.5)
+    x, scale, gain, hc, reads = torch.randn((batch, streams, width), generator=g), torch.randn(width, generator=g), torch.randn(width, generator=g), _coefficients(g, streams), torch.randn(streams, generator=g)
+    d = {m: v.to(cuda) for m, v in dict(a=a, w=w, w2=w2, x=x, scale=scale, gain=gain, reads=reads, **hc).items()}
+    lib = _lib.load_dense()
+    parts = lib.ajqd_dense_out_parts(batch, width)
+    args = (_p(d["a"]), _p(d["w"]), _p(d["x"]), _p(d["scale"]), _p(d["out"]), _p(d["mix"]), _p(d["reads"]))
+    u, y = torch.empty((batch, width), device=cuda), torch.empty((2, batch, n), device=cuda)
+    scaled, sums = torch.empty((batch, width), dtype=torch.bfloat16, device=cuda), torch.empty((batch, parts), device=cuda)
+    _ok(lib.ajqd_dense_out_streams(*args, _p(u), streams, batch, k, width, _st()))
+    after = d["x"].clone()
+    d["x"].copy_(x)
+    _ok(lib.ajqd_dense_out_streams_scaled(*args, _p(d["gain"]), _p(scaled), _p(sums), streams, batch, k, width, _st()))
+    assert torch.equal(after, d["x"]) and torch.equal(scaled, (u * d["gain"]).bfloat16())
+    assert _rel(sums.sum(1), u.double().square().sum(1)) < 1e-6
+    normed = dense._add_norms(u, None, None, None, d["gain"], None, 1e-3, 0, width, torch.bfloat16)[0]
+    for i, more in enumerate((dict(n1=_p(normed)), dict(n1=_p(scaled), sums=_p(sums), parts=parts))):
+        _ok(lib.ajqd_dense_in(ctypes.byref(_lib.DenseInArgs(w1=_p(d["w2"]), y1=y[i].data_ptr(), batch=batch, true_width=width, width=width, tiles1=n // 16,
+                                                            eps=1e-3, **more)), _st()))
+    assert _rel(y[1], y[0]) < 6e-3
+    assert lib.ajqd_dense_in(ctypes.byref(_lib.DenseInArgs(w1=_p(d["w2"]), y1=_p(y), batch=batch, true_width=width, width=width, tiles1=n // 16, n1=_p(scaled),
+                                                           sums=_p(sums), parts=parts, center=1, eps=1e-3)), _st()) < 0
