@@ -124,4 +124,26 @@ __device__ __forceinline__ float team_sum16(float v) {
   return v;
 }
 
+// max / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 (a lane quarter's place in the wave):
+// v_permlane16_swap and v_permlane32_swap hand every lane its partner's value in one VALU
+// instruction each, without a trip through the LDS crossbar.
+__device__ __forceinline__ float quad_max(float x) {
+  typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+  uint32_t b = __float_as_uint(x);
+  u32x2v s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  x = fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
+  b = __float_as_uint(x);
+  s = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
+}
+__device__ __forceinline__ float quad_sum(float x) {
+  typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+  uint32_t b = __float_as_uint(x);
+  u32x2v s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  x = __uint_as_float(s.x) + __uint_as_float(s.y);
+  b = __float_as_uint(x);
+  s = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return __uint_as_float(s.x) + __uint_as_float(s.y);
+}
+
 }  // namespace ajq

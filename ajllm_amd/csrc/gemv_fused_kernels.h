@@ -17,6 +17,9 @@
 // row's sum of squares: every wave reduces its slice per row, the eight partial sums meet in
 // LDS behind one barrier (the weight loads are in flight meanwhile).  Workgroup 0 writes the
 // updated residual stream, to a buffer other than the one being read.
+// What bounds these launches is the chain of round trips to memory, so no load may wait for another's value: the activations'
+// way into LDS has no branch and no select that would draw a load into itself (kProNormSums used to fetch h and the gain only
+// after the row sums had arrived: a 12-layer int4 step of width 2048 at batch 1 took 0.326 ms with that, 0.313 without).
 #pragma once
 #include "gemv_kernels.h"
 #include "decode_kernels.h"
@@ -140,8 +143,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
     for (int u = 0; u < kPartLoads; ++u) {
       const int j = piece + u * kLanesPerRow;
       const bool live = 4 * j < S && row < M;  // (idle lanes re-read the first 16 bytes)
-      const float4 t = *reinterpret_cast<const float4*>(src1 + (live ? (size_t)row * S + 4 * j : 0));
-      sums[u] = live ? t : float4{0.f, 0.f, 0.f, 0.f};
+      sums[u] = *reinterpret_cast<const float4*>(src1 + (live ? (size_t)row * S + 4 * j : 0));
     }
   }
   if (kW4) {  // before the weights: scales and zero-points are there when the first tile lands
@@ -160,7 +162,9 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   constexpr bool kResid = kOut == kOutResid;
   constexpr int kLiveRows = MROWS < 4 ? MROWS : 4;
   float h_old[kLiveRows], gain_n = 0.f;
-  if (kResid) {  // behind the weights in issue order, used at the very end
+  uint32_t scale_bits = 0;  // (what is used at the very end goes behind the weights in issue order)
+  if (!kW4) scale_bits = scales8[nt * kTileN + nl];
+  if (kResid) {
     gain_n = gain[nt * kTileN + nl];
 #pragma unroll
     for (int i = 0; i < kLiveRows; ++i) h_old[i] = res_h_in[(size_t)min(4 * kc + i, M - 1) * N + nt * kTileN + nl];
@@ -208,11 +212,16 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
     // a row's total in its first lane, then through the wave's own LDS words to whoever holds a piece of the row
     float total = 0.f;
 #pragma unroll
-    for (int u = 0; u < kPartLoads; ++u) total += (sums[u].x + sums[u].y) + (sums[u].z + sums[u].w);
+    for (int u = 0; u < kPartLoads; ++u) {
+      // (the idle lanes' words are dropped here and not at the load, which would become a branch of its own)
+      asm volatile("" : "+v"(sums[u].x), "+v"(sums[u].y), "+v"(sums[u].z), "+v"(sums[u].w));
+      const bool live = 4 * (lane % kLanesPerRow + u * kLanesPerRow) < S && lane / kLanesPerRow < M;
+      total += live ? (sums[u].x + sums[u].y) + (sums[u].z + sums[u].w) : 0.f;
+    }
     if (kLanesPerRow >= 16) {
-      total = team_sum16(total);  // DPP row rotates inside each 16 lanes, then the crossbar for whole rows of 16
-#pragma unroll
-      for (int off = 16; off < kLanesPerRow; off <<= 1) total += __shfl_xor(total, off);
+      total = team_sum16(total);  // DPP row rotates inside each 16 lanes, then lane swaps for whole rows of 16
+      if (kLanesPerRow == 64) total = quad_sum(total);
+      else if (kLanesPerRow == 32) total += __shfl_xor(total, 16);
     } else {
 #pragma unroll
       for (int off = kLanesPerRow / 2; off > 0; off >>= 1) total += __shfl_xor(total, off);
@@ -222,7 +231,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
     for (int i = 0; i < kXLoads; ++i) {
       const int v = min(lane + 64 * i, kVecs - 1);
       // one row: every lane already holds its total
-      const Divisor by_rms(sqrtf((MROWS > 1 ? ssq[(v / kVecPerRow) * kWaves + wave] : total) / (float)K + eps));
+      const Divisor by_rms(sqrtf((MROWS > 1 ? ssq[(v / kVecPerRow) * kWaves + wave] : total) / (float)(kWaves * kSlice) + eps));  // (K, so a product where it is a power of two)
       const float4 h0 = a0[i][0], h1 = a0[i][1], g0v = a2[i][0], g1v = a2[i][1];
       xv[i][0] = by_rms.divide(h0.x) * g0v.x; xv[i][1] = by_rms.divide(h0.y) * g0v.y;
       xv[i][2] = by_rms.divide(h0.z) * g0v.z; xv[i][3] = by_rms.divide(h0.w) * g0v.w;
@@ -249,8 +258,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
 #pragma unroll
       for (int j = 0; j < kCpl; ++j)
         if (sgrp + 4 * j < S) mloc = fmaxf(mloc, pm[q][j].x);
-      float mall = fmaxf(mloc, __shfl_xor(mloc, 16));
-      mall = fmaxf(mall, __shfl_xor(mall, 32));
+      const float mall = quad_max(mloc);
       float L = 0.f, A[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < kCpl; ++j) {
@@ -261,13 +269,9 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
           A[4] += pa[q][j][1].x * cw; A[5] += pa[q][j][1].y * cw; A[6] += pa[q][j][1].z * cw; A[7] += pa[q][j][1].w * cw;
         }
       }
-      L += __shfl_xor(L, 16);
-      L += __shfl_xor(L, 32);
+      L = quad_sum(L);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        A[e] += __shfl_xor(A[e], 16);
-        A[e] += __shfl_xor(A[e], 32);
-      }
+      for (int e = 0; e < 8; ++e) A[e] = quad_sum(A[e]);
       if (sgrp == 0) {
         u32x4_t pk;
         pk.x = pack2_bf16(A[0] / L, A[1] / L);
@@ -278,17 +282,17 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
       }
     }
   }
-  // bf16, into the wave's own LDS rows
+  // bf16, into the wave's own LDS rows.  Lanes past the slice write its last vector once more (the same value): a branch here
+  // would draw the loads of h and gain into itself, behind the wait for the row sums.
 #pragma unroll
   for (int i = 0; i < (kPro == kProMerge ? 0 : kXLoads); ++i) {
-    const int v = lane + 64 * i;
+    const int v = min(lane + 64 * i, kVecs - 1);
     u32x4_t pk;
     pk.x = pack2_bf16(xv[i][0], xv[i][1]);
     pk.y = pack2_bf16(xv[i][2], xv[i][3]);
     pk.z = pack2_bf16(xv[i][4], xv[i][5]);
     pk.w = pack2_bf16(xv[i][6], xv[i][7]);
-    if ((i + 1) * 64 <= kVecs || v < kVecs)
-      *reinterpret_cast<u32x4_t*>(xs + (v / kVecPerRow) * kStride + 8 * (v % kVecPerRow)) = pk;
+    *reinterpret_cast<u32x4_t*>(xs + (v / kVecPerRow) * kStride + 8 * (v % kVecPerRow)) = pk;
   }
 
   // ---- the matmul, as in dequant_gemv_kernel.  What depends on the activations alone comes first, while the
@@ -347,6 +351,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
 
   // ---- the waves' partial sums meet in LDS; wave 0 adds them in wave order
   asm volatile("" : "+v"(acc));
+  if (!kW4) asm volatile("" : "+v"(scale_bits));
   constexpr int kLive = MROWS < 4 ? MROWS : 4;
   typedef float live_t __attribute__((ext_vector_type(kLive == 3 ? 4 : kLive)));
   live_t* redv = reinterpret_cast<live_t*>(red);
@@ -364,7 +369,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   for (int u = 1; u < kWaves; ++u) sum += part[u];
   const int n = nt * kTileN + nl;
   float cs = 1.0f;
-  if (!kW4) cs = f16_bits_to_f32(scales8[n]);
+  if (!kW4) cs = f16_bits_to_f32(scale_bits);
   if (kResid) {
     const int ntiles = N / kTileN;
 #pragma unroll

@@ -169,13 +169,14 @@ __device__ __forceinline__ void dequant_gemv_body(
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 
   // slice of a batch -> wave-private LDS.  LDS operations of one wave execute in order, so the reads of the
-  // previous batch are already done.
+  // previous batch are already done.  Lanes past the slice write its last vector once more (the same value to the same
+  // place): a branch here would draw the load of the slice into itself, behind the weights in issue order, and all that
+  // is formed from the activations would wait for the weights.
   auto stage = [&](const Batch& b) {
 #pragma unroll
     for (int i = 0; i < kXLoads; ++i) {
-      const int v = lane + 64 * i;
-      if ((i + 1) * 64 <= kVecs || v < kVecs)
-        *reinterpret_cast<u32x4_t*>(xs + (v / kVecPerRow) * kStride + 8 * (v % kVecPerRow)) = b.x[i];
+      const int v = min(lane + 64 * i, kVecs - 1);
+      *reinterpret_cast<u32x4_t*>(xs + (v / kVecPerRow) * kStride + 8 * (v % kVecPerRow)) = b.x[i];
     }
   };
   // kSingle: formed from the activations alone, before the weights have landed (see the kSingle branch below)
@@ -250,14 +251,16 @@ __device__ __forceinline__ void dequant_gemv_body(
   };
 
   // two register sets, ping-pong: the next batch is in flight while one is computed
-  // ---- what the epilogue variants need from memory is requested behind the first batch of weights
+  // ---- what the end of the kernel (the W8 scales, the epilogue variants) needs from memory is requested behind the first batch of weights
   // (vector loads return in issue order: in front of them it would delay the HBM requests) and used at
   // the end
   constexpr int kLiveRows = MROWS < 4 ? MROWS : 4;
   float* red2 = red + kWaves * 64 * 4;  // [16][kWaves] shares of the rows' sums of squares
   float4 ssq_share[2];
   float h_old[kLiveRows], gain_n = 0.f;
+  uint32_t scale_bits = 0;
   auto epilogue_loads = [&]() {
+    if (!kW4) scale_bits = scales8[nt * kTileN + nl];
     if (kEpi & kEpiRowScale) {
       const int m = lane & 15, c = lane >> 4;
 #pragma unroll
@@ -311,6 +314,7 @@ __device__ __forceinline__ void dequant_gemv_body(
   // (the empty asm pins the accumulator here: otherwise the compiler sinks the
   // epilogue arithmetic, and the loads that feed it, into the conditional store)
   asm volatile("" : "+v"(acc));
+  if (!kW4) asm volatile("" : "+v"(scale_bits));  // (and its load would follow it, a round trip to memory behind the barrier)
   constexpr int kLive = MROWS < 4 ? MROWS : 4;  // accumulator components that hold rows < MROWS
   typedef float live_t __attribute__((ext_vector_type(kLive == 3 ? 4 : kLive)));
   live_t* redv = reinterpret_cast<live_t*>(red);
@@ -322,8 +326,7 @@ __device__ __forceinline__ void dequant_gemv_body(
     // this wave's share of the rows' sums of squares: lane (row m = lane & 15, quarter c) holds 8 parts
     float sh = ((ssq_share[0].x + ssq_share[0].y) + (ssq_share[0].z + ssq_share[0].w)) +
                ((ssq_share[1].x + ssq_share[1].y) + (ssq_share[1].z + ssq_share[1].w));
-    sh += __shfl_xor(sh, 16);
-    sh += __shfl_xor(sh, 32);
+    sh = quad_sum(sh);
     if (kc == 0) red2[nl * kWaves + wave] = sh;
   }
   __syncthreads();
@@ -336,7 +339,7 @@ __device__ __forceinline__ void dequant_gemv_body(
   for (int w = 1; w < kWaves; ++w) sum += part[w];
   const int n = nt * kTileN + nl;
   float cs = 1.0f;
-  if (!kW4) cs = f16_bits_to_f32(scales8[n]);  // per-output-channel scale, once
+  if (!kW4) cs = f16_bits_to_f32(scale_bits);  // per-output-channel scale, once
   float rstd[kLive];
 #pragma unroll
   for (int i = 0; i < kLive; ++i) {

@@ -61,28 +61,6 @@ __device__ __forceinline__ u32x4_t to_bf16x8(const Raw8F32& r) {
 }
 __device__ __forceinline__ u32x4_t to_bf16x8(const u32x4_t& r) { return r; }
 
-// max / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 (the lanes that share a query row):
-// v_permlane16_swap and v_permlane32_swap hand every lane its partner's value in one VALU
-// instruction each, without a trip through the LDS crossbar.
-__device__ __forceinline__ float quad_max(float x) {
-  typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
-  uint32_t b = __float_as_uint(x);
-  u32x2v s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-  x = fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
-  b = __float_as_uint(x);
-  s = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-  return fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
-}
-__device__ __forceinline__ float quad_sum(float x) {
-  typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
-  uint32_t b = __float_as_uint(x);
-  u32x2v s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-  x = __uint_as_float(s.x) + __uint_as_float(s.y);
-  b = __float_as_uint(x);
-  s = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-  return __uint_as_float(s.x) + __uint_as_float(s.y);
-}
-
 typedef short pf_i16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) pf_i16x4_t pf_lds_i16x4_t;
 typedef __attribute__((address_space(3))) const u32x4_t pf_lds_u32x4_t;
