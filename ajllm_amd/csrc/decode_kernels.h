@@ -192,35 +192,37 @@ __device__ __forceinline__ void widen2(uint32_t w, float& lo, float& hi) {  // t
   lo = __uint_as_float(w << 16);
   hi = __uint_as_float(w & 0xFFFF0000u);
 }
-// p: the lane's first dimension of the row
-template <bool kStream, int HD>
-__device__ __forceinline__ KvRow<HD / 16> load_row(const float* p) {
-  using LD = LaneDims<float, HD>;
-  KvRow<HD / 16> r;
-  if constexpr (LD::DPL == 2) {
-    const u32x2_t a = load_kv<kStream>(reinterpret_cast<const u32x2_t*>(p));
-    r.v[0] = __uint_as_float(a.x); r.v[1] = __uint_as_float(a.y);
-  } else {
-    const u32x4_t a = load_kv<kStream>(reinterpret_cast<const u32x4_t*>(p));
-    r.v[0] = __uint_as_float(a.x); r.v[1] = __uint_as_float(a.y); r.v[2] = __uint_as_float(a.z); r.v[3] = __uint_as_float(a.w);
-    if constexpr (LD::DPL == 8) {
-      const u32x4_t b = load_kv<kStream>(reinterpret_cast<const u32x4_t*>(p + LD::second));
-      r.v[4] = __uint_as_float(b.x); r.v[5] = __uint_as_float(b.y); r.v[6] = __uint_as_float(b.z); r.v[7] = __uint_as_float(b.w);
+// A row of the cache as loaded (the lane's dimensions; p: the first of them) and widened to fp32 when it is used, so that a row
+// on its way from memory costs no more registers than its bytes.
+template <typename CacheT, int HD> struct RawRow {
+  static constexpr int words = (HD / 16) * (int)sizeof(CacheT) / 4;  // 8, 4, 2 (fp32) or 4, 2, 1 (bf16)
+  uint32_t w[words];
+};
+template <bool kStream, int HD, typename CacheT>
+__device__ __forceinline__ RawRow<CacheT, HD> load_raw(const CacheT* p) {
+  constexpr int words = RawRow<CacheT, HD>::words;
+  RawRow<CacheT, HD> r;
+  if constexpr (words >= 4) {
+#pragma unroll
+    for (int h = 0; h < words / 4; ++h) {
+      const u32x4_t a = load_kv<kStream>(reinterpret_cast<const u32x4_t*>(p + h * LaneDims<CacheT, HD>::second));
+      r.w[4 * h] = a.x; r.w[4 * h + 1] = a.y; r.w[4 * h + 2] = a.z; r.w[4 * h + 3] = a.w;
     }
+  } else if constexpr (words == 2) {
+    const u32x2_t a = load_kv<kStream>(reinterpret_cast<const u32x2_t*>(p));
+    r.w[0] = a.x; r.w[1] = a.y;
+  } else {
+    r.w[0] = load_kv<kStream>(reinterpret_cast<const uint32_t*>(p));
   }
   return r;
 }
-template <bool kStream, int HD>
-__device__ __forceinline__ KvRow<HD / 16> load_row(const uint16_t* p) {
+template <typename CacheT, int HD>
+__device__ __forceinline__ KvRow<HD / 16> widen_row(const RawRow<CacheT, HD>& raw) {
   KvRow<HD / 16> r;
-  if constexpr (HD / 16 == 8) {
-    const u32x4_t v = load_kv<kStream>(reinterpret_cast<const u32x4_t*>(p));
-    widen2(v.x, r.v[0], r.v[1]); widen2(v.y, r.v[2], r.v[3]); widen2(v.z, r.v[4], r.v[5]); widen2(v.w, r.v[6], r.v[7]);
-  } else if constexpr (HD / 16 == 4) {
-    const u32x2_t v = load_kv<kStream>(reinterpret_cast<const u32x2_t*>(p));
-    widen2(v.x, r.v[0], r.v[1]); widen2(v.y, r.v[2], r.v[3]);
-  } else {
-    widen2(load_kv<kStream>(reinterpret_cast<const uint32_t*>(p)), r.v[0], r.v[1]);
+#pragma unroll
+  for (int i = 0; i < RawRow<CacheT, HD>::words; ++i) {
+    if constexpr (sizeof(CacheT) == 4) r.v[i] = __uint_as_float(raw.w[i]);
+    else widen2(raw.w[i], r.v[2 * i], r.v[2 * i + 1]);
   }
   return r;
 }
@@ -290,7 +292,9 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_kernel(const float* _
   const int rows = (int)p + 1;
   const int per = (rows + S - 1) / S;
   const int t_begin = s * per;
-  int t_end = min(rows, t_begin + per);
+  const int t_end = min(rows, t_begin + per);
+  // the step's own row: the chunk that owns it rotates the key, stores both and attends from registers (team 0)
+  const bool own = kStream ? (((int)p / (2 * kTeams)) % S) == s : (t_begin <= (int)p && (int)p < t_end);
   const int d0 = LD::per_lane * c;      // the lane's first dimension
   // kStep: cosines / sines of the lane's DPL / 2 pairs (interleaved pairs never straddle a lane's four)
   float cs[DPL / 2], sn[DPL / 2];
@@ -334,12 +338,43 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_kernel(const float* _
   };
   Row qr[R];
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    qr[r] = load_act(kStep ? qkv_row + (size_t)(hk * R + r) * hd : q + (size_t)(bh0 + r) * hd + d0);
-    if (kStep) rotate(qr[r]);
+  for (int r = 0; r < R; ++r) qr[r] = load_act(kStep ? qkv_row + (size_t)(hk * R + r) * hd : q + (size_t)(bh0 + r) * hd + d0);
+  Row kn{}, vn{};  // (fetched by every chunk, see below)
+  if (kStep) {
+    kn = load_act(qkv_row + (size_t)(H + hk) * hd);
+    vn = load_act(qkv_row + (size_t)(H + Hkv + hk) * hd);
   }
+  // rows first .. limit-1 in steps of `stride`, two rows per team at work and the next two on their way.  The first two are
+  // requested right behind the queries: every row of the launch waits for *pos, none for another row's arithmetic.
+  // (Past the end: a row that is there, fetched for nothing.)
+  // What bounds a decode step's launch is this chain of round trips: 12 layers of 16 heads on fp32 rows at batch 1 take 282 us a
+  // step where requesting rows pair by pair, each pair behind the one before, took 289 (context 577; at 2048 328 and 340).
   const CacheT* kbase = kcache + (size_t)bk * max_len * hd + d0;
   const CacheT* vbase = vcache + (size_t)bk * max_len * hd + d0;
+  const int first = kStream ? 2 * kTeams * s + team : t_begin + team;
+  const int limit = kStream ? ((kStep && own) ? (int)p : rows) : ((kStep && own) ? (int)p : t_end);
+  const int stride = kStream ? 2 * kTeams * S : 2 * kTeams;
+  RawRow<CacheT, HD> kr[2], vr[2];
+  auto request = [&](int t) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const size_t at = (size_t)max(min(t + u * kTeams, limit - 1), 0) * hd;
+      kr[u] = load_raw<kStream, HD>(kbase + at);
+      vr[u] = load_raw<kStream, HD>(vbase + at);
+    }
+  };
+  // (four heads on fp32 rows fill the 128 registers of a 16-wave workgroup's lanes: no rows ahead there)
+  constexpr bool kAhead = !(kWaves == 16 && R == 4 && RawRow<CacheT, HD>::words == 8);
+  __builtin_amdgcn_sched_barrier(0);
+  if (kAhead) request(first);
+  __builtin_amdgcn_sched_barrier(0);
+  if (kStep) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) rotate(qr[r]);
+    // the step's own row is here by now as well; without this the compiler fetches it in the owner's branch, a round trip of its own
+#pragma unroll
+    for (int i = 0; i < DPL; ++i) asm volatile("" : "+v"(kn.v[i]), "+v"(vn.v[i]));
+  }
   const float scale2 = scale * kLog2e;  // maxima and the partial results' maxima are base-2 exponents
   float m[R], l[R], acc[R][DPL];
 #pragma unroll
@@ -397,33 +432,19 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_kernel(const float* _
       for (int i = 0; i < DPL; ++i) acc[r][i] += w * v.v[i];
     }
   };
-  // the step's own row: the chunk that owns it rotates the key, stores both and attends from registers (team 0)
-  const bool own = kStream ? (((int)p / (2 * kTeams)) % S) == s : (t_begin <= (int)p && (int)p < t_end);
-  if (kStep && own) {
-    t_end = (int)p;
-    if (team == 0) {
-      Row kn = load_act(qkv_row + (size_t)(H + hk) * hd);
-      Row vn = load_act(qkv_row + (size_t)(H + Hkv + hk) * hd);
-      rotate(kn);
-      store_row<HD>(kcache + ((size_t)bk * max_len + p) * hd + d0, kn);
-      store_row<HD>(vcache + ((size_t)bk * max_len + p) * hd + d0, vn);
-      row(kn, vn);
-    }
+  if (kStep && own && team == 0) {
+    rotate(kn);
+    store_row<HD>(kcache + ((size_t)bk * max_len + p) * hd + d0, kn);
+    store_row<HD>(vcache + ((size_t)bk * max_len + p) * hd + d0, vn);
+    row(kn, vn);
   }
-  // rows first .. limit-1 in steps of `stride`, two rows per team in flight
-  const int first = kStream ? 2 * kTeams * s + team : t_begin + team;
-  const int limit = kStream ? ((kStep && own) ? (int)p : rows) : t_end;
-  const int stride = kStream ? 2 * kTeams * S : 2 * kTeams;
   for (int t = first; t < limit; t += stride) {
-    if (t + kTeams < limit) {
-      const Row k0 = load_row<kStream, HD>(kbase + (size_t)t * hd), k1 = load_row<kStream, HD>(kbase + (size_t)(t + kTeams) * hd);
-      const Row v0 = load_row<kStream, HD>(vbase + (size_t)t * hd), v1 = load_row<kStream, HD>(vbase + (size_t)(t + kTeams) * hd);
-      row(k0, v0);
-      row(k1, v1);
-    } else {
-      const Row k0 = load_row<kStream, HD>(kbase + (size_t)t * hd), v0 = load_row<kStream, HD>(vbase + (size_t)t * hd);
-      row(k0, v0);
-    }
+    if (!kAhead) request(t);
+    const Row k0 = widen_row<CacheT, HD>(kr[0]), v0 = widen_row<CacheT, HD>(vr[0]);
+    const Row k1 = widen_row<CacheT, HD>(kr[1]), v1 = widen_row<CacheT, HD>(vr[1]);
+    if (kAhead && t + stride < limit) request(t + stride);
+    row(k0, v0);
+    if (t + kTeams < limit) row(k1, v1);
   }
   // Sixteen partial results meet in LDS: the 16 teams of a 4-wave workgroup, or the 16 waves of the large one,
   // whose four teams are first merged inside the wave (lanes 16 and 32 apart hold the same dimensions).
@@ -499,15 +520,18 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(const float* __restrict_
 #pragma unroll
   for (int s = 0; s < 16; ++s)
     a[s] = *reinterpret_cast<const float2*>(src + min(s, S - 1) * stride + 4 + 2 * dl);
-  float M = ml.x;
-#pragma unroll
-  for (int off = 8; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off));
+  float M = ml.x;  // (the four quarters of the wave hold the same 16 values)
+  M = fmaxf(M, row_ror<8>(M));
+  M = fmaxf(M, row_ror<4>(M));
+  M = fmaxf(M, row_ror<2>(M));
+  M = fmaxf(M, row_ror<1>(M));
   const float mine = ml.x == -INFINITY ? 0.f : exp2_hw(ml.x - M);  // weight of chunk lane % 16 (base-2 maxima)
   float L = 0.f;
   float2 A = float2{0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < 16; ++s) {
-    const float c = __shfl(mine, s), l = __shfl(ml.y, s);
+    const float c = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), s));
+    const float l = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ml.y), s));
     if (s < S) {
       L += l * c;
       A.x += a[s].x * c;
