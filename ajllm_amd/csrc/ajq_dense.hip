@@ -392,7 +392,7 @@ int ajqd_latent_absorb(const float* y, int ldy, const ajqd_latent_shape* shape, 
   const int groups = (shape->rankp / 16 + 3) / 4;
   LatentAbsorb d{y, (const uint16_t*)ukt, latent_gain, cosine, sine, positions64(pos), (uint16_t*)q, (uint16_t*)ring,
                  batch, ldy, table_rows, cap, groups, device_shape(shape)};
-  hipLaunchKernelGGL(latent_absorb_kernel, dim3(shape->heads * groups + 4, (batch + kGemvBatch - 1) / kGemvBatch), dim3(256), 0,
+  hipLaunchKernelGGL(latent_absorb_kernel, dim3(shape->heads * groups + 4 + shape->heads, (batch + kGemvBatch - 1) / kGemvBatch), dim3(256), 0,
                      (hipStream_t)stream, d);
   return check_launch("ajqd_latent_absorb");
 }
@@ -422,9 +422,13 @@ int ajqd_latent_decode(const void* q, const void* ring, const int64_t* pos, floa
     return fail(AJQ_ERR_SHAPE, "ajqd_latent_decode: unsupported shape (batch=%d chunks=%d)", batch, chunks);
   LatentDecode d{(const uint16_t*)q, (const uint16_t*)ring, positions64(pos), partial,
                  heads_at(partial, batch, heads, chunks, rankp), batch, heads, rankp, rankp + rotp, cap, chunks, first_column / 32, scale * kLog2eF};
-  const long long blocks = (long long)latent_head_groups(heads) * chunks * batch;
+  // Two head tiles share a workgroup and its rows where there is more than one workgroup per CU; below that one each, on twice
+  // the CUs: 32 heads, rows of 576, a chunk per 64 of 560 rows, 1 / 8 / 16 sequences (two tiles make 10 / 80 / 160 workgroups):
+  // 8.8 / 9.8 / 10.6 us with two, 6.1 / 7.3 / 13.0 with one.
+  const long long singles = (long long)((heads + 15) / 16) * chunks * batch;
+  const bool two = heads > 16 && singles > kDecodeWorkgroups;
+  const long long blocks = two ? (long long)((heads + 31) / 32) * chunks * batch : singles;
   if (blocks > 0x7FFFFFFFll) return fail(AJQ_ERR_SHAPE, "ajqd_latent_decode: too many workgroups");
-  const bool two = heads > 16;
   auto go = [&](auto kernel, int ks) {
     const int bytes = latent_decode_lds(ks, two ? 2 : 1);
     if (int e = allow_lds(kernel, bytes, "ajqd_latent_decode")) return e;
@@ -452,12 +456,22 @@ int ajqd_latent_expand(const float* partial, const float* sink, const float* gat
     return fail(AJQ_ERR_SHAPE, "ajqd_latent_expand: unsupported shape (batch=%d heads=%d chunks=%d rankp=%d vdimp=%d)", batch,
                 heads, chunks, rankp, vdimp);
   if (rankp > kExpandRank) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_latent_expand: latents of %d are not built", rankp);
-  const bool few = batch <= kExpandBatch;
-  const int tw = few ? 2 : 8, groups = (vdimp / 16 + tw - 1) / tw, bytes = 2 * kExpandBatch * (rankp + 8);
-  LatentExpand d{partial, heads_at(partial, batch, heads, chunks, rankp), sink, gate, (const uint16_t*)uv, (uint16_t*)out, batch, heads, chunks, rankp, vdimp, gate_ld, out_ld, groups};
-  hipLaunchKernelGGL(few ? latent_expand_kernel<2> : latent_expand_kernel<8>, dim3(heads * groups, (batch + kExpandBatch - 1) / kExpandBatch), dim3(512), bytes,
-                     (hipStream_t)stream, d);
-  return check_launch("ajqd_latent_expand");
+  // A workgroup reads a part of a head's weights and the chunks' sums of a few sequences, at what one CU takes in: the cut that
+  // makes both small and still leaves no more than one workgroup per CU.  (512 x 128 weights, 10 chunks: 16 heads, 8 sequences: 5.6 us
+  // with 2 tiles x 2 sequences, 7.9 with 8 x 4; 32 heads, 8 sequences: 7.5 with 8 x 1, 8.1 with 8 x 4, 11.5 with 2 x 2, and with
+  // 32 chunks 8.8 with 8 x 1, 13.8 with 8 x 4; 16 sequences: 7.9 with 8 x 2, 8.4 with 8 x 4, 13.7 with 8 x 1.)
+  auto go = [&](auto kernel, int tw, int eb) {
+    const int groups = (vdimp / 16 + tw - 1) / tw, bytes = 2 * eb * (rankp + 8);
+    LatentExpand d{partial, heads_at(partial, batch, heads, chunks, rankp), sink, gate, (const uint16_t*)uv, (uint16_t*)out, batch, heads, chunks, rankp, vdimp, gate_ld, out_ld, groups};
+    hipLaunchKernelGGL(kernel, dim3(heads * groups, (batch + eb - 1) / eb), dim3(512), bytes, (hipStream_t)stream, d);
+    return check_launch("ajqd_latent_expand");
+  };
+  auto fits = [&](int tw, int eb) { return (long long)heads * ((vdimp / 16 + tw - 1) / tw) * ((batch + eb - 1) / eb) <= kDecodeWorkgroups; };
+  if (fits(2, 2)) return go(latent_expand_kernel<2, 2>, 2, 2);
+  if (batch <= 4) return go(latent_expand_kernel<2, 4>, 2, 4);
+  if (fits(8, 1)) return go(latent_expand_kernel<8, 1>, 8, 1);
+  if (fits(8, 2)) return go(latent_expand_kernel<8, 2>, 8, 2);
+  return go(latent_expand_kernel<8, 4>, 8, 4);
 }
 
 // ---- several residual streams

@@ -461,7 +461,10 @@ struct LatentAbsorb {
   int batch, ldy, table_rows, cap, groups;  // groups: workgroups per head (4 tiles of 16 latent columns each)
   LatentShape s;
 };
-// Grid (H * groups + 4, batch blocks); the last four workgroups of a batch block make the cache rows, a wave each.
+// Grid (H * groups + 4 + H, batch blocks).  Behind the products' workgroups four make the cache rows, a wave each, and one per head
+// rotates the rotated part of its queries: those hang on the position and then on its angles, two round trips more than a
+// product takes.  A cache row's operands are requested at once (8 sequences, 32 heads, 512 + 64 columns: 4.9 us a launch, 5.5 with the
+// rotations ahead of the first product of a head and a wait per 256 columns of a row).
 __global__ __launch_bounds__(256) void latent_absorb_kernel(LatentAbsorb a) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
   const int b0 = blockIdx.y * kGemvBatch, nb = min(kGemvBatch, a.batch - b0);
@@ -470,46 +473,74 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(LatentAbsorb a) {
   const int p = clamped_position(a.pos, 0, a.table_rows);
   const float* cs = a.cosine + (size_t)p * (s.rot >> 1);
   const float* sn = a.sine + (size_t)p * (s.rot >> 1);
-  if ((int)blockIdx.x >= s.heads * a.groups) {
-    const int b = 4 * ((int)blockIdx.x - s.heads * a.groups) + wave;
+  const int extra = (int)blockIdx.x - s.heads * a.groups;
+  if (extra >= 4) {
+    const int head = extra - 4;
+    for (int i = threadIdx.x; i < nb * s.rotp; i += 256) {
+      const int b = b0 + i / s.rotp, d = i % s.rotp;
+      a.q[((size_t)b * s.heads + head) * width + s.rankp + d] =
+          f32_to_bf16_rne(rotated(a.y + (size_t)b * a.ldy + head * dq + s.dimp, d, s.rot, cs, sn));
+    }
+    return;
+  }
+  if (extra >= 0) {
+    const int b = 4 * extra + wave;
     if (b < nb) {
       const float* lat = a.y + (size_t)(b0 + b) * a.ldy + s.heads * dq;
-      float ss = 0.f;
-      for (int i = 4 * lane; i < s.rankp; i += 256) {  // padding columns are zero
-        const float4 v = load4(lat + i);
-        ss += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
-      }
-      const Divisor by(sqrtf(wave_sum64(ss) / (float)s.rank + s.eps));
       uint16_t* dst = a.ring + ((size_t)(b0 + b) * a.cap + p % a.cap) * width;
-      for (int i = 4 * lane; i < s.rankp; i += 256) {
-        const float4 v = load4(lat + i), w = load4(a.latent_gain + i);
-        store4(dst + i, float4{by.divide(v.x) * w.x, by.divide(v.y) * w.y, by.divide(v.z) * w.z, by.divide(v.w) * w.w});
+      constexpr int kKeep = 2;  // the first 512 columns stay in registers
+      float4 v[kKeep], w[kKeep];
+#pragma unroll
+      for (int j = 0; j < kKeep; ++j) {
+        const int i = min(4 * lane + 256 * j, s.rankp - 4);
+        v[j] = load4(lat + i);
+        w[j] = load4(a.latent_gain + i);
       }
       for (int i = lane; i < s.rotp; i += 64) dst[s.rankp + i] = f32_to_bf16_rne(rotated(lat + s.rankp, i, s.rot, cs, sn));
+      float ss = 0.f;
+      auto square = [&](const float4& u) { ss += (u.x * u.x + u.y * u.y) + (u.z * u.z + u.w * u.w); };  // padding columns are zero
+#pragma unroll
+      for (int j = 0; j < kKeep; ++j)
+        if (4 * lane + 256 * j < s.rankp) square(v[j]);
+      for (int i = 4 * lane + 256 * kKeep; i < s.rankp; i += 256) square(load4(lat + i));
+      const Divisor by(sqrtf(wave_sum64(ss) / (float)s.rank + s.eps));
+      auto put = [&](int i, const float4& u, const float4& k) {
+        store4(dst + i, float4{by.divide(u.x) * k.x, by.divide(u.y) * k.y, by.divide(u.z) * k.z, by.divide(u.w) * k.w});
+      };
+#pragma unroll
+      for (int j = 0; j < kKeep; ++j)
+        if (4 * lane + 256 * j < s.rankp) put(4 * lane + 256 * j, v[j], w[j]);
+      for (int i = 4 * lane + 256 * kKeep; i < s.rankp; i += 256) put(i, load4(lat + i), load4(a.latent_gain + i));
     }
     return;
   }
   const int h = blockIdx.x / a.groups, grp = blockIdx.x % a.groups;
-  if (grp == 0) {
-    for (int i = threadIdx.x; i < nb * s.rotp; i += 256) {
-      const int b = b0 + i / s.rotp, d = i % s.rotp;
-      a.q[((size_t)b * s.heads + h) * width + s.rankp + d] =
-          f32_to_bf16_rne(rotated(a.y + (size_t)b * a.ldy + h * dq + s.dimp, d, s.rot, cs, sn));
-    }
-  }
   const int tile = 4 * grp + wave;
   if (16 * tile >= s.rankp) return;
   const uint16_t* wrow = a.ukt + ((size_t)h * s.rankp + 16 * tile + r) * s.dimp;
-  const float* xr = a.y + (size_t)(b0 + min(r, nb - 1)) * a.ldy + h * dq + 8 * g;
-  f32x4_t acc[1][1] = {};
-  tile_steps<1, 1>(wrow, s.dimp, 0, (s.dimp + 31) >> 5, g, acc, [&](int, int st) {
-    if (r >= nb) return u32x4_t{0u, 0u, 0u, 0u};
-    const float4 u = load4(xr + 32 * st), v = load4(xr + 32 * st + 4);
-    return u32x4_t{pack2_bf16(u.x, u.y), pack2_bf16(u.z, u.w), pack2_bf16(v.x, v.y), pack2_bf16(v.z, v.w)};
-  });
+  const float* xr = a.y + (size_t)(b0 + min(r, nb - 1)) * a.ldy + h * dq;  // (columns past the batch repeat the last one, and are not stored)
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  constexpr int kSteps = 4;
+  for (int k0 = 8 * g; k0 < s.dimp + 8 * g; k0 += 32 * kSteps) {
+    u32x4_t w[kSteps];
+    float4 u[kSteps], v[kSteps];
+#pragma unroll
+    for (int i = 0; i < kSteps; ++i) {
+      const int k = min(k0 + 32 * i, s.dimp - 8);
+      w[i] = *reinterpret_cast<const u32x4_t*>(wrow + k);
+      u[i] = load4(xr + k);
+      v[i] = load4(xr + k + 4);
+    }
+#pragma unroll
+    for (int i = 0; i < kSteps; ++i) {
+      const u32x4_t none = {0u, 0u, 0u, 0u};
+      const u32x4_t x = {pack2_bf16(u[i].x, u[i].y), pack2_bf16(u[i].z, u[i].w), pack2_bf16(v[i].x, v[i].y), pack2_bf16(v[i].z, v[i].w)};
+      const bool live = k0 + 32 * i < s.dimp;
+      acc = mfma16(live ? w[i] : none, live ? x : none, acc);
+    }
+  }
   if (r < nb)
-    store4(a.q + ((size_t)(b0 + r) * s.heads + h) * width + 16 * tile + 4 * g,
-           float4{acc[0][0][0], acc[0][0][1], acc[0][0][2], acc[0][0][3]});
+    store4(a.q + ((size_t)(b0 + r) * s.heads + h) * width + 16 * tile + 4 * g, float4{acc[0], acc[1], acc[2], acc[3]});
 }
 
 // One chunk of cache rows against 16 HT heads of one sequence, in the latent space: row j of the ring
@@ -536,6 +567,7 @@ __host__ __device__ constexpr long long latent_sums_at(int b, int tile, int chun
   return (((long long)b * ((heads + 15) / 16) + tile) * chunks + chunk) * 16 * rankp;
 }
 constexpr int kLatentRows = 64;
+constexpr int kBufferWord3 = 0x00020000;  // last word of a raw buffer descriptor: 32-bit elements, no swizzle
 constexpr int kLatentPBytes = (kLatentRows + 8) * 2;
 constexpr int latent_decode_lds(int ks, int ht) { return ks * 8192 + ht * 16 * kLatentPBytes; }  // two stages of ks / 2 panels
 template <int KS, int RT, int HT>
@@ -559,13 +591,17 @@ __global__ __launch_bounds__(256 * HT) void latent_decode_kernel(LatentDecode a)
   }
   const int b = unit / a.chunks, chunk = unit % a.chunks, h0 = 16 * (HT * group + ht);
   const int cw = a.width >> 3;
-  u32x4_t qf[KS];  // requested before the position is known
-  const uint16_t* qsrc = a.q + ((size_t)b * a.heads + min(h0 + r, a.heads - 1)) * a.width + 8 * g;
+  // Requested before the position is known and in one go, through a buffer descriptor of the sequence's queries: chunks past the
+  // width are addressed past its end, which reads as zeros (left out by a branch, each was waited for before the next was
+  // requested; cleared by selects, 18 of them cost a microsecond of arithmetic).
+  u32x4_t qf[KS];
+  const uint32_t q_bytes = 2u * (uint32_t)(a.heads * a.width);  // (a launch's queries of one sequence stay far below 2 GiB)
+  const __amdgpu_buffer_rsrc_t q_rows =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.q) + (size_t)b * a.heads * a.width, 0, (int)q_bytes, kBufferWord3);
+  const uint32_t q_at = 2u * (uint32_t)(min(h0 + r, a.heads - 1) * a.width);
 #pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    qf[s] = u32x4_t{0u, 0u, 0u, 0u};
-    if (4 * s + g < cw) qf[s] = *reinterpret_cast<const u32x4_t*>(qsrc + 32 * s);
-  }
+  for (int s = 0; s < KS; ++s)
+    qf[s] = __builtin_amdgcn_raw_buffer_load_b128(q_rows, (int)(4 * s + g < cw ? q_at + 16u * (uint32_t)(4 * s + g) : q_bytes), 0, 0);
   const int valid = (int)min(max(*a.pos, 0ll), (long long)a.cap - 1) + 1;  // rows the ring holds
   const int per = (((valid + a.chunks - 1) / a.chunks) + kLatentRows - 1) & ~(kLatentRows - 1);
   const int begin = chunk * per, end = min(valid, begin + per);
@@ -588,6 +624,10 @@ __global__ __launch_bounds__(256 * HT) void latent_decode_kernel(LatentDecode a)
       }
     };
     fetch(begin);
+    // (the queries are waited for here, where the first block is on its way, and not in the loop, where the wait would be for the
+    // block ahead as well)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));
     // keys: row 16 part + r, chunk 4 (s & 1) + g of panel s / 2
     const uint32_t k_rd[2] = {lds0 + (uint32_t)((16 * part + r) * 128 + 16 * (g ^ (r & 6 | r >> 3))),
                               lds0 + (uint32_t)((16 * part + r) * 128 + 16 * ((4 + g) ^ (r & 6 | r >> 3)))};
@@ -602,9 +642,37 @@ __global__ __launch_bounds__(256 * HT) void latent_decode_kernel(LatentDecode a)
       if (j0 + kLatentRows < end) fetch(j0 + kLatentRows);
       const uint32_t stage = (uint32_t)((((j0 - begin) / kLatentRows) & 1) * kStage);
       f32x4_t sc[2] = {};
+      auto fragment = [&](int s) { return pf_read128(k_rd[s & 1] + stage + (uint32_t)((s >> 1) * kPanel)); };
+      // the usual two starts: fragments are read kBatch at a time, ahead of the products of the ones before (left to the compiler,
+      // and more so with a branch per step, each read waits for the product before it)
+      auto scores_from = [&](auto from) {
+        constexpr int kFrom = decltype(from)::value, kBatch = 4;
+        u32x4_t ka[2][kBatch];
+        auto read = [&](int s0) {
 #pragma unroll
-      for (int s = 0; s < KS; ++s)
-        if (s >= a.key_step) sc[s & 1] = mfma16(pf_read128(k_rd[s & 1] + stage + (uint32_t)((s >> 1) * kPanel)), qf[s], sc[s & 1]);
+          for (int i = 0; i < kBatch; ++i)
+            if (s0 + i < KS) ka[((s0 - kFrom) / kBatch) & 1][i] = fragment(s0 + i);
+        };
+        read(kFrom);
+#pragma unroll
+        for (int s0 = kFrom; s0 < KS; s0 += kBatch) {
+          if (s0 + kBatch < KS) read(s0 + kBatch);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < kBatch; ++i)
+            if (s0 + i < KS) sc[(s0 + i) & 1] = mfma16(ka[((s0 - kFrom) / kBatch) & 1][i], qf[s0 + i], sc[(s0 + i) & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      if (a.key_step == 0) {
+        scores_from(std::integral_constant<int, 0>{});
+      } else if (a.key_step == KS / 2) {
+        scores_from(std::integral_constant<int, KS / 2>{});
+      } else {
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+          if (s >= a.key_step) sc[s & 1] = mfma16(fragment(s), qf[s], sc[s & 1]);
+      }
       // score i: key j0 + 16 part + 4 g + i, head h0 + r
       float p[4], mx = -INFINITY;
 #pragma unroll
@@ -667,19 +735,19 @@ struct LatentExpand {
   uint16_t* out;            // [B, out_ld], head h at column h * vdimp
   int batch, heads, chunks, rankp, vdimp, gate_ld, out_ld, groups;  // groups: workgroups per head
 };
-constexpr int kLatentMaxChunks = 32, kExpandBatch = 4, kExpandRank = 512;
-// A workgroup of 8 waves per (head, TW 16-column tiles of values, 4 sequences): the chunks are merged by all threads, then
+constexpr int kLatentMaxChunks = 32, kExpandRank = 512;
+// A workgroup of 8 waves per (head, TW 16-column tiles of values, EB sequences): the chunks are merged by all threads, then
 // 8 / TW waves per tile expand the merged latents, a part of them each; their weights are requested first.  One CU takes in
-// some 40 KB per microsecond: for few sequences a head's weights (128 KB at 512 x 128) want several workgroups (TW = 2),
-// for more the merge, which every workgroup of a head repeats, wants few (TW = 8).  Grid (H * groups, batch blocks).
-template <int TW>
+// some 40 KB per microsecond, and that is what bounds a launch: a head's weights (128 KB at 512 x 128) divided by the tiles, a
+// sequence's chunks (2 KB each) times EB, which every workgroup of a head repeats.  Grid (H * groups, batch blocks).
+template <int TW, int EB>
 __global__ __launch_bounds__(512) void latent_expand_kernel(LatentExpand a) {
   constexpr int kParts = 8 / TW, kSteps = kExpandRank / 32 / kParts;
-  extern __shared__ __attribute__((aligned(16))) uint16_t merged[];   // [kExpandBatch][rankp + 8] bf16
-  __shared__ float weight[kExpandBatch][kLatentMaxChunks];
+  extern __shared__ __attribute__((aligned(16))) uint16_t merged[];   // [EB][rankp + 8] bf16
+  __shared__ float weight[EB][kLatentMaxChunks];
   __shared__ float4 part[512];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
-  const int b0 = blockIdx.y * kExpandBatch, nb = min(kExpandBatch, a.batch - b0);
+  const int b0 = blockIdx.y * EB, nb = min(EB, a.batch - b0);
   const int h = blockIdx.x / a.groups, tile = TW * (blockIdx.x % a.groups) + wave / kParts;
   const int ld = a.rankp + 8;
   const u32x4_t zero = {0u, 0u, 0u, 0u};
@@ -706,6 +774,7 @@ __global__ __launch_bounds__(512) void latent_expand_kernel(LatentExpand a) {
     for (int k = 0; k < kAhead; ++k) ahead[k] = load4(src + (size_t)min(s0 + k * split, a.chunks - 1) * (16 * a.rankp));
   };
   request(tid % span, which);
+  const float gate = a.gate ? a.gate[(size_t)(b0 + min(r, nb - 1)) * a.gate_ld + h] : 0.f;
   if (wave < nb) {  // a wave per sequence, a lane per chunk
     const bool mine = lane < a.chunks;
     const float2 ml = mine ? a.heads_in[((size_t)(b0 + wave) * a.heads + h) * a.chunks + lane] : float2{-INFINITY, 0.f};
@@ -759,7 +828,7 @@ __global__ __launch_bounds__(512) void latent_expand_kernel(LatentExpand a) {
     acc[0] += v.x; acc[1] += v.y; acc[2] += v.z; acc[3] += v.w;
   }
   if (r >= nb) return;
-  const float f = a.gate ? sigmoid_f32(a.gate[(size_t)(b0 + r) * a.gate_ld + h]) : 1.f;
+  const float f = a.gate ? sigmoid_f32(gate) : 1.f;
   store4(a.out + (size_t)(b0 + r) * a.out_ld + (size_t)h * a.vdimp + 16 * tile + 4 * g,
          float4{acc[0] * f, acc[1] * f, acc[2] * f, acc[3] * f});
 }

@@ -21,11 +21,16 @@ template <> __device__ __forceinline__ float from_f32<float>(float v) { return v
 template <> __device__ __forceinline__ uint16_t from_f32<uint16_t>(float v) { return f32_to_bf16_rne(v); }
 
 __device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 load4(const uint16_t* p) {
-  const u32x2_t v = *reinterpret_cast<const u32x2_t*>(p);
+__device__ __forceinline__ float4 widen4(const u32x2_t& v) {
   return float4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u), __uint_as_float(v.y << 16),
                 __uint_as_float(v.y & 0xFFFF0000u)};
 }
+__device__ __forceinline__ float4 widen4(const float4& v) { return v; }
+__device__ __forceinline__ float4 load4(const uint16_t* p) { return widen4(*reinterpret_cast<const u32x2_t*>(p)); }
+// four elements as they lie, for loads that are not to be waited for yet
+template <typename T> struct Raw4;
+template <> struct Raw4<float> { typedef float4 type; };
+template <> struct Raw4<uint16_t> { typedef u32x2_t type; };
 __device__ __forceinline__ void store4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ __forceinline__ void store4(uint16_t* p, float4 v) {
   *reinterpret_cast<u32x2_t*>(p) = u32x2_t{pack2_bf16(v.x, v.y), pack2_bf16(v.z, v.w)};
@@ -38,8 +43,7 @@ __device__ __forceinline__ Float8 load8(const float* p) {
   const float4 a = load4(p), b = load4(p + 4);
   return Float8{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
 }
-__device__ __forceinline__ Float8 load8(const uint16_t* p) {
-  const u32x4_t q = *reinterpret_cast<const u32x4_t*>(p);
+__device__ __forceinline__ Float8 widen8(const u32x4_t& q) {
   Float8 f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -48,6 +52,7 @@ __device__ __forceinline__ Float8 load8(const uint16_t* p) {
   }
   return f;
 }
+__device__ __forceinline__ Float8 load8(const uint16_t* p) { return widen8(*reinterpret_cast<const u32x4_t*>(p)); }
 __device__ __forceinline__ void store8(float* p, const Float8& f) {
   store4(p, float4{f.v[0], f.v[1], f.v[2], f.v[3]});
   store4(p + 4, float4{f.v[4], f.v[5], f.v[6], f.v[7]});
@@ -57,15 +62,14 @@ __device__ __forceinline__ void store8(uint16_t* p, const Float8& f) {
                                            pack2_bf16(f.v[6], f.v[7])};
 }
 
-__device__ __forceinline__ float wave_sum64(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
-}
+// over a wave, the result in every lane: rotations inside the rows of 16 lanes, then lane swaps
+__device__ __forceinline__ float wave_sum64(float v) { return quad_sum(team_sum16(v)); }
 __device__ __forceinline__ float wave_max64(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-  return v;
+  v = fmaxf(v, row_ror<8>(v));
+  v = fmaxf(v, row_ror<4>(v));
+  v = fmaxf(v, row_ror<2>(v));
+  v = fmaxf(v, row_ror<1>(v));
+  return quad_max(v);
 }
 // sum over a 256-thread workgroup, the result in every thread (`part`: four floats of LDS)
 __device__ __forceinline__ float block_sum256(float v, float* part) {
@@ -112,7 +116,9 @@ __global__ __launch_bounds__(256) void embed_kernel(const long long* __restrict_
 // x[m, :] += delta[m, :] + again[m, :] + step[:] (each optional; written back when any is given), then for j = 1, 2
 // (each optional) out_j[m, :] = (x - mean) / sqrt(variance + eps) * gain_j.  `center` = 0 leaves the mean in: an RMS
 // norm.  Statistics over the first D of Dp columns, fp32, deviations squared after the mean is known.
-// One workgroup per row; the first 8192 columns stay in registers between the passes.
+// One workgroup per row; the first 8192 columns stay in registers between the passes.  A decode step has a handful of rows, so
+// a launch is bounded by its round trips to memory: all that a row needs, the gain included, is requested before the first
+// sum (8 rows of 4096: 5.0 us, 6.4 where every vector of every operand was waited for in turn).
 template <typename T, typename DeltaT>
 __global__ __launch_bounds__(256) void add_norms_kernel(float* __restrict__ x, const DeltaT* __restrict__ delta,
                                                         const float* __restrict__ again, const float* __restrict__ step,
@@ -123,7 +129,7 @@ __global__ __launch_bounds__(256) void add_norms_kernel(float* __restrict__ x, c
   __shared__ float part[4];
   const size_t base = (size_t)blockIdx.x * Dp;
   const bool changed = delta || again || step;
-  auto take = [&](int i) {
+  auto take = [&](int i) {  // (columns past the registers)
     float4 v = load4(x + base + i);
     if (delta) {
       const float4 d = load4(delta + base + i);
@@ -140,16 +146,57 @@ __global__ __launch_bounds__(256) void add_norms_kernel(float* __restrict__ x, c
     if (changed) store4(x + base + i, v);
     return v;
   };
-  float4 keep[kKeep];
+  const float4 zero = float4{0.f, 0.f, 0.f, 0.f};
+  float4 keep[kKeep], gain[kKeep];  // (gain: of the first output there is)
+  auto column = [&](int j) { return 4 * ((int)threadIdx.x + 256 * j); };
+#pragma unroll
+  for (int j = 0; j < kKeep; ++j) {
+    keep[j] = zero;
+    if (column(j) < Dp) keep[j] = load4(x + base + column(j));
+  }
+  auto fetch_gain = [&] {
+    const float* from = out1 ? gain1 : gain2;
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) {
+      gain[j] = zero;
+      if (from && column(j) < Dp) gain[j] = load4(from + column(j));
+    }
+  };
+  if (delta) {
+    typename Raw4<DeltaT>::type d[kKeep];
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) {
+      d[j] = {};
+      if (column(j) < Dp) d[j] = *reinterpret_cast<const typename Raw4<DeltaT>::type*>(delta + base + column(j));
+    }
+    fetch_gain();
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) {
+      const float4 v = widen4(d[j]);
+      keep[j].x += v.x; keep[j].y += v.y; keep[j].z += v.z; keep[j].w += v.w;
+    }
+  } else {
+    fetch_gain();
+  }
+  auto add = [&](const float* from) {
+    float4 d[kKeep];
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) {
+      d[j] = zero;
+      if (column(j) < Dp) d[j] = load4(from + column(j));
+    }
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) {
+      keep[j].x += d[j].x; keep[j].y += d[j].y; keep[j].z += d[j].z; keep[j].w += d[j].w;
+    }
+  };
+  if (again) add(again + base);
+  if (step) add(step);
   float sum = 0.f;
 #pragma unroll
   for (int j = 0; j < kKeep; ++j) {
-    const int i = 4 * (threadIdx.x + 256 * j);
-    keep[j] = float4{0.f, 0.f, 0.f, 0.f};
-    if (i < Dp) {
-      keep[j] = take(i);
-      sum += (keep[j].x + keep[j].y) + (keep[j].z + keep[j].w);  // padding columns are zero
-    }
+    if (changed && column(j) < Dp) store4(x + base + column(j), keep[j]);
+    sum += (keep[j].x + keep[j].y) + (keep[j].z + keep[j].w);  // padding columns are zero
   }
   for (int i = 4 * (threadIdx.x + 256 * kKeep); i < Dp; i += 1024) {
     const float4 v = take(i);
@@ -175,8 +222,7 @@ __global__ __launch_bounds__(256) void add_norms_kernel(float* __restrict__ x, c
   }
   for (int i = 4 * (threadIdx.x + 256 * kKeep); i < Dp; i += 1024) square(i, load4(x + base + i));
   const Divisor by(sqrtf(block_sum256(ss, part) / (float)D + eps));
-  auto put = [&](int i, const float4& v, const float* gain, T* out) {
-    const float4 g = load4(gain + i);
+  auto put = [&](int i, const float4& v, const float4& g, T* out) {
     store4(out + base + i, float4{by.divide(v.x - mean) * g.x, by.divide(v.y - mean) * g.y, by.divide(v.z - mean) * g.z,
                                   by.divide(v.w - mean) * g.w});  // gains are zero in the padding columns
   };
@@ -184,14 +230,14 @@ __global__ __launch_bounds__(256) void add_norms_kernel(float* __restrict__ x, c
   for (int j = 0; j < kKeep; ++j) {
     const int i = 4 * (threadIdx.x + 256 * j);
     if (i < Dp) {
-      if (out1) put(i, keep[j], gain1, out1);
-      if (out2) put(i, keep[j], gain2, out2);
+      put(i, keep[j], gain[j], out1 ? out1 : out2);
+      if (out1 && out2) put(i, keep[j], load4(gain2 + i), out2);
     }
   }
   for (int i = 4 * (threadIdx.x + 256 * kKeep); i < Dp; i += 1024) {
     const float4 v = load4(x + base + i);
-    if (out1) put(i, v, gain1, out1);
-    if (out2) put(i, v, gain2, out2);
+    if (out1) put(i, v, load4(gain1 + i), out1);
+    if (out2) put(i, v, load4(gain2 + i), out2);
   }
 }
 

@@ -155,6 +155,17 @@ __global__ __launch_bounds__(256) void group_merge_kernel(GroupMerge a) {
   const int b = blockIdx.x / heads, head = blockIdx.x % heads, h = head % a.share;
   const int unit = b * a.groups + head / a.share;
   const int quads = a.dimp >> 2, split = max(1, min(256 / quads, a.chunks)), which = tid / quads;
+  // what the sums need from memory, before the chunks' weights are known: a launch is one round trip, not three
+  const int c = 4 * (tid % quads);
+  const float* src = a.sums + latent_sums_at(unit, h >> 4, 0, a.share, a.chunks, a.dimp) + 256 * (c >> 4) + 16 * (h & 15) + (c & 15);
+  constexpr int kAhead = 4;
+  float4 ahead[kAhead], z = float4{0.f, 0.f, 0.f, 0.f};
+  auto request = [&](int s0) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) ahead[k] = load4(src + (size_t)min(s0 + k * split, a.chunks - 1) * (16 * a.dimp));
+  };
+  request(which);
+  if (a.gate) z = load4(a.gate + (size_t)b * a.gate_ld + (size_t)head * a.dimp + c);
   if (tid < 64) {  // a lane per chunk
     const bool mine = lane < a.chunks;
     const float2 ml = mine ? a.heads_in[((size_t)unit * a.share + h) * a.chunks + lane] : float2{-INFINITY, 0.f};
@@ -164,14 +175,17 @@ __global__ __launch_bounds__(256) void group_merge_kernel(GroupMerge a) {
     if (mine) weight[lane] = e / total;
   }
   __syncthreads();
-  const int c = 4 * (tid % quads);
   float4 sum = float4{0.f, 0.f, 0.f, 0.f};
   if (which < split) {
-    const float* src = a.sums + latent_sums_at(unit, h >> 4, 0, a.share, a.chunks, a.dimp) + 256 * (c >> 4) + 16 * (h & 15) + (c & 15);
-    for (int s = which; s < a.chunks; s += split) {
-      const float4 v = load4(src + (size_t)s * (16 * a.dimp));
-      const float f = weight[s];
-      sum.x = fmaf(v.x, f, sum.x); sum.y = fmaf(v.y, f, sum.y); sum.z = fmaf(v.z, f, sum.z); sum.w = fmaf(v.w, f, sum.w);
+    for (int s0 = which; s0 < a.chunks; s0 += kAhead * split) {
+      if (s0 > which) request(s0);
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        if (s0 + k * split >= a.chunks) break;
+        const float4 v = ahead[k];
+        const float f = weight[s0 + k * split];
+        sum.x = fmaf(v.x, f, sum.x); sum.y = fmaf(v.y, f, sum.y); sum.z = fmaf(v.z, f, sum.z); sum.w = fmaf(v.w, f, sum.w);
+      }
     }
   }
   part[tid] = sum;
@@ -182,7 +196,6 @@ __global__ __launch_bounds__(256) void group_merge_kernel(GroupMerge a) {
     sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
   }
   if (a.gate) {
-    const float4 z = load4(a.gate + (size_t)b * a.gate_ld + (size_t)head * a.dimp + c);
     sum.x *= sigmoid_f32(z.x); sum.y *= sigmoid_f32(z.y); sum.z *= sigmoid_f32(z.z); sum.w *= sigmoid_f32(z.w);
   }
   store4(a.out + (size_t)b * a.out_ld + (size_t)head * a.dimp + c, sum);

@@ -82,6 +82,33 @@ def test_add_norms(cuda, dtype, true_width):
             assert (out[:, true_width:] == 0).all()
 
 
+@pytest.mark.parametrize("width", [16, 1040, 8192, 8208])   # one lane's worth, a ragged second turn, the registers' end and past it
+@pytest.mark.parametrize("delta, again, step, outputs", [(None, False, False, 1), ("f32", False, True, 2), ("bf16", True, False, 1), ("bf16", False, False, 0)])
+def test_add_norms_with_operands_left_out(cuda, width, delta, again, step, outputs):
+    """Every operand of ajqd_add_norms is optional; ``outputs``: 0 none, 1 the second alone, 2 both.  The sum is fp32 (three additions:
+    < 4 ulp of its parts), the norm's relative error at most 2^-9 of bf16 and a few fp32 roundings."""
+    g = torch.Generator().manual_seed(width)
+    rand = lambda *s: torch.randn(s, generator=g)
+    rows = 3
+    x, d, e, s, g1, g2 = rand(rows, width) + 1, rand(rows, width), rand(rows, width), rand(width), rand(width), rand(width)
+    if delta == "bf16":
+        d = d.to(torch.bfloat16)
+    total = x.double() + (d.double() if delta else 0) + (e.double() if again else 0) + (s.double() if step else 0)
+    dev = [t.to(cuda) for t in (x, d, e, s, g1, g2)]
+    out = torch.full((2, rows, width), 9.0, dtype=torch.bfloat16, device=cuda)
+    ptr = lambda t, wanted: t.data_ptr() if wanted else None
+    _ok(_lib.load_dense().ajqd_add_norms(
+        dev[0].data_ptr(), ptr(dev[1], delta), _lib.AJQD_BF16 if delta == "bf16" else _lib.AJQD_F32, ptr(dev[2], again), ptr(dev[3], step),
+        ptr(dev[4], outputs == 2), ptr(dev[5], outputs), 1e-5, 1, ptr(out[0], outputs == 2), ptr(out[1], outputs), rows, width, width,
+        _lib.AJQD_BF16, _st()))
+    assert float((dev[0].cpu().double() - total).abs().max()) < 4 * 2.0 ** -23 * 16
+    for i, gain in ((0, g1), (1, g2)):
+        if outputs == 2 or (outputs == 1 and i == 1):
+            assert _rel(out[i].float(), O.layer_norm(total, gain.double(), 1e-5)) < 4e-3
+        else:
+            assert (out[i] == 9.0).all()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_embedding_and_device_side_position(cuda, dtype):
     table, pos = torch.randn(19, 32).to(dtype), torch.randn(40, 32).to(dtype)
@@ -280,6 +307,16 @@ def test_latent_decode_and_expand_against_plain(cuda, shape):
                                    out.data_ptr(), heads * vdim + 8, batch, heads, chunks, rank, vdim, _st()))
         assert _rel(out[:, : heads * vdim], want.reshape(batch, -1)) < 8e-3, chunks
         assert (out[:, heads * vdim:] == 5.0).all()
+
+
+@pytest.mark.parametrize("shape", [
+    (8, 32, 512, 64, 128, 100, 99),     # a workgroup per head and sequence
+    (33, 16, 512, 64, 128, 70, 65),     # four sequences per workgroup, the last block with one; one head tile
+    (17, 32, 128, 64, 128, 300, 290),   # two sequences per workgroup, an odd count; head tiles alone or in pairs by the chunks
+])
+def test_cuts_of_latent_decode_and_expand(cuda, shape):
+    """The splits of work that the shapes above do not reach, against the same oracle."""
+    test_latent_decode_and_expand_against_plain(cuda, shape)
 
 
 # ------------------------------------------------------------------ the decoder against the plain implementation
