@@ -10,9 +10,14 @@
 namespace ajq {
 
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
+  // lanes l and l ^ 32, then ^ 16, by swaps, then rotations inside the rows of 16: as xor steps 32 ... 1, bit for bit, without the
+  // trips through the LDS crossbar
+  typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+  uint32_t b = __float_as_uint(v);
+  u32x2v s = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  b = __float_as_uint(__uint_as_float(s.x) + __uint_as_float(s.y));
+  s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  return team_sum16(__uint_as_float(s.x) + __uint_as_float(s.y));
 }
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
@@ -23,7 +28,7 @@ __device__ __forceinline__ float wave_max(float v) {
 // hidden[b, :] += delta[b, :] (when delta != nullptr; written back), then
 // out[b, :] = bf16( (hidden / sqrt(mean(hidden^2) + eps)) * gain ).
 // One 256-thread workgroup per row; D % 4 == 0.  The first 4096 elements of a row (four float4 per thread)
-// and their gains stay in registers between the two passes: one memory round trip for the usual widths.
+// and their gains stay in registers between the two passes and are requested together: one memory round trip for the usual widths.
 __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ hidden, const float* __restrict__ delta,
                                                           const float* __restrict__ gain, float eps,
                                                           uint16_t* __restrict__ out, int D) {
@@ -34,26 +39,43 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ hi
   const float4* g4 = reinterpret_cast<const float4*>(gain);
   const int n4 = D >> 2;
   float ss = 0.f;
-  auto take = [&](int i) {
+  auto square = [&](const float4& v) { ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w; };
+  float4 keep[kKeep], g[kKeep];
+#pragma unroll
+  for (int j = 0; j < kKeep; ++j) {
+    const int i = threadIdx.x + 256 * j;
+    keep[j] = g[j] = float4{0.f, 0.f, 0.f, 0.f};
+    if (i < n4) {
+      keep[j] = h4[i];
+      g[j] = g4[i];
+    }
+  }
+  if (d4) {
+    float4 d[kKeep];
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) {
+      const int i = threadIdx.x + 256 * j;
+      d[j] = float4{0.f, 0.f, 0.f, 0.f};
+      if (i < n4) d[j] = d4[i];
+    }
+#pragma unroll
+    for (int j = 0; j < kKeep; ++j) {
+      const int i = threadIdx.x + 256 * j;
+      keep[j].x += d[j].x; keep[j].y += d[j].y; keep[j].z += d[j].z; keep[j].w += d[j].w;
+      if (i < n4) h4[i] = keep[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kKeep; ++j) square(keep[j]);
+  for (int i = threadIdx.x + 256 * kKeep; i < n4; i += 256) {
     float4 v = h4[i];
     if (d4) {
       const float4 d = d4[i];
       v.x += d.x; v.y += d.y; v.z += d.z; v.w += d.w;
       h4[i] = v;
     }
-    ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
-    return v;
-  };
-  float4 keep[kKeep], g[kKeep];
-#pragma unroll
-  for (int j = 0; j < kKeep; ++j) {
-    const int i = threadIdx.x + 256 * j;
-    if (i < n4) {
-      keep[j] = take(i);
-      g[j] = g4[i];
-    }
+    square(v);
   }
-  for (int i = threadIdx.x + 256 * kKeep; i < n4; i += 256) take(i);
   ss = wave_sum(ss);
   __shared__ float part[4];
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;

@@ -56,23 +56,42 @@ struct SkinnySplit {
 // What becomes of one finished unit of a 32-row block that starts at row m0: row tile `tile` of N, 16-row block r;
 // lane (nl, kc) holds rows 4 kc + i of the block in component i, column nl of the tile.  Channel scale (int8),
 // the rows' norm factors, then the plain store, the residual form or the SwiGLU gate on interleaved rows.
+// What that needs from memory is requested ahead of the unit's sum (skinny_unit_operands): fetched where they are used, the four
+// old residuals were a round trip each, behind the store of the one before.
+struct SkinnyUnitOperands {
+  uint32_t scale_bits;
+  float gain, h_old[4];
+};
 template <bool kW4, int kEpi>
-__device__ __forceinline__ void skinny_finish_unit(const f32x4_t& sum, int tile, int r, const float (&rstd)[4], int m0, int M,
-                                                   int N, int lane, void* __restrict__ y, int out_f32,
-                                                   const uint16_t* __restrict__ scales8, const GemvEpilogue& ep) {
+__device__ __forceinline__ SkinnyUnitOperands skinny_unit_operands(int tile, int r, int m0, int M, int N, int lane,
+                                                                   const uint16_t* __restrict__ scales8, const GemvEpilogue& ep) {
+  SkinnyUnitOperands o{};
+  const int n = tile * kTileN + (lane & 15);
+  if (!kW4) o.scale_bits = scales8[n];
+  if (kEpi & kEpiResidual) {
+    o.gain = ep.gain[n];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o.h_old[i] = ep.h_in[(size_t)min(m0 + 16 * r + 4 * (lane >> 4) + i, M - 1) * N + n];
+  }
+  return o;
+}
+template <bool kW4, int kEpi>
+__device__ __forceinline__ void skinny_finish_unit(const f32x4_t& sum, const SkinnyUnitOperands& operands, int tile, int r,
+                                                   const float (&rstd)[4], int m0, int M, int N, int lane, void* __restrict__ y,
+                                                   int out_f32, const GemvEpilogue& ep) {
   const int nl = lane & 15, kc = lane >> 4;
   const int ntiles = N / kTileN;
   const int n = tile * kTileN + nl;
   float cs = 1.0f;
-  if (!kW4) cs = f16_bits_to_f32(scales8[n]);  // per-output-channel scale, once
+  if (!kW4) cs = f16_bits_to_f32(operands.scale_bits);  // per-output-channel scale, once
   if (kEpi & kEpiResidual) {
-    const float gain_n = ep.gain[n];
+    const float gain_n = operands.gain;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int m = m0 + 16 * r + 4 * kc + i;
       float v = sum[i] * cs * rstd[i];
       asm volatile("" : "+v"(v));  // no fused multiply-add: bit for bit the plain output, then the add
-      const float h = (m < M ? ep.h_in[(size_t)m * N + n] : 0.f) + v;
+      const float h = operands.h_old[i] + v;
       if (m < M) {
         ep.h_out[(size_t)m * N + n] = h;
         if (ep.xt) ep.xt[(size_t)m * N + n] = f32_to_bf16_rne(h * gain_n);
@@ -376,6 +395,7 @@ __device__ __forceinline__ void dequant_skinny_body(
   for (int u = wave; u < NT * MB; u += kWaves) {
     const int t = u / MB, r = u % MB;
     if (nt0 + t >= ntiles) break;
+    const SkinnyUnitOperands operands = skinny_unit_operands<kW4, kEpi>(nt0 + t, r, m0, M, N, lane, scales8, ep);
     f32x4_t sum;
     if constexpr (kSplitK) {
       const unsigned long long* src = reinterpret_cast<const unsigned long long*>(shared_partial) + ((size_t)u * 64 + lane) * 2;
@@ -386,8 +406,18 @@ __device__ __forceinline__ void dequant_skinny_body(
         return f32x4_t{__uint_as_float((uint32_t)lo), __uint_as_float((uint32_t)(lo >> 32)), __uint_as_float((uint32_t)hi),
                        __uint_as_float((uint32_t)(hi >> 32))};
       };
-      sum = fetch(0);
-      for (int q = 1; q < S; ++q) sum += fetch(q);
+      // four parts requested together, added in split order (one after the other: a round trip to memory each)
+      constexpr int kTogether = 4;
+      for (int q0 = 0; q0 < S; q0 += kTogether) {
+        f32x4_t part[kTogether];
+#pragma unroll
+        for (int k = 0; k < kTogether; ++k) part[k] = fetch(min(q0 + k, S - 1));
+        if (q0 == 0) sum = part[0];
+        else sum += part[0];
+#pragma unroll
+        for (int k = 1; k < kTogether; ++k)
+          if (q0 + k < S) sum += part[k];
+      }
     } else {
       sum = unit_sum(u);
     }
@@ -401,7 +431,7 @@ __device__ __forceinline__ void dequant_skinny_body(
         rstd[i] = rsqrtf(total * ep.inv_k + ep.eps);
       }
     }
-    skinny_finish_unit<kW4, kEpi>(sum, nt0 + t, r, rstd, m0, M, N, lane, y, out_f32, scales8, ep);
+    skinny_finish_unit<kW4, kEpi>(sum, operands, nt0 + t, r, rstd, m0, M, N, lane, y, out_f32, ep);
   }
 }
 
