@@ -859,6 +859,13 @@ int launch_gemv_pro(int M, int K, const uint32_t* wq, const uint32_t* meta, cons
 #define AJQ_PRO(W, T, R)                                                                                              \
   return launch_gemv_pro_cfg<W, T, R, kW4, kPro, kOut>(M, K, wq, meta, scales8, N, y, out_f32, src0, src1, gain, eps, \
                                                        h_out, stream, S)
+  // One row with its norm from the sums: four waves of twice the groups.  Every wave forms the norm's divisor for itself, and with
+  // eight a launch of many workgroups is bounded by that arithmetic (int4, K = 2048, N = 6144 / 11264 / 32000: 3.87 / 4.93 / 9.24 us
+  // with eight waves, 3.67 / 4.57 / 8.19 with four; K = 1024, N = 11264: 4.18 / 3.59; int8, K = 2048, N = 11264: 6.25 / 6.12).
+  if constexpr (kPro == kProNormSums) {
+    if (M <= 1 && K == 1024) AJQ_PRO(4, 2, 1);
+    if (M <= 1 && K == 2048) AJQ_PRO(4, 4, 1);
+  }
   if (K == 1024) {
     if (M <= 1) AJQ_PRO(8, 1, 1);
     if (M <= 4) AJQ_PRO(8, 1, 4);

@@ -626,6 +626,13 @@ def test_gemv_residual_then_rowscale_against_the_oracle(cuda, scheme, m, k1, d, 
                   _lib.AJQ_OUT_F32, 0, st) != 0
 
 
+@pytest.mark.parametrize("scheme", ["w4", "w8"])
+@pytest.mark.parametrize("m,k1,d,n2", [(1, 1024, 1024, 32), (1, 2048, 2048, 11264), (2, 2048, 1024, 512)])
+def test_norm_from_sums_on_one_row(cuda, scheme, m, k1, d, n2):
+    """One row takes workgroups of four waves, two rows those of eight: the fewest row tiles, and many, of either."""
+    test_gemv_residual_then_rowscale_against_the_oracle(cuda, scheme, m, k1, d, n2)
+
+
 # (M, N, K) of the routes that cut K: every row-block height at its edges, a last column block cut short, parts of unequal length, one
 # part only; the tiles' shifted and short last row tile; and shapes beside the rules' lines
 _SPLIT_SHAPES = [(17, 2064, 14336), (32, 4096, 8320), (33, 4112, 5632), (48, 16016, 1408), (49, 8208, 3072), (64, 3088, 8192), (37, 33008, 640),
