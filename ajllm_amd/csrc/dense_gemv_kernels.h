@@ -98,7 +98,7 @@ constexpr int kStreamBlock = 128;
 constexpr int stream_lds(int waves, int rows, int rt, int bt, int uq) {
   return waves * uq * rt * rows * 256 > rt * bt * waves * 1024 ? waves * uq * rt * rows * 256 : rt * bt * waves * 1024;
 }
-template <int kWaves, int ROWS, int RT, int BT, int UQ, typename Between, typename XFn>
+template <int kWaves, int ROWS, int RT, int BT, int UQ, bool kXFirst = true, typename Between, typename XFn>
 __device__ __forceinline__ void stream_rows(const uint16_t* __restrict__ w, int K, int wave, int lane, unsigned char* lds,
                                             f32x4_t (&acc)[RT][BT], Between&& between, XFn&& x) {
   static_assert(ROWS == 16 || ROWS == 8, "tiles of 16 or 8 rows");
@@ -156,10 +156,11 @@ __device__ __forceinline__ void stream_rows(const uint16_t* __restrict__ w, int 
         }
   };
   if (count >= UQ) load_w(0, begin);
+  if (kXFirst && count >= UQ) load_x(0, begin);
   between();
   int s = begin, left = count;
   if (left >= UQ) {
-    load_x(0, s);
+    if (!kXFirst) load_x(0, s);
     for (; left >= 3 * UQ; left -= 2 * UQ, s += 2 * UQ) {
       load_w(1, s + UQ);
       load_x(1, s + UQ);
@@ -304,7 +305,7 @@ __global__ __launch_bounds__(64 * kWaves) void dense_in_kernel(DenseIn a) {
       }
       __syncthreads();
     };
-    stream_rows<kWaves, 16, RT, BT, 1>(wrow, a.Dp, wave, lane, lds, acc, norm, [&](int t, int s) {
+    stream_rows<kWaves, 16, RT, BT, 1, false>(wrow, a.Dp, wave, lane, lds, acc, norm, [&](int t, int s) {
       return *reinterpret_cast<const u32x4_t*>(normed + min(16 * t + r, nb - 1) * stride + 8 * g + 32 * s);
     });
   } else {
@@ -315,8 +316,14 @@ __global__ __launch_bounds__(64 * kWaves) void dense_in_kernel(DenseIn a) {
       for (int row = threadIdx.x >> 4; row < nb; row += 4 * kWaves) {
         const float* part = a.sums + (size_t)(b0 + row) * a.parts;
         float ss = 0.f;
-#pragma unroll 8
-        for (int i = r; i < a.parts; i += 16) ss += part[i];
+        constexpr int kTogether = 16;
+        for (int i0 = r; i0 < a.parts; i0 += 16 * kTogether) {
+          float p[kTogether];
+#pragma unroll
+          for (int k = 0; k < kTogether; ++k) p[k] = part[min(i0 + 16 * k, a.parts - 1)];
+#pragma unroll
+          for (int k = 0; k < kTogether; ++k) ss += i0 + 16 * k < a.parts ? p[k] : 0.f;
+        }
         ss = team_sum16(ss);
         if (r == 0) stat[row] = 1.0f / sqrtf(ss / (float)a.D + a.eps);
       }
@@ -369,22 +376,17 @@ __global__ __launch_bounds__(64 * kWaves) void dense_out_kernel(DenseOut a) {
   const bool writes = wave < RT * BT && 4 * g < ROWS;
   const int row = 16 * (wave % BT) + r, column = first + ROWS * (wave / BT) + 4 * g;
   const size_t place = (size_t)(b0 + min(row, nb - 1)) * a.Dp + column;
-  float4 v = float4{0.f, 0.f, 0.f, 0.f};
-  if (writes) {
-    v = load4(a.x + place);
-    if (a.again) {
-      const float4 e = load4(a.again + place);
-      v.x += e.x; v.y += e.y; v.z += e.z; v.w += e.w;
-    }
-    if (a.step) {
-      const float4 e = load4(a.step + column);
-      v.x += e.x; v.y += e.y; v.z += e.z; v.w += e.w;
-    }
-  }
+  // (and added behind it: an addition here would have that wave wait before it asks for its first weights)
+  float4 v = float4{0.f, 0.f, 0.f, 0.f}, again = v, step = v;
+  if (writes) v = load4(a.x + place);
+  if (writes && a.again) again = load4(a.again + place);
+  if (writes && a.step) step = load4(a.step + column);
   f32x4_t acc[RT][BT] = {};
   stream_rows<kWaves, ROWS, RT, BT, UQ>(a.w + (size_t)first * a.K, a.K, wave, lane, lds, acc, [] {}, [&](int t, int s) {
     return *reinterpret_cast<const u32x4_t*>(xr + (size_t)min(16 * t + r, nb - 1) * a.K + 32 * s);
   });
+  if (a.again) { v.x += again.x; v.y += again.y; v.z += again.z; v.w += again.w; }
+  if (a.step) { v.x += step.x; v.y += step.y; v.z += step.z; v.w += step.w; }
 #pragma unroll
   for (int i = 0; i < RT * BT; ++i) {
     const f32x4_t& sum = acc[i / BT][i % BT];
@@ -421,6 +423,24 @@ __global__ __launch_bounds__(64 * kWaves) void dense_out_streams_kernel(DenseOut
 #pragma unroll
   for (int s = 0; s < MAXS; ++s)
     if (writes && s < a.streams) v[s] = load4(x + (size_t)s * a.Dp);
+  // and the column's factors and, for few streams, the coefficients: fetched where the epilogue uses them they were five round trips
+  // to memory, one after the other, at the end of every launch (4 sequences, K = 8192, 2048 columns, two streams: 7.9 us, 7.2 now)
+  constexpr bool kHold = MAXS <= 4;
+  constexpr int kC = kHold ? MAXS : 1;
+  float4 f = float4{0.f, 0.f, 0.f, 0.f}, k = f;
+  float c_out[kC], c_next[kC], c_mix[kC * kC];
+  if (writes) f = load4(a.scale + column);
+  if (writes && !a.u) k = load4(a.gain + column);
+  if constexpr (kHold) {
+#pragma unroll
+    for (int t = 0; t < kC; ++t) {
+      const int to = min(t, a.streams - 1);
+      c_out[t] = a.out[to];
+      c_next[t] = a.next ? a.next[to] : 1.f;
+#pragma unroll
+      for (int s = 0; s < kC; ++s) c_mix[s * kC + t] = a.mix[min(s, a.streams - 1) * a.streams + to];
+    }
+  }
   f32x4_t acc[RT][BT] = {};
   stream_rows<kWaves, ROWS, RT, BT, UQ>(a.w + (size_t)first * a.K, a.K, wave, lane, lds, acc, [] {}, [&](int t, int s) {
     return *reinterpret_cast<const u32x4_t*>(xr + (size_t)min(16 * t + r, nb - 1) * a.K + 32 * s);
@@ -429,17 +449,19 @@ __global__ __launch_bounds__(64 * kWaves) void dense_out_streams_kernel(DenseOut
   for (int i = 0; i < RT * BT; ++i) {
     if (wave != i || !writes || row >= nb) continue;
     const f32x4_t& sum = acc[i / BT][i % BT];
-    const float4 f = load4(a.scale + column);
-    mix_streams<MAXS>(v, a.streams, a.out, a.mix, float4{sum[0] * f.x, sum[1] * f.y, sum[2] * f.z, sum[3] * f.w});
+    const float4 y = float4{sum[0] * f.x, sum[1] * f.y, sum[2] * f.z, sum[3] * f.w};
+    if constexpr (kHold) mix_streams_by<MAXS>(v, a.streams, [&](int t) { return c_out[t]; }, [&](int s, int t) { return c_mix[s * kC + t]; }, y);
+    else mix_streams<MAXS>(v, a.streams, a.out, a.mix, y);
 #pragma unroll
     for (int s = 0; s < MAXS; ++s)
       if (s < a.streams) store4(x + (size_t)s * a.Dp, v[s]);
-    const float4 read = read_streams<MAXS>(v, a.streams, a.next);
+    float4 read;
+    if constexpr (kHold) read = read_streams_by<MAXS>(v, a.streams, [&](int s) { return c_next[s]; });
+    else read = read_streams<MAXS>(v, a.streams, a.next);
     if (a.u) {
       store4(a.u + (size_t)(b0 + row) * a.Dp + column, read);
       continue;
     }
-    const float4 k = load4(a.gain + column);
     store4(a.scaled + (size_t)(b0 + row) * a.Dp + column, float4{read.x * k.x, read.y * k.y, read.z * k.z, read.w * k.w});
     // (the lanes of a row are 16 apart, and all of them here)
     float ss = (read.x * read.x + read.y * read.y) + (read.z * read.z + read.w * read.w);

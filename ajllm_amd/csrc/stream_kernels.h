@@ -37,19 +37,20 @@ __global__ __launch_bounds__(256) void embed_streams_kernel(const long long* __r
 }
 
 // Four columns of every stream: update by `y` (already scaled), weighted sum for the next reader.
-// `in` null: the plain sum.  Coefficients are uniform over the launch.
-template <int MAXS>
-__device__ __forceinline__ void mix_streams(float4 (&v)[MAXS], int S, const float* __restrict__ out, const float* __restrict__ mix, float4 y) {
+// Coefficients come from out(t), mix(s, t) and in(s), or from memory, where they are uniform over the launch (`in` null: the
+// plain sum).
+template <int MAXS, typename Out, typename Mix>
+__device__ __forceinline__ void mix_streams_by(float4 (&v)[MAXS], int S, Out&& out, Mix&& mix, float4 y) {
   float4 w[MAXS];
 #pragma unroll
   for (int t = 0; t < MAXS; ++t) {
     if (t >= S) continue;
-    const float o = out[t];
+    const float o = out(t);
     w[t] = float4{o * y.x, o * y.y, o * y.z, o * y.w};
 #pragma unroll
     for (int s = 0; s < MAXS; ++s) {
       if (s >= S) continue;
-      const float f = mix[s * S + t];
+      const float f = mix(s, t);
       w[t].x = fmaf(f, v[s].x, w[t].x); w[t].y = fmaf(f, v[s].y, w[t].y);
       w[t].z = fmaf(f, v[s].z, w[t].z); w[t].w = fmaf(f, v[s].w, w[t].w);
     }
@@ -59,15 +60,23 @@ __device__ __forceinline__ void mix_streams(float4 (&v)[MAXS], int S, const floa
     if (t < S) v[t] = w[t];
 }
 template <int MAXS>
-__device__ __forceinline__ float4 read_streams(const float4 (&v)[MAXS], int S, const float* __restrict__ in) {
+__device__ __forceinline__ void mix_streams(float4 (&v)[MAXS], int S, const float* __restrict__ out, const float* __restrict__ mix, float4 y) {
+  mix_streams_by<MAXS>(v, S, [&](int t) { return out[t]; }, [&](int s, int t) { return mix[s * S + t]; }, y);
+}
+template <int MAXS, typename In>
+__device__ __forceinline__ float4 read_streams_by(const float4 (&v)[MAXS], int S, In&& in) {
   float4 u = float4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < MAXS; ++s) {
     if (s >= S) continue;
-    const float f = in ? in[s] : 1.f;
+    const float f = in(s);
     u.x = fmaf(f, v[s].x, u.x); u.y = fmaf(f, v[s].y, u.y); u.z = fmaf(f, v[s].z, u.z); u.w = fmaf(f, v[s].w, u.w);
   }
   return u;
+}
+template <int MAXS>
+__device__ __forceinline__ float4 read_streams(const float4 (&v)[MAXS], int S, const float* __restrict__ in) {
+  return read_streams_by<MAXS>(v, S, [&](int s) { return in ? in[s] : 1.f; });
 }
 
 // With delta: x <- mixed streams + out * (scale * delta), written back.  Then u = sum in[s] x_s (kept if `u` is given) and
