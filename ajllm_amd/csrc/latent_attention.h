@@ -15,7 +15,7 @@
 // Scores, weights and sums are fp32; exponents are taken in base 2, scores multiplied by scale * log2(e).
 #pragma once
 #include "dense_kernels.h"
-#include "prefill_attention.h"  // also dma16, the fragment reads and quad_max / quad_sum
+#include "prefill_attention.h"  // also dma16 and the fragment reads
 
 namespace ajq {
 
