@@ -385,8 +385,10 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_kernel(const float* _
       vr[u] = load_raw<kStream, HD>(vbase + at);
     }
   };
-  // (four heads on fp32 rows fill the 128 registers of a 16-wave workgroup's lanes: no rows ahead there)
-  constexpr bool kAhead = !(kWaves == 16 && R == 4 && RawRow<CacheT, HD>::words == 8);
+  // (In 16-wave workgroups only where a lane's part of a row is 8 bytes: with more the waves hide the trips as it is and the rows
+  // ahead cost a little: 64 sequences, 32 heads of 64 on 8 cache heads, 900 rows: fp32 44.8 us ahead, 43.1 not, bf16 31.6 and
+  // 33.7; 16 heads of 128 on 8, bf16: 46.9 and 46.1.  And 128 registers do not hold four heads of 128 with fp32 rows ahead.)
+  constexpr bool kAhead = kWaves == 4 || RawRow<CacheT, HD>::words <= 2;
   __builtin_amdgcn_sched_barrier(0);
   if (kAhead) request(first);
   __builtin_amdgcn_sched_barrier(0);
