@@ -146,4 +146,15 @@ __device__ __forceinline__ float quad_sum(float x) {
   return __uint_as_float(s.x) + __uint_as_float(s.y);
 }
 
+// over a wave, the result in every lane: lanes l and l ^ 32 by a swap, then ^ 16, then rotations inside the rows of 16.  The order of
+// addition is that of xor steps 32, 16, .., 1, bit for bit, without their trips through the LDS crossbar.
+__device__ __forceinline__ float wave_sum(float v) {
+  typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+  uint32_t b = __float_as_uint(v);
+  u32x2v s = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  b = __float_as_uint(__uint_as_float(s.x) + __uint_as_float(s.y));
+  s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  return team_sum16(__uint_as_float(s.x) + __uint_as_float(s.y));
+}
+
 }  // namespace ajq

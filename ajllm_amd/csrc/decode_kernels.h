@@ -9,16 +9,6 @@
 
 namespace ajq {
 
-__device__ __forceinline__ float wave_sum(float v) {
-  // lanes l and l ^ 32, then ^ 16, by swaps, then rotations inside the rows of 16: as xor steps 32 ... 1, bit for bit, without the
-  // trips through the LDS crossbar
-  typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
-  uint32_t b = __float_as_uint(v);
-  u32x2v s = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-  b = __float_as_uint(__uint_as_float(s.x) + __uint_as_float(s.y));
-  s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-  return team_sum16(__uint_as_float(s.x) + __uint_as_float(s.y));
-}
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));

@@ -251,7 +251,7 @@ __global__ __launch_bounds__(64 * kWaves) void dense_in_kernel(DenseIn a) {
     constexpr int kThreads = 64 * kWaves, kKeep = 4;
     const int stride = a.Dp + 8;
     auto block_sum = [&](float v) {
-      v = wave_sum64(v);
+      v = wave_sum(v);
       __syncthreads();
       if (lane == 0) stat[wave] = v;
       __syncthreads();
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(LatentAbsorb a) {
       for (int j = 0; j < kKeep; ++j)
         if (4 * lane + 256 * j < s.rankp) square(v[j]);
       for (int i = 4 * lane + 256 * kKeep; i < s.rankp; i += 256) square(load4(lat + i));
-      const Divisor by(sqrtf(wave_sum64(ss) / (float)s.rank + s.eps));
+      const Divisor by(sqrtf(wave_sum(ss) / (float)s.rank + s.eps));
       auto put = [&](int i, const float4& u, const float4& k) {
         store4(dst + i, float4{by.divide(u.x) * k.x, by.divide(u.y) * k.y, by.divide(u.z) * k.z, by.divide(u.w) * k.w});
       };
@@ -804,7 +804,7 @@ __global__ __launch_bounds__(512) void latent_expand_kernel(LatentExpand a) {
     const float sink2 = a.sink ? a.sink[h] * kLog2eF : -INFINITY;
     const float top = fmaxf(wave_max64(mx), sink2);
     const float e = mx == -INFINITY ? 0.f : exp2f(mx - top);
-    const float total = wave_sum64(sum * e) + (a.sink ? exp2f(sink2 - top) : 0.f);
+    const float total = wave_sum(sum * e) + (a.sink ? exp2f(sink2 - top) : 0.f);
     if (lane < kLatentMaxChunks) weight[wave][lane] = mine ? e / total : 0.f;
   }
   __syncthreads();

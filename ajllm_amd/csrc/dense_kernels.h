@@ -62,8 +62,7 @@ __device__ __forceinline__ void store8(uint16_t* p, const Float8& f) {
                                            pack2_bf16(f.v[6], f.v[7])};
 }
 
-// over a wave, the result in every lane: rotations inside the rows of 16 lanes, then lane swaps
-__device__ __forceinline__ float wave_sum64(float v) { return quad_sum(team_sum16(v)); }
+// over a wave, the result in every lane (sums: wave_sum)
 __device__ __forceinline__ float wave_max64(float v) {
   v = fmaxf(v, row_ror<8>(v));
   v = fmaxf(v, row_ror<4>(v));
@@ -73,7 +72,7 @@ __device__ __forceinline__ float wave_max64(float v) {
 }
 // sum over a 256-thread workgroup, the result in every thread (`part`: four floats of LDS)
 __device__ __forceinline__ float block_sum256(float v, float* part) {
-  v = wave_sum64(v);
+  v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -399,7 +398,7 @@ __global__ __launch_bounds__(256) void matvec_kernel(const T* __restrict__ w, co
     acc = fmaf(a.z, v.z, acc);
     acc = fmaf(a.w, v.w, acc);
   }
-  acc = wave_sum64(acc);
+  acc = wave_sum(acc);
   if (lane == 0) y[(size_t)b * y_batch + (size_t)g * y_group + n] = from_f32<O>(acc);
 }
 

@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) void group_merge_kernel(GroupMerge a) {
     const float2 ml = mine ? a.heads_in[((size_t)unit * a.share + h) * a.chunks + lane] : float2{-INFINITY, 0.f};
     const float top = wave_max64(ml.x);
     const float e = ml.x == -INFINITY ? 0.f : exp2f(ml.x - top);
-    const float total = wave_sum64(ml.y * e);
+    const float total = wave_sum(ml.y * e);
     if (mine) weight[lane] = e / total;
   }
   __syncthreads();

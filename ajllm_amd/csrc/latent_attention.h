@@ -94,7 +94,7 @@ __global__ __launch_bounds__(64) void windowed_attention_kernel(WindowedAttentio
     const float m_new = fmaxf(mx, wave_max64(s));
     const float corr = mx == -INFINITY ? 0.f : exp2f(mx - m_new);
     const float w = s == -INFINITY ? 0.f : exp2f(s - m_new);
-    total = total * corr + wave_sum64(w);
+    total = total * corr + wave_sum(w);
     mx = m_new;
     weight[lane] = w;
     __syncthreads();

@@ -109,6 +109,18 @@ def test_add_norms_with_operands_left_out(cuda, width, delta, again, step, outpu
             assert (out[i] == 9.0).all()
 
 
+def test_sums_over_a_wave_start_with_lanes_32_apart(cuda):
+    """The order of addition is part of a norm's result: of 256 columns, four to a lane, 2^25 and -2^25 lie 32 lanes apart and cancel
+    before the 1 one lane on is added (in another order it is rounded away), so the mean is 1 / 256 and not 0."""
+    x = torch.zeros(1, 256)
+    x[0, 0], x[0, 128], x[0, 4] = 2.0 ** 25, -2.0 ** 25, 1.0
+    out, dx, gain = torch.empty((1, 256), device=cuda), x.to(cuda), torch.ones(256, device=cuda)
+    _ok(_lib.load_dense().ajqd_add_norms(dx.data_ptr(), None, _lib.AJQD_F32, None, None, gain.data_ptr(), None, 1e-5, 1, out.data_ptr(), None,
+                                         1, 256, 256, _lib.AJQD_F32, _st()))
+    want = -(1 / 256) / x.double().std(correction=0)
+    assert torch.allclose(out[0, 5:128].cpu().double(), want.expand(123), rtol=1e-5, atol=0)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_embedding_and_device_side_position(cuda, dtype):
     table, pos = torch.randn(19, 32).to(dtype), torch.randn(40, 32).to(dtype)
