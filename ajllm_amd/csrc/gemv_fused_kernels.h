@@ -314,7 +314,12 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   }
   const W4Consts w4c = w4_consts();
   const u32x4_t ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
-  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  // Four waves of twice the groups keep the sums of their two halves apart: added up like those of eight waves, the outputs are
+  // the same bit for bit.
+  constexpr int kHalves = kWaves == 4 ? 2 : 1;
+  static_assert(TPW % kHalves == 0, "whole groups per half");
+  f32x4_t acc[kHalves] = {};
+  auto half = [](int p) { return p * kHalves / TPW; };
   if constexpr (kValuSums) {  // the same arithmetic as dequant_gemv_body, bit for bit
 #pragma unroll
     for (int p = 0; p < TPW; ++p) {
@@ -322,7 +327,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) part = mfma16(fragment(p, j), w4_unpack(w[p][0][j], w4c), part);
 #pragma unroll
-      for (int i = 0; i < MROWS; ++i) acc[i] += sc[p] * (part[i] - zc[p] * gs[i][p]);
+      for (int i = 0; i < MROWS; ++i) acc[half(p)][i] += sc[p] * (part[i] - zc[p] * gs[i][p]);
     }
   } else if (kW4) {
 #pragma unroll
@@ -335,7 +340,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
         asum = mfma16(a, ones, asum);
       }
 #pragma unroll
-      for (int i = 0; i < (MROWS < 4 ? MROWS : 4); ++i) acc[i] += sc[p] * (part[i] - zc[p] * asum[i]);
+      for (int i = 0; i < (MROWS < 4 ? MROWS : 4); ++i) acc[half(p)][i] += sc[p] * (part[i] - zc[p] * asum[i]);
     }
   } else {
 #pragma unroll
@@ -345,28 +350,34 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
         const u32x4_t a = fragment(p, j);
         const u32x2_t lo = w8_to_bf16(w[p][j >> 1][2 * (j & 1)]);
         const u32x2_t hi = w8_to_bf16(w[p][j >> 1][2 * (j & 1) + 1]);
-        acc = mfma16(a, u32x4_t{lo.x, lo.y, hi.x, hi.y}, acc);
+        acc[half(p)] = mfma16(a, u32x4_t{lo.x, lo.y, hi.x, hi.y}, acc[half(p)]);
       }
   }
 
   // ---- the waves' partial sums meet in LDS; wave 0 adds them in wave order
-  asm volatile("" : "+v"(acc));
+#pragma unroll
+  for (int u = 0; u < kHalves; ++u) asm volatile("" : "+v"(acc[u]));
   if (!kW4) asm volatile("" : "+v"(scale_bits));
   constexpr int kLive = MROWS < 4 ? MROWS : 4;
   typedef float live_t __attribute__((ext_vector_type(kLive == 3 ? 4 : kLive)));
   live_t* redv = reinterpret_cast<live_t*>(red);
-  live_t mine;
 #pragma unroll
-  for (int i = 0; i < kLive; ++i) mine[i] = acc[i];
-  if (kc < kRowQuads) redv[wave * (16 * kRowQuads) + lane] = mine;
+  for (int u = 0; u < kHalves; ++u) {
+    live_t mine;
+#pragma unroll
+    for (int i = 0; i < kLive; ++i) mine[i] = acc[u][i];
+    if (kc < kRowQuads) redv[(wave * kHalves + u) * (16 * kRowQuads) + lane] = mine;
+  }
   __syncthreads();
   if (wave != 0 || kc >= kRowQuads) return;
-  live_t part[kWaves];
+  constexpr int kParts = kWaves * kHalves;
+  static_assert(16 * kRowQuads * kLive * kHalves <= 256, "a wave's words of the reduction");
+  live_t part[kParts];
 #pragma unroll
-  for (int u = 0; u < kWaves; ++u) part[u] = redv[u * (16 * kRowQuads) + lane];
+  for (int u = 0; u < kParts; ++u) part[u] = redv[u * (16 * kRowQuads) + lane];
   live_t sum = part[0];
 #pragma unroll
-  for (int u = 1; u < kWaves; ++u) sum += part[u];
+  for (int u = 1; u < kParts; ++u) sum += part[u];
   const int n = nt * kTileN + nl;
   float cs = 1.0f;
   if (!kW4) cs = f16_bits_to_f32(scale_bits);

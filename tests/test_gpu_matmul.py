@@ -633,6 +633,26 @@ def test_norm_from_sums_on_one_row(cuda, scheme, m, k1, d, n2):
     test_gemv_residual_then_rowscale_against_the_oracle(cuda, scheme, m, k1, d, n2)
 
 
+@pytest.mark.parametrize("scheme", ["w4", "w8"])
+@pytest.mark.parametrize("k,n", [(1024, 48), (2048, 48), (2048, 8208)])
+def test_norm_from_sums_adds_in_one_order(cuda, scheme, k, n):
+    """One row's four waves add up in the order of two rows' eight: the same bits (the rows' sums of squares are whole numbers, so
+    that the norm itself does not hang on an order)."""
+    from ajllm_amd import _lib
+
+    lib = _lib.load()
+    _, wq, meta = _quantized(scheme, n, k, 41 + k + n, cuda)
+    g = torch.Generator().manual_seed(k + n)
+    h, gain = torch.randn(2, k, generator=g).to(cuda), torch.randn(k, generator=g).to(cuda)
+    ssq = torch.randint(1, 64, (2, k // 16), generator=g).float().to(cuda)
+    fn = lib.ajq_w4a16_gemv_norm_sums if scheme == "w4" else lib.ajq_w8a16_gemv_norm_sums
+    ys = [torch.empty((m, n), device=cuda) for m in (1, 2)]
+    for m, y in zip((1, 2), ys):
+        _lib.check(fn(h.data_ptr(), ssq.data_ptr(), k // 16, gain.data_ptr(), 1e-5, m, k, wq.data_ptr(), meta.data_ptr(), n, y.data_ptr(),
+                      _lib.AJQ_OUT_F32, 0, torch.cuda.current_stream().cuda_stream), "gemv_norm_sums")
+    assert torch.equal(ys[0][0], ys[1][0])
+
+
 # (M, N, K) of the routes that cut K: every row-block height at its edges, a last column block cut short, parts of unequal length, one
 # part only; the tiles' shifted and short last row tile; and shapes beside the rules' lines
 _SPLIT_SHAPES = [(17, 2064, 14336), (32, 4096, 8320), (33, 4112, 5632), (48, 16016, 1408), (49, 8208, 3072), (64, 3088, 8192), (37, 33008, 640),
