@@ -188,24 +188,28 @@ def quantize_pack_w4(weight: torch.Tensor) -> tuple[torch.Tensor, ...]:
 _OUT_FLAGS = {torch.bfloat16: _lib.AJQ_OUT_BF16, torch.float32: _lib.AJQ_OUT_F32}
 
 
-def _matmul(w4: bool, x: torch.Tensor, k: int, wq: torch.Tensor, aux: torch.Tensor, out_dtype: torch.dtype, kernel: str) -> torch.Tensor:
+def _matmul(w4: bool, x: torch.Tensor, wq: torch.Tensor, aux: torch.Tensor, out_dtype: torch.dtype, kernel: str) -> torch.Tensor:
     """One product through the C ABI.  A decode step makes one of these per projection and token: as little Python as the
-    checks need (5 us of 15 per call with device and stream objects made anew, 9 all told without)."""
+    checks need (5 us of 15 per call with device and stream objects made anew, 9 all told without).  The kernels take a
+    matrix's extent from its packed tensors, so the rows and the W8 scales are held against those."""
     if not x.is_cuda:
         _require_cuda(x)
+    tiles, k = wq.shape[0], wq.shape[1] * (GROUP if w4 else 64)
     if x.dim() != 2 or x.shape[1] != k:
         raise ValueError(f"x must be [M, {k}], got {tuple(x.shape)}")
     if x.dtype is not torch.bfloat16:
         raise ValueError("activations must be bfloat16")
+    if not w4 and aux.numel() != tiles * TILE_N:
+        raise ValueError(f"scales must have {tiles * TILE_N} entries (rows padded to a multiple of 16)")
     flag = _OUT_FLAGS.get(out_dtype)
     if flag is None:
         raise ValueError("out_dtype must be torch.bfloat16 or torch.float32")
     if not x.is_contiguous():
         x = x.contiguous()
-    m, n16, index = x.shape[0], wq.shape[0] * TILE_N, x.device.index
+    m, n16, index = x.shape[0], tiles * TILE_N, x.device.index
     if index != torch.cuda.current_device():
         with torch.cuda.device(index):
-            return _matmul(w4, x, k, wq, aux, out_dtype, kernel)
+            return _matmul(w4, x, wq, aux, out_dtype, kernel)
     y = x.new_empty((m, n16), dtype=out_dtype)
     if m == 0:
         return y
@@ -229,7 +233,7 @@ def w4a16_matmul(
     kernel: str = "auto",
 ) -> torch.Tensor:
     """y[M, N16] = x[M, K] @ W_hat^T for private W4 tensors.  ``kernel``: auto | gemv | gemm."""
-    return _matmul(True, x, wq.shape[1] * GROUP, wq, meta, out_dtype, kernel)
+    return _matmul(True, x, wq, meta, out_dtype, kernel)
 
 
 def w8a16_matmul(
@@ -237,11 +241,7 @@ def w8a16_matmul(
     kernel: str = "auto",
 ) -> torch.Tensor:
     """y[M, N16] = x[M, K] @ W_hat^T for private W8 tensors; ``scales`` fp16 [N16]."""
-    if not x.is_cuda:
-        _require_cuda(x)
-    if scales.numel() != wq.shape[0] * TILE_N:
-        raise ValueError(f"scales must have {wq.shape[0] * TILE_N} entries (rows padded to a multiple of 16)")
-    return _matmul(False, x, wq.shape[1] * 64, wq, scales, out_dtype, kernel)
+    return _matmul(False, x, wq, scales, out_dtype, kernel)
 
 
 # --------------------------------------------------------------------------- the layer
@@ -361,11 +361,10 @@ class QuantLinear(nn.Module):
         x = inputs if inputs.dim() == 2 and inputs.shape[1] == k else inputs.reshape(-1, k)
         if x.dtype is not torch.bfloat16:
             x = x.to(torch.bfloat16)
-        w4 = self.scheme != "w8a16"
         if k % GROUP != 0:  # W8 with in_features off the kernels' 128-column grid
             x = torch.nn.functional.pad(x, (0, self.padded_in_features - k))
         kernel_out = torch.float32 if want is torch.float32 else torch.bfloat16
-        y = _matmul(w4, x, self.padded_in_features if k % GROUP else k, wq, buffers["meta"], kernel_out, "auto")
+        y = _matmul(self.scheme != "w8a16", x, wq, buffers["meta"], kernel_out, "auto")
         if y.shape[1] != self.out_features:
             y = y[:, : self.out_features]
         if kernel_out is not want:

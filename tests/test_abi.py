@@ -193,3 +193,36 @@ def test_bench_refuses_more_than_one_gpu():
     proc = subprocess.run([sys.executable, str(Path(__file__).resolve().parents[1] / "bench.py"), "--gpus", "2"],
                           capture_output=True, text=True, timeout=300)
     assert proc.returncode != 0 and "one GPU" in (proc.stderr + proc.stdout)
+
+
+@pytest.mark.parametrize("scheme,fault", [("w4a16_g128", "columns"), ("w8a16", "columns"), ("w8a16", "scales"), ("w4a16_g128", "in_features"),
+                                          ("w8a16", "in_features")])
+def test_a_layer_whose_tensors_do_not_fit_is_refused_ahead_of_the_library(monkeypatch, scheme, fault):
+    """A packed tensor of another width, W8 scales of another length or an edited in_features would have the kernels walk the weights
+    with a stride that is not theirs.  Host tensors stand in for device tensors: the library is not reached."""
+    import torch
+
+    from ajllm_amd import QuantLinear, quant
+
+    class Library:
+        def __getattr__(self, name):
+            raise AssertionError(f"{name} reached")
+
+    monkeypatch.setattr(quant, "_require_cuda", lambda *tensors: None)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: None)   # (a host tensor's device index)
+    monkeypatch.setattr(_lib, "load", lambda: Library())
+    w4 = scheme == "w4a16_g128"
+    layer = QuantLinear(256, 48, scheme)
+    layer.wq = torch.zeros((3, 2 if w4 else 4, 64, 4), dtype=torch.int32)
+    layer.meta = torch.zeros((3, 2, 16), dtype=torch.int32) if w4 else torch.zeros(48, dtype=torch.float16)
+    x = torch.zeros((2, 256), dtype=torch.bfloat16)
+    with pytest.raises(AssertionError, match="reached"):
+        layer(x)
+    if fault == "columns":
+        layer.wq = torch.zeros((3, 4 if w4 else 8, 64, 4), dtype=torch.int32)
+    elif fault == "scales":
+        layer.meta = torch.zeros(32, dtype=torch.float16)
+    else:
+        layer.in_features, x = 512, torch.zeros((2, 512), dtype=torch.bfloat16)
+    with pytest.raises(ValueError):
+        layer(x)
