@@ -1320,7 +1320,9 @@ int ajq_w4a16_matmul(const uint16_t* x, int M, int K, const uint32_t* wq, const 
                      void* workspace, size_t workspace_bytes, void* stream) {
   if (int s = check_matmul_args("ajq_w4a16_matmul", x, M, K, wq, meta, N, y, out_dtype, kGroup)) return s;
   const SplitRoute r = split_route(M, N, K, true, workspace, workspace_bytes);
-  if (r.kind == kRouteWhole) return ajq_w4a16_gemm(x, M, K, wq, meta, N, y, out_dtype, workspace, workspace_bytes, stream);
+  // (kRouteMid reads four meta words at a time, the others one)
+  if (r.kind == kRouteWhole || (r.kind == kRouteMid && !aligned16(meta)))
+    return ajq_w4a16_gemm(x, M, K, wq, meta, N, y, out_dtype, workspace, workspace_bytes, stream);
   if (int s = launch_split<true>(r, x, M, K, wq, meta, nullptr, N, y, out_dtype == AJQ_OUT_F32, workspace, (hipStream_t)stream)) return s;
   return check_launch("ajq_w4a16_matmul");
 }

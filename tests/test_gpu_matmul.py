@@ -690,6 +690,29 @@ def test_matmul_split_into_parts_of_k(cuda, scheme, m, n, k):
     assert torch.equal(run(nbytes, 0, torch.bfloat16), y32.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("scheme,m,n,k", [("w4", 40, 4096, 5632), ("w8", 40, 4096, 5632), ("w8", 100, 4096, 11008)])
+def test_matmul_takes_its_whole_route_where_factors_are_not_aligned(cuda, scheme, m, n, k):
+    """Meta words and scales may lie anywhere for the kernels that read them one by one: so for the fastest route, which reads several at
+    a time where it cuts K, and runs as the plain entry point does where they do not lie on its grid."""
+    from ajllm_amd import _lib
+
+    lib, w4 = _lib.load(), scheme == "w4"
+    w_hat, wq, meta = _quantized(scheme, n, k, 77, cuda)
+    off = torch.empty(meta.numel() + 1, dtype=meta.dtype, device=cuda)[1:].view(meta.shape)
+    off.copy_(meta)
+    x = make_activations(m, k, 5, True).to(cuda)
+    nbytes = lib.ajq_matmul_scratch_bytes(m, n, k, int(w4))
+    assert nbytes > 0
+    ws, stream = torch.empty(nbytes, dtype=torch.uint8, device=cuda), torch.cuda.current_stream().cuda_stream
+    y, whole = torch.empty((m, n), device=cuda), torch.empty((m, n), device=cuda)
+    head = lambda to: (x.data_ptr(), m, k, wq.data_ptr(), off.data_ptr(), n, to.data_ptr(), _lib.AJQ_OUT_F32)
+    _lib.check((lib.ajq_w4a16_matmul if w4 else lib.ajq_w8a16_matmul)(*head(y), ws.data_ptr(), nbytes, stream), "matmul")
+    _lib.check(lib.ajq_w4a16_gemm(*head(whole), ws.data_ptr(), nbytes, stream) if w4 else lib.ajq_w8a16_gemm(*head(whole), stream), "gemm")
+    assert torch.equal(y, whole)
+    max_abs, rel = errors(y.double().cpu(), (x.double() @ w_hat.to(cuda).double().t()).cpu())
+    assert max_abs <= 2e-3 and rel <= 1e-5, (max_abs, rel)
+
+
 def test_quant_linear_refuses_what_does_not_fit(cuda):
     """Rows of another width are refused, also where their elements would make whole rows; empty inputs and any leading sizes are taken."""
     from ajllm_amd import QuantLinear
