@@ -175,7 +175,7 @@ class DenseInArgs(ctypes.Structure):
 
     _fields_ = ([(n, c_void_p) for n in ("x", "n1", "n2", "gain1", "gain2", "w1", "w2", "y1", "gated")]
                 + [(n, c_int) for n in ("batch", "true_width", "width", "tiles1", "tiles2", "gated_ld", "act", "center", "pairs")]
-                + [("eps", c_float), ("sums", c_void_p), ("parts", c_int)])
+                + [("eps", c_float)])
 
 
 class KeyValueSplitArgs(ctypes.Structure):
@@ -217,6 +217,7 @@ DENSE_SIGNATURES: dict[str, tuple] = {
     "ajqd_windowed_prefill_supported": (c_int, [_I, _I, _I]),
     "ajqd_windowed_prefill": (c_int, [ctypes.POINTER(WindowedAttentionArgs), _P]),
     "ajqd_dense_in": (c_int, [ctypes.POINTER(DenseInArgs), _P]),
+    "ajqd_dense_in_scaled": (c_int, [ctypes.POINTER(DenseInArgs), _P, _I, _P]),
     "ajqd_dense_out": (c_int, [_P, _P, _P, _P, _P, _I, _I, _I, _P]),
     "ajqd_latent_absorb": (c_int, [_P, _I, ctypes.POINTER(LatentShape), _P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _P]),
     "ajqd_latent_decode_chunks": (c_int, [_I, _I, _I, _I, _I]),

@@ -310,23 +310,22 @@ int ajqd_windowed_prefill(const ajqd_windowed_attention_args* args, void* stream
   }
 }
 
-int ajqd_dense_in(const ajqd_dense_in_args* a, void* stream) {
+static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* sums, int parts, void* stream) {
   if (!a || (a->x ? (a->tiles1 && !a->gain1) || (a->tiles2 && !a->gain2) : (a->tiles1 && !a->n1) || (a->tiles2 && !a->n2)) ||
       (a->tiles1 && (!a->w1 || !a->y1)) || (a->tiles2 && (!a->w2 || !a->gated)))
-    return fail(AJQ_ERR_NULL, "ajqd_dense_in: null pointer argument");
+    return fail(AJQ_ERR_NULL, "%s: null pointer argument", name);
   if (a->batch < 1 || a->true_width < 1 || a->width < a->true_width || a->width % 8 || a->tiles1 < 0 || a->tiles2 < 0 ||
       a->tiles1 + a->tiles2 < 1 || (a->tiles2 && (a->gated_ld < (a->pairs ? 8 : 16) * a->tiles2 || a->gated_ld % 4)))
-    return fail(AJQ_ERR_SHAPE, "ajqd_dense_in: unsupported shape (batch=%d width=%d/%d tiles=%d+%d)", a->batch, a->true_width,
-                a->width, a->tiles1, a->tiles2);
-  if (a->act < 0 || a->act > AJQD_ACT_SQUARED_RELU) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_dense_in: unknown activation");
-  if (a->sums && (a->x || a->center || a->parts < 1)) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_dense_in: sums of squares go with scaled rows of an RMS norm");
-  if (a->x && a->batch > 4) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_dense_in: the norm prologue takes at most 4 rows");
+    return fail(AJQ_ERR_SHAPE, "%s: unsupported shape (batch=%d width=%d/%d tiles=%d+%d)", name, a->batch, a->true_width, a->width,
+                a->tiles1, a->tiles2);
+  if (a->act < 0 || a->act > AJQD_ACT_SQUARED_RELU) return fail(AJQ_ERR_UNSUPPORTED, "%s: unknown activation", name);
+  if (a->x && a->batch > 4) return fail(AJQ_ERR_UNSUPPORTED, "%s: the norm prologue takes at most 4 rows", name);
   DenseIn d;
   d.x = a->x; d.n1 = (const uint16_t*)a->n1; d.n2 = (const uint16_t*)a->n2; d.gain1 = a->gain1; d.gain2 = a->gain2;
   d.w1 = (const uint16_t*)a->w1; d.w2 = (const uint16_t*)a->w2; d.y1 = a->y1; d.gated = (uint16_t*)a->gated;
   d.batch = a->batch; d.D = a->true_width; d.Dp = a->width; d.tiles1 = a->tiles1; d.tiles2 = a->tiles2;
   d.gated_ld = a->gated_ld; d.act = a->act; d.center = a->center; d.pairs = a->pairs; d.eps = a->eps;
-  d.sums = a->sums; d.parts = a->parts;
+  d.sums = sums; d.parts = parts;
   // more than 16 sequences: two batch tiles and (from two tiles of rows on) two row tiles per workgroup
   const bool wide = a->batch > kGemvBatch;
   const int block = wide ? 2 * kGemvBatch : kGemvBatch;
@@ -334,9 +333,9 @@ int ajqd_dense_in(const ajqd_dense_in_args* a, void* stream) {
   const dim3 grid((a->tiles1 + rt - 1) / rt + (a->tiles2 + rt - 1) / rt, (a->batch + block - 1) / block);
   const int bytes = a->x ? 2 * a->batch * (a->width + 8) : 0;
   auto go = [&](auto kernel, int threads) {
-    if (int e = allow_lds(kernel, bytes, "ajqd_dense_in")) return e;
+    if (int e = allow_lds(kernel, bytes, name)) return e;
     hipLaunchKernelGGL(kernel, grid, dim3(threads), bytes, (hipStream_t)stream, d);
-    return check_launch("ajqd_dense_in");
+    return check_launch(name);
   };
   if (a->x) {
     // (rows so long that a workgroup's staging would not fit beside them run on two waves)
@@ -344,6 +343,14 @@ int ajqd_dense_in(const ajqd_dense_in_args* a, void* stream) {
     return go(dense_in_kernel<4, true, 1, 1>, 256);
   }
   return rt == 2 ? go(dense_in_kernel<4, false, 2, 2>, 256) : wide ? go(dense_in_kernel<4, false, 1, 2>, 256) : go(dense_in_kernel<4, false, 1, 1>, 256);
+}
+
+int ajqd_dense_in(const ajqd_dense_in_args* a, void* stream) { return dense_in("ajqd_dense_in", a, nullptr, 0, stream); }
+
+int ajqd_dense_in_scaled(const ajqd_dense_in_args* a, const float* sums, int parts, void* stream) {
+  if (!a || !sums) return fail(AJQ_ERR_NULL, "ajqd_dense_in_scaled: null pointer argument");
+  if (a->x || a->center || parts < 1) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_dense_in_scaled: sums of squares go with scaled rows of an RMS norm");
+  return dense_in("ajqd_dense_in_scaled", a, sums, parts, stream);
 }
 
 // How dense_out and dense_out_streams cut [width, k]: up to 128 tiles of 16 rows leave half the CUs idle, tiles of 8 rows on eight

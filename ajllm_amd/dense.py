@@ -238,5 +238,9 @@ class DenseLM(nn.Module):
             gated=gated, batch=batch, true_width=self.d_model, width=w.shape[1],
             tiles1=w1.shape[0] // 16 if w1 is not None else 0,
             tiles2=w2.shape[0] // 16 if w2 is not None else 0, gated_ld=gated_ld, act=act, center=center,
-            pairs=int(pairs), eps=eps, sums=_ptr(sums), parts=sums.shape[1] if sums is not None else 0)
-        _lib.check_dense(_lib.load_dense().ajqd_dense_in(ctypes.byref(args), _stream()), "dense_in")
+            pairs=int(pairs), eps=eps)
+        lib = _lib.load_dense()
+        if sums is None:
+            _lib.check_dense(lib.ajqd_dense_in(ctypes.byref(args), _stream()), "dense_in")
+        else:
+            _lib.check_dense(lib.ajqd_dense_in_scaled(ctypes.byref(args), _ptr(sums), sums.shape[1], _stream()), "dense_in_scaled")

@@ -107,13 +107,14 @@ typedef struct {
   void* gated;
   int32_t batch, true_width, width, tiles1, tiles2, gated_ld, act, center, pairs;
   float eps;
-  const float* sums;   /* or NULL: n1 / n2 are rows times the gain of an RMS norm, [batch, parts] their rows' sums of squares in parts */
-  int32_t parts;
 } ajqd_dense_in_args;
 /* y1 = norm1(x) w1^T (fp32), gated = act(norm2(x) w_gate^T) * (norm2(x) w_up^T) (bf16; w2 holds both in blocks of 8 rows), or
  * act(norm2(x) w2^T) with pairs = 0.  With x the norms are formed by the
  * product's own workgroups (batch <= 4); with n1 / n2 the normed bf16 rows are read.  tiles: output rows / 16. */
 int ajqd_dense_in(const ajqd_dense_in_args* args, void* stream);
+/* the same with n1 / n2 not normed yet: rows times the gain of an RMS norm (x NULL, center 0), whose factor goes to the outputs;
+ * sums [batch, parts] holds the rows' sums of squares in parts */
+int ajqd_dense_in_scaled(const ajqd_dense_in_args* args, const float* sums, int parts, void* stream);
 
 /* x += in w^T (+ again) (+ step); in [batch, k] bf16, w [width, k] bf16, x / again [batch, width], step [width] fp32 */
 int ajqd_dense_out(const void* in, const void* w, float* x, const float* again, const float* step, int batch, int k,
@@ -150,7 +151,7 @@ int ajqd_streams_norm(float* x, const float* delta, const float* scale, const fl
 /* one decode step in bf16: the same update with delta = in w^T as its epilogue, u = sum_s next[s] x_s (next NULL: plain) */
 int ajqd_dense_out_streams(const void* in, const void* w, float* x, const float* scale, const float* out, const float* mix,
                            const float* next, float* u, int streams, int batch, int k, int width, void* stream);
-/* the same, and in u's place what a following ajqd_dense_in takes with `sums`: scaled = bf16(u gain) [batch, width] and u's sums of
+/* the same, and in u's place what a following ajqd_dense_in_scaled takes: scaled = bf16(u gain) [batch, width] and u's sums of
  * squares per tile [batch, ajqd_dense_out_parts(batch, width)] */
 int ajqd_dense_out_streams_scaled(const void* in, const void* w, float* x, const float* scale, const float* out, const float* mix,
                                   const float* next, const float* gain, void* scaled, float* sums, int streams, int batch, int k, int width,

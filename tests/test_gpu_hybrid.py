@@ -794,9 +794,9 @@ def test_norm_carried_to_the_outputs(cuda, batch, width, streams):
     assert torch.equal(after, d["x"]) and torch.equal(scaled, (u * d["gain"]).bfloat16())
     assert _rel(sums.sum(1), u.double().square().sum(1)) < 1e-6
     normed = dense._add_norms(u, None, None, None, d["gain"], None, 1e-3, 0, width, torch.bfloat16)[0]
-    for i, more in enumerate((dict(n1=_p(normed)), dict(n1=_p(scaled), sums=_p(sums), parts=parts))):
-        _ok(lib.ajqd_dense_in(ctypes.byref(_lib.DenseInArgs(w1=_p(d["w2"]), y1=y[i].data_ptr(), batch=batch, true_width=width, width=width, tiles1=n // 16,
-                                                            eps=1e-3, **more)), _st()))
+    product = lambda rows, to, **more: ctypes.byref(_lib.DenseInArgs(w1=_p(d["w2"]), y1=to.data_ptr(), batch=batch, true_width=width, width=width,
+                                                                     tiles1=n // 16, eps=1e-3, n1=_p(rows), **more))
+    _ok(lib.ajqd_dense_in(product(normed, y[0]), _st()))
+    _ok(lib.ajqd_dense_in_scaled(product(scaled, y[1]), _p(sums), parts, _st()))
     assert _rel(y[1], y[0]) < 6e-3
-    assert lib.ajqd_dense_in(ctypes.byref(_lib.DenseInArgs(w1=_p(d["w2"]), y1=_p(y), batch=batch, true_width=width, width=width, tiles1=n // 16, n1=_p(scaled),
-                                                           sums=_p(sums), parts=parts, center=1, eps=1e-3)), _st()) < 0
+    assert lib.ajqd_dense_in_scaled(product(scaled, y, center=1), _p(sums), parts, _st()) < 0

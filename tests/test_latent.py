@@ -1,9 +1,12 @@
 """Dorutar on the host: the plain implementation (oracle/dorutar.py) against itself and against closed forms, the
 registry and the checkpoint reader, the packed weights, the ring cache's bookkeeping and the dense library's ABI."""
 
+import ctypes
 import json
 import math
 import re
+import shutil
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -246,6 +249,21 @@ def test_dense_library_refuses_bad_arguments_before_any_launch():
     assert lib.ajqd_latent_decode_chunks(1, 32, 512, 64, 1024) == 16 and lib.ajqd_latent_decode_chunks(1, 32, 528, 64, 1024) == 0
     dense_in = _lib.DenseInArgs(x=p, gain1=p, w1=p, y1=p, batch=5, true_width=16, width=16, tiles1=1)
     assert lib.ajqd_dense_in(ctypes.byref(dense_in), None) == -4                                # norm prologue: at most 4 rows
+    assert lib.ajqd_dense_in_scaled(ctypes.byref(dense_in), p, 1, None) == -4                   # rows that are scaled, not normed
+    assert lib.ajqd_dense_in_scaled(ctypes.byref(dense_in), None, 1, None) == -1
+
+
+@pytest.mark.skipif(shutil.which("gcc") is None, reason="needs a C compiler")
+def test_argument_structs_keep_their_layout(tmp_path):
+    """A C program passes these structs by address, so a field added to one is read past the end of what a program built with the
+    header of before hands over: sizes as they were published, the same in C and in the bindings."""
+    sizes = {"windowed_attention": 184, "dense_in": 112, "key_value_split": 136, "scan": 128, "scan_step": 136}
+    lines = "".join(f"_Static_assert(sizeof(ajqd_{n}_args) == {b}, \"{n}\");\n" for n, b in sizes.items())
+    (tmp_path / "sizes.c").write_text('#include "ajq_dense.h"\n' + lines)
+    done = subprocess.run(["gcc", "-std=c11", "-fsyntax-only", f"-I{HEADER.parent}", str(tmp_path / "sizes.c")], capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr
+    for n, b in sizes.items():
+        assert ctypes.sizeof(getattr(_lib, "".join(w.capitalize() for w in n.split("_")) + "Args")) == b, n
 
 
 def test_trace_replay_refuses_bad_steps():
