@@ -146,6 +146,14 @@ __device__ __forceinline__ float quad_sum(float x) {
   return __uint_as_float(s.x) + __uint_as_float(s.y);
 }
 
+// Between lanes that hand words to each other through their wave's own LDS.  The hardware runs a wave's LDS operations in order; for
+// the compiler they are accesses of unrelated threads, and this keeps them in order there too.  No instruction.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // over a wave, the result in every lane: lanes l and l ^ 32 by a swap, then ^ 16, then rotations inside the rows of 16.  The order of
 // addition is that of xor steps 32, 16, .., 1, bit for bit, without their trips through the LDS crossbar.
 __device__ __forceinline__ float wave_sum(float v) {

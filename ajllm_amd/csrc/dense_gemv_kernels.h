@@ -144,6 +144,7 @@ __device__ __forceinline__ void stream_rows(const uint16_t* __restrict__ w, int 
       for (int n = 0; n < RT; ++n)
 #pragma unroll
         for (int j = 0; j < kLoads; ++j) put(i, n, j, wr[buf][i][n][j]);
+    wave_lds_order();
 #pragma unroll
     for (int i = 0; i < UQ; ++i)
 #pragma unroll
@@ -154,6 +155,7 @@ __device__ __forceinline__ void stream_rows(const uint16_t* __restrict__ w, int 
 #pragma unroll
           for (int t = 0; t < BT; ++t) acc[n][t] = mfma16(f, xr[buf][i][t][s], acc[n][t]);
         }
+    wave_lds_order();  // (the next block's puts overwrite what was read here)
   };
   if (count >= UQ) load_w(0, begin);
   if (kXFirst && count >= UQ) load_x(0, begin);
@@ -200,6 +202,7 @@ __device__ __forceinline__ void stream_rows(const uint16_t* __restrict__ w, int 
           v = *reinterpret_cast<const u32x4_t*>(base + n * tile + (size_t)q * 256 + at[j]);
         put(0, n, j, v);
       }
+    wave_lds_order();
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
@@ -209,6 +212,7 @@ __device__ __forceinline__ void stream_rows(const uint16_t* __restrict__ w, int 
 #pragma unroll
         for (int n = 0; n < RT; ++n) acc[n][t] = mfma16(operand(0, n, k), v, acc[n][t]);
       }
+    wave_lds_order();
   }
   __syncthreads();
   meet<kWaves, RT, BT>(acc, reinterpret_cast<float*>(lds), wave, lane);
