@@ -1079,8 +1079,8 @@ int launch_split(const SplitRoute& r, const uint16_t* x, int M, int K, const uin
     auto kernel = dequant_gemm128_kernel<kW4, 4, false, true>;
     constexpr size_t lds = kW4 ? kG1LdsBytesW4 : kG1LdsBytesW8;
     if (int s = allow_big_lds(kernel, lds)) return s;
-    const int units = (N + kG1BN - 1) / kG1BN * r.S, tm = (M + kG1BM - 1) / kG1BM;
-    hipLaunchKernelGGL(kernel, dim3(8 * ((units + 7) / 8) * tm), dim3(512), lds, stream, x, M, K, reinterpret_cast<const u32x4_t*>(wq),
+    const int grid = gemm_split_grid((M + kG1BM - 1) / kG1BM, (N + kG1BN - 1) / kG1BN, r.S);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), lds, stream, x, M, K, reinterpret_cast<const u32x4_t*>(wq),
                        meta, scales8, reinterpret_cast<const u32x4_t*>(workspace), N, parts, 1, r.S);
   }
   if (r.S > 1) {

@@ -690,6 +690,19 @@ def test_matmul_split_into_parts_of_k(cuda, scheme, m, n, k):
     assert torch.equal(run(nbytes, 0, torch.bfloat16), y32.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("scheme,m,n,k,parts", [("w8", 257, 3440, 6016, 3), ("w4", 277, 3504, 6912, 3), ("w8", 1144, 1760, 5120, 2)])
+def test_tiles_in_parts_where_column_blocks_do_not_come_out_even(cuda, scheme, m, n, k, parts):
+    """Column blocks times parts that, dealt to the 8 XCDs in turn, would give one of them more workgroups than its CUs: the order of
+    workgroups in which every XCD takes as many."""
+    from ajllm_amd import _lib
+
+    tiles, blocks, w4 = -(-m // 128), -(-n // 128), scheme == "w4"
+    assert tiles * blocks * parts <= 256 and -(-blocks * parts // 8) * tiles > 32
+    sums = -(-(k // 128 * m * 16) // 256) * 256 if w4 else 0
+    assert _lib.load().ajq_matmul_scratch_bytes(m, n, k, int(w4)) == sums + 4 * parts * m * n
+    test_matmul_split_into_parts_of_k(cuda, scheme, m, n, k)
+
+
 @pytest.mark.parametrize("scheme,m,n,k", [("w4", 40, 4096, 5632), ("w8", 40, 4096, 5632), ("w8", 100, 4096, 11008)])
 def test_matmul_takes_its_whole_route_where_factors_are_not_aligned(cuda, scheme, m, n, k):
     """Meta words and scales may lie anywhere for the kernels that read them one by one: so for the fastest route, which reads several at
