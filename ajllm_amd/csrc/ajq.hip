@@ -1009,9 +1009,11 @@ MatmulKernel pick_matmul_kernel(int M, int N, int K, bool w4) {
 
 // ---- routes that cut K into parts and add the parts' sums in a second launch: shapes whose output is too small to fill the chip
 // and whose K is long.  They need a workspace, so only ajq_*_matmul takes them.
-//  * kRouteMid (gemm_mid_kernels.h): 17 .. 48 rows, int8 up to 64, K other than the resident form's 2048 and 4096, from 16 (int4:
-//    20) million weights on; up to 32 rows only K > 8192.  Below that the streaming kernel's one launch is the faster (3840 x 4816,
-//    32 rows, int8: 10.6 against 11.1 us; 8192 x 8192, 20 rows: 18.6 / 20.6; int4 at 64 rows, K = 14336: 21.0 / 20.1, 11008: 18.3 / 18.7);
+//  * kRouteMid (gemm_mid_kernels.h): 17 .. 48 rows, int8 up to 64 (from 24 million weights on above 48), K other than the resident
+//    form's 2048 and 4096, from 16 (int4: 20) million weights on; up to 32 rows only K > 8192.  Below that the streaming kernel's one
+//    launch is the faster (3840 x 4816, 32 rows, int8: 10.6 against 11.1 us; 8192 x 8192, 20 rows: 18.6 / 20.6; int4 at 64 rows, K =
+//    14336: 21.0 / 20.1, 11008: 18.3 / 18.7).  And not where the streaming kernel's workgroups happen to fill their round, as the two
+//    estimates of mid_is_faster say (int8, 44 rows, 2432 -> 7872: 9.3 against 11.7 us; int4, 37 rows, 3328 -> 7696: 10.8 / 11.9);
 //  * kRouteTiles (gemm128_kernels.h): where the estimate says so by a clear margin.  A k-block of a 128 x 128 tile takes 0.76 us
 //    (int8) / 0.80 (int4) whether 32 or 256 workgroups run, so 256 / tiles parts of K cost that much less: K = 14336, N = 4096, int8 /
 //    int4: 256 rows 65 -> 39 / 54 -> 42 us, 512 rows 91 -> 64 / 97 -> 70; K = 5632, N = 2048, 384 rows, int8 30 -> 19.  The other side
@@ -1025,6 +1027,22 @@ struct SplitRoute {
   int S = 1, mb = 0;
   size_t sums = 0, bytes = 0;   // int4 tiles: bytes of group sums ahead of the parts; all of the workspace
 };
+// Estimates in microseconds, fitted to 2400 random shapes within the limits above (int8 4 %, int4 2.5 % rms).  Streaming kernel: a launch, a start per
+// round of 256 workgroups, columns in groups of 128 for each of eight waves by row tiles per workgroup, the weights' bytes from HBM and,
+// per block of 32 rows, from L2.  In parts: two launches, a turn of 128 columns per team by row blocks, the weights, the parts' sums.
+// On 1000 other shapes the route without them was more than 2 % slower than the streaming kernel on 56 (by up to 20 %), with them on 15
+// (by up to 5 %, and to 3 % where both sides run the same kernel).
+bool mid_is_faster(int M, int N, int K, bool w4, int S, int mb) {
+  constexpr double kStreamTiles[2][3] = {{0.112, 0.150, 0.206}, {0.107, 0.116, 0.186}}, kTurn[2][3] = {{0.70, 0.76, 0.90}, {0.79, 0.97, 0.97}};
+  const int G = K / kGroup, tiles = w4 ? skinny_row_tiles<true>(M, N) : skinny_row_tiles<false>(M, N), mblocks = (M + 31) / 32;
+  const double weights = (double)N * K / 1e6;
+  const int rounds = ((N / kTileN + tiles - 1) / tiles * mblocks + 255) / 256, groups = (G + 7) / 8 * 8;
+  const double whole = 2.0 + rounds * ((w4 ? 1.8 : 0.73) + groups * kStreamTiles[w4][tiles / 2]) +
+                       weights * (w4 ? 0.023 + 0.019 * mblocks : 0.048 + 0.037 * mblocks);
+  const int turns = (G + S * kMidTeams - 1) / (S * kMidTeams);
+  const double parts = 6.05 + turns * kTurn[w4][mb - 2] + weights * (w4 ? 0.013 : 0.078) + (double)S * M * N / 1e6 * (w4 ? 1.82 : 1.29);
+  return parts < 0.98 * whole;
+}
 size_t group_sum_bytes(int M, int K) { return (size_t)(K / kGroup) * M * 16; }
 SplitRoute pick_split(int M, int N, int K, bool w4) {
   SplitRoute r;
@@ -1037,6 +1055,8 @@ SplitRoute pick_split(int M, int N, int K, bool w4) {
     r.mb = M <= 32 ? 2 : M <= 48 ? 3 : 4;
     const int blocks = (N + kMidColumns - 1) / kMidColumns;
     r.S = std::max(1, std::min(std::min(256 / blocks, 16), G / kMidTeams));
+    // (from 128 column blocks on the streaming kernel's workgroups never fit one round)
+    if (blocks < 128 && !mid_is_faster(M, N, K, w4, r.S, r.mb)) return SplitRoute{};
     r.kind = kRouteMid;
     r.bytes = r.S > 1 ? (size_t)r.S * M * N * 4 : 0;
     return r;

@@ -703,7 +703,7 @@ def test_tiles_in_parts_where_column_blocks_do_not_come_out_even(cuda, scheme, m
     test_matmul_split_into_parts_of_k(cuda, scheme, m, n, k)
 
 
-@pytest.mark.parametrize("scheme,m,n,k", [("w4", 40, 4096, 5632), ("w8", 40, 4096, 5632), ("w8", 100, 4096, 11008)])
+@pytest.mark.parametrize("scheme,m,n,k", [("w4", 40, 2048, 14336), ("w8", 40, 4096, 5632), ("w8", 100, 4096, 11008)])
 def test_matmul_takes_its_whole_route_where_factors_are_not_aligned(cuda, scheme, m, n, k):
     """Meta words and scales may lie anywhere for the kernels that read them one by one: so for the fastest route, which reads several at
     a time where it cuts K, and runs as the plain entry point does where they do not lie on its grid."""
