@@ -653,10 +653,34 @@ def test_norm_from_sums_adds_in_one_order(cuda, scheme, k, n):
     assert torch.equal(ys[0][0], ys[1][0])
 
 
-# (M, N, K) of the routes that cut K: every row-block height at its edges, a last column block cut short, parts of unequal length, one
-# part only; the tiles' shifted and short last row tile; and shapes beside the rules' lines
-_SPLIT_SHAPES = [(17, 2064, 14336), (32, 4096, 8320), (33, 4112, 5632), (48, 16016, 1408), (49, 8208, 3072), (64, 3088, 8192), (37, 33008, 640),
-                 (65, 4112, 8192), (128, 2576, 11008), (129, 4096, 5632), (200, 4112, 8320), (333, 2064, 5760), (384, 4096, 6144), (700, 2048, 8192)]
+# (M, N, K) of the routes that cut K, and into how many parts (int4, int8; 0: the whole-K route).  Every row-block height at its edges, a
+# last column block cut short, parts of unequal length, the tiles' shifted last row tile and, below 128 rows, their repeated last
+# row; one part (which needs no workspace, so that it counts as 0 here); and shapes beside the rules' lines.
+_SPLIT_SHAPES = {(17, 2064, 14336): (15, 15), (32, 4096, 8320): (8, 0), (32, 3088, 9088): (10, 10), (33, 4112, 5632): (7, 7), (48, 16016, 1408): (2, 2),
+                 (48, 3088, 8192): (0, 10), (49, 8208, 3072): (0, 3), (64, 3088, 8192): (0, 10), (37, 33008, 640): (0, 0), (65, 4112, 8192): (0, 0),
+                 (65, 7056, 14336): (0, 4), (65, 7680, 14336): (0, 4), (100, 4096, 11008): (0, 8), (128, 2576, 11008): (0, 12), (129, 4096, 5632): (0, 0),
+                 (163, 4560, 14336): (3, 3), (200, 4112, 8320): (0, 3), (261, 2064, 14336): (5, 5), (333, 2064, 5760): (0, 0), (333, 4096, 14336): (2, 2),
+                 (384, 4096, 6144): (2, 2), (700, 2048, 8192): (2, 2)}
+
+
+def _parts_of_k(lib, w4: bool, m: int, n: int, k: int) -> int:
+    """Parts the fastest route cuts K into: what its workspace holds beside int4 tiles' group sums (0: none beyond the plain route's)."""
+    nbytes = lib.ajq_matmul_scratch_bytes(m, n, k, int(w4))
+    if nbytes == (lib.ajq_w4a16_gemm_workspace_bytes_for(m, n, k) if w4 else 0):
+        return 0
+    if w4 and m > 64:
+        nbytes -= -(-(k // 128 * m * 16) // 256) * 256
+    assert nbytes % (4 * m * n) == 0
+    return nbytes // (4 * m * n)
+
+
+@pytest.mark.parametrize("m,n,k", _SPLIT_SHAPES)
+@pytest.mark.parametrize("scheme", ["w4", "w8"])
+def test_matmul_takes_the_route_its_shape_asks_for(cuda, scheme, m, n, k):
+    """The shapes below run on the routes they are meant for."""
+    from ajllm_amd import _lib
+
+    assert _parts_of_k(_lib.load(), scheme == "w4", m, n, k) == _SPLIT_SHAPES[m, n, k][scheme == "w8"]
 
 
 @pytest.mark.parametrize("m,n,k", _SPLIT_SHAPES)
@@ -698,8 +722,7 @@ def test_tiles_in_parts_where_column_blocks_do_not_come_out_even(cuda, scheme, m
 
     tiles, blocks, w4 = -(-m // 128), -(-n // 128), scheme == "w4"
     assert tiles * blocks * parts <= 256 and -(-blocks * parts // 8) * tiles > 32
-    sums = -(-(k // 128 * m * 16) // 256) * 256 if w4 else 0
-    assert _lib.load().ajq_matmul_scratch_bytes(m, n, k, int(w4)) == sums + 4 * parts * m * n
+    assert _parts_of_k(_lib.load(), w4, m, n, k) == parts
     test_matmul_split_into_parts_of_k(cuda, scheme, m, n, k)
 
 
