@@ -140,16 +140,44 @@ def test_quantize_and_pack_in_one_pass(cuda, n, k, odd):
     layer = QuantLinear.from_weight(w.to(cuda), "w4a16_g128")
     with np.errstate(all="ignore"):
         q, s, z = qspec.quantize_w4_g128(w.numpy())
-    if not odd:   # (the statement leaves the codes of quotients that are no number open)
-        assert np.array_equal(layer.qweight.cpu().numpy(), qspec.pack_int4(q)) and np.array_equal(layer.zeros.cpu().numpy(), z)
-    assert np.array_equal(layer.scales.cpu().numpy().view(np.uint16), s.view(np.uint16)) or odd
+    # (the statement leaves groups that hold an infinity or NaN open)
+    stated = np.isfinite(w.numpy()).reshape(n, k // 128, 128).all(2)
+    assert odd or stated.all()
+    assert np.array_equal(layer.qweight.cpu().numpy().reshape(n, k // 128, 16)[stated], qspec.pack_int4(q).reshape(n, k // 128, 16)[stated])
+    assert np.array_equal(layer.zeros.cpu().numpy()[stated], z[stated])
+    assert np.array_equal(layer.scales.cpu().numpy().view(np.uint16)[stated], s.view(np.uint16)[stated])
     wq, meta = repack_w4(layer.qweight, layer.scales, layer.zeros)
     assert torch.equal(layer.wq, wq) and torch.equal(layer.meta, meta)
     for cols in (k, k - 4):   # W8 columns need no grid
         layer = QuantLinear.from_weight(w[:, :cols].contiguous().to(cuda), "w8a16")
         with np.errstate(all="ignore"):
             q, s = qspec.quantize_w8(w[:, :cols].numpy())
-        if not odd:
-            assert np.array_equal(layer.qweight.cpu().numpy(), q) and np.array_equal(layer.scales.cpu().numpy().view(np.uint16), s.view(np.uint16))
+        stated = np.isfinite(w[:, :cols].numpy()).all(1)
+        assert np.array_equal(layer.qweight.cpu().numpy()[stated], q[stated])
+        assert np.array_equal(layer.scales.cpu().numpy().view(np.uint16)[stated], s.view(np.uint16)[stated])
         assert torch.equal(layer.wq, repack_w8(layer.qweight))
         assert torch.equal(layer.meta.view(torch.int16), _pad_rows(layer.scales, layer.wq.shape[0] * 16).view(torch.int16))
+
+
+@pytest.mark.parametrize("beside", [False, True])
+def test_quantize_w4_around_the_bound_of_the_short_quotient(cuda, beside):
+    """Groups of a small spread around a large offset: quotients up to 2^21 take three instructions, larger ones the division, one choice
+    for the rows and groups of a wavefront.  Both sides of the bound, alone and ``beside`` ordinary groups; codes, zero-points and
+    scales bit for bit."""
+    from ajllm_amd import QuantLinear
+
+    g = torch.Generator().manual_seed(5)
+    steps = torch.randint(0, 16, (16, 4, 128), generator=g).float()
+    steps[..., 0], steps[..., 1] = 0, 15
+    offsets = torch.tensor([2.0 ** 21 - 15, 2.0 ** 21 - 14.75, 2.0 ** 21 - 16, 2.0 ** 20, 2.0 ** 22, -2.0 ** 21, -2.0 ** 21 - 0.25, -2.0 ** 21 - 1])
+    w = offsets.repeat(2)[:, None, None] + steps          # a spread of 15: the scale is 1, and the bound 2^21
+    w[8:] = 3e6 * offsets[:, None, None].sign() + 0.25 * steps[8:]      # a scale of 1/4 far beyond it
+    largest = w.abs().amax(2)
+    assert (largest[:8] <= 2 ** 21).any() and (largest[:8] > 2 ** 21).any() and (largest[8:] > 2 ** 19).all()
+    if beside:
+        w[:, 1:3] = torch.randn(16, 2, 128, generator=g) * 0.02
+    w = w.reshape(16, 512)
+    layer = QuantLinear.from_weight(w.to(cuda), "w4a16_g128")
+    q, s, z = qspec.quantize_w4_g128(w.numpy())
+    assert np.array_equal(layer.qweight.cpu().numpy(), qspec.pack_int4(q)) and np.array_equal(layer.zeros.cpu().numpy(), z)
+    assert np.array_equal(layer.scales.cpu().numpy().view(np.uint16), s.view(np.uint16))
