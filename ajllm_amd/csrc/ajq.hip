@@ -1085,10 +1085,11 @@ int launch_split(const SplitRoute& r, const uint16_t* x, int M, int K, const uin
                  int N, void* y, int out_f32, void* workspace, hipStream_t stream) {
   float* parts = reinterpret_cast<float*>(static_cast<char*>(workspace) + r.sums);
   if (r.kind == kRouteMid) {
-    auto kernel = r.mb == 2 ? dequant_gemm_mid_kernel<kW4, 2> : r.mb == 3 ? dequant_gemm_mid_kernel<kW4, 3> : dequant_gemm_mid_kernel<kW4, 4>;
+    auto kernel = r.mb == 2 ? dequant_gemm_mid_kernel<kW4, 2> : dequant_gemm_mid_kernel<kW4, 3>;
+    if constexpr (!kW4)
+      if (r.mb == 4) kernel = dequant_gemm_mid_kernel<kW4, 4>;
     if (int s = allow_big_lds(kernel, mid_lds_bytes(r.mb))) return s;
-    const int units = (N + kMidColumns - 1) / kMidColumns * r.S;
-    hipLaunchKernelGGL(kernel, dim3(8 * ((units + 7) / 8)), dim3(64 * kMidWaves * kMidTeams), mid_lds_bytes(r.mb), stream, x, M, K,
+    hipLaunchKernelGGL(kernel, dim3((N + kMidColumns - 1) / kMidColumns * r.S), dim3(64 * kMidWaves * kMidTeams), mid_lds_bytes(r.mb), stream, x, M, K,
                        reinterpret_cast<const u32x4_t*>(wq), meta, scales8, N, r.S, y, out_f32, parts);
   } else {
     if (kW4) {

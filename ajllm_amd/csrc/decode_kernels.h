@@ -9,12 +9,6 @@
 
 namespace ajq {
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off));
-  return v;
-}
-
 // hidden[b, :] += delta[b, :] (when delta != nullptr; written back), then
 // out[b, :] = bf16( (hidden / sqrt(mean(hidden^2) + eps)) * gain ).
 // One 256-thread workgroup per row; D % 4 == 0.  The first 4096 elements of a row (four float4 per thread)

@@ -24,38 +24,27 @@ namespace ajq {
 
 constexpr int kGemvBatch = 16;
 
-// acc[n][t] += W[rows of row tile n, steps begin .. end) x_t; `wrow` points at this lane's row of the first tile (a tile is
-// 16 K elements further), `x(t, step)` gives the B fragment of batch tile t (batch column r, k = 32 step + 8 g ..), both
-// zero past K.  A weight fragment meets BT batch tiles, an activation fragment RT row tiles.
-template <int RT, int BT, typename XFn>
-__device__ __forceinline__ void tile_steps(const uint16_t* __restrict__ wrow, int K, int begin, int end, int g,
-                                           f32x4_t (&acc)[RT][BT], XFn&& x) {
-  constexpr int kUnroll = 8 / RT;
+// acc += W[16 rows, steps begin .. end) x; `wrow` points at this lane's row, `x(step)` gives the B fragment (batch column r, k = 32
+// step + 8 g ..), both zero past K.
+template <typename XFn>
+__device__ __forceinline__ void tile_steps(const uint16_t* __restrict__ wrow, int K, int begin, int end, int g, f32x4_t& acc, XFn&& x) {
+  constexpr int kUnroll = 8;
   const u32x4_t zero = {0u, 0u, 0u, 0u};
   for (int s0 = begin; s0 < end; s0 += kUnroll) {
-    u32x4_t w[kUnroll][RT], v[kUnroll][BT];
+    u32x4_t w[kUnroll], v[kUnroll];
 #pragma unroll
     for (int i = 0; i < kUnroll; ++i) {
       const int k = 32 * (s0 + i) + 8 * g;
-#pragma unroll
-      for (int n = 0; n < RT; ++n) {
-        w[i][n] = zero;
-        if (s0 + i < end && k < K) w[i][n] = *reinterpret_cast<const u32x4_t*>(wrow + (size_t)n * 16 * K + k);
-      }
+      w[i] = zero;
+      if (s0 + i < end && k < K) w[i] = *reinterpret_cast<const u32x4_t*>(wrow + k);
     }
 #pragma unroll
-    for (int i = 0; i < kUnroll; ++i)
+    for (int i = 0; i < kUnroll; ++i) {
+      v[i] = zero;
+      if (s0 + i < end && 32 * (s0 + i) + 8 * g < K) v[i] = x(s0 + i);
+    }
 #pragma unroll
-      for (int t = 0; t < BT; ++t) {
-        v[i][t] = zero;
-        if (s0 + i < end && 32 * (s0 + i) + 8 * g < K) v[i][t] = x(t, s0 + i);
-      }
-#pragma unroll
-    for (int i = 0; i < kUnroll; ++i)
-#pragma unroll
-      for (int n = 0; n < RT; ++n)
-#pragma unroll
-        for (int t = 0; t < BT; ++t) acc[n][t] = mfma16(w[i][n], v[i][t], acc[n][t]);
+    for (int i = 0; i < kUnroll; ++i) acc = mfma16(w[i], v[i], acc);
   }
 }
 

@@ -1,5 +1,5 @@
 // Dequant matmul of 17 to 64 rows where the activations do not stay resident in registers (skinny_resident_kernels.h: K = 2048 and
-// 4096): blocks of 16 MB rows x 128 columns, K cut into S parts.
+// 4096): one block of 16 MB rows x 128 columns, K cut into S parts.
 //
 // What it is for: dequant_skinny_kernel gives every workgroup of one to four 16-column tiles its own copy of 32 rows of activations,
 // which the L2s deliver at 14 TB/s at most, twice as many bytes as int8 weights; rows past 32 read the weights again.
@@ -38,11 +38,8 @@ __global__ __launch_bounds__(64 * kMidWaves * kMidTeams) void dequant_gemm_mid_k
   extern __shared__ __attribute__((aligned(16))) unsigned char mid_lds[];
   const int lane = threadIdx.x & 63, nl = lane & 15, kc = lane >> 4;
   const int all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wave = all % kMidWaves, team = all / kMidWaves;
-  const int ntiles = N / kTileN, nblocks = (ntiles + kMidWaves * NW - 1) / (kMidWaves * NW), mblocks = (M + kRows - 1) / kRows;
-  // the row blocks of one (column block, part of K) meet the same weights: consecutive slots of one XCD
-  const int unit = (int)(blockIdx.x & 7) + 8 * ((int)(blockIdx.x >> 3) / mblocks), m0 = (int)(blockIdx.x >> 3) % mblocks * kRows;
-  if (unit >= nblocks * S) return;
-  const int nt0 = unit / S * (kMidWaves * NW) + wave * NW, split = unit % S;
+  const int ntiles = N / kTileN;
+  const int nt0 = (int)blockIdx.x / S * (kMidWaves * NW) + wave * NW, split = (int)blockIdx.x % S;
   const int G = K / kGroup, part0 = split * kMidTeams + team, parts = S * kMidTeams;
   const int begin = (int)((long long)G * part0 / parts), count = (int)((long long)G * (part0 + 1) / parts) - begin;
   // (every team takes as many turns: the barriers are the workgroup's)
@@ -53,7 +50,7 @@ __global__ __launch_bounds__(64 * kMidWaves * kMidTeams) void dequant_gemm_mid_k
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
     const int row = 4 * (MB * wave + i) + kc;
-    x_at[i] = (uint32_t)min(m0 + row, M - 1) * (2u * K) + 16u * nl;
+    x_at[i] = (uint32_t)min(row, M - 1) * (2u * K) + 16u * nl;
     x_to[i] = (uint32_t)(row * 256 + ((nl ^ (row & 15)) << 4));
   }
   unsigned char* const slots = mid_lds + team * (2 * kGroupBytes);
@@ -165,7 +162,7 @@ __global__ __launch_bounds__(64 * kMidWaves * kMidTeams) void dequant_gemm_mid_k
     }
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
-      const int m = m0 + 16 * i + nl;
+      const int m = 16 * i + nl;
       if (m >= M) continue;
       const f32x4_t v = {acc[n][i][0] * cs[0], acc[n][i][1] * cs[1], acc[n][i][2] * cs[2], acc[n][i][3] * cs[3]};
       if (S > 1) *reinterpret_cast<f32x4_t*>(partial + ((size_t)split * M + m) * N + col) = v;

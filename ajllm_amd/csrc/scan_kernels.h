@@ -488,8 +488,8 @@ __global__ __launch_bounds__(256) void scan_step_kernel(ScanStep a) {
   }
   __syncthreads();
   if (tile) {
-    f32x4_t acc[1][1] = {};
-    auto operand = [&](int, int s) {
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    auto operand = [&](int s) {
       return r < nb ? *reinterpret_cast<const u32x4_t*>(low + r * ld + 32 * s + 8 * g) : u32x4_t{0u, 0u, 0u, 0u};
     };
 #pragma unroll
@@ -497,12 +497,12 @@ __global__ __launch_bounds__(256) void scan_step_kernel(ScanStep a) {
       if (32 * s < a.rank) {
         const u32x4_t none = {0u, 0u, 0u, 0u};
         const bool live = 32 * s + 8 * g < a.rank;
-        acc[0][0] = mfma16(live ? w[s] : none, live ? operand(0, s) : none, acc[0][0]);
+        acc = mfma16(live ? w[s] : none, live ? operand(s) : none, acc);
       }
-    tile_steps<1, 1>(wrow, a.rank, kSteps, (a.rank + 31) >> 5, g, acc, operand);
+    tile_steps(wrow, a.rank, kSteps, (a.rank + 31) >> 5, g, acc, operand);
     if (r < nb) {
-      store4(dt_s + r * 64 + 16 * wave + 4 * g, float4{softplus_f32(acc[0][0][0] + dt_bias.x), softplus_f32(acc[0][0][1] + dt_bias.y),
-                                                       softplus_f32(acc[0][0][2] + dt_bias.z), softplus_f32(acc[0][0][3] + dt_bias.w)});
+      store4(dt_s + r * 64 + 16 * wave + 4 * g, float4{softplus_f32(acc[0] + dt_bias.x), softplus_f32(acc[1] + dt_bias.y),
+                                                       softplus_f32(acc[2] + dt_bias.z), softplus_f32(acc[3] + dt_bias.w)});
     }
   }
   __syncthreads();
