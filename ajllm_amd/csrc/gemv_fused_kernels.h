@@ -19,7 +19,9 @@
 // updated residual stream, to a buffer other than the one being read.
 // What bounds these launches is the chain of round trips to memory, so no load may wait for another's value: the activations'
 // way into LDS has no branch and no select that would draw a load into itself (kProNormSums used to fetch h and the gain only
-// after the row sums had arrived: a 12-layer int4 step of width 2048 at batch 1 took 0.326 ms with that, 0.313 without).
+// after the row sums had arrived: a 12-layer int4 step of width 2048 at batch 1 took 0.326 ms with that, 0.313 without).  Several
+// rows with their sums are the exception: up to sixteen vectors of sums, the rows and the gains held at once cost more registers than the
+// trip is worth (int8, K = 1024, N = 11264, 12 rows: 12.2 us so, 9.0 with the sums dropped at the load; K = 2048, 4 rows: 7.7 / 7.2).
 #pragma once
 #include "gemv_kernels.h"
 #include "decode_kernels.h"
@@ -137,6 +139,9 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   constexpr int kLanesPerRow = 64 / MROWS;
   constexpr int kPartLoads = kPro == kProNormSums ? (64 + kLanesPerRow - 1) / kLanesPerRow : 1;  // up to 256 parts
   float4 sums[kPartLoads];
+  // what the activations need is held from its request on; several rows and their sums only where that was the faster
+  // (int8, K = 4096, N = 11264, 4 rows: 12.4 us, 14.3 without; int4 gains nothing from it)
+  constexpr bool kHeld = kPro != kProNormSums || MROWS == 1 || (!kW4 && MROWS <= 4 && kWaves * kSlice == 4096);
   if (kPro == kProNormSums) {
     const int row = lane / kLanesPerRow, piece = lane % kLanesPerRow;
 #pragma unroll
@@ -144,6 +149,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
       const int j = piece + u * kLanesPerRow;
       const bool live = 4 * j < S && row < M;  // (idle lanes re-read the first 16 bytes)
       sums[u] = *reinterpret_cast<const float4*>(src1 + (live ? (size_t)row * S + 4 * j : 0));
+      if (!kHeld) sums[u] = live ? sums[u] : float4{0.f, 0.f, 0.f, 0.f};
     }
   }
   if (kW4) {  // before the weights: scales and zero-points are there when the first tile lands
@@ -163,7 +169,8 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   constexpr int kLiveRows = MROWS < 4 ? MROWS : 4;
   float h_old[kLiveRows], gain_n = 0.f;
   uint32_t scale_bits = 0;  // (what is used at the very end goes behind the weights in issue order)
-  if (!kW4) scale_bits = scales8[nt * kTileN + nl];
+  constexpr bool kScaleAhead = !kW4 && kHeld;
+  if (kScaleAhead) scale_bits = scales8[nt * kTileN + nl];
   if (kResid) {
     gain_n = gain[nt * kTileN + nl];
 #pragma unroll
@@ -214,8 +221,8 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
 #pragma unroll
     for (int u = 0; u < kPartLoads; ++u) {
       // (the idle lanes' words are dropped here and not at the load, which would become a branch of its own)
-      asm volatile("" : "+v"(sums[u].x), "+v"(sums[u].y), "+v"(sums[u].z), "+v"(sums[u].w));
-      const bool live = 4 * (lane % kLanesPerRow + u * kLanesPerRow) < S && lane / kLanesPerRow < M;
+      if (kHeld) asm volatile("" : "+v"(sums[u].x), "+v"(sums[u].y), "+v"(sums[u].z), "+v"(sums[u].w));
+      const bool live = !kHeld || (4 * (lane % kLanesPerRow + u * kLanesPerRow) < S && lane / kLanesPerRow < M);
       total += live ? (sums[u].x + sums[u].y) + (sums[u].z + sums[u].w) : 0.f;
     }
     if (kLanesPerRow >= 16) {
@@ -284,15 +291,17 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   }
   // bf16, into the wave's own LDS rows.  Lanes past the slice write its last vector once more (the same value): a branch here
   // would draw the loads of h and gain into itself, behind the wait for the row sums.
+  constexpr bool kAllStore = kHeld;
 #pragma unroll
   for (int i = 0; i < (kPro == kProMerge ? 0 : kXLoads); ++i) {
-    const int v = min(lane + 64 * i, kVecs - 1);
+    const int v = kAllStore ? min(lane + 64 * i, kVecs - 1) : lane + 64 * i;
     u32x4_t pk;
     pk.x = pack2_bf16(xv[i][0], xv[i][1]);
     pk.y = pack2_bf16(xv[i][2], xv[i][3]);
     pk.z = pack2_bf16(xv[i][4], xv[i][5]);
     pk.w = pack2_bf16(xv[i][6], xv[i][7]);
-    *reinterpret_cast<u32x4_t*>(xs + (v / kVecPerRow) * kStride + 8 * (v % kVecPerRow)) = pk;
+    if (kAllStore || (i + 1) * 64 <= kVecs || v < kVecs)
+      *reinterpret_cast<u32x4_t*>(xs + (v / kVecPerRow) * kStride + 8 * (v % kVecPerRow)) = pk;
   }
 
   // ---- the matmul, as in dequant_gemv_kernel.  What depends on the activations alone comes first, while the
@@ -357,7 +366,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   // ---- the waves' partial sums meet in LDS; wave 0 adds them in wave order
 #pragma unroll
   for (int u = 0; u < kHalves; ++u) asm volatile("" : "+v"(acc[u]));
-  if (!kW4) asm volatile("" : "+v"(scale_bits));
+  if (kScaleAhead) asm volatile("" : "+v"(scale_bits));
   constexpr int kLive = MROWS < 4 ? MROWS : 4;
   typedef float live_t __attribute__((ext_vector_type(kLive == 3 ? 4 : kLive)));
   live_t* redv = reinterpret_cast<live_t*>(red);
@@ -380,7 +389,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   for (int u = 1; u < kParts; ++u) sum += part[u];
   const int n = nt * kTileN + nl;
   float cs = 1.0f;
-  if (!kW4) cs = f16_bits_to_f32(scale_bits);
+  if (!kW4) cs = f16_bits_to_f32(kScaleAhead ? scale_bits : (uint32_t)scales8[n]);
   if (kResid) {
     const int ntiles = N / kTileN;
 #pragma unroll
