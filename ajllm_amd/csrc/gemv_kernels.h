@@ -256,14 +256,16 @@ __device__ __forceinline__ void dequant_gemv_body(
   // the end.  The scales only where that batch is the only one (int8, one row, 2048 -> 2048: 2.95 us, 2.99 with them fetched behind
   // the barrier; 5 rows, 4096 -> 14336: 12.4 and 13.0).  In the loop they are one more word among the batches' waits and cost more
   // than the trip they save (9 rows, 3840 -> 4816: 9.3 us, 8.9 without; 3 rows, 11008 -> 4096: 11.0 and 10.8; one, 1024 -> 4096: 3.36
-  // and 3.25).
+  // and 3.25), and so they do beside the row sums (16 rows, 2048 -> 4096: 5.19 and 4.74) or the old residuals of several rows (5
+  // rows, 4096 -> 19664: 18.3 and 17.0) and in workgroups of eleven waves (one row, 5632 -> 18096: 19.3 and 17.4).
   constexpr int kLiveRows = MROWS < 4 ? MROWS : 4;
   float* red2 = red + kWaves * 64 * 4;  // [16][kWaves] shares of the rows' sums of squares
   float4 ssq_share[2];
   float h_old[kLiveRows], gain_n = 0.f;
   uint32_t scale_bits = 0;
+  constexpr bool kScaleAhead = !kW4 && kSingle && kWaves <= 8 && !(kEpi & kEpiRowScale) && (MROWS == 1 || !(kEpi & kEpiResidual));
   auto epilogue_loads = [&]() {
-    if (!kW4 && kSingle) scale_bits = scales8[nt * kTileN + nl];
+    if (kScaleAhead) scale_bits = scales8[nt * kTileN + nl];
     if (kEpi & kEpiRowScale) {
       const int m = lane & 15, c = lane >> 4;
 #pragma unroll
@@ -317,7 +319,7 @@ __device__ __forceinline__ void dequant_gemv_body(
   // (the empty asm pins the accumulator here: otherwise the compiler sinks the
   // epilogue arithmetic, and the loads that feed it, into the conditional store)
   asm volatile("" : "+v"(acc));
-  if (!kW4 && kSingle) asm volatile("" : "+v"(scale_bits));  // (and its load would follow it, a round trip to memory behind the barrier)
+  if (kScaleAhead) asm volatile("" : "+v"(scale_bits));  // (and its load would follow it, a round trip to memory behind the barrier)
   constexpr int kLive = MROWS < 4 ? MROWS : 4;  // accumulator components that hold rows < MROWS
   typedef float live_t __attribute__((ext_vector_type(kLive == 3 ? 4 : kLive)));
   live_t* redv = reinterpret_cast<live_t*>(red);
@@ -342,7 +344,7 @@ __device__ __forceinline__ void dequant_gemv_body(
   for (int w = 1; w < kWaves; ++w) sum += part[w];
   const int n = nt * kTileN + nl;
   float cs = 1.0f;
-  if (!kW4) cs = f16_bits_to_f32(kSingle ? scale_bits : (uint32_t)scales8[n]);  // per-output-channel scale, once
+  if (!kW4) cs = f16_bits_to_f32(kScaleAhead ? scale_bits : (uint32_t)scales8[n]);  // per-output-channel scale, once
   float rstd[kLive];
 #pragma unroll
   for (int i = 0; i < kLive; ++i) {
