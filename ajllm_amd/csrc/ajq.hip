@@ -204,7 +204,9 @@ static int quantize_w8(const char* name, const float* W, int N, int K, int8_t* q
     return fail(AJQ_ERR_SHAPE, "%s: need N >= 1 and K a positive multiple of 4 (got N=%d, K=%d)", name, N, K);
   if (!aligned16(W) || (reinterpret_cast<uintptr_t>(q) & 3u) || (reinterpret_cast<uintptr_t>(wq) & 3u))
     return fail(AJQ_ERR_ALIGN, "%s: W must be 16-byte, q and wq 4-byte aligned", name);
-  if (K > kQuantizeW8RowMaxK) {
+  // (canonical codes of short rows: nothing to gain from a row held in registers; 14336 x 128: 12.4 us with that, 10.8
+  // without, 500 x 1024: 3.0 / 2.8, but 2048 x 1024: 4.2 / 4.7)
+  if (K > kQuantizeW8RowMaxK || (!wq && (K <= 256 || (K <= 1024 && N <= 1024)))) {
     if (wq) return fail(AJQ_ERR_UNSUPPORTED, "%s: K=%d is above %d (quantize and repack one after the other)", name, K, kQuantizeW8RowMaxK);
     hipLaunchKernelGGL(quantize_w8_kernel, dim3(N), dim3(256), 0, st, W, K, q, scales);
     return check_launch(name);
@@ -234,11 +236,15 @@ static int quantize_w4(const char* name, const float* W, int N, int K, int32_t* 
     return fail(AJQ_ERR_SHAPE, "%s: need N >= 1 and K a positive multiple of 128 (got N=%d, K=%d)", name, N, K);
   if (!aligned16(W) || !aligned16(wq)) return fail(AJQ_ERR_ALIGN, "%s: W and wq must be 16-byte aligned", name);
   const int G = K / kGroup;
-  const long long tiles = (N + kTileN - 1) / kTileN;
-  const long long blocks = tiles * ((G + kQuantizeGroups - 1) / kQuantizeGroups);
+  const long long groups = (long long)N * G, tiles = (N + kTileN - 1) / kTileN;
+  const long long blocks = wq ? tiles * ((G + kQuantizeGroups - 1) / kQuantizeGroups) : (groups + 15) / 16;
   if (blocks > 0x7FFFFFFFLL) return fail(AJQ_ERR_SHAPE, "%s: too many groups", name);
-  hipLaunchKernelGGL(quantize_w4_kernel, dim3((unsigned)blocks), dim3(256), 0, st, W, N, G, reinterpret_cast<uint32_t*>(qweight),
-                     scales, zeros, reinterpret_cast<u32x4_t*>(wq), meta);
+  if (wq)
+    hipLaunchKernelGGL(quantize_w4_kernel, dim3((unsigned)blocks), dim3(256), 0, st, W, N, G, reinterpret_cast<uint32_t*>(qweight),
+                       scales, zeros, reinterpret_cast<u32x4_t*>(wq), meta);
+  else
+    hipLaunchKernelGGL(quantize_w4_codes_kernel, dim3((unsigned)blocks), dim3(256), 0, st, W, groups, reinterpret_cast<uint32_t*>(qweight),
+                       scales, zeros);
   return check_launch(name);
 }
 
