@@ -310,6 +310,7 @@ int ajqd_windowed_prefill(const ajqd_windowed_attention_args* args, void* stream
   }
 }
 
+constexpr int kTwoWaveColumns = 256;  // products of one or two blocks of columns run on two waves (stream_rows)
 static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* sums, int parts, void* stream) {
   if (!a || (a->x ? (a->tiles1 && !a->gain1) || (a->tiles2 && !a->gain2) : (a->tiles1 && !a->n1) || (a->tiles2 && !a->n2)) ||
       (a->tiles1 && (!a->w1 || !a->y1)) || (a->tiles2 && (!a->w2 || !a->gated)))
@@ -329,7 +330,8 @@ static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* 
   // more than 16 sequences: two batch tiles and (from two tiles of rows on) two row tiles per workgroup
   const bool wide = a->batch > kGemvBatch;
   const int block = wide ? 2 * kGemvBatch : kGemvBatch;
-  const int rt = wide && a->tiles1 != 1 && a->tiles2 != 1 ? 2 : 1;
+  const bool few = a->width <= kTwoWaveColumns;
+  const int rt = wide && !few && a->tiles1 != 1 && a->tiles2 != 1 ? 2 : 1;
   const dim3 grid((a->tiles1 + rt - 1) / rt + (a->tiles2 + rt - 1) / rt, (a->batch + block - 1) / block);
   const int bytes = a->x ? 2 * a->batch * (a->width + 8) : 0;
   auto go = [&](auto kernel, int threads) {
@@ -339,9 +341,13 @@ static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* 
   };
   if (a->x) {
     // (rows so long that a workgroup's staging would not fit beside them run on two waves)
-    if (bytes > 140 * 1024) return go(dense_in_kernel<2, true, 1, 1>, 128);
+    // (and rows of more than 4096 columns on eight, whose registers hold them between the norm's passes: 8192 columns, 4 rows, 0 + 13648: 59.9
+    // us on eight waves of the half-line form before, 96.7 on four of this one; 2016 + 6912: 43.7, 70.9, and 46.6 on eight)
+    if (bytes > 140 * 1024 || few) return go(dense_in_kernel<2, true, 1, 1>, 128);
+    if (a->width > 4096 && bytes <= 120 * 1024) return go(dense_in_kernel<8, true, 1, 1>, 512);
     return go(dense_in_kernel<4, true, 1, 1>, 256);
   }
+  if (few) return wide ? go(dense_in_kernel<2, false, 1, 2>, 128) : go(dense_in_kernel<2, false, 1, 1>, 128);
   return rt == 2 ? go(dense_in_kernel<4, false, 2, 2>, 256) : wide ? go(dense_in_kernel<4, false, 1, 2>, 256) : go(dense_in_kernel<4, false, 1, 1>, 256);
 }
 
@@ -354,21 +360,25 @@ int ajqd_dense_in_scaled(const ajqd_dense_in_args* a, const float* sums, int par
 }
 
 // How dense_out and dense_out_streams cut [width, k]: up to 128 tiles of 16 rows leave half the CUs idle, tiles of 8 rows on eight
-// waves use them all (2048 x 8192: 9.4 -> 7.9 us at 4 sequences, 19.1 -> 17.9 at 32).  More than 16 sequences read each weight
+// waves use them all (2048 x 8192: 9.4 -> 7.9 us at 4 sequences, 19.1 -> 17.9 at 32), where K gives each of them a block (1024 x 512: 3.0 us
+// with them, 2.5 without).  More than 16 sequences read each weight
 // fragment twice: from 512 tiles on two row tiles per workgroup share the activations (35424 x 4096: 84 -> 65 us), below that a
-// workgroup has two blocks in flight instead (4096 x 18432: 44.2 -> 42.6).
+// workgroup has two blocks in flight instead (4096 x 18432: 44.2 -> 42.6) where K gives each wave several (5120 x 256, 64 sequences: 9.1 us
+// with two, 5.1 with one).  K of one or two blocks: two waves (32000 x 128, one sequence: 5.2 us on four, 4.4 on two).
 struct OutCut {
   int rows, rt, bt;
   dim3 grid;
   int threads;
 };
-OutCut out_cut(int batch, int width) {
+OutCut out_cut(int batch, int width, int k, bool sums) {
   OutCut c;
   c.bt = batch > kGemvBatch ? 2 : 1;
-  c.rows = width / 16 <= 128 ? 8 : 16;
+  const int blocks = (batch + kGemvBatch * c.bt - 1) / (kGemvBatch * c.bt);
+  c.rows = (long long)(width / 16) * blocks <= 128 && (sums || k >= 1024) ? 8 : 16;
+  const bool few = c.rows == 16 && c.bt == 1 && k <= kTwoWaveColumns;
   c.rt = c.bt == 2 && width >= 8192 && width % 32 == 0 ? 2 : 1;
-  c.grid = dim3(width / (c.rows * c.rt), (batch + kGemvBatch * c.bt - 1) / (kGemvBatch * c.bt));
-  c.threads = c.rows == 8 ? 512 : 256;
+  c.grid = dim3(width / (c.rows * c.rt), blocks);
+  c.threads = c.rows == 8 ? 512 : few ? 128 : 256;
   return c;
 }
 
@@ -378,13 +388,16 @@ int ajqd_dense_out(const void* in, const void* w, float* x, const float* again, 
   if (batch < 1 || k < 8 || k % 8 || width < 16 || width % 16)
     return fail(AJQ_ERR_SHAPE, "ajqd_dense_out: unsupported shape (batch=%d k=%d width=%d)", batch, k, width);
   DenseOut d{(const uint16_t*)in, (const uint16_t*)w, x, again, step, batch, k, width};
-  const OutCut c = out_cut(batch, width);
+  const OutCut c = out_cut(batch, width, k, false);
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, c.grid, dim3(c.threads), 0, (hipStream_t)stream, d);
     return check_launch("ajqd_dense_out");
   };
   if (c.rows == 8) return c.bt == 2 ? go(dense_out_kernel<8, 8, 1, 2, 1>) : go(dense_out_kernel<8, 8, 1, 1, 1>);
-  return c.rt == 2 ? go(dense_out_kernel<4, 16, 2, 2, 1>) : c.bt == 2 ? go(dense_out_kernel<4, 16, 1, 2, 2>) : go(dense_out_kernel<4, 16, 1, 1, 1>);
+  if (c.threads == 128) return go(dense_out_kernel<2, 16, 1, 1, 1>);
+  if (c.rt == 2) return go(dense_out_kernel<4, 16, 2, 2, 1>);
+  if (c.bt == 2) return k < 2048 ? go(dense_out_kernel<4, 16, 1, 2, 1>) : go(dense_out_kernel<4, 16, 1, 2, 2>);
+  return go(dense_out_kernel<4, 16, 1, 1, 1>);
 }
 
 int ajqd_latent_absorb(const float* y, int ldy, const ajqd_latent_shape* shape, const void* ukt, const float* latent_gain,
@@ -526,7 +539,7 @@ static int dense_out_streams(const char* name, DenseOutStreams d, void* stream) 
   if (int e = check_streams(streams, name)) return e;
   if (batch < 1 || k < 8 || k % 8 || width < 16 || width % 16)
     return fail(AJQ_ERR_SHAPE, "%s: unsupported shape (batch=%d k=%d width=%d)", name, batch, k, width);
-  const OutCut c = out_cut(batch, width);
+  const OutCut c = out_cut(batch, width, k, !d.u);
   auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, c.grid, dim3(c.threads), 0, (hipStream_t)stream, d);
     return check_launch(name);
@@ -534,8 +547,10 @@ static int dense_out_streams(const char* name, DenseOutStreams d, void* stream) 
   auto pick = [&](auto room) {
     constexpr int M = decltype(room)::value;
     if (c.rows == 8) return c.bt == 2 ? go(dense_out_streams_kernel<8, 8, 1, 2, 1, M>) : go(dense_out_streams_kernel<8, 8, 1, 1, 1, M>);
-    return c.rt == 2 ? go(dense_out_streams_kernel<4, 16, 2, 2, 1, M>) : c.bt == 2 ? go(dense_out_streams_kernel<4, 16, 1, 2, 2, M>)
-                                                                                  : go(dense_out_streams_kernel<4, 16, 1, 1, 1, M>);
+    if (c.threads == 128) return go(dense_out_streams_kernel<2, 16, 1, 1, 1, M>);
+    if (c.rt == 2) return go(dense_out_streams_kernel<4, 16, 2, 2, 1, M>);
+    if (c.bt == 2) return k < 2048 ? go(dense_out_streams_kernel<4, 16, 1, 2, 1, M>) : go(dense_out_streams_kernel<4, 16, 1, 2, 2, M>);
+    return go(dense_out_streams_kernel<4, 16, 1, 1, 1, M>);
   };
   switch (stream_room(streams)) {
     case 2: return pick(std::integral_constant<int, 2>{});
@@ -551,7 +566,7 @@ int ajqd_dense_out_streams(const void* in, const void* w, float* x, const float*
                                                                      nullptr, nullptr, batch, k, width, streams}, stream);
 }
 
-int ajqd_dense_out_parts(int batch, int width) { return batch < 1 || width < 16 || width % 16 ? 0 : width / out_cut(batch, width).rows; }
+int ajqd_dense_out_parts(int batch, int width) { return batch < 1 || width < 16 || width % 16 ? 0 : width / out_cut(batch, width, kTwoWaveColumns, true).rows; }
 
 int ajqd_dense_out_streams_scaled(const void* in, const void* w, float* x, const float* scale, const float* out, const float* mix,
                                   const float* next, const float* gain, void* scaled, float* sums, int streams, int batch, int k, int width,

@@ -773,6 +773,25 @@ def test_streamed_products(cuda, batch, k, width):
         assert _rel(y, normed.double() @ w.double().T) < 1e-3   # (a norm rounded the other way moves an operand by 2^-8)
 
 
+@pytest.mark.parametrize("batch,k,width", [(1, 8, 48), (17, 24, 64), (2, 256, 2064), (16, 264, 2064), (33, 1000, 2064), (40, 1032, 48), (48, 1016, 16),
+                                           (64, 256, 5120), (33, 2056, 1040), (17, 72, 8224)])
+def test_streamed_products_of_short_rows(cuda, batch, k, width):
+    """The same where K is less than one block, one or two (two wavefronts), or ends inside a block with several batch tiles, on one and
+    two blocks of sequences."""
+    test_streamed_products(cuda, batch, k, width)
+
+
+@pytest.mark.parametrize("batch,k", [(4, 256), (3, 264), (2, 4096), (4, 4104), (4, 8192), (3, 8200), (4, 15432), (4, 17928)])
+def test_norm_prologue_on_two_four_and_eight_waves(cuda, batch, k):
+    """dense_in with the norm inside, at the row lengths where its workgroups change; an operand rounded the other way moves by 2^-8."""
+    g, n = torch.Generator().manual_seed(k + batch), 48
+    rows, gain, w = torch.randn((batch, k), generator=g), torch.randn(k, generator=g), _bf(g, n, k, std=k ** -0.5)
+    y, dr, dg, dw = torch.empty((batch, n), device=cuda), rows.to(cuda), gain.to(cuda), w.to(cuda)
+    _ok(_lib.load_dense().ajqd_dense_in(ctypes.byref(_lib.DenseInArgs(x=_p(dr), gain1=_p(dg), w1=_p(dw), y1=_p(y), batch=batch, true_width=k, width=k,
+                                                                      tiles1=n // 16, eps=1e-3)), _st()))
+    assert _rel(y, O.centered_rms_norm(rows, gain - 1, 1e-3).bfloat16().double() @ w.double().T) < 1e-3
+
+
 @pytest.mark.parametrize("batch", [1, 5, 16, 17, 33])
 @pytest.mark.parametrize("width,streams", [(48, 1), (2048, 2), (2064, 3)])
 def test_norm_carried_to_the_outputs(cuda, batch, width, streams):
