@@ -552,8 +552,10 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(LatentAbsorb a) {
   const uint16_t* wrow = a.ukt + ((size_t)h * s.rankp + 16 * tile + r) * s.dimp;
   const float* xr = a.y + (size_t)(b0 + min(r, nb - 1)) * a.ldy + h * dq;  // (columns past the batch repeat the last one, and are not stored)
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  constexpr int kSteps = 4;
-  for (int k0 = 8 * g; k0 < s.dimp + 8 * g; k0 += 32 * kSteps) {
+  // (as many steps together as a head has, at most four: repeated ones cost their loads, 5.6 us instead of 3.5 at 48 sequences, 20
+  // heads of 32 columns, latents of 512)
+  auto steps = [&](auto together, int k0) {
+    constexpr int kSteps = decltype(together)::value;
     u32x4_t w[kSteps];
     float4 u[kSteps], v[kSteps];
 #pragma unroll
@@ -570,6 +572,13 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(LatentAbsorb a) {
       const bool live = k0 + 32 * i < s.dimp;
       acc = mfma16(live ? w[i] : none, live ? x : none, acc);
     }
+  };
+  if (s.dimp <= 32) {
+    steps(std::integral_constant<int, 1>{}, 8 * g);
+  } else if (s.dimp <= 64) {
+    steps(std::integral_constant<int, 2>{}, 8 * g);
+  } else {
+    for (int k0 = 8 * g; k0 < s.dimp + 8 * g; k0 += 128) steps(std::integral_constant<int, 4>{}, k0);
   }
   if (r < nb)
     store4(a.q + ((size_t)(b0 + r) * s.heads + h) * width + 16 * tile + 4 * g, float4{acc[0], acc[1], acc[2], acc[3]});
