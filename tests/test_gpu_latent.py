@@ -325,6 +325,7 @@ def test_latent_decode_and_expand_against_plain(cuda, shape):
     (8, 32, 512, 64, 128, 100, 99),     # a workgroup per head and sequence
     (33, 16, 512, 64, 128, 70, 65),     # four sequences per workgroup, the last block with one; one head tile
     (17, 32, 128, 64, 128, 300, 290),   # two sequences per workgroup, an odd count; head tiles alone or in pairs by the chunks
+    (5, 6, 512, 16, 128, 70, 69),       # two value tiles and two sequences per workgroup, with many chunks a head and a sequence
 ])
 def test_cuts_of_latent_decode_and_expand(cuda, shape):
     """The splits of work that the shapes above do not reach, against the same oracle."""
