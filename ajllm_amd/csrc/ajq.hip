@@ -868,6 +868,7 @@ int launch_gemv_pro(int M, int K, const uint32_t* wq, const uint32_t* meta, cons
   // One row with its norm from the sums: four waves of twice the groups.  Every wave forms the norm's divisor for itself, and with
   // eight a launch of many workgroups is bounded by that arithmetic (int4, K = 2048, N = 6144 / 11264 / 32000: 3.87 / 4.93 / 9.24 us
   // with eight waves, 3.67 / 4.57 / 8.19 with four; K = 1024, N = 11264: 4.18 / 3.59; int8, K = 2048, N = 11264: 6.25 / 6.12).
+  // K = 4096 has eight: a quarter of its columns is more than one load per lane, and that form is not built.
   if constexpr (kPro == kProNormSums) {
     if (M <= 1 && K == 1024) AJQ_PRO(4, 2, 1);
     if (M <= 1 && K == 2048) AJQ_PRO(4, 4, 1);
@@ -985,11 +986,16 @@ int check_pro(const char* name, int M, int K, const void* a, const void* b) {
   return AJQ_OK;
 }
 
-// Which kernel runs a matmul of M >= 17 rows.  All three times are modelled from measurements
-// at K = 4096 (microseconds per k-block of 128 and round of 256 workgroups, one workgroup per CU).
-//  * 256 x 128 tiles: about 1.8 us.
-//  * 128 x 128 tiles (M >= 128): about 1.25 us (W4) / 1.15 us (W8): they win where the big tiles
-//    leave CUs idle (M = 1024 on N = 4096 is 128 big tiles or 256 small ones).
+// Which kernel runs a matmul of M >= 17 rows.  All three times are estimated, in microseconds per k-block of 128 and round of 256
+// workgroups, one workgroup per CU; the weights below settle the choice and are not the kernels' times.  Those (25 shapes of 333 to
+// 5328 rows, both schemes, graph replays) depend on how full the rounds are:
+//  * 256 x 128 tiles, weight 1.8: 1.6 to 2.0 (W4) / 1.6 to 1.8 (W8) in full rounds, down to 1.4 / 1.15 with half of the last one empty.
+//  * 128 x 128 tiles (M >= 128), weight 1.25 (W4) / 1.15 (W8): 0.9 to 1.1 in full rounds, 0.75 to 0.85 with half of one empty, 1.4 from
+//    thirty rounds on.  They win where the big tiles leave CUs idle (M = 1024 on N = 4096 is 128 big tiles or 256 small ones: 51 /
+//    39 us W4, 45 / 36 W8).
+// So the estimate is wrong where the big tiles' second round is nearly empty: W8, 4096 -> 14336, 640 rows 99.0 us against 85.3 with the
+// other kernel; 4096 -> 6144, 1500 rows 94.6 / 77.7; W4, 4096 -> 28672, 333 rows 109.5 / 101.2.  On 42 of the 50 the choice is
+// the faster kernel or within 3 % of it.
 //  * the weight-streaming kernel sustains about 400 TFLOP/s for M >= 256 and is the only one below
 //    M = 128.
 #ifndef AJQ_GEMM_TILE
@@ -1021,7 +1027,7 @@ MatmulKernel pick_matmul_kernel(int M, int N, int K, bool w4) {
 //    14336: 21.0 / 20.1, 11008: 18.3 / 18.7).  And not where the streaming kernel's workgroups happen to fill their round, as the two
 //    estimates of mid_is_faster say (int8, 44 rows, 2432 -> 7872: 9.3 against 11.7 us; int4, 37 rows, 3328 -> 7696: 10.8 / 11.9);
 //  * kRouteTiles (gemm128_kernels.h): where the estimate says so by a clear margin.  A k-block of a 128 x 128 tile takes 0.76 us
-//    (int8) / 0.80 (int4) whether 32 or 256 workgroups run, so 256 / tiles parts of K cost that much less: K = 14336, N = 4096, int8 /
+//    (int8) / 0.80 (int4) in this estimate, whether 32 or 256 workgroups run, so 256 / tiles parts of K cost that much less: K = 14336, N = 4096, int8 /
 //    int4: 256 rows 65 -> 39 / 54 -> 42 us, 512 rows 91 -> 64 / 97 -> 70; K = 5632, N = 2048, 384 rows, int8 30 -> 19.  The other side
 //    of the estimate: the streaming kernel at 420 (int8) / 440 TFLOP/s up to 128 rows and 470 above, whole 128- and 256-row tiles
 //    by rounds.  K = 2048 and 4096 stay with the resident form up to 256 rows (int4: 512: 27.3 us against 30.2), int4 below 160
