@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   constexpr int kLiveRows = MROWS < 4 ? MROWS : 4;
   float h_old[kLiveRows], gain_n = 0.f;
   uint32_t scale_bits = 0;  // (what is used at the very end goes behind the weights in issue order)
-  constexpr bool kScaleAhead = !kW4 && kHeld;
+  constexpr bool kScaleAhead = !kW4 && kHeld && (kPro != kProMerge || MROWS == 1);
   if (kScaleAhead) scale_bits = scales8[nt * kTileN + nl];
   if (kResid) {
     gain_n = gain[nt * kTileN + nl];
@@ -259,13 +259,25 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
     // 8 dimensions 8c .. 8c + 7; maxima, denominators and sums meet across the quarters, quarter 0
     // normalises and stages the 8 activations
     const int sgrp = lane >> 4, c = lane & 15;
+    // One row: swaps of lane halves, the quicker way to a result.  Several rows of several heads keep the vector units busy with them and go
+    // through the LDS crossbar beside those (4 rows, 2048 -> 6144: 14.6 us, 16.3 with swaps; the same sums).
+    constexpr bool kSwaps = MROWS == 1;
+    auto crossbar_max = [](float v) {
+      v = fmaxf(v, __shfl_xor(v, 16));
+      return fmaxf(v, __shfl_xor(v, 32));
+    };
+    auto over_quarters = [](float v) {
+      if (kSwaps) return quad_sum(v);
+      v += __shfl_xor(v, 16);
+      return v + __shfl_xor(v, 32);
+    };
 #pragma unroll
     for (int q = 0; q < kPairs; ++q) {
       float mloc = -INFINITY;
 #pragma unroll
       for (int j = 0; j < kCpl; ++j)
         if (sgrp + 4 * j < S) mloc = fmaxf(mloc, pm[q][j].x);
-      const float mall = quad_max(mloc);
+      const float mall = kSwaps ? quad_max(mloc) : crossbar_max(mloc);
       float L = 0.f, A[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < kCpl; ++j) {
@@ -276,9 +288,9 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
           A[4] += pa[q][j][1].x * cw; A[5] += pa[q][j][1].y * cw; A[6] += pa[q][j][1].z * cw; A[7] += pa[q][j][1].w * cw;
         }
       }
-      L = quad_sum(L);
+      L = over_quarters(L);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) A[e] = quad_sum(A[e]);
+      for (int e = 0; e < 8; ++e) A[e] = over_quarters(A[e]);
       if (sgrp == 0) {
         u32x4_t pk;
         pk.x = pack2_bf16(A[0] / L, A[1] / L);
