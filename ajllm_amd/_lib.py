@@ -178,6 +178,13 @@ class DenseInArgs(ctypes.Structure):
                 + [("eps", c_float)])
 
 
+class ProductArgs(ctypes.Structure):
+    """``ajqd_product_args``"""
+
+    _fields_ = ([(n, c_void_p) for n in ("x", "w", "y")]
+                + [(n, c_int) for n in ("rows", "n", "k", "ldx", "ldy", "out_dtype", "act", "pairs")])
+
+
 class KeyValueSplitArgs(ctypes.Structure):
     """``ajqd_key_value_split_args``"""
 
@@ -212,6 +219,8 @@ DENSE_SIGNATURES: dict[str, tuple] = {
                                   _I, _P, _L, _P, _I, _P]),
     "ajqd_ring_copy": (c_int, [_P, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "ajqd_gated_activation": (c_int, [_P, _I, _P, _I, _I, _I, _I, _I, _P]),
+    "ajqd_product_better": (c_int, [_I, _I, _I]),
+    "ajqd_product": (c_int, [ctypes.POINTER(ProductArgs), _P]),
     "ajqd_matvec": (c_int, [_P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "ajqd_windowed_attention": (c_int, [ctypes.POINTER(WindowedAttentionArgs), _I, _I, _P]),
     "ajqd_windowed_prefill_supported": (c_int, [_I, _I, _I]),

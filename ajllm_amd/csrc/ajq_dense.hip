@@ -1,9 +1,11 @@
 // C ABI of libajq_dense.so (include/ajq_dense.h): argument validation, launch geometry, error reporting.
+#include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
 
 #include "../../include/ajq_dense.h"
 #include "ajq_common.h"
+#include "dense_gemm_kernels.h"
 #include "dense_kernels.h"
 #include "latent_attention.h"
 #include "dense_gemv_kernels.h"
@@ -115,6 +117,52 @@ int launch_prefill_vt(int vt, const WindowedAttention& w, hipStream_t stream) {
     case 6: return launch_prefill<KS, 6>(w, stream);
     case 8: return launch_prefill<KS, 8>(w, stream);
     default: return launch_prefill<KS, 16>(w, stream);
+  }
+}
+
+// ---- products of many rows: tiles of 64 QM x 128 QN.  Microseconds of a tile that has a CU to itself, of its 64 k, and of its output's
+// bytes per element; and of the launch.  Fitted to 330 random products (32 .. 8192 rows, 256 .. 29000 columns, k up to 18000): the tile
+// chosen with them takes 1 % longer than the best one on average.
+struct ProductTile {
+  int qm, qn;
+  float launch, tile, step, out;
+};
+constexpr ProductTile kProductTiles[] = {{4, 2, 0.0f, 4.28f, 0.985f, 0.684f}, {3, 2, 0.0f, 3.86f, 0.797f, 0.53f}, {2, 2, 0.0f, 3.21f, 0.568f, 0.426f},
+                                         {3, 1, 0.28f, 2.66f, 0.505f, 0.295f}, {2, 1, 1.34f, 1.32f, 0.399f, 0.237f}, {1, 1, 1.96f, 0.57f, 0.312f, 0.138f}};
+constexpr int kCus = 256;
+long long product_tiles(int qm, int qn, int rows, int n) { return (long long)((rows + 64 * qm - 1) / (64 * qm)) * ((n + 128 * qn - 1) / (128 * qn)); }
+int pick_product_tile(int rows, int n, int k, int out_bytes) {
+  int best = 0;
+  float least = 0.f;
+  for (int i = 0; i < (int)(sizeof(kProductTiles) / sizeof(kProductTiles[0])); ++i) {
+    const ProductTile& t = kProductTiles[i];
+    const float turns = (float)product_tiles(t.qm, t.qn, rows, n) / kCus;
+    // two tiles of one column quadrant share a CU, and a round that they fill half takes half as long
+    const float rounds = t.qn == 2 || turns <= 1.f ? ceilf(turns) : 0.5f * ceilf(2.f * turns);
+    const float us = t.launch + rounds * (t.tile + t.step * (float)(k / 64) + t.out * (float)out_bytes);
+    if (i == 0 || us < least) { best = i; least = us; }
+  }
+  return best;
+}
+template <int QM, int QN, int EPI>
+int launch_product(const DenseGemm& a, hipStream_t stream) {
+  constexpr int bytes = tile_lds_bytes(64 * QM, 128 * QN, EPI);
+  auto kernel = dense_gemm_kernel<QM, QN, EPI>;
+  if (int e = allow_lds(kernel, bytes, "ajqd_product")) return e;
+  const long long blocks = product_tiles(QM, QN, a.m, a.n);
+  if (blocks > 0x7FFFFFFFll) return fail(AJQ_ERR_SHAPE, "ajqd_product: too many workgroups");
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kTileThreads), bytes, stream, a);
+  return check_launch("ajqd_product");
+}
+template <int EPI>
+int launch_product_tile(int tile, const DenseGemm& a, hipStream_t stream) {
+  switch (tile) {
+    case 0: return launch_product<4, 2, EPI>(a, stream);
+    case 1: return launch_product<3, 2, EPI>(a, stream);
+    case 2: return launch_product<2, 2, EPI>(a, stream);
+    case 3: return launch_product<3, 1, EPI>(a, stream);
+    case 4: return launch_product<2, 1, EPI>(a, stream);
+    default: return launch_product<1, 1, EPI>(a, stream);
   }
 }
 
@@ -256,6 +304,30 @@ int ajqd_gated_activation(const void* y, int y_dtype, void* out, int out_ld, int
                        out_ld, rows, width, act);
   });
   return check_launch("ajqd_gated_activation");
+}
+
+int ajqd_product_better(int rows, int n, int k) {
+  if (rows < 1 || n < 16 || n % 16 || k < 64 || k % 64) return 0;
+  // A workgroup goes through all of k, the vendor's kernels cut it: few tiles and a long k are theirs (61 rows, 8576 -> 528: 37 us
+  // against 20; 919 rows, 15488 -> 640: 78 against 53).  Up to k = 2048 (13 us in one wave of workgroups) or from a tile per
+  // CU on this one is the faster (geometric mean over the 330 products 0.61 of the vendor's time).
+  return k <= 2048 || product_tiles(1, 1, rows, n) >= kCus;
+}
+
+int ajqd_product(const ajqd_product_args* a, void* stream) {
+  if (!a || !a->x || !a->w || !a->y) return fail(AJQ_ERR_NULL, "ajqd_product: null pointer argument");
+  const int columns = a->pairs ? a->n / 2 : a->n, multiple = a->out_dtype == AJQD_F32 ? 4 : 8;
+  if (a->rows < 1 || a->n < 16 || a->n % 16 || a->k < 64 || a->k % 64 || a->k > (1 << 22) || a->ldx < a->k || a->ldx > (1 << 22) || a->ldy < columns)
+    return fail(AJQ_ERR_SHAPE, "ajqd_product: unsupported shape (rows=%d n=%d k=%d ldx=%d ldy=%d)", a->rows, a->n, a->k, a->ldx, a->ldy);
+  if (!known(a->out_dtype) || a->act < -1 || a->act > AJQD_ACT_SQUARED_RELU || (a->out_dtype == AJQD_F32 && a->act >= 0) || (a->pairs && a->act < 0))
+    return fail(AJQ_ERR_UNSUPPORTED, "ajqd_product: unsupported output (dtype=%d act=%d pairs=%d)", a->out_dtype, a->act, a->pairs);
+  if (a->ldx % 8 || a->ldy % multiple || !aligned16(a->x) || !aligned16(a->w) || !aligned16(a->y))
+    return fail(AJQ_ERR_ALIGN, "ajqd_product: rows must start on 16-byte boundaries");
+  DenseGemm d{(const uint16_t*)a->x, (const uint16_t*)a->w, a->y, a->rows, a->n, a->k, a->ldx, a->ldy, a->act};
+  const int tile = pick_product_tile(a->rows, a->n, a->k, a->out_dtype == AJQD_F32 ? 4 : a->pairs ? 1 : 2);
+  if (a->out_dtype == AJQD_F32) return launch_product_tile<kTileF32>(tile, d, (hipStream_t)stream);
+  if (a->act < 0) return launch_product_tile<kTileBf16>(tile, d, (hipStream_t)stream);
+  return a->pairs ? launch_product_tile<kTilePairs>(tile, d, (hipStream_t)stream) : launch_product_tile<kTileAct>(tile, d, (hipStream_t)stream);
 }
 
 int ajqd_matvec(const void* w, const void* x, int x_batch, int x_group, void* y, int y_batch, int y_group, int groups,

@@ -80,8 +80,25 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+def _own_product(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``x w^T`` (``w`` contiguous) is this library's product: bf16 rows that start on 16-byte boundaries, and a size at
+    which it is the faster one."""
+    return (x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0
+            and bool(_lib.load_dense().ajqd_product_better(x.shape[0], w.shape[0], w.shape[1])))
+
+
+def _product_into(x: torch.Tensor, w: torch.Tensor, y: int, ldy: int, out_dtype: torch.dtype, act: int = -1, pairs: bool = False) -> None:
+    args = _lib.ProductArgs(x=_ptr(x), w=_ptr(w), y=y, rows=x.shape[0], n=w.shape[0], k=w.shape[1], ldx=x.stride(0), ldy=ldy,
+                            out_dtype=_flag(out_dtype), act=act, pairs=int(pairs))
+    _lib.check_dense(_lib.load_dense().ajqd_product(ctypes.byref(args), _stream()), "product")
+
+
 def _product(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
-    """``x w^T`` of many rows (the vendor library's product, fp32 accumulation)."""
+    """``x w^T`` of many rows, fp32 accumulation (fp32 rows, and few tiles of a long product: the vendor library's)."""
+    if _own_product(x, w):
+        y = torch.empty((x.shape[0], w.shape[0]), dtype=out_dtype, device=x.device)
+        _product_into(x, w, _ptr(y), w.shape[0], out_dtype)
+        return y
     if x.dtype == out_dtype:
         return torch.mm(x, w.t())
     return torch.mm(x, w.t(), out_dtype=out_dtype)

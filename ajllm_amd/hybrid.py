@@ -30,8 +30,8 @@ import torch
 from torch import nn
 
 from . import _lib
-from .dense import (NORM_PROLOGUE_ROWS, DenseLM, FrequencyScaling, Loop, _add_norms, _flag, _matvec, _padded, _product, _ptr,
-                    _stream, _up, rotary_frequencies)
+from .dense import (NORM_PROLOGUE_ROWS, DenseLM, FrequencyScaling, Loop, _add_norms, _flag, _matvec, _own_product, _padded, _product,
+                    _product_into, _ptr, _stream, _up, rotary_frequencies)
 from .modeling import Embedding, Linear, PlainFeedForward, RingCache, RMSNorm, build_feed_forward, build_norm, register_architecture
 
 UNBOUNDED = 1 << 30   # context length of a model without a position table
@@ -303,12 +303,20 @@ class HybridLM(DenseLM):
             elif isinstance(w, PackedScan):
                 mixed = self._scan(h, w, cache, run, batch, seq, start)
             else:
-                mixed = self._activated(_product(h, w.w_in, h.dtype), w.act)
+                mixed = self._fed_forward(h, w)
             delta, done = _product(mixed, w.w_out, torch.float32), sub
             if residuals is not None and (k + 1 == len(order) or order[k + 1][0] != run):
                 total = (sub.mix.sum(dim=1)[:, None] * x).sum(dim=1) + sub.writes.sum() * (sub.scale * delta)
                 residuals.append(total[:, : self.d_model].view(batch, seq, -1))
         return self._streams_norm(x, delta, done, None), None
+
+    def _fed_forward(self, h: torch.Tensor, w: PackedFeedForward) -> torch.Tensor:
+        """``act(h w_in^T)``: one launch where the product is this library's."""
+        if not _own_product(h, w.w_in):
+            return self._activated(_product(h, w.w_in, h.dtype), w.act)
+        y = torch.empty((h.shape[0], w.width), dtype=h.dtype, device=h.device)
+        _product_into(h, w.w_in, _ptr(y), w.width, h.dtype, w.act)
+        return y
 
     def _activated(self, y: torch.Tensor, act: int) -> torch.Tensor:
         _lib.check_dense(_lib.load_dense().ajqd_activation(_ptr(y), _ptr(y), y.numel(), act, _flag(y.dtype), _stream()), "activation")
@@ -374,7 +382,7 @@ class HybridLM(DenseLM):
         ring, state = (cache.rings[run], cache.states[run]) if cache is not None else (None, None)
         x = self._convolved(y, w, ring, start, None, seq)
         low = _product(x, w.w_low, h.dtype)
-        raw = torch.mm(low[:, : w.rank], w.w_dt.t())
+        raw = _product(low[:, : w.rank], w.w_dt, h.dtype)
         out = self._recur(x, raw, low, y, w, state, batch, seq, start, None)
         keep = min(seq, w.taps - 1)
         if ring is not None and keep > 0:

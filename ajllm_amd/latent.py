@@ -28,8 +28,8 @@ import torch
 from torch import nn
 
 from . import _lib
-from .dense import (NORM_PROLOGUE_ROWS, DenseLM, Loop, _add_norms, _flag, _matvec, _padded, _product, _ptr, _stream, _up,
-                    rotary_frequencies)
+from .dense import (NORM_PROLOGUE_ROWS, DenseLM, Loop, _add_norms, _flag, _matvec, _own_product, _padded, _product, _product_into, _ptr,
+                    _stream, _up, rotary_frequencies)
 from .modeling import Embedding, GatedFeedForward, Linear, RingCache, RMSNorm, build_norm, register_architecture
 
 
@@ -252,7 +252,10 @@ class LatentLM(DenseLM):
                 _lib.check_dense(lib.ajqd_windowed_attention(ctypes.byref(args), _flag(dtype), _flag(dtype), st), "windowed_attention")
             del kv, q
             if w.w2 is not None:
-                self._gate(_product(n2, w.w2, dtype), joined, w)
+                if _own_product(n2, w.w2):
+                    _product_into(n2, w.w2, self._gated_columns(joined, w), w.joined, dtype, w.act, pairs=True)
+                else:
+                    self._gate(_product(n2, w.w2, dtype), joined, w)
             delta = _product(joined, w.wo, torch.float32)
             if ring is not None:
                 keep = min(seq, ring.shape[1])
@@ -262,9 +265,14 @@ class LatentLM(DenseLM):
                 residuals.append((x + delta)[:, : self.d_model].view(batch, seq, -1))
         return x, delta
 
+    @staticmethod
+    def _gated_columns(joined: torch.Tensor, w: PackedBlock) -> int:
+        """Where the feed-forward columns of ``joined`` begin."""
+        return joined.data_ptr() + w.heads * w.vdimp * joined.element_size()
+
     def _gate(self, y: torch.Tensor, joined: torch.Tensor, w: PackedBlock) -> None:
         """The gated activation of ``y`` into the feed-forward columns of ``joined``."""
-        at = joined.data_ptr() + w.heads * w.vdimp * joined.element_size()
+        at = self._gated_columns(joined, w)
         _lib.check_dense(_lib.load_dense().ajqd_gated_activation(_ptr(y), _flag(y.dtype), at, w.joined, y.shape[0], w.ff, w.act,
                                                                  _flag(joined.dtype), _stream()), "gated_activation")
 

@@ -71,6 +71,19 @@ int ajqd_gated_activation(const void* y, int y_dtype, void* out, int out_ld, int
 int ajqd_matvec(const void* w, const void* x, int x_batch, int x_group, void* y, int y_batch, int y_group, int groups,
                 int n, int k, int batch, int dtype, int out_dtype, void* stream);
 
+/* ---- products of many rows in bf16 */
+typedef struct {
+  const void *x, *w;
+  void* y;
+  int32_t rows, n, k, ldx, ldy, out_dtype, act, pairs;
+} ajqd_product_args;
+/* y [rows, n] = x [rows, k] w [n, k]^T, fp32 sums, out_dtype; k a multiple of 64, n of 16; ldx, ldy in elements.  act >= 0 (bf16 out):
+ * act(y), or with pairs (w's rows in blocks of 8 gates and their 8 ups) act(gate) * up, [rows, n / 2].
+ * ajqd_product_better says whether this is the faster way to make the product (the vendor's cuts a long K where the output
+ * has few tiles). */
+int ajqd_product_better(int rows, int n, int k);
+int ajqd_product(const ajqd_product_args* args, void* stream);
+
 typedef struct {
   const void *q, *k1, *k2, *v;
   const float *sink, *gates;

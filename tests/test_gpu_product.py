@@ -1,0 +1,76 @@
+"""Products of many rows (``ajqd_product``) against float64, over every tile that the sizes choose and its edges."""
+
+import ctypes
+
+import pytest
+import torch
+
+from ajllm_amd import _lib
+
+PLAIN, ACT, PAIRS = "plain", "act", "pairs"
+ACTS = {
+    "relu": torch.relu, "silu": torch.nn.functional.silu, "squared_relu": lambda z: torch.relu(z).square(),
+    "gelu_tanh": lambda z: torch.nn.functional.gelu(z, approximate="tanh"),
+}
+
+
+def _args(x, w, y, rows, n, k, ldx, ldy, out=_lib.AJQD_BF16, act=-1, pairs=0):
+    return _lib.ProductArgs(x=x, w=w, y=y, rows=rows, n=n, k=k, ldx=ldx, ldy=ldy, out_dtype=out, act=act, pairs=pairs)
+
+
+# (rows, n, k): the smallest; a row and a tile's rows around 64; tiles of 64 x 128, 192 x 128, 128 x 128, 128 x 256, 192 x 256,
+# 256 x 256 with remainders on both sides; one, two, an odd and an even number of 64-k steps
+SIZES = [(1, 16, 64), (63, 144, 64), (65, 272, 192), (500, 1008, 320), (257, 16000, 192), (1025, 4112, 320), (4097, 4112, 64),
+         (1537, 4080, 64), (2040, 4080, 640), (2049, 5008, 128), (3000, 4048, 640), (3080, 8080, 64), (4000, 4016, 192)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,out", [(PLAIN, torch.float32), (PLAIN, torch.bfloat16), (ACT, torch.bfloat16), (PAIRS, torch.bfloat16)])
+@pytest.mark.parametrize("rows,n,k", SIZES)
+def test_product(cuda, rows, n, k, kind, out):
+    lib = _lib.load_dense()
+    g = torch.Generator(device=cuda).manual_seed(rows + n + k)
+    ldx = k + 24
+    x = torch.randn((rows, ldx), generator=g, device=cuda).to(torch.bfloat16)
+    w = (torch.randn((n, k), generator=g, device=cuda) * k ** -0.5).to(torch.bfloat16)
+    sums = x[:, :k].double() @ w.double().t()
+    # fp32 sums of k terms: k roundings of 2^-24 of the terms' absolute sum
+    slack = k * 2.0 ** -24 * (x[:, :k].double().abs() @ w.double().t().abs())
+    for name in (["relu"] if kind == PLAIN else ACTS):
+        want, bound = sums, slack
+        if kind == ACT:
+            want = ACTS[name](sums)
+            # slopes: below 1.2, for the square 2 |z|; the functions themselves within 2^-20 of |z| in fp32
+            bound = slack * (2 * sums.abs() + slack if name == "squared_relu" else 1.2) + 2.0 ** -20 * want.abs().maximum(sums.abs())
+        if kind == PAIRS:
+            gate, up = (t.reshape(rows, -1) for t in sums.view(rows, -1, 2, 8).unbind(2))
+            gs, us = (t.reshape(rows, -1) for t in slack.view(rows, -1, 2, 8).unbind(2))
+            a = ACTS[name](gate)
+            ab = gs * (2 * gate.abs() + gs if name == "squared_relu" else 1.2) + 2.0 ** -20 * a.abs().maximum(gate.abs())
+            want, bound = a * up, ab * up.abs() + a.abs() * us + ab * us
+        ldy = want.shape[1] + 8
+        y = torch.full((rows + 1, ldy), float("nan"), dtype=out, device=cuda)
+        act = -1 if kind == PLAIN else _lib.AJQD_ACTIVATIONS[name]
+        args = _args(x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, n, k, ldx, ldy,
+                     _lib.AJQD_F32 if out == torch.float32 else _lib.AJQD_BF16, act, int(kind == PAIRS))
+        _lib.check_dense(lib.ajqd_product(ctypes.byref(args), torch.cuda.current_stream().cuda_stream), "product")
+        got = y[:rows, : want.shape[1]].double()
+        if out == torch.bfloat16:
+            bound = bound + 2.0 ** -8 * (want.abs() + bound)   # to the nearest of 8 significant bits
+        assert bool(((got - want).abs() <= bound + 1e-30).all()), (name, float(((got - want).abs() - bound).max()))
+        assert bool(y[rows:].isnan().all()) and bool(y[:, want.shape[1]:].isnan().all()), "written outside the result"
+
+
+def test_product_refuses_what_it_does_not_make():
+    lib = _lib.load_dense()
+    buf = ctypes.create_string_buffer(4096 + 16)
+    p = (ctypes.addressof(buf) + 15) & ~15   # host memory: only its address is looked at
+    assert lib.ajqd_product(None, None) == -1
+    for change, status in ((dict(x=None), -1), (dict(rows=0), -2), (dict(n=24), -2), (dict(k=96), -2), (dict(ldx=56), -2), (dict(ldy=8), -2),
+                           (dict(ldx=68), -3), (dict(ldy=20), -3), (dict(w=p + 8), -3), (dict(out=2), -4), (dict(act=4), -4),
+                           (dict(out=_lib.AJQD_F32, act=0), -4), (dict(pairs=1), -4)):
+        args = _args(**{**dict(x=p, w=p, y=p, rows=1, n=16, k=64, ldx=64, ldy=16), **change})
+        assert lib.ajqd_product(ctypes.byref(args), None) == status, change
+    assert lib.ajqd_product_better(500, 4096, 4096) == 1 and lib.ajqd_product_better(1, 16, 64) == 1
+    assert lib.ajqd_product_better(919, 640, 15488) == 0          # few tiles, long sums
+    assert not any(lib.ajqd_product_better(*s) for s in ((500, 4096, 96), (500, 24, 64), (0, 16, 64), (500, 4096, 0)))
