@@ -15,6 +15,7 @@
 #include "gemm_split_kernels.h"
 #include "gemm_wide_kernels.h"
 #include "gemm128_kernels.h"
+#include "gemm_turns_kernels.h"
 #include "gemm_mid_kernels.h"
 #include "skinny_kernels.h"
 #include "skinny_resident_kernels.h"
@@ -116,11 +117,11 @@ int check_matmul_args(const char* name, const void* x, int M, int K, const void*
   return AJQ_OK;
 }
 
-// 256-row tiles on 32x32x16 MFMA; M >= 256 (the last row tile is shifted, not masked).  Shapes with enough tiles
-// take 256 x 256 ones (gemm_wide_kernels.h); otherwise 256 x 128: W8 with K % 256 == 0
+// 256-row tiles on 32x32x16 MFMA; M >= 256 (the last row tile is shifted, not masked).  int4 shapes with enough tiles take 256 x 256
+// ones (gemm_wide_kernels.h); otherwise 256 x 128: W8 with K % 256 == 0
 // runs the ring kernel (four compute waves that unpack their own weights, a loader wave); W4, and W8 on any other
 // K % 128 == 0, the split-role kernel (four compute waves, four producers that dequantize once per workgroup; W4
-// needs no group sums there).
+// needs no group sums there).  (int8 on 256 x 256 and three smaller tiles: gemm_turns_kernels.h.)
 #ifndef AJQ_GEMM_WIDE
 #define AJQ_GEMM_WIDE 1
 #endif
@@ -128,7 +129,7 @@ template <bool kW4, bool kGate = false>
 int launch_gemm256(const uint16_t* x, int M, int K, const uint32_t* wq, const uint32_t* meta, const uint16_t* scales8,
                    int N, void* y, int out_f32, hipStream_t stream) {
   const int tiles = ((M + kG2BM - 1) / kG2BM) * ((N + kG2BN - 1) / kG2BN);
-  if (!kGate || (N / 2) % (kGWBN / 2) == 0) {
+  if (kW4 && (!kGate || (N / 2) % (kGWBN / 2) == 0)) {
     // 256 x 256 tiles move half the activation bytes per MFMA and measure 9-15 % faster per flop, but there are half
     // as many of them: they run when that still fills the CUs' rounds better (a wide tile takes 2 / 1.12 narrow ones)
     const long long wide = (long long)((M + kGWBM - 1) / kGWBM) * ((N + kGWBN - 1) / kGWBN);
@@ -152,6 +153,19 @@ int launch_gemm256(const uint16_t* x, int M, int K, const uint32_t* wq, const ui
   if (int s = allow_big_lds(split, kGSLdsBytes)) return s;
   hipLaunchKernelGGL(split, dim3(tiles), dim3(kGSThreads), kGSLdsBytes, stream, x, M, K,
                      reinterpret_cast<const u32x4_t*>(wq), meta, scales8, N, y, out_f32);
+  return AJQ_OK;
+}
+
+// int8 tiles of waves that take turns
+template <bool kGate, int QM, int QN>
+int launch_turns(const uint16_t* x, int M, int K, const uint32_t* wq, const uint16_t* scales8, int N, void* y, int out_f32,
+                 hipStream_t stream) {
+  constexpr int BM = 64 * QM, BN = 128 * QN, bytes = gemm_turns_lds(BM, BN);
+  auto kernel = dequant_gemm_turns_kernel<kGate, QM, QN>;
+  if (int s = allow_big_lds(kernel, bytes)) return s;
+  const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  hipLaunchKernelGGL(kernel, dim3(tiles), dim3(kTurnsThreads), bytes, stream, x, M, K, reinterpret_cast<const u32x4_t*>(wq), scales8, N, y,
+                     out_f32);
   return AJQ_OK;
 }
 
@@ -986,28 +1000,57 @@ int check_pro(const char* name, int M, int K, const void* a, const void* b) {
   return AJQ_OK;
 }
 
-// Which kernel runs a matmul of M >= 17 rows.  All three times are estimated, in microseconds per k-block of 128 and round of 256
+// Which kernel runs a matmul of M >= 17 rows.
+//
+// Three times are estimated, in microseconds per k-block of 128 and round of 256
 // workgroups, one workgroup per CU; the weights below settle the choice and are not the kernels' times.  Those (25 shapes of 333 to
-// 5328 rows, both schemes, graph replays) depend on how full the rounds are:
-//  * 256 x 128 tiles, weight 1.8: 1.6 to 2.0 (W4) / 1.6 to 1.8 (W8) in full rounds, down to 1.4 / 1.15 with half of the last one empty.
-//  * 128 x 128 tiles (M >= 128), weight 1.25 (W4) / 1.15 (W8): 0.9 to 1.1 in full rounds, 0.75 to 0.85 with half of one empty, 1.4 from
-//    thirty rounds on.  They win where the big tiles leave CUs idle (M = 1024 on N = 4096 is 128 big tiles or 256 small ones: 51 /
-//    39 us W4, 45 / 36 W8).
-// So the estimate is wrong where the big tiles' second round is nearly empty: W8, 4096 -> 14336, 640 rows 99.0 us against 85.3 with the
-// other kernel; 4096 -> 6144, 1500 rows 94.6 / 77.7; W4, 4096 -> 28672, 333 rows 109.5 / 101.2.  On 42 of the 50 the choice is
-// the faster kernel or within 3 % of it.
+// 5328 rows, graph replays) depend on how full the rounds are:
+//  * 256 x 128 tiles, weight 1.8: 1.6 to 2.0 (int4) in full rounds, down to 1.4 with half of the last one empty.
+//  * 128 x 128 tiles (M >= 128), weight 1.25 (int8 1.15): 0.9 to 1.1 in full rounds, 0.75 to 0.85 with half of one empty, 1.4 from
+//    thirty rounds on.  They win where the big tiles leave CUs idle (M = 1024 on N = 4096 is 128 big tiles or 256 small ones: int4 51 /
+//    39 us).
 //  * the weight-streaming kernel sustains about 400 TFLOP/s for M >= 256 and is the only one below
 //    M = 128.
+// For int4 they decide (wrongly where the big tiles' second round is nearly empty: 4096 -> 28672, 333 rows 109.5 us against 101.2 with
+// the other kernel); for int8 they say where tiles are taken at all, or where a second estimate does.
+//
+// int8: the times of six tile kernels in microseconds as fitted to 740 random products (129 .. 8192 rows, 1024 .. 32000 columns, K
+// 1024 .. 14336; 4 to 7 % rms).  A round that is partly filled costs `least` of a full one and the rest by its filling: fewer tiles at
+// once run at a higher clock.  Over 520 of the shapes the choice takes 0.94 of the time (geometric mean) of a choice between the
+// last two kernels, 256 x 256 tiles that read ahead of their MFMAs and the streaming kernel by the weights above.  Tiles are taken
+// beyond those weights where they are estimated to be faster than 440 TFLOP/s (229 rows, 3200 -> 8432: 35.7 -> 23.7 us).
 #ifndef AJQ_GEMM_TILE
 #define AJQ_GEMM_TILE 0  // 0: by the estimate; 128 or 256: that tile kernel for every M it can run
 #endif
-enum MatmulKernel { kStreaming, kTiles256, kTiles128 };
+enum MatmulKernel { kStreaming, kTiles256, kTiles128, kTurns256, kTurns192, kTurns128, kTurns192Narrow };
+struct TileTimes {
+  MatmulKernel kernel;
+  int bm, bn, least_rows;
+  double launch, tile, step, least;
+};
+constexpr TileTimes kW8Tiles[] = {{kTurns256, 256, 256, 256, 1.91, 8.84, 1.441, 0.727}, {kTurns192, 192, 256, 17, 1.11, 7.51, 1.132, 0.811},
+                                  {kTurns128, 128, 256, 17, 1.00, 5.16, 0.861, 0.802},  {kTurns192Narrow, 192, 128, 17, 5.18, 0.69, 0.705, 0.894},
+                                  {kTiles256, 256, 128, 256, 0.25, 6.51, 0.776, 0.656}, {kTiles128, 128, 128, 128, 0.04, 4.31, 0.499, 0.694}};
+double w8_tiles_us(int M, int N, int K, MatmulKernel& which) {
+  double least = 1e30;
+  for (const TileTimes& t : kW8Tiles) {
+    if (M < t.least_rows) continue;
+    const long long tiles = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const double filled = (double)(tiles % 256) / 256, rounds = (double)(tiles / 256) + (filled > 0 ? t.least + (1 - t.least) * filled : 0);
+    const double us = t.launch + rounds * (t.tile + t.step * (K / 64));
+    if (us < least) {
+      least = us;
+      which = t.kernel;
+    }
+  }
+  return least;
+}
 MatmulKernel pick_matmul_kernel(int M, int N, int K, bool w4) {
   if (AJQ_GEMM_TILE == 128 && M >= kG1BM) return kTiles128;
   if (AJQ_GEMM_TILE == 256 && M >= kG2BM) return kTiles256;
   if (M < kG1BM) return kStreaming;
   const double G = (double)(K / kGroup);
-  const double us_stream = 2.0 * M * N * (double)K / 400e6;
+  const double flops = 2.0 * M * N * (double)K, us_stream = flops / 400e6;
   double us_big = 1e30;
   if (M >= kGemm256MinM) {
     const long long tiles = (long long)((M + kG2BM - 1) / kG2BM) * ((N + kG2BN - 1) / kG2BN);
@@ -1015,8 +1058,26 @@ MatmulKernel pick_matmul_kernel(int M, int N, int K, bool w4) {
   }
   const long long small_ = (long long)((M + kG1BM - 1) / kG1BM) * ((N + kG1BN - 1) / kG1BN);
   const double us_small = (double)((small_ + 255) / 256) * G * (w4 ? 1.25 : 1.15) + 5.0;
-  if (us_stream <= us_big && us_stream <= us_small) return kStreaming;
+  const bool stream = us_stream <= us_big && us_stream <= us_small;
+  if (!w4) {
+    MatmulKernel which = kStreaming;
+    const double us = w8_tiles_us(M, N, K, which);
+    return stream && us >= 0.95 * (flops / 440e6 + 2.0) ? kStreaming : which;
+  }
+  if (stream) return kStreaming;
   return us_small < us_big ? kTiles128 : kTiles256;
+}
+template <bool kGate>
+int launch_w8_tiles(MatmulKernel which, const uint16_t* x, int M, int K, const uint32_t* wq, const uint16_t* scales, int N, void* y, int out_f32,
+                    hipStream_t stream) {
+  switch (which) {
+    case kTurns256: return launch_turns<kGate, 4, 2>(x, M, K, wq, scales, N, y, out_f32, stream);
+    case kTurns192: return launch_turns<kGate, 3, 2>(x, M, K, wq, scales, N, y, out_f32, stream);
+    case kTurns128: return launch_turns<kGate, 2, 2>(x, M, K, wq, scales, N, y, out_f32, stream);
+    case kTurns192Narrow: return launch_turns<kGate, 3, 1>(x, M, K, wq, scales, N, y, out_f32, stream);
+    case kTiles128: return launch_gemm128<false, kGate>(x, M, K, wq, nullptr, scales, nullptr, N, y, out_f32, stream);
+    default: return launch_gemm256<false, kGate>(x, M, K, wq, nullptr, scales, N, y, out_f32, stream);
+  }
 }
 
 // ---- routes that cut K into parts and add the parts' sums in a second launch: shapes whose output is too small to fill the chip
@@ -1085,6 +1146,8 @@ SplitRoute pick_split(int M, int N, int K, bool w4) {
   if (M >= kGemm256MinM)
     other = std::min(other, (double)(((M + 255) / 256 * tn + 255) / 256) * G * (w4 ? 1.45 : 1.15) + 5.0);
   if (split >= 0.88 * other) return r;
+  MatmulKernel which;
+  if (!w4 && w8_tiles_us(M, N, K, which) < 0.9 * split) return r;
   r.kind = kRouteTiles;
   r.S = S;
   r.sums = w4 ? (group_sum_bytes(M, K) + 255) / 256 * 256 : 0;
@@ -1397,10 +1460,7 @@ int ajq_w8a16_gemm(const uint16_t* x, int M, int K, const uint32_t* wq, const ui
   }
   if ((long long)M * K * 2 >= (1LL << 32))
     return fail(AJQ_ERR_SHAPE, "ajq_w8a16_gemm: M * K = %lld exceeds the 32-bit activation offsets", (long long)M * K);
-  if (int s = which == kTiles128
-                  ? launch_gemm128<false>(x, M, K, wq, nullptr, scales, nullptr, N, y, out_f32, (hipStream_t)stream)
-                  : launch_gemm256<false>(x, M, K, wq, nullptr, scales, N, y, out_f32, (hipStream_t)stream))
-    return s;
+  if (int s = launch_w8_tiles<false>(which, x, M, K, wq, scales, N, y, out_f32, (hipStream_t)stream)) return s;
   return check_launch("ajq_w8a16_gemm");
 }
 
@@ -1442,10 +1502,7 @@ int ajq_w8a16_gemm_gate(const uint16_t* x, int M, int K, const uint32_t* wq, con
                 N2, K);
   if ((long long)M * K * 2 >= (1LL << 32))
     return fail(AJQ_ERR_SHAPE, "ajq_w8a16_gemm_gate: M * K = %lld exceeds the 32-bit activation offsets", (long long)M * K);
-  if (int s = pick_matmul_kernel(M, N2, K, false) == kTiles128
-                  ? launch_gemm128<false, true>(x, M, K, wq, nullptr, scales, nullptr, N2, y, 0, (hipStream_t)stream)
-                  : launch_gemm256<false, true>(x, M, K, wq, nullptr, scales, N2, y, 0, (hipStream_t)stream))
-    return s;
+  if (int s = launch_w8_tiles<true>(pick_matmul_kernel(M, N2, K, false), x, M, K, wq, scales, N2, y, 0, (hipStream_t)stream)) return s;
   return check_launch("ajq_w8a16_gemm_gate");
 }
 

@@ -40,12 +40,6 @@ constexpr int tile_lds_bytes(int bm, int bn, int epi) {
   return stages > out ? stages : out;
 }
 
-__device__ __forceinline__ void tile_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 // A quadrant of a wave: QM x QN blocks of 16 x 16; BM = 64 QM, BN = 128 QN.
 template <int QM, int QN, int EPI>
 __global__ __launch_bounds__(kTileThreads) void dense_gemm_kernel(DenseGemm a) {
@@ -61,13 +55,9 @@ __global__ __launch_bounds__(kTileThreads) void dense_gemm_kernel(DenseGemm a) {
   const int wm = wave >> 2, wn = wave & 3;
   const int r = lane & 15, g = lane >> 4;
   const int steps = a.k >> 6;
-  // Work order.  XCD k (workgroups are dealt to the XCDs round-robin) takes a contiguous part of the tiles, which are numbered in
-  // bands of eight row tiles, so that what runs on it at once shares rows and columns in its L2 (2800 x 8192 x 2048: 98 -> 78 us).
-  const int tiles_m = (a.m + BM - 1) / BM, tiles_n = (a.n + BN - 1) / BN;
-  const int tiles = tiles_m * tiles_n, xcd = blockIdx.x & 7, part = tiles >> 3, rest = tiles & 7;
-  const int id = xcd * part + min(xcd, rest) + (int)(blockIdx.x >> 3);
-  const int band = id / (8 * tiles_n), in_band = id - band * 8 * tiles_n, high = min(8, tiles_m - 8 * band);
-  const int m0 = (8 * band + in_band % high) * BM, n0 = in_band / high * BN;
+  int tile_m, tile_n;
+  tile_place((a.m + BM - 1) / BM, (a.n + BN - 1) / BN, tile_m, tile_n);
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
 
   // ---- requests: eight rows of 128 bytes each; chunk c of a half's row r sits in slot c ^ ((r >> 1) & 7), so that the 16 rows
   // a fragment read meets lie in distinct banks.  Rows past the end repeat the last one.
@@ -154,8 +144,8 @@ __global__ __launch_bounds__(kTileThreads) void dense_gemm_kernel(DenseGemm a) {
   request_a(min(1, last), 1, 0);
   request_b(min(1, last), 1, 0);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kYounger) : "memory");
-  tile_barrier();
-  if (wm == 1) tile_barrier();
+  turn_barrier();
+  if (wm == 1) turn_barrier();
 
   auto step = [&](int j, auto bc) {
     constexpr int cur = decltype(bc)::value, nxt = cur ^ 1;
@@ -164,31 +154,31 @@ __global__ __launch_bounds__(kTileThreads) void dense_gemm_kernel(DenseGemm a) {
     read_b(cur, 0);
     request_b(j1, nxt, 1);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kYounger) : "memory");
-    tile_barrier();
+    turn_barrier();
     products(0, 0);
-    tile_barrier();
+    turn_barrier();
     read_b(cur, 1);
     request_a(j1, nxt, 1);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kYounger) : "memory");
-    tile_barrier();
+    turn_barrier();
     products(0, 1);
-    tile_barrier();
+    turn_barrier();
     read_a(cur, 1);
     request_a(j2, cur, 0);
-    tile_barrier();
+    turn_barrier();
     products(1, 1);
-    tile_barrier();
+    turn_barrier();
     request_b(j2, cur, 0);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kYounger) : "memory");
-    tile_barrier();
+    turn_barrier();
     products(1, 0);
-    tile_barrier();
+    turn_barrier();
   };
   for (int j = 0; j < steps; j += 2) {
     step(j, std::integral_constant<int, 0>{});
     if (j + 1 < steps) step(j + 1, std::integral_constant<int, 1>{});
   }
-  if (wm == 0) tile_barrier();
+  if (wm == 0) turn_barrier();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   // ---- the result leaves through LDS in whole rows of the tile, 16 bytes per lane
