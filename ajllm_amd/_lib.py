@@ -251,6 +251,7 @@ DENSE_SIGNATURES: dict[str, tuple] = {
 _lib: ctypes.CDLL | None = None
 _dense_lib: ctypes.CDLL | None = None
 _bench_lib: ctypes.CDLL | None = None
+_native = None
 
 
 def load_bench() -> ctypes.CDLL:
@@ -286,6 +287,22 @@ def load() -> ctypes.CDLL:
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+def load_native():
+    """The extension module, bound to the operator library on first use (built by ``python -m ajllm_amd.build``)."""
+    global _native
+    if _native is None:
+        try:
+            from . import _native as module
+        except ImportError as error:
+            raise RuntimeError("ajllm_amd/_native.so is missing or does not fit this interpreter: build it with "
+                               "`python -m ajllm_amd.build`") from error
+        lib = load()
+        module.bind(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in (
+            "ajq_w4a16_gemv", "ajq_w8a16_gemv", "ajq_w4a16_matmul", "ajq_w8a16_matmul", "ajq_matmul_scratch_bytes")))
+        _native = module
+    return _native
 
 
 def load_dense() -> ctypes.CDLL:

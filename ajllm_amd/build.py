@@ -1,4 +1,5 @@
-"""Compile the HIP sources in ``csrc/`` into ``libajq.so`` and ``libajq_dense.so`` next to this file.
+"""Compile the HIP sources in ``csrc/`` into ``libajq.so`` and ``libajq_dense.so`` next to this file, and the extension module
+``_native.so``.
 
 Cross-compiles for gfx950 with hipcc; needs no GPU.  Run as
 ``python -m ajllm_amd.build`` or call :func:`build_library`.
@@ -19,6 +20,9 @@ LIBRARY = PACKAGE_DIR / "libajq.so"
 # without waiting for the quantized matmuls to compile
 DENSE_SOURCE = PACKAGE_DIR / "csrc" / "ajq_dense.hip"
 DENSE_LIBRARY = PACKAGE_DIR / "libajq_dense.so"
+# a quantized layer's forward without the interpreter: an extension module that calls the operator library
+NATIVE_SOURCE = PACKAGE_DIR / "csrc" / "native_linear.cpp"
+NATIVE_MODULE = PACKAGE_DIR / "_native.so"
 # measurement probes for bench.py (include/ajq_bench.h); the operator library does not depend on it
 BENCH_SOURCE = PACKAGE_DIR / "csrc" / "ajq_bench.hip"
 BENCH_LIBRARY = PACKAGE_DIR / "libajq_bench.so"
@@ -66,6 +70,30 @@ def ensure_dense_library() -> Path:
     return DENSE_LIBRARY
 
 
+def build_native_module(verbose: bool = False) -> Path:
+    """The extension module, by the host compiler (it holds no device code)."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    libraries = Path(torch.__file__).resolve().parent / "lib"
+    rocm = Path(shutil.which("hipcc") or "/opt/rocm/bin/hipcc").resolve().parents[1]
+    tmp = NATIVE_MODULE.with_suffix(".so.tmp%d" % os.getpid())
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{p}" for p in include_paths()),
+           f"-I{rocm / 'include'}", "-I/opt/rocm/include", f"-I{sysconfig.get_paths()['include']}", str(NATIVE_SOURCE), "-o", str(tmp),
+           f"-L{libraries}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        tmp.unlink(missing_ok=True)
+        raise RuntimeError(f"g++ failed ({proc.returncode}):\n{proc.stderr}")
+    os.replace(tmp, NATIVE_MODULE)
+    return NATIVE_MODULE
+
+
 def build_bench_library(verbose: bool = False) -> Path:
     return build_library(verbose, BENCH_SOURCE, BENCH_LIBRARY)
 
@@ -73,4 +101,5 @@ def build_bench_library(verbose: bool = False) -> Path:
 if __name__ == "__main__":
     print(build_library(verbose=True))
     print(build_dense_library(verbose=True))
+    print(build_native_module(verbose=True))
     print(build_bench_library(verbose=True))

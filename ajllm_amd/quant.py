@@ -35,6 +35,15 @@ _raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(torch._C, "_cuda_get
     lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
+_linear = None   # the extension module's function, once it is bound
+
+
+def _bound_linear():
+    global _linear
+    _linear = _lib.load_native().linear
+    return _linear
+
+
 def _require_cuda(*tensors: torch.Tensor) -> None:
     for t in tensors:
         if not t.is_cuda:
@@ -189,7 +198,7 @@ _OUT_FLAGS = {torch.bfloat16: _lib.AJQ_OUT_BF16, torch.float32: _lib.AJQ_OUT_F32
 
 
 def _matmul(w4: bool, x: torch.Tensor, wq: torch.Tensor, aux: torch.Tensor, out_dtype: torch.dtype, kernel: str) -> torch.Tensor:
-    """One product through the C ABI.  A decode step makes one of these per projection and token: as little Python as the
+    """One product through the C ABI, with as little Python as the
     checks need (5 us of 15 per call with device and stream objects made anew, 9 all told without).  The kernels take a
     matrix's extent from its packed tensors, so the rows and the W8 scales are held against those."""
     if not x.is_cuda:
@@ -353,7 +362,13 @@ class QuantLinear(nn.Module):
             self.prepare()
 
     def forward(self, inputs: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.Tensor:
-        buffers, k, want = self._buffers, self.in_features, out_dtype or inputs.dtype
+        buffers = self._buffers
+        # bf16 rows as the kernels take them: one call of native code, which leaves everything else to the lines below it
+        y = (_linear or _bound_linear())(inputs, buffers["wq"], buffers["meta"], self.scheme != "w8a16", self.in_features, self.out_features,
+                                         out_dtype)
+        if y is not None:
+            return y
+        k, want = self.in_features, out_dtype or inputs.dtype
         wq = buffers["wq"]
         if wq is None:
             raise RuntimeError("QuantLinear has no weights: build it with from_linear()/from_weight()")
