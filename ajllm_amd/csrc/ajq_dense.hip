@@ -1,4 +1,5 @@
 // C ABI of libajq_dense.so (include/ajq_dense.h): argument validation, launch geometry, error reporting.
+#include <algorithm>
 #include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -189,22 +190,31 @@ int launch_scan(const Scan& a, int batch, hipStream_t stream) {
   const long long lanes = (long long)batch * a.inner;
   auto go = [&](auto kernel, int per_channel) {
     const int channels = 256 / per_channel;
-    hipLaunchKernelGGL(kernel, dim3((a.inner + channels - 1) / channels, batch), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL(kernel, dim3((a.inner + channels - 1) / channels, batch), dim3(256), 0, stream, a, ScanParts{});
     return check_launch("ajqd_scan");
   };
   const bool few = lanes * 4 < 2 * 65536, fewer = lanes * 8 < 2 * 65536;  // (65536 lanes: a wave on every SIMD)
   const int n = a.states;
-  if (n <= 16 && fewer) return go(scan_kernel<T, 16, 1>, 16);
-  if (n <= 16 && few) return go(scan_kernel<T, 8, 2>, 8);
-  if (n <= 16) return go(scan_kernel<T, 4, 4>, 4);
-  if (n <= 32 && fewer) return go(scan_kernel<T, 16, 2>, 16);
-  if (n <= 32 && few) return go(scan_kernel<T, 8, 4>, 8);
-  if (n <= 24) return go(scan_kernel<T, 4, 6>, 4);
-  if (n <= 32) return go(scan_kernel<T, 4, 8>, 4);
-  if (n <= 64) return few ? go(scan_kernel<T, 16, 4>, 16) : go(scan_kernel<T, 8, 8>, 8);
-  if (n <= 128) return go(scan_kernel<T, 16, 8>, 16);
-  if (n <= 256) return go(scan_kernel<T, 32, 8>, 32);
+  if (n <= 16 && fewer) return go(scan_kernel<T, 16, 1, kScanWhole>, 16);
+  if (n <= 16 && few) return go(scan_kernel<T, 8, 2, kScanWhole>, 8);
+  if (n <= 16) return go(scan_kernel<T, 4, 4, kScanWhole>, 4);
+  if (n <= 32 && fewer) return go(scan_kernel<T, 16, 2, kScanWhole>, 16);
+  if (n <= 32 && few) return go(scan_kernel<T, 8, 4, kScanWhole>, 8);
+  if (n <= 24) return go(scan_kernel<T, 4, 6, kScanWhole>, 4);
+  if (n <= 32) return go(scan_kernel<T, 4, 8, kScanWhole>, 4);
+  if (n <= 64) return few ? go(scan_kernel<T, 16, 4, kScanWhole>, 16) : go(scan_kernel<T, 8, 8, kScanWhole>, 8);
+  if (n <= 128) return go(scan_kernel<T, 16, 8, kScanWhole>, 16);
+  if (n <= 256) return go(scan_kernel<T, 32, 8, kScanWhole>, 32);
   return fail(AJQ_ERR_UNSUPPORTED, "ajqd_scan: %d states per channel (up to 256 are built)", n);
+}
+// In parts: four lanes per channel, the fewest there are (the part's own work counts now, not the length of its loop).
+constexpr int kScanPartLanes = 4, kScanPartTokens = 32;  // a part is a multiple of the kernel's tile
+template <typename T, int NS>
+int launch_scan_parts(const Scan& a, int batch, int count, const ScanParts& parts, hipStream_t stream) {
+  const int channels = 256 / kScanPartLanes, blocks = (a.inner + channels - 1) / channels;
+  hipLaunchKernelGGL((scan_kernel<T, kScanPartLanes, NS, kScanEnds>), dim3(blocks, batch, count - 1), dim3(256), 0, stream, a, parts);
+  hipLaunchKernelGGL((scan_kernel<T, kScanPartLanes, NS, kScanPart>), dim3(blocks, batch, count), dim3(256), 0, stream, a, parts);
+  return check_launch("ajqd_scan_in_parts");
 }
 
 
@@ -744,19 +754,61 @@ int ajqd_conv_silu(const void* y, int ldy, void* ring, const float* weight, cons
   return check_launch("ajqd_conv_silu");
 }
 
-int ajqd_scan(const ajqd_scan_args* a, int dtype, void* stream) {
+}  // extern "C"
+namespace {
+int check_scan(const char* name, const ajqd_scan_args* a, int dtype) {
   if (!a || !a->x || !a->dt || !a->low || !a->z || !a->a2 || !a->d || !a->dt_bias || !a->out || (!a->state && (a->start > 0 || a->pos)))
-    return fail(AJQ_ERR_NULL, "ajqd_scan: null pointer argument");
+    return fail(AJQ_ERR_NULL, "%s: null pointer argument", name);
   if (a->batch < 1 || a->batch > 65535 || a->seq < 1 || a->inner < 8 || a->inner % 8 || a->states < 4 || a->states % 4 || a->start < 0 ||
       a->dt_ld < a->inner || a->dt_ld % 8 || a->z_ld < a->inner || a->z_ld % 8 || a->out_ld < a->inner || a->out_ld % 8 || a->b_col < 0 ||
       a->c_col < 0 || a->low_ld < a->b_col + a->states || a->low_ld < a->c_col + a->states || (a->pos && a->seq != 1))
-    return fail(AJQ_ERR_SHAPE, "ajqd_scan: unsupported shape (batch=%d seq=%d inner=%d states=%d)", a->batch, a->seq, a->inner, a->states);
-  if (!known(dtype)) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_scan: unknown dtype %d", dtype);
+    return fail(AJQ_ERR_SHAPE, "%s: unsupported shape (batch=%d seq=%d inner=%d states=%d)", name, a->batch, a->seq, a->inner, a->states);
+  if (!known(dtype)) return fail(AJQ_ERR_UNSUPPORTED, "%s: unknown dtype %d", name, dtype);
   if (!aligned16(a->x) || !aligned16(a->dt) || !aligned16(a->z) || !aligned16(a->out) || !aligned16(a->d) || !aligned16(a->dt_bias))
-    return fail(AJQ_ERR_ALIGN, "ajqd_scan: rows must be 16-byte aligned");
-  Scan s{a->x, a->dt, a->low, a->z, a->a2, a->d, a->dt_bias, a->state, a->start, positions64(a->pos), a->seq, a->inner, a->states,
-         a->dt_ld, a->low_ld, a->b_col, a->c_col, a->z_ld, a->out_ld, a->out};
+    return fail(AJQ_ERR_ALIGN, "%s: rows must be 16-byte aligned", name);
+  return AJQ_OK;
+}
+Scan device_scan(const ajqd_scan_args* a) {
+  return Scan{a->x, a->dt, a->low, a->z, a->a2, a->d, a->dt_bias, a->state, a->start, positions64(a->pos), a->seq, a->inner, a->states,
+              a->dt_ld, a->low_ld, a->b_col, a->c_col, a->z_ld, a->out_ld, a->out};
+}
+}  // namespace
+extern "C" {
+
+int ajqd_scan(const ajqd_scan_args* a, int dtype, void* stream) {
+  if (int e = check_scan("ajqd_scan", a, dtype)) return e;
+  const Scan s = device_scan(a);
   return dtype == AJQD_BF16 ? launch_scan<uint16_t>(s, a->batch, (hipStream_t)stream) : launch_scan<float>(s, a->batch, (hipStream_t)stream);
+}
+
+int ajqd_scan_parts(int batch, int seq, int inner, int states) {
+  if (batch < 1 || seq < 1 || inner < 8 || states < 1 || states > 16) return 1;
+  // The states are gone through twice then, so it pays where one piece leaves a SIMD with fewer than four waves (us, one piece against
+  // parts: 8192 channels, 1500 tokens 168 / 120, 192 tokens 30 / 23; 2048 channels, 2048 tokens 160 / 53, 192 tokens 16.5 / 13.9; 12288
+  // channels, 700 tokens 97 / 85; but 16384, 700 tokens 106 / 106, and 128 tokens of 8192 channels 15.2 / 16.9).  About four waves on
+  // every SIMD, parts of one tile of tokens at least: few parts of a short prompt are slower than one piece (300 tokens of 2048
+  // channels: 23 in one, 37 in two, 19 in six).
+  const long long channels = (long long)batch * inner;
+  if (channels >= 16384 || seq < 192) return 1;
+  const long long tiles = (seq + kScanPartTokens - 1) / kScanPartTokens;
+  return (int)std::min({tiles, std::max(6LL, 4 * 65536 / (channels * kScanPartLanes)), 128LL});  // (a part goes through all ends before it)
+}
+size_t ajqd_scan_workspace(int batch, int inner, int states, int parts) {
+  return parts > 1 ? ((size_t)parts * states + parts - 1) * batch * inner * sizeof(float) : 0;
+}
+int ajqd_scan_in_parts(const ajqd_scan_args* a, int parts, float* workspace, int dtype, void* stream) {
+  if (int e = check_scan("ajqd_scan_in_parts", a, dtype)) return e;
+  if (parts < 2) return ajqd_scan(a, dtype, stream);
+  if (a->states > 16 || a->pos) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_scan_in_parts: up to 16 states of a prompt are built (%d)", a->states);
+  if (!workspace) return fail(AJQ_ERR_NULL, "ajqd_scan_in_parts: null workspace");
+  const int tiles = (a->seq + kScanPartTokens - 1) / kScanPartTokens, length = (tiles + parts - 1) / parts * kScanPartTokens;
+  const int count = (a->seq + length - 1) / length;
+  if (count < 2) return ajqd_scan(a, dtype, stream);
+  if (count > 65535) return fail(AJQ_ERR_SHAPE, "ajqd_scan_in_parts: %d parts", count);
+  const ScanParts cut{workspace, workspace + (size_t)count * a->batch * a->inner * a->states, length};
+  const Scan s = device_scan(a);
+  return dtype == AJQD_BF16 ? launch_scan_parts<uint16_t, 4>(s, a->batch, count, cut, (hipStream_t)stream)
+                            : launch_scan_parts<float, 4>(s, a->batch, count, cut, (hipStream_t)stream);
 }
 
 int ajqd_scan_splits(int batch, int inner) {

@@ -159,16 +159,29 @@ constexpr int scan_tile() {
   while (t * L * NS > 4096) t /= 2;
   return t;
 }
-template <typename T, int L, int NS>
-__global__ __launch_bounds__(256) void scan_kernel(Scan a) {
+//
+// Few channels leave the chip to a wave or two per SIMD and their latencies (8192 channels of 16 states, 1500 tokens: 168 us, of which
+// the arithmetic is 70; in parts 120).  Then time is cut into `parts` (ScanParts): a first launch (kScanEnds) takes every part but the
+// last one through the states alone, from zero (the first part from where the sequence stands), and leaves their ends and sums of dt; in
+// a second one (kScanPart) a part starts from the ends before it, S = 2^(a2 sum dt) S + end, and makes its outputs.
+enum { kScanWhole = 0, kScanEnds = 1, kScanPart = 2 };
+struct ScanParts {
+  float* ends;   // [parts, B, states / 4, inner, 4]: the state ahead of the first part, then every part's end
+  float* sums;   // [parts - 1, B, inner]: a part's sum of dt
+  int length;    // of a part, in tokens
+};
+template <typename T, int L, int NS, int kRole>
+__global__ __launch_bounds__(256) void scan_kernel(Scan a, ScanParts parts) {
   constexpr int CH = 256 / L, kT = scan_tile<L, NS>(), kN = L * NS, kVec = kT * CH / 8, kPitch = CH + 4, kTogether = 4;
   static_assert(kT % kTogether == 0, "whole groups of tokens");
   static_assert(kVec >= 1 && kVec <= 256, "at most one vector of 8 channels per thread");
   __shared__ __attribute__((aligned(16))) float dt_s[kT * kPitch], dx_s[kT * kPitch], b_s[kT * kN], c_s[kT * kN];
   const int tid = threadIdx.x, ch = tid / L, part = tid % L;
   const int b = blockIdx.y, c0 = blockIdx.x * CH, c = c0 + ch;
+  const int cut = kRole == kScanWhole ? 0 : (int)blockIdx.z;
+  const int begin = kRole == kScanWhole ? 0 : cut * parts.length, end = kRole == kScanWhole ? a.seq : min(a.seq, begin + parts.length);
   const bool mine = c < a.inner;
-  float s[NS], a2[NS];
+  float s[NS], a2[NS], whole_dt = 0.f;
   const bool carried = a.state && (a.start > 0 || (a.pos && *a.pos > 0));
   float* state = a.state + (size_t)b * a.inner * a.states;
   auto place = [&](int n) { return ((size_t)(n >> 2) * a.inner + c) * 4 + (n & 3); };
@@ -177,7 +190,24 @@ __global__ __launch_bounds__(256) void scan_kernel(Scan a) {
     const int n = part * NS + i;
     const bool real = mine && n < a.states;
     a2[i] = real ? a.a2[place(n)] : 0.f;
-    s[i] = real && carried ? state[place(n)] : 0.f;
+    s[i] = kRole != kScanPart && real && carried && cut == 0 ? state[place(n)] : 0.f;
+  }
+  const size_t planes = (size_t)a.inner * a.states, batch_planes = (size_t)gridDim.y * planes;
+  if (kRole == kScanEnds && cut == 0 && mine)  // (the last part of the second launch writes `state` while others start)
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+      if (part * NS + i < a.states) parts.ends[b * planes + place(part * NS + i)] = s[i];
+  if (kRole == kScanPart && mine) {
+    const float* ends = parts.ends + b * planes;
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+      if (part * NS + i < a.states) s[i] = ends[(cut ? batch_planes : 0) + place(part * NS + i)];
+    for (int q = 1; q < cut; ++q) {
+      const float sum = parts.sums[((size_t)q * gridDim.y + b) * a.inner + c];
+#pragma unroll
+      for (int i = 0; i < NS; ++i)
+        if (part * NS + i < a.states) s[i] = fmaf(__builtin_amdgcn_exp2f(sum * a2[i]), s[i], ends[(q + 1) * batch_planes + place(part * NS + i)]);
+    }
   }
   // this thread's vector of a tile: token vt, channels vc ..
   const int vt = tid / (CH / 8), vl = 8 * (tid % (CH / 8)), vc = c0 + vl;
@@ -196,24 +226,24 @@ __global__ __launch_bounds__(256) void scan_kernel(Scan a) {
   }
   auto request = [&](int t0) {
     const int t = t0 + vt;
-    if (stages && t < a.seq) {
+    if (stages && t < end) {
       nx = load8(xp + (size_t)t * a.inner);
       nd = load8(dp + (size_t)t * a.dt_ld);
-      nz = load8(zp + (size_t)t * a.z_ld);
+      if (kRole != kScanEnds) nz = load8(zp + (size_t)t * a.z_ld);
     }
 #pragma unroll
     for (int k = 0; k < kLow; ++k) {
       const int i = tid + 256 * k, u = t0 + i / kN, n = i % kN;
       nb[k] = nc[k] = 0.f;
-      if (i < kT * kN && u < a.seq && n < a.states) {
+      if (i < kT * kN && u < end && n < a.states) {
         nb[k] = to_f32(lp[(size_t)u * a.low_ld + a.b_col + n]);
-        nc[k] = to_f32(lp[(size_t)u * a.low_ld + a.c_col + n]);
+        if (kRole != kScanEnds) nc[k] = to_f32(lp[(size_t)u * a.low_ld + a.c_col + n]);
       }
     }
   };
-  request(0);
-  for (int t0 = 0; t0 < a.seq; t0 += kT) {
-    const int count = min(kT, a.seq - t0);
+  request(begin);
+  for (int t0 = begin; t0 < end; t0 += kT) {
+    const int count = min(kT, end - t0);
     const Float8 x = nx, z = nz;
     if (tid < kVec) {
       float* dts = dt_s + vt * kPitch + vl;
@@ -234,11 +264,11 @@ __global__ __launch_bounds__(256) void scan_kernel(Scan a) {
       const int i = tid + 256 * k;
       if (i < kT * kN) {
         b_s[i] = nb[k];
-        c_s[i] = nc[k];
+        if (kRole != kScanEnds) c_s[i] = nc[k];
       }
     }
     __syncthreads();
-    if (t0 + kT < a.seq) request(t0 + kT);
+    if (t0 + kT < end) request(t0 + kT);
     // (tokens past the end: dt = 0 leaves the states alone)  A group's operands are read ahead of the arithmetic of the one before.
     Operands<kTogether, NS> next;
     auto read = [&](int u) {
@@ -249,7 +279,7 @@ __global__ __launch_bounds__(256) void scan_kernel(Scan a) {
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
           next.b[k][i] = b_s[(u + k) * kN + part * NS + i];
-          next.c[k][i] = c_s[(u + k) * kN + part * NS + i];
+          if (kRole != kScanEnds) next.c[k][i] = c_s[(u + k) * kN + part * NS + i];
         }
       }
     };
@@ -268,9 +298,11 @@ __global__ __launch_bounds__(256) void scan_kernel(Scan a) {
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
           s[i] = fmaf(f[k][i], s[i], now.dx[k] * now.b[k][i]);
-          y[k] = fmaf(s[i], now.c[k][i], y[k]);
+          if (kRole != kScanEnds) y[k] = fmaf(s[i], now.c[k][i], y[k]);
         }
+        if (kRole == kScanEnds) whole_dt += now.dt[k];
       }
+      if (kRole == kScanEnds) continue;
 #pragma unroll
       for (int k = 0; k < kTogether; ++k) y[k] = team_sum<L>(y[k]);
       if (part == 0)
@@ -278,16 +310,20 @@ __global__ __launch_bounds__(256) void scan_kernel(Scan a) {
         for (int k = 0; k < kTogether; ++k) dx_s[(u + k) * kPitch + ch] = y[k];
     }
     __syncthreads();
-    if (stages && vt < count) {
+    if (kRole != kScanEnds && stages && vt < count) {
       const float* ys = dx_s + vt * kPitch + vl;
       Float8 o;
 #pragma unroll
       for (int e = 0; e < 8; ++e) o.v[e] = fmaf(skip.v[e], x.v[e], ys[e]) * silu_for<T>(z.v[e]);
       store8(op + (size_t)(t0 + vt) * a.out_ld, o);
     }
-    __syncthreads();
+    if (kRole != kScanEnds) __syncthreads();
   }
-  if (a.state && mine)
+  if (kRole == kScanEnds) {
+    if (mine && part == 0) parts.sums[((size_t)cut * gridDim.y + b) * a.inner + c] = whole_dt;
+    state = parts.ends + (cut + 1) * batch_planes + b * planes;
+  }
+  if ((kRole == kScanEnds || (a.state && end == a.seq)) && mine)
 #pragma unroll
     for (int i = 0; i < NS; ++i)
       if (part * NS + i < a.states) state[place(part * NS + i)] = s[i];

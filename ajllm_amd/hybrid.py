@@ -406,7 +406,13 @@ class HybridLM(DenseLM):
             x=_ptr(x), dt=_ptr(raw), low=_ptr(low), z=y.data_ptr() + w.inner * y.element_size(), a2=_ptr(w.a2), d=_ptr(w.skip),
             dt_bias=_ptr(w.dt_bias), state=_ptr(state), pos=_ptr(pos), out=_ptr(out), batch=batch, seq=seq, start=start, inner=w.inner,
             states=w.states, dt_ld=raw.shape[1], low_ld=low.shape[1], b_col=w.rank, c_col=w.rank + w.states, z_ld=y.shape[1], out_ld=out.shape[1])
-        _lib.check_dense(_lib.load_dense().ajqd_scan(ctypes.byref(args), _flag(x.dtype), _stream()), "scan")
+        lib = _lib.load_dense()
+        parts = lib.ajqd_scan_parts(batch, seq, w.inner, w.states) if pos is None else 1
+        if parts > 1:
+            room = torch.empty(lib.ajqd_scan_workspace(batch, w.inner, w.states, parts), dtype=torch.uint8, device=x.device)
+            _lib.check_dense(lib.ajqd_scan_in_parts(ctypes.byref(args), parts, _ptr(room), _flag(x.dtype), _stream()), "scan_in_parts")
+        else:
+            _lib.check_dense(lib.ajqd_scan(ctypes.byref(args), _flag(x.dtype), _stream()), "scan")
         return out
 
     # ---- one token per sequence, at the device-side position ``cache.position``

@@ -213,6 +213,11 @@ typedef struct {
 /* dt = softplus(dt + dt_bias); S = 2^(dt a2) S + dt x B; out = (S C + d x) silu(z), token by token; state (optional) is read
  * unless the first token's position is 0, and written.  x, dt, low (B | C), z, out in dtype, one row per token. */
 int ajqd_scan(const ajqd_scan_args* args, int dtype, void* stream);
+/* the same for prompts (no pos, up to 16 states) with time cut into `parts`, two launches; workspace of ajqd_scan_workspace bytes.
+ * ajqd_scan_parts says how many parts pay (1: none) */
+int ajqd_scan_parts(int batch, int seq, int inner, int states);
+size_t ajqd_scan_workspace(int batch, int inner, int states, int parts);
+int ajqd_scan_in_parts(const ajqd_scan_args* args, int parts, float* workspace, int dtype, void* stream);
 /* one decode step in bf16: y fp32 [batch, ldy] = (columns to convolve: inner | z: inner).  ajqd_scan_project convolves and
  * multiplies by w [rows, inner] = (dt rank | B | C | padding), leaving `splits` parts [splits, batch, rows];
  * ajqd_scan_step adds them and does the rest (w_dt [inner, rank]) -> out bf16 [batch, out_ld] */
