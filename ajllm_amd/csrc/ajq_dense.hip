@@ -122,27 +122,39 @@ int launch_prefill_vt(int vt, const WindowedAttention& w, hipStream_t stream) {
 }
 
 // ---- products of many rows: tiles of 64 QM x 128 QN.  Microseconds of a tile that has a CU to itself, of its 64 k, and of its output's
-// bytes per element; and of the launch.  Fitted to 330 random products (32 .. 8192 rows, 256 .. 29000 columns, k up to 18000): the tile
-// chosen with them takes 1 % longer than the best one on average.
+// bytes per element; and of the launch.  Fitted to the times of 345 random products (1 .. 9000 rows, 64 .. 22000 columns, k up to 18000;
+// every tile, k in one piece and in up to 24 parts) in a row of milliseconds with weights that are in no cache, as a model's are: the tile
+// and parts chosen with them take 1.3 % longer than the best ones on average.  (Fitted to short runs on weights that stay cached, 1500
+// rows, 16384 -> 4096 came out as one piece: 162 us against 155 in two parts there, but 188 against 168 in a model.)
 struct ProductTile {
   int qm, qn;
   float launch, tile, step, out;
 };
-constexpr ProductTile kProductTiles[] = {{4, 2, 0.0f, 4.28f, 0.985f, 0.684f}, {3, 2, 0.0f, 3.86f, 0.797f, 0.53f}, {2, 2, 0.0f, 3.21f, 0.568f, 0.426f},
-                                         {3, 1, 0.28f, 2.66f, 0.505f, 0.295f}, {2, 1, 1.34f, 1.32f, 0.399f, 0.237f}, {1, 1, 1.96f, 0.57f, 0.312f, 0.138f}};
+constexpr ProductTile kProductTiles[] = {{4, 2, 0.0f, 3.606f, 1.038f, 0.603f}, {3, 2, 0.0f, 2.748f, 0.883f, 0.58f}, {2, 2, 0.0f, 1.862f, 0.709f, 0.522f},
+                                         {3, 1, 0.925f, 1.376f, 0.573f, 0.299f}, {2, 1, 0.941f, 0.78f, 0.473f, 0.323f}, {1, 1, 1.982f, 0.0f, 0.381f, 0.209f}};
+constexpr float kSharedTile = 1.224f;                        // of two tiles on one CU, against half of each alone
+constexpr float kSumLaunch = 2.392f, kSumMegabyte = 0.299f;   // adding the parts: the launch, and what it reads and writes
+constexpr int kProductParts[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
 constexpr int kCus = 256;
 long long product_tiles(int qm, int qn, int rows, int n) { return (long long)((rows + 64 * qm - 1) / (64 * qm)) * ((n + 128 * qn - 1) / (128 * qn)); }
-int pick_product_tile(int rows, int n, int k, int out_bytes) {
+// steps of 64 k in a part, and the parts that come of it
+int part_steps(int k, int parts) { return (k / 64 + parts - 1) / parts; }
+int whole_parts(int k, int parts) { const int steps = part_steps(k, parts); return (k / 64 + steps - 1) / steps; }
+float product_us(const ProductTile& t, int rows, int n, int k, int out_bytes, int parts) {
+  const float turns = (float)product_tiles(t.qm, t.qn, rows, n) * whole_parts(k, parts) / kCus;
+  // two tiles of one column quadrant share a CU, and a round that they fill half takes half as long
+  const float rounds = t.qn == 2 || turns <= 1.f ? ceilf(turns) : 0.5f * kSharedTile * ceilf(2.f * turns);
+  const float us = t.launch + rounds * (t.tile + t.step * (float)part_steps(k, parts) + t.out * (float)(parts > 1 ? 4 : out_bytes));
+  return parts == 1 ? us : us + kSumLaunch + kSumMegabyte * 1e-6f * (float)rows * (float)n * (float)(4 * parts + out_bytes);
+}
+int pick_product_tile(int rows, int n, int k, int out_bytes, int parts, float* us = nullptr) {
   int best = 0;
   float least = 0.f;
   for (int i = 0; i < (int)(sizeof(kProductTiles) / sizeof(kProductTiles[0])); ++i) {
-    const ProductTile& t = kProductTiles[i];
-    const float turns = (float)product_tiles(t.qm, t.qn, rows, n) / kCus;
-    // two tiles of one column quadrant share a CU, and a round that they fill half takes half as long
-    const float rounds = t.qn == 2 || turns <= 1.f ? ceilf(turns) : 0.5f * ceilf(2.f * turns);
-    const float us = t.launch + rounds * (t.tile + t.step * (float)(k / 64) + t.out * (float)out_bytes);
-    if (i == 0 || us < least) { best = i; least = us; }
+    const float now = product_us(kProductTiles[i], rows, n, k, out_bytes, parts);
+    if (i == 0 || now < least) { best = i; least = now; }
   }
+  if (us) *us = least;
   return best;
 }
 template <int QM, int QN, int EPI>
@@ -152,7 +164,7 @@ int launch_product(const DenseGemm& a, hipStream_t stream) {
   if (int e = allow_lds(kernel, bytes, "ajqd_product")) return e;
   const long long blocks = product_tiles(QM, QN, a.m, a.n);
   if (blocks > 0x7FFFFFFFll) return fail(AJQ_ERR_SHAPE, "ajqd_product: too many workgroups");
-  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kTileThreads), bytes, stream, a);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks, (a.k + a.part - 1) / a.part), dim3(kTileThreads), bytes, stream, a);
   return check_launch("ajqd_product");
 }
 template <int EPI>
@@ -318,26 +330,71 @@ int ajqd_gated_activation(const void* y, int y_dtype, void* out, int out_ld, int
 
 int ajqd_product_better(int rows, int n, int k) {
   if (rows < 1 || n < 16 || n % 16 || k < 64 || k % 64) return 0;
-  // A workgroup goes through all of k, the vendor's kernels cut it: few tiles and a long k are theirs (61 rows, 8576 -> 528: 37 us
-  // against 20; 919 rows, 15488 -> 640: 78 against 53).  Up to k = 2048 (13 us in one wave of workgroups) or from a tile per
-  // CU on this one is the faster (geometric mean over the 330 products 0.61 of the vendor's time).
+  // A workgroup goes through all of k here: few tiles and a long k are made faster in parts (or by the vendor's kernels, which cut k as
+  // well) with the activation behind them (61 rows, 8576 -> 528: 37 us against 20; 919 rows, 15488 -> 640: 78 against 53).  Up to k = 2048
+  // (13 us in one wave of workgroups) or from a tile per CU on one piece is the faster.
   return k <= 2048 || product_tiles(1, 1, rows, n) >= kCus;
 }
 
-int ajqd_product(const ajqd_product_args* a, void* stream) {
-  if (!a || !a->x || !a->w || !a->y) return fail(AJQ_ERR_NULL, "ajqd_product: null pointer argument");
+}  // extern "C"
+namespace {
+int check_product(const char* name, const ajqd_product_args* a) {
+  if (!a || !a->x || !a->w || !a->y) return fail(AJQ_ERR_NULL, "%s: null pointer argument", name);
   const int columns = a->pairs ? a->n / 2 : a->n, multiple = a->out_dtype == AJQD_F32 ? 4 : 8;
   if (a->rows < 1 || a->n < 16 || a->n % 16 || a->k < 64 || a->k % 64 || a->k > (1 << 22) || a->ldx < a->k || a->ldx > (1 << 22) || a->ldy < columns)
-    return fail(AJQ_ERR_SHAPE, "ajqd_product: unsupported shape (rows=%d n=%d k=%d ldx=%d ldy=%d)", a->rows, a->n, a->k, a->ldx, a->ldy);
+    return fail(AJQ_ERR_SHAPE, "%s: unsupported shape (rows=%d n=%d k=%d ldx=%d ldy=%d)", name, a->rows, a->n, a->k, a->ldx, a->ldy);
   if (!known(a->out_dtype) || a->act < -1 || a->act > AJQD_ACT_SQUARED_RELU || (a->out_dtype == AJQD_F32 && a->act >= 0) || (a->pairs && a->act < 0))
-    return fail(AJQ_ERR_UNSUPPORTED, "ajqd_product: unsupported output (dtype=%d act=%d pairs=%d)", a->out_dtype, a->act, a->pairs);
+    return fail(AJQ_ERR_UNSUPPORTED, "%s: unsupported output (dtype=%d act=%d pairs=%d)", name, a->out_dtype, a->act, a->pairs);
   if (a->ldx % 8 || a->ldy % multiple || !aligned16(a->x) || !aligned16(a->w) || !aligned16(a->y))
-    return fail(AJQ_ERR_ALIGN, "ajqd_product: rows must start on 16-byte boundaries");
-  DenseGemm d{(const uint16_t*)a->x, (const uint16_t*)a->w, a->y, a->rows, a->n, a->k, a->ldx, a->ldy, a->act};
-  const int tile = pick_product_tile(a->rows, a->n, a->k, a->out_dtype == AJQD_F32 ? 4 : a->pairs ? 1 : 2);
+    return fail(AJQ_ERR_ALIGN, "%s: rows must start on 16-byte boundaries", name);
+  return AJQ_OK;
+}
+}  // namespace
+extern "C" {
+
+int ajqd_product(const ajqd_product_args* a, void* stream) {
+  if (int e = check_product("ajqd_product", a)) return e;
+  DenseGemm d{(const uint16_t*)a->x, (const uint16_t*)a->w, a->y, a->rows, a->n, a->k, a->ldx, a->ldy, a->act, a->k};
+  const int tile = pick_product_tile(a->rows, a->n, a->k, a->out_dtype == AJQD_F32 ? 4 : a->pairs ? 1 : 2, 1);
   if (a->out_dtype == AJQD_F32) return launch_product_tile<kTileF32>(tile, d, (hipStream_t)stream);
   if (a->act < 0) return launch_product_tile<kTileBf16>(tile, d, (hipStream_t)stream);
   return a->pairs ? launch_product_tile<kTilePairs>(tile, d, (hipStream_t)stream) : launch_product_tile<kTileAct>(tile, d, (hipStream_t)stream);
+}
+
+int ajqd_product_parts(int rows, int n, int k, int out_dtype) {
+  if (rows < 1 || n < 16 || n % 16 || k < 64 || k % 64 || !known(out_dtype)) return 0;
+  // Few tiles leave the chip idle for all of k: then its parts are made side by side, as many as the estimates say.  Against the vendor's
+  // products over the 345: 0.45 of their time (110 rows, 16960 -> 4544: 33 us, theirs 101, in one piece 83; 463 rows, 11392 -> 384: 15,
+  // 27, 56; 1500 rows, 8192 -> 288: 20, 22, 42); two are slower by more than 4 %, 4 rows against 11280 x 15872 most (75, 62).  Large
+  // outputs stay in one piece (4096 rows, 18432 -> 4096: 413 us, in two parts 447).
+  int best = 1;
+  float least = 0.f, us;
+  for (int parts : kProductParts) {
+    // (what the estimates were fitted to; 128 MiB of sums at most)
+    if (parts > 1 && (k / parts < 256 || (long long)rows * n * parts > (1LL << 25))) continue;
+    pick_product_tile(rows, n, k, out_dtype == AJQD_F32 ? 4 : 2, parts, &us);
+    if (parts == 1 || us < least) { best = parts; least = us; }
+  }
+  return whole_parts(k, best);
+}
+size_t ajqd_product_workspace(int rows, int n, int parts) { return parts > 1 ? (size_t)parts * rows * n * sizeof(float) : 0; }
+int ajqd_product_in_parts(const ajqd_product_args* a, int parts, float* workspace, void* stream) {
+  if (int e = check_product("ajqd_product_in_parts", a)) return e;
+  if (a->act >= 0) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_product_in_parts: an activation takes the product in one piece");
+  if (parts > 1) parts = whole_parts(a->k, parts);
+  if (parts < 2) return ajqd_product(a, stream);
+  if (!workspace) return fail(AJQ_ERR_NULL, "ajqd_product_in_parts: null workspace");
+  if (!aligned16(workspace)) return fail(AJQ_ERR_ALIGN, "ajqd_product_in_parts: the workspace must start on a 16-byte boundary");
+  const long long blocks = ((long long)a->rows * (a->n / 8) + 255) / 256;
+  if (parts > 65535 || blocks > 0x7FFFFFFFll) return fail(AJQ_ERR_SHAPE, "ajqd_product_in_parts: too many workgroups");
+  const int out_bytes = a->out_dtype == AJQD_F32 ? 4 : 2, tile = pick_product_tile(a->rows, a->n, a->k, out_bytes, parts);
+  const DenseGemm d{(const uint16_t*)a->x, (const uint16_t*)a->w, workspace, a->rows, a->n, a->k, a->ldx, a->n, -1, 64 * part_steps(a->k, parts)};
+  if (int e = launch_product_tile<kTileF32>(tile, d, (hipStream_t)stream)) return e;
+  if (out_bytes == 4)
+    hipLaunchKernelGGL(sum_parts_kernel<float>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, workspace, parts, a->rows, a->n, (float*)a->y, a->ldy);
+  else
+    hipLaunchKernelGGL(sum_parts_kernel<uint16_t>, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, workspace, parts, a->rows, a->n, (uint16_t*)a->y, a->ldy);
+  return check_launch("ajqd_product_in_parts");
 }
 
 int ajqd_matvec(const void* w, const void* x, int x_batch, int x_group, void* y, int y_batch, int y_group, int groups,

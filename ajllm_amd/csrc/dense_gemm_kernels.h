@@ -9,8 +9,8 @@
 // The two waves of a SIMD take turns: a quadrant is a part that reads LDS and asks for data and a part that is nothing but MFMA, a
 // barrier ends each part, and the second four waves run one part behind the first.  So one wave's MFMA always runs beside the
 // other's reads.  Eight waves that all read ahead of their own MFMAs (ring of four 32-k stages, one barrier per stage, the
-// order left to the compiler) reached 1.31 PFLOP/s at 8192 x 8192 x 8192, this 1.53; there the clock is what limits (the
-// vendor's product: 1.61).
+// order left to the compiler) reached 1.31 PFLOP/s at 8192 x 8192 x 8192, this 1.62; there the clock is what limits (the
+// vendor's product: 1.61 to 1.65).
 //
 // Hazards.  A request goes to a place that was read two quadrants before: the wave that is a part behind has waited for those
 // reads (its products consumed them) ahead of a barrier that the requesting wave has passed.  A half is read in the quadrant after
@@ -28,6 +28,7 @@ struct DenseGemm {
   const uint16_t *x, *w;
   void* y;
   int m, n, k, ldx, ldy, act;
+  int part;  // of k, a workgroup row's (gridDim.y); more than one: fp32 planes [parts][m][ldy]
 };
 
 // What becomes of the sums: fp32, bf16, bf16(act(sum)), or bf16(act(gate) * up) of w's rows in blocks of 8 gates and their 8 ups.
@@ -54,15 +55,15 @@ __global__ __launch_bounds__(kTileThreads) void dense_gemm_kernel(DenseGemm a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 2, wn = wave & 3;
   const int r = lane & 15, g = lane >> 4;
-  const int steps = a.k >> 6;
+  const int k0 = (int)blockIdx.y * a.part, steps = min(a.part, a.k - k0) >> 6;
   int tile_m, tile_n;
   tile_place((a.m + BM - 1) / BM, (a.n + BN - 1) / BN, tile_m, tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
 
   // ---- requests: eight rows of 128 bytes each; chunk c of a half's row r sits in slot c ^ ((r >> 1) & 7), so that the 16 rows
   // a fragment read meets lie in distinct banks.  Rows past the end repeat the last one.
-  const char* a_base = reinterpret_cast<const char*>(a.x) + (size_t)m0 * a.ldx * 2;
-  const char* b_base = reinterpret_cast<const char*>(a.w) + (size_t)n0 * a.k * 2;
+  const char* a_base = reinterpret_cast<const char*>(a.x) + ((size_t)m0 * a.ldx + k0) * 2;
+  const char* b_base = reinterpret_cast<const char*>(a.w) + ((size_t)n0 * a.k + k0) * 2;
   uint32_t a_voff[2][RA], b_voff[2][RB], a_to[RA], b_to[RB];
 #pragma unroll
   for (int h = 0; h < RA; ++h) {
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(kTileThreads) void dense_gemm_kernel(DenseGemm a) {
   auto col_of = [&](int hb, int t) { return hb * (BN / 2) + (wn * QN + t) * 16 + 4 * g; };
   if constexpr (EPI == kTileF32) {
     constexpr int kStride = BN * 4 + 16, kPieces = BN / 4;
-    float* y = reinterpret_cast<float*>(a.y);
+    float* y = reinterpret_cast<float*>(a.y) + (size_t)blockIdx.y * a.m * a.ldy;
 #pragma unroll
     for (int ha = 0; ha < 2; ++ha) {  // (half the rows at a time)
       __syncthreads();
@@ -241,6 +242,22 @@ __global__ __launch_bounds__(kTileThreads) void dense_gemm_kernel(DenseGemm a) {
       if (m0 + row < a.m && n < out_n) *reinterpret_cast<u32x4_t*>(reinterpret_cast<uint16_t*>(a.y) + (size_t)(m0 + row) * a.ldy + n) = v;
     }
   }
+}
+
+// y = the sum of a product's parts: eight columns of a row per thread.  Bound by its bytes, which come from the last-level cache where the
+// parts have just been written (3.3 TB/s over the launch, 1500 x 4096 in two parts).
+template <typename O>
+__global__ __launch_bounds__(256) void sum_parts_kernel(const float* planes, int parts, int m, int n, O* y, int ldy) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, pieces = (size_t)m * (n / 8);
+  if (i >= pieces) return;
+  Float8 v = load8(planes + i * 8);
+#pragma unroll 4
+  for (int p = 1; p < parts; ++p) {
+    const Float8 u = load8(planes + ((size_t)p * pieces + i) * 8);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v.v[e] += u.v[e];
+  }
+  store8(y + i / (n / 8) * ldy + i % (n / 8) * 8, v);
 }
 
 }  // namespace ajq

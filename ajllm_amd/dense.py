@@ -80,25 +80,37 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+def _product_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether this library's product reads ``x``: bf16 rows that start on 16-byte boundaries (``w`` contiguous)."""
+    return x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0
+
+
 def _own_product(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ``x w^T`` (``w`` contiguous) is this library's product: bf16 rows that start on 16-byte boundaries, and a size at
-    which it is the faster one."""
-    return (x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0
-            and bool(_lib.load_dense().ajqd_product_better(x.shape[0], w.shape[0], w.shape[1])))
+    """Whether ``act(x w^T)`` is this library's product: rows that it reads, and a size at which it is the faster one."""
+    return _product_rows(x, w) and bool(_lib.load_dense().ajqd_product_better(x.shape[0], w.shape[0], w.shape[1]))
+
+
+def _product_args(x: torch.Tensor, w: torch.Tensor, y: int, ldy: int, out_dtype: torch.dtype, act: int, pairs: bool) -> _lib.ProductArgs:
+    return _lib.ProductArgs(x=_ptr(x), w=_ptr(w), y=y, rows=x.shape[0], n=w.shape[0], k=w.shape[1], ldx=x.stride(0), ldy=ldy,
+                            out_dtype=_flag(out_dtype), act=act, pairs=int(pairs))
 
 
 def _product_into(x: torch.Tensor, w: torch.Tensor, y: int, ldy: int, out_dtype: torch.dtype, act: int = -1, pairs: bool = False) -> None:
-    args = _lib.ProductArgs(x=_ptr(x), w=_ptr(w), y=y, rows=x.shape[0], n=w.shape[0], k=w.shape[1], ldx=x.stride(0), ldy=ldy,
-                            out_dtype=_flag(out_dtype), act=act, pairs=int(pairs))
+    args = _product_args(x, w, y, ldy, out_dtype, act, pairs)
     _lib.check_dense(_lib.load_dense().ajqd_product(ctypes.byref(args), _stream()), "product")
 
 
 def _product(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
-    """``x w^T`` of many rows, fp32 accumulation (fp32 rows, and few tiles of a long product: the vendor library's)."""
-    if _own_product(x, w):
-        y = torch.empty((x.shape[0], w.shape[0]), dtype=out_dtype, device=x.device)
-        _product_into(x, w, _ptr(y), w.shape[0], out_dtype)
-        return y
+    """``x w^T`` of many rows, fp32 accumulation (fp32 rows, and columns off the kernel's grid: the vendor library's)."""
+    if _product_rows(x, w):
+        lib = _lib.load_dense()
+        parts = lib.ajqd_product_parts(x.shape[0], w.shape[0], w.shape[1], _flag(out_dtype))
+        if parts:
+            y = torch.empty((x.shape[0], w.shape[0]), dtype=out_dtype, device=x.device)
+            args = _product_args(x, w, _ptr(y), w.shape[0], out_dtype, -1, False)
+            room = torch.empty(lib.ajqd_product_workspace(x.shape[0], w.shape[0], parts), dtype=torch.uint8, device=x.device) if parts > 1 else None
+            _lib.check_dense(lib.ajqd_product_in_parts(ctypes.byref(args), parts, _ptr(room), _stream()), "product")
+            return y
     if x.dtype == out_dtype:
         return torch.mm(x, w.t())
     return torch.mm(x, w.t(), out_dtype=out_dtype)

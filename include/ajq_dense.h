@@ -79,10 +79,15 @@ typedef struct {
 } ajqd_product_args;
 /* y [rows, n] = x [rows, k] w [n, k]^T, fp32 sums, out_dtype; k a multiple of 64, n of 16; ldx, ldy in elements.  act >= 0 (bf16 out):
  * act(y), or with pairs (w's rows in blocks of 8 gates and their 8 ups) act(gate) * up, [rows, n / 2].
- * ajqd_product_better says whether this is the faster way to make the product (the vendor's cuts a long K where the output
- * has few tiles). */
+ * ajqd_product_better says whether this is the faster way to make a product with an activation (the vendor's cuts a long K where the
+ * output has few tiles). */
 int ajqd_product_better(int rows, int n, int k);
 int ajqd_product(const ajqd_product_args* args, void* stream);
+/* The same without an activation, K cut into parts whose fp32 sums (workspace of ajqd_product_workspace bytes, 16-byte aligned) a second
+ * launch adds.  ajqd_product_parts: in how many parts it is made fastest; 0 where it is not made. */
+int ajqd_product_parts(int rows, int n, int k, int out_dtype);
+size_t ajqd_product_workspace(int rows, int n, int parts);
+int ajqd_product_in_parts(const ajqd_product_args* args, int parts, float* workspace, void* stream);
 
 typedef struct {
   const void *q, *k1, *k2, *v;

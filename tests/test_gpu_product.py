@@ -61,6 +61,43 @@ def test_product(cuda, rows, n, k, kind, out):
         assert bool(y[rows:].isnan().all()) and bool(y[:, want.shape[1]:].isnan().all()), "written outside the result"
 
 
+# a part of one and of several 64-k steps, a last part that is shorter, more parts than steps, remainders of every tile's sides
+PARTS = [(1, 16, 128, 2), (65, 272, 192, 3), (130, 144, 448, 3), (500, 1008, 320, 4), (257, 4112, 640, 4), (1025, 1040, 832, 7), (33, 48, 320, 9)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,n,k,parts", PARTS)
+def test_product_in_parts(cuda, rows, n, k, parts, out):
+    lib = _lib.load_dense()
+    g = torch.Generator(device=cuda).manual_seed(rows + n + k)
+    ldx, ldy = k + 24, n + 8
+    x = torch.randn((rows, ldx), generator=g, device=cuda).to(torch.bfloat16)
+    w = (torch.randn((n, k), generator=g, device=cuda) * k ** -0.5).to(torch.bfloat16)
+    want = x[:, :k].double() @ w.double().t()
+    bound = k * 2.0 ** -24 * (x[:, :k].double().abs() @ w.double().t().abs())   # (as above: k roundings, wherever they fall)
+    y = torch.full((rows + 1, ldy), float("nan"), dtype=out, device=cuda)
+    room = torch.full((lib.ajqd_product_workspace(rows, n, parts) // 4 + 64,), float("nan"), device=cuda)
+    assert room.numel() == parts * rows * n + 64
+    args = _args(x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, n, k, ldx, ldy, _lib.AJQD_F32 if out == torch.float32 else _lib.AJQD_BF16)
+    _lib.check_dense(lib.ajqd_product_in_parts(ctypes.byref(args), parts, room.data_ptr(), torch.cuda.current_stream().cuda_stream), "product")
+    if out == torch.bfloat16:
+        bound = bound + 2.0 ** -8 * (want.abs() + bound)
+    assert bool(((y[:rows, :n].double() - want).abs() <= bound + 1e-30).all())
+    assert bool(y[rows:].isnan().all()) and bool(y[:, n:].isnan().all()) and bool(room[-64:].isnan().all()), "written outside the result"
+
+
+def test_parts_are_for_few_tiles_and_long_sums():
+    lib, bf16, f32 = _lib.load_dense(), _lib.AJQD_BF16, _lib.AJQD_F32
+    assert lib.ajqd_product_parts(500, 4096, 4096, f32) >= 1 and lib.ajqd_product_parts(1, 16, 64, bf16) == 1
+    assert lib.ajqd_product_parts(1500, 288, 8192, bf16) > 1 and lib.ajqd_product_parts(110, 4544, 16960, bf16) > 1
+    assert lib.ajqd_product_parts(4096, 4096, 18432, f32) == 1 and lib.ajqd_product_parts(8192, 8192, 512, bf16) == 1
+    assert not any(lib.ajqd_product_parts(*s, bf16) for s in ((500, 4096, 96), (500, 24, 64), (0, 16, 64), (500, 4096, 0)))
+    for rows, n, k in ((3, 64, 320), (700, 288, 8192), (64, 4096, 1088), (9000, 16, 18368)):
+        parts = lib.ajqd_product_parts(rows, n, k, f32)   # no part is empty, and the sums fit 128 MiB
+        assert (parts - 1) * (-(-(k // 64) // parts)) < k // 64 and (parts == 1 or lib.ajqd_product_workspace(rows, n, parts) <= 1 << 27)
+
+
 def test_product_refuses_what_it_does_not_make():
     lib = _lib.load_dense()
     buf = ctypes.create_string_buffer(4096 + 16)
@@ -74,3 +111,6 @@ def test_product_refuses_what_it_does_not_make():
     assert lib.ajqd_product_better(500, 4096, 4096) == 1 and lib.ajqd_product_better(1, 16, 64) == 1
     assert lib.ajqd_product_better(919, 640, 15488) == 0          # few tiles, long sums
     assert not any(lib.ajqd_product_better(*s) for s in ((500, 4096, 96), (500, 24, 64), (0, 16, 64), (500, 4096, 0)))
+    for change, status in ((dict(rows=0), -2), (dict(ldy=20), -3), (dict(act=1), -4), (dict(k=128, ldx=128), -1)):   # (the last: no workspace)
+        args = _args(**{**dict(x=p, w=p, y=p, rows=1, n=16, k=64, ldx=64, ldy=16), **change})
+        assert lib.ajqd_product_in_parts(ctypes.byref(args), 2, None, None) == status, change
