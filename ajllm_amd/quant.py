@@ -38,8 +38,11 @@ _raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(torch._C, "_cuda_get
 _linear = None   # the extension module's function, once it is bound
 
 
-def _bound_linear():
+def _bound_linear(inputs):
+    """The native forward, bound at the first call with a device tensor (ahead of that the general path answers, which refuses)."""
     global _linear
+    if not getattr(inputs, "is_cuda", False):
+        return lambda *args: None
     _linear = _lib.load_native().linear
     return _linear
 
@@ -364,7 +367,7 @@ class QuantLinear(nn.Module):
     def forward(self, inputs: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.Tensor:
         buffers = self._buffers
         # bf16 rows as the kernels take them: one call of native code, which leaves everything else to the lines below it
-        y = (_linear or _bound_linear())(inputs, buffers["wq"], buffers["meta"], self.scheme != "w8a16", self.in_features, self.out_features,
+        y = (_linear or _bound_linear(inputs))(inputs, buffers["wq"], buffers["meta"], self.scheme != "w8a16", self.in_features, self.out_features,
                                          out_dtype)
         if y is not None:
             return y

@@ -237,3 +237,19 @@ def test_routes_that_cut_k_leave_full_rounds_of_the_streaming_kernel_alone():
         assert lib.ajq_matmul_scratch_bytes(m, n, k, w4) == 0, (w4, m, n, k)
     for w4, m, n, k, parts in ((0, 37, 4096, 14336, 8), (1, 37, 4096, 14336, 8), (0, 44, 4096, 7808, 8), (1, 44, 8320, 5120, 3), (0, 62, 16384, 8448, 2)):
         assert lib.ajq_matmul_scratch_bytes(m, n, k, w4) == 4 * parts * m * n, (w4, m, n, k)
+
+
+def test_host_tensors_are_refused_ahead_of_the_extension_module(monkeypatch):
+    """A host tensor gets the general path's error in a process that has not bound the module (or has not built it)."""
+    import torch
+
+    from ajllm_amd import QuantLinear, quant
+
+    def load():
+        raise AssertionError("bound")
+    monkeypatch.setattr(quant, "_linear", None)
+    monkeypatch.setattr(_lib, "load_native", load)
+    layer = QuantLinear(256, 48, "w8a16")
+    layer.wq, layer.meta = torch.zeros((3, 4, 64, 4), dtype=torch.int32), torch.zeros(48, dtype=torch.float16)
+    with pytest.raises(ValueError, match="device tensors only"):
+        layer(torch.zeros((2, 256), dtype=torch.bfloat16))
