@@ -2,8 +2,8 @@
 mechanism, and ``DenseLM``, whose ``forward(token_ids, cache)`` is the one step function: whole prompts, portions of
 prompts and single tokens; ``modeling.greedy_decode``, the decoders of ``decoding`` and ``trace`` call it.
 
-All of it runs on a ROCm device, weights and activations in bf16 or fp32 (plain matrix products of prompts are the vendor
-library's).  There is no CPU path.
+All of it runs on a ROCm device, weights and activations in bf16 or fp32 (the plain matrix products of fp32 prompts are the
+vendor library's).  There is no CPU path.
 """
 
 from __future__ import annotations

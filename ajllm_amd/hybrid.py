@@ -14,7 +14,7 @@ arguments:
 
 Whatever the dtype, fp32: residual streams, norms, angles, attention scores and sums, gates, step sizes, decays and states.
 
-A prompt runs on the vendor library's products with this library's kernels between them.  A single token runs on matrix-
+A prompt runs on tile products (fp32: the vendor library's) with kernels of one job each between them.  A single token runs on matrix-
 vector kernels with what surrounds them folded in: the product that ends a sublayer updates all streams and forms the next
 sublayer's input; attention treats a key / value head as a sequence of its own for the latent decode kernel (a cache row is
 value and key at once); the scan's projection convolves its own operands.

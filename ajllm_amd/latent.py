@@ -11,8 +11,8 @@ arguments:
                          learned offset for the stream it starts from, the later ones take the embedding in again as well
 * ``LatentLM``           the decoder (``dense.DenseLM``)
 
-All of it runs on the operators of ``libajq_dense.so`` on a ROCm device, weights and activations in bf16 or fp32 (plain
-matrix products of prompts are the vendor library's).  There is no CPU path.  The residual stream, norms, angles,
+All of it runs on the operators of ``libajq_dense.so`` on a ROCm device, weights and activations in bf16 or fp32 (the plain
+matrix products of fp32 prompts are the vendor library's).  There is no CPU path.  The residual stream, norms, angles,
 attention scores and sums, gates and logits are fp32 in both.
 
 A prompt expands keys and values per head (two products per position, then attention at the head width); a single token
