@@ -244,8 +244,8 @@ __global__ __launch_bounds__(kTileThreads) void dense_gemm_kernel(DenseGemm a) {
   }
 }
 
-// y = the sum of a product's parts: eight columns of a row per thread.  Bound by its bytes, which come from the last-level cache where the
-// parts have just been written (3.3 TB/s over the launch, 1500 x 4096 in two parts).
+// y = the sum of a product's parts: eight columns of a row per thread.  Bound by its bytes, read where the parts have just been written
+// (1500 x 4096 in two parts: 13.1 us, 5.6 TB/s).
 template <typename O>
 __global__ __launch_bounds__(256) void sum_parts_kernel(const float* planes, int parts, int m, int n, O* y, int ldy) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, pieces = (size_t)m * (n / 8);
