@@ -1062,7 +1062,8 @@ MatmulKernel pick_matmul_kernel(int M, int N, int K, bool w4) {
   if (!w4) {
     MatmulKernel which = kStreaming;
     const double us = w8_tiles_us(M, N, K, which);
-    return stream && us >= 0.95 * (flops / 440e6 + 2.0) ? kStreaming : which;
+    // (the tile kernels' offsets into the activations are 32 bits wide: from 4 GiB on, what the streaming kernel takes stays with it)
+    return stream && (us >= 0.95 * (flops / 440e6 + 2.0) || (long long)M * K * 2 >= (1LL << 32)) ? kStreaming : which;
   }
   if (stream) return kStreaming;
   return us_small < us_big ? kTiles128 : kTiles256;

@@ -239,6 +239,15 @@ def test_routes_that_cut_k_leave_full_rounds_of_the_streaming_kernel_alone():
         assert lib.ajq_matmul_scratch_bytes(m, n, k, w4) == 4 * parts * m * n, (w4, m, n, k)
 
 
+def test_activations_beyond_the_tile_kernels_offsets_stay_with_the_streaming_kernel():
+    """Few columns and 4 GiB of activations or more: the streaming kernel addresses them, the int8 tile kernels (faster by the estimate) do
+    not, with the gate or without.  Just below, they are taken."""
+    lib = _lib.load()
+    for m, n, k in ((7009, 256, 306432), (2284, 768, 940416), (12500, 128, 171904)):
+        assert m * k * 2 >= 1 << 32 and lib.ajq_gemm_gate_supported(m, n, k, 0) == 0, (m, n, k)
+        assert lib.ajq_gemm_gate_supported(m - 24, n, k, 0) == 1, (m, n, k)
+
+
 def test_host_tensors_are_refused_ahead_of_the_extension_module(monkeypatch):
     """A host tensor gets the general path's error in a process that has not bound the module (or has not built it)."""
     import torch
