@@ -381,7 +381,7 @@ size_t ajqd_product_workspace(int rows, int n, int parts) { return parts > 1 ? (
 int ajqd_product_in_parts(const ajqd_product_args* a, int parts, float* workspace, void* stream) {
   if (int e = check_product("ajqd_product_in_parts", a)) return e;
   if (a->act >= 0) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_product_in_parts: an activation takes the product in one piece");
-  if (parts > 1) parts = whole_parts(a->k, parts);
+  if (parts > 1) parts = whole_parts(a->k, std::min(parts, a->k / 64));
   if (parts < 2) return ajqd_product(a, stream);
   if (!workspace) return fail(AJQ_ERR_NULL, "ajqd_product_in_parts: null workspace");
   if (!aligned16(workspace)) return fail(AJQ_ERR_ALIGN, "ajqd_product_in_parts: the workspace must start on a 16-byte boundary");
@@ -858,7 +858,9 @@ int ajqd_scan_in_parts(const ajqd_scan_args* a, int parts, float* workspace, int
   if (parts < 2) return ajqd_scan(a, dtype, stream);
   if (a->states > 16 || a->pos) return fail(AJQ_ERR_UNSUPPORTED, "ajqd_scan_in_parts: up to 16 states of a prompt are built (%d)", a->states);
   if (!workspace) return fail(AJQ_ERR_NULL, "ajqd_scan_in_parts: null workspace");
-  const int tiles = (a->seq + kScanPartTokens - 1) / kScanPartTokens, length = (tiles + parts - 1) / parts * kScanPartTokens;
+  const int tiles = (a->seq + kScanPartTokens - 1) / kScanPartTokens;
+  parts = std::min(parts, tiles);
+  const int length = (tiles + parts - 1) / parts * kScanPartTokens;
   const int count = (a->seq + length - 1) / length;
   if (count < 2) return ajqd_scan(a, dtype, stream);
   if (count > 65535) return fail(AJQ_ERR_SHAPE, "ajqd_scan_in_parts: %d parts", count);

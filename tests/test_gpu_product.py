@@ -114,3 +114,12 @@ def test_product_refuses_what_it_does_not_make():
     for change, status in ((dict(rows=0), -2), (dict(ldy=20), -3), (dict(act=1), -4), (dict(k=128, ldx=128), -1)):   # (the last: no workspace)
         args = _args(**{**dict(x=p, w=p, y=p, rows=1, n=16, k=64, ldx=64, ldy=16), **change})
         assert lib.ajqd_product_in_parts(ctypes.byref(args), 2, None, None) == status, change
+
+
+def test_more_parts_than_there_is_to_cut():
+    """Any number of parts is one: the sums that round it up must not overflow."""
+    lib = _lib.load_dense()
+    buf = ctypes.create_string_buffer(4096 + 16)
+    p = (ctypes.addressof(buf) + 15) & ~15   # host memory: only its address is looked at
+    args = _args(x=p, w=p, y=p, rows=1, n=16, k=128, ldx=128, ldy=16)
+    assert lib.ajqd_product_in_parts(ctypes.byref(args), 2**31 - 1, None, None) == -1   # (no workspace)

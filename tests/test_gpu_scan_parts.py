@@ -48,3 +48,14 @@ def test_parts_are_for_few_channels_and_long_prompts():
     assert lib.ajqd_scan_parts(1, 1500, 8192, 16) > 1 and lib.ajqd_scan_parts(2, 192, 2048, 4) > 1
     assert lib.ajqd_scan_parts(1, 100, 8192, 16) == 1 and lib.ajqd_scan_parts(4, 700, 4096, 16) == 1 and lib.ajqd_scan_parts(1, 1500, 8192, 32) == 1
     assert lib.ajqd_scan_workspace(1, 8192, 16, 1) == 0
+
+
+def test_more_parts_than_tokens():
+    """Any number of parts is one: the sums that round it up must not overflow.  (More parts than a grid has rows: refused, not launched.)"""
+    lib = _lib.load_dense()
+    buf = ctypes.create_string_buffer(4096 + 16)
+    p = (ctypes.addressof(buf) + 15) & ~15   # host memory: only its address is looked at
+    args = _lib.ScanArgs(x=p, dt=p, low=p, z=p, a2=p, d=p, dt_bias=p, state=None, pos=None, out=p, batch=1, seq=65540 * 32, start=0, inner=8,
+                         states=4, dt_ld=8, low_ld=8, b_col=0, c_col=4, z_ld=8, out_ld=8)
+    for parts in (65540, 2**31 - 1):
+        assert lib.ajqd_scan_in_parts(ctypes.byref(args), parts, p, _lib.AJQD_BF16, None) == -2
