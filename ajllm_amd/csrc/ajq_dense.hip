@@ -136,6 +136,8 @@ constexpr float kSharedTile = 1.224f;                        // of two tiles on 
 constexpr float kSumLaunch = 2.392f, kSumMegabyte = 0.299f;   // adding the parts: the launch, and what it reads and writes
 constexpr int kProductParts[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
 constexpr int kCus = 256;
+constexpr int kProductMaxK = 1 << 22;   // of a row's elements too: a tile's offsets are 32 bits
+bool product_made(int rows, int n, int k) { return rows >= 1 && n >= 16 && n % 16 == 0 && k >= 64 && k % 64 == 0 && k <= kProductMaxK; }
 long long product_tiles(int qm, int qn, int rows, int n) { return (long long)((rows + 64 * qm - 1) / (64 * qm)) * ((n + 128 * qn - 1) / (128 * qn)); }
 // steps of 64 k in a part, and the parts that come of it
 int part_steps(int k, int parts) { return (k / 64 + parts - 1) / parts; }
@@ -329,7 +331,7 @@ int ajqd_gated_activation(const void* y, int y_dtype, void* out, int out_ld, int
 }
 
 int ajqd_product_better(int rows, int n, int k) {
-  if (rows < 1 || n < 16 || n % 16 || k < 64 || k % 64) return 0;
+  if (!product_made(rows, n, k)) return 0;
   // A workgroup goes through all of k here: few tiles and a long k are made faster in parts (or by the vendor's kernels, which cut k as
   // well) with the activation behind them (61 rows, 8576 -> 528: 37 us against 20; 919 rows, 15488 -> 640: 78 against 53).  Up to k = 2048
   // (13 us in one wave of workgroups) or from a tile per CU on one piece is the faster.
@@ -341,7 +343,7 @@ namespace {
 int check_product(const char* name, const ajqd_product_args* a) {
   if (!a || !a->x || !a->w || !a->y) return fail(AJQ_ERR_NULL, "%s: null pointer argument", name);
   const int columns = a->pairs ? a->n / 2 : a->n, multiple = a->out_dtype == AJQD_F32 ? 4 : 8;
-  if (a->rows < 1 || a->n < 16 || a->n % 16 || a->k < 64 || a->k % 64 || a->k > (1 << 22) || a->ldx < a->k || a->ldx > (1 << 22) || a->ldy < columns)
+  if (!product_made(a->rows, a->n, a->k) || a->ldx < a->k || a->ldx > kProductMaxK || a->ldy < columns)
     return fail(AJQ_ERR_SHAPE, "%s: unsupported shape (rows=%d n=%d k=%d ldx=%d ldy=%d)", name, a->rows, a->n, a->k, a->ldx, a->ldy);
   if (!known(a->out_dtype) || a->act < -1 || a->act > AJQD_ACT_SQUARED_RELU || (a->out_dtype == AJQD_F32 && a->act >= 0) || (a->pairs && a->act < 0))
     return fail(AJQ_ERR_UNSUPPORTED, "%s: unsupported output (dtype=%d act=%d pairs=%d)", name, a->out_dtype, a->act, a->pairs);
@@ -362,7 +364,7 @@ int ajqd_product(const ajqd_product_args* a, void* stream) {
 }
 
 int ajqd_product_parts(int rows, int n, int k, int out_dtype) {
-  if (rows < 1 || n < 16 || n % 16 || k < 64 || k % 64 || !known(out_dtype)) return 0;
+  if (!product_made(rows, n, k) || !known(out_dtype)) return 0;
   // Few tiles leave the chip idle for all of k: then its parts are made side by side, as many as the estimates say.  Against the vendor's
   // products over the 345: 0.45 of their time (110 rows, 16960 -> 4544: 33 us, theirs 101, in one piece 83; 463 rows, 11392 -> 384: 15,
   // 27, 56; 1500 rows, 8192 -> 288: 20, 22, 42); two are slower by more than 4 %, 4 rows against 11280 x 15872 most (75, 62).  Large

@@ -77,7 +77,7 @@ typedef struct {
   void* y;
   int32_t rows, n, k, ldx, ldy, out_dtype, act, pairs;
 } ajqd_product_args;
-/* y [rows, n] = x [rows, k] w [n, k]^T, fp32 sums, out_dtype; k a multiple of 64, n of 16; ldx, ldy in elements.  act >= 0 (bf16 out):
+/* y [rows, n] = x [rows, k] w [n, k]^T, fp32 sums, out_dtype; k a multiple of 64, n of 16; ldx, ldy in elements, k and ldx up to 2^22.  act >= 0 (bf16 out):
  * act(y), or with pairs (w's rows in blocks of 8 gates and their 8 ups) act(gate) * up, [rows, n / 2].
  * ajqd_product_better says whether this is the faster way to make a product with an activation (the vendor's cuts a long K where the
  * output has few tiles). */

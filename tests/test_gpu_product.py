@@ -5,7 +5,7 @@ import ctypes
 import pytest
 import torch
 
-from ajllm_amd import _lib
+from ajllm_amd import _lib, dense
 
 PLAIN, ACT, PAIRS = "plain", "act", "pairs"
 ACTS = {
@@ -92,7 +92,7 @@ def test_parts_are_for_few_tiles_and_long_sums():
     assert lib.ajqd_product_parts(500, 4096, 4096, f32) >= 1 and lib.ajqd_product_parts(1, 16, 64, bf16) == 1
     assert lib.ajqd_product_parts(1500, 288, 8192, bf16) > 1 and lib.ajqd_product_parts(110, 4544, 16960, bf16) > 1
     assert lib.ajqd_product_parts(4096, 4096, 18432, f32) == 1 and lib.ajqd_product_parts(8192, 8192, 512, bf16) == 1
-    assert not any(lib.ajqd_product_parts(*s, bf16) for s in ((500, 4096, 96), (500, 24, 64), (0, 16, 64), (500, 4096, 0)))
+    assert not any(lib.ajqd_product_parts(*s, bf16) for s in ((500, 4096, 96), (500, 24, 64), (0, 16, 64), (500, 4096, 0), (2, 16, (1 << 22) + 64)))
     for rows, n, k in ((3, 64, 320), (700, 288, 8192), (64, 4096, 1088), (9000, 16, 18368)):
         parts = lib.ajqd_product_parts(rows, n, k, f32)   # no part is empty, and the sums fit 128 MiB
         assert (parts - 1) * (-(-(k // 64) // parts)) < k // 64 and (parts == 1 or lib.ajqd_product_workspace(rows, n, parts) <= 1 << 27)
@@ -110,10 +110,24 @@ def test_product_refuses_what_it_does_not_make():
         assert lib.ajqd_product(ctypes.byref(args), None) == status, change
     assert lib.ajqd_product_better(500, 4096, 4096) == 1 and lib.ajqd_product_better(1, 16, 64) == 1
     assert lib.ajqd_product_better(919, 640, 15488) == 0          # few tiles, long sums
-    assert not any(lib.ajqd_product_better(*s) for s in ((500, 4096, 96), (500, 24, 64), (0, 16, 64), (500, 4096, 0)))
+    assert not any(lib.ajqd_product_better(*s) for s in ((500, 4096, 96), (500, 24, 64), (0, 16, 64), (500, 4096, 0), (4096, 4096, (1 << 22) + 64)))
     for change, status in ((dict(rows=0), -2), (dict(ldy=20), -3), (dict(act=1), -4), (dict(k=128, ldx=128), -1)):   # (the last: no workspace)
         args = _args(**{**dict(x=p, w=p, y=p, rows=1, n=16, k=64, ldx=64, ldy=16), **change})
         assert lib.ajqd_product_in_parts(ctypes.byref(args), 2, None, None) == status, change
+
+
+def test_rows_that_the_product_does_not_read_are_left_to_the_vendors():
+    """Which answers, or says what does not fit: only the forms that the kernel reads are taken to it."""
+    w = torch.zeros((32, 64), dtype=torch.bfloat16)
+    x = torch.zeros((4, 88), dtype=torch.bfloat16)
+    far = torch.zeros(3 * (1 << 22), dtype=torch.bfloat16)   # (not touched)
+    assert dense._product_rows(x[:, :64], w) and dense._product_rows(far.as_strided((3, 64), (1 << 22, 1)), w)
+    for rows, weights in ((x[:, :72], w), (x[:, :64].float(), w), (x[:, :64], w.float()), (x[:, 4:68], w), (x[:, :64], torch.zeros((64, 32), dtype=w.dtype).t()),
+                          (x[:, :64], torch.zeros((32, 128), dtype=w.dtype)[:, ::2]), (x[:1, :64].expand(4, 64), w), (x.as_strided((4, 64), (8, 1)), w),
+                          (far.as_strided((2, 64), ((1 << 22) + 8, 1)), w), (x[:, :64], w.to("meta"))):
+        assert not dense._product_rows(rows, weights), (rows.shape, rows.stride(), weights.stride())
+    with pytest.raises(RuntimeError):
+        dense._product(x[:, :72], w, torch.bfloat16)
 
 
 def test_more_parts_than_there_is_to_cut():
