@@ -295,6 +295,10 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+class NativeModuleMissing(RuntimeError):
+    """The extension module cannot be imported (the operator library may well be there)."""
+
+
 def load_native():
     """The extension module, bound to the operator library on first use (built by ``python -m ajllm_amd.build``)."""
     global _native
@@ -302,8 +306,8 @@ def load_native():
         try:
             from . import _native as module
         except ImportError as error:
-            raise RuntimeError("ajllm_amd/_native.so is missing or does not fit this interpreter: build it with "
-                               "`python -m ajllm_amd.build`") from error
+            raise NativeModuleMissing("ajllm_amd/_native.so is missing or does not fit this interpreter: build it with "
+                                      "`python -m ajllm_amd.build`") from error
         lib = load()
         module.bind(*(ctypes.cast(getattr(lib, name), c_void_p).value for name in (
             "ajq_w4a16_gemv", "ajq_w8a16_gemv", "ajq_w4a16_matmul", "ajq_w8a16_matmul", "ajq_matmul_scratch_bytes")))

@@ -2,7 +2,8 @@
 ``_native.so``.
 
 Cross-compiles for gfx950 with hipcc; needs no GPU.  Run as
-``python -m ajllm_amd.build`` or call :func:`build_library`.
+``python -m ajllm_amd.build`` or call :func:`build_library`, which makes all that a quantized layer needs
+(without the extension module its calls take longer on the host).
 """
 
 from __future__ import annotations

@@ -14,6 +14,8 @@ ROCm device; there is no CPU path here.
 
 from __future__ import annotations
 
+import warnings
+
 import torch
 from torch import nn
 
@@ -39,12 +41,21 @@ _linear = None   # the extension module's function, once it is bound
 
 
 def _bound_linear(inputs):
-    """The native forward, bound at the first call with a device tensor (ahead of that the general path answers, which refuses)."""
+    """The native forward, bound at the first call with a device tensor (ahead of that the general path answers, which refuses).  Without
+    the extension module, or with one built for another interpreter, the general path answers every call."""
     global _linear
     if not getattr(inputs, "is_cuda", False):
-        return lambda *args: None
-    _linear = _lib.load_native().linear
+        return _leave
+    try:
+        _linear = _lib.load_native().linear
+    except _lib.NativeModuleMissing as error:
+        _linear = _leave
+        warnings.warn(f"{error}; until then a quantized layer's call takes the longer way through the interpreter", RuntimeWarning, stacklevel=3)
     return _linear
+
+
+def _leave(*args) -> None:
+    """In the native forward's place: every call is left to the general path."""
 
 
 def _require_cuda(*tensors: torch.Tensor) -> None:

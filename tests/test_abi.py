@@ -262,3 +262,22 @@ def test_host_tensors_are_refused_ahead_of_the_extension_module(monkeypatch):
     layer.wq, layer.meta = torch.zeros((3, 4, 64, 4), dtype=torch.int32), torch.zeros(48, dtype=torch.float16)
     with pytest.raises(ValueError, match="device tensors only"):
         layer(torch.zeros((2, 256), dtype=torch.bfloat16))
+
+
+def test_a_layer_does_without_the_extension_module(monkeypatch):
+    """Where the module is missing, or was built for another interpreter, the general path answers: with one warning, not with an error."""
+    import sys
+    from types import SimpleNamespace
+
+    import ajllm_amd
+    from ajllm_amd import quant
+
+    monkeypatch.setattr(quant, "_linear", None)
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.delattr(ajllm_amd, "_native", raising=False)
+    monkeypatch.setitem(sys.modules, "ajllm_amd._native", None)   # an import of it fails
+    with pytest.warns(RuntimeWarning, match="_native.so is missing"):
+        first = quant._bound_linear(SimpleNamespace(is_cuda=True))
+    assert first() is None and quant._linear is first
+    with pytest.raises(RuntimeError, match="ajllm_amd.build"):
+        _lib.load_native()

@@ -93,6 +93,15 @@ def test_anything_else_takes_the_general_path(cuda, calls):
         torch.func.vmap(layer)(x[:, None])
 
 
+def test_without_the_module(cuda, calls, monkeypatch):
+    layer, x = _layer("w4a16_g128", 1000, 256, cuda), _x(cuda, 2, 3, 256)
+    want = layer(x)
+    assert not calls
+    monkeypatch.setattr(quant, "_linear", quant._leave)
+    got = layer(x)
+    assert len(calls) == 1 and torch.equal(got, want) and got.stride() == want.stride()
+
+
 def test_on_a_stream_and_in_a_graph(cuda):
     layer, x = _layer("w8a16", 4096, 14336, cuda), _x(cuda, 37, 14336)
     want = layer(x)
