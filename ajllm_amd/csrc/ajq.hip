@@ -125,22 +125,25 @@ int check_matmul_args(const char* name, const void* x, int M, int K, const void*
 #ifndef AJQ_GEMM_WIDE
 #define AJQ_GEMM_WIDE 1
 #endif
+bool takes_wide_tiles(int M, int N, bool gate) {
+  if (!AJQ_GEMM_WIDE || (gate && (N / 2) % (kGWBN / 2) != 0)) return false;
+  // 256 x 256 tiles move half the activation bytes per MFMA and measure 9-15 % faster per flop, but there are half
+  // as many of them: they run when that still fills the CUs' rounds better (a wide tile takes 2 / 1.12 narrow ones)
+  const long long wide = (long long)((M + kGWBM - 1) / kGWBM) * ((N + kGWBN - 1) / kGWBN);
+  const int tiles = ((M + kG2BM - 1) / kG2BM) * ((N + kG2BN - 1) / kG2BN);
+  return (double)((wide + 255) / 256) * (2.0 / 1.12) < (double)((tiles + 255) / 256);
+}
 template <bool kW4, bool kGate = false>
 int launch_gemm256(const uint16_t* x, int M, int K, const uint32_t* wq, const uint32_t* meta, const uint16_t* scales8,
                    int N, void* y, int out_f32, hipStream_t stream) {
   const int tiles = ((M + kG2BM - 1) / kG2BM) * ((N + kG2BN - 1) / kG2BN);
-  if (kW4 && (!kGate || (N / 2) % (kGWBN / 2) == 0)) {
-    // 256 x 256 tiles move half the activation bytes per MFMA and measure 9-15 % faster per flop, but there are half
-    // as many of them: they run when that still fills the CUs' rounds better (a wide tile takes 2 / 1.12 narrow ones)
+  if (kW4 && takes_wide_tiles(M, N, kGate)) {
     const long long wide = (long long)((M + kGWBM - 1) / kGWBM) * ((N + kGWBN - 1) / kGWBN);
-    const double cost_wide = (double)((wide + 255) / 256) * (2.0 / 1.12), cost_narrow = (double)((tiles + 255) / 256);
-    if (AJQ_GEMM_WIDE && cost_wide < cost_narrow) {
-      auto kernel = dequant_gemm256w_kernel<kW4, kGate>;
-      if (int s = allow_big_lds(kernel, kGWLdsBytes)) return s;
-      hipLaunchKernelGGL(kernel, dim3((unsigned)wide), dim3(kGWThreads), kGWLdsBytes, stream, x, M, K,
-                         reinterpret_cast<const u32x4_t*>(wq), meta, scales8, N, y, out_f32);
-      return AJQ_OK;
-    }
+    auto kernel = dequant_gemm256w_kernel<kW4, kGate>;
+    if (int s = allow_big_lds(kernel, kGWLdsBytes)) return s;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)wide), dim3(kGWThreads), kGWLdsBytes, stream, x, M, K,
+                       reinterpret_cast<const u32x4_t*>(wq), meta, scales8, N, y, out_f32);
+    return AJQ_OK;
   }
   if (!kW4 && K % 256 == 0) {
     auto ring = dequant_gemm256r_w8_kernel<kGate>;
@@ -1019,6 +1022,10 @@ int check_pro(const char* name, int M, int K, const void* a, const void* b) {
 // once run at a higher clock.  Over 520 of the shapes the choice takes 0.94 of the time (geometric mean) of a choice between the
 // last two kernels, 256 x 256 tiles that read ahead of their MFMAs and the streaming kernel by the weights above.  Tiles are taken
 // beyond those weights where they are estimated to be faster than 440 TFLOP/s (229 rows, 3200 -> 8432: 35.7 -> 23.7 us).
+// Checked on 350 others (K from 128 on, both output types) against the choice between the last two: 0.93 of its time; 3 slower by more
+// than 5 % (2477 rows, 256 -> 2768: 10.5 us, 11.6).  The 192 x 128 tile's own time is from these: K below 1024 was not among the 740,
+// and the 0.69 fitted to them had it run where it is the slower one (fp32, 2994 rows, 128 -> 4544: 17.9 us, now 15.8; 1143 rows,
+// 896 -> 23984: 74.4, now 64.2).
 #ifndef AJQ_GEMM_TILE
 #define AJQ_GEMM_TILE 0  // 0: by the estimate; 128 or 256: that tile kernel for every M it can run
 #endif
@@ -1029,7 +1036,7 @@ struct TileTimes {
   double launch, tile, step, least;
 };
 constexpr TileTimes kW8Tiles[] = {{kTurns256, 256, 256, 256, 1.91, 8.84, 1.441, 0.727}, {kTurns192, 192, 256, 17, 1.11, 7.51, 1.132, 0.811},
-                                  {kTurns128, 128, 256, 17, 1.00, 5.16, 0.861, 0.802},  {kTurns192Narrow, 192, 128, 17, 5.18, 0.69, 0.705, 0.894},
+                                  {kTurns128, 128, 256, 17, 1.00, 5.16, 0.861, 0.802},  {kTurns192Narrow, 192, 128, 17, 5.18, 2.00, 0.705, 0.894},
                                   {kTiles256, 256, 128, 256, 0.25, 6.51, 0.776, 0.656}, {kTiles128, 128, 128, 128, 0.04, 4.31, 0.499, 0.694}};
 double w8_tiles_us(int M, int N, int K, MatmulKernel& which) {
   double least = 1e30;
@@ -1463,6 +1470,19 @@ int ajq_w8a16_gemm(const uint16_t* x, int M, int K, const uint32_t* wq, const ui
     return fail(AJQ_ERR_SHAPE, "ajq_w8a16_gemm: M * K = %lld exceeds the 32-bit activation offsets", (long long)M * K);
   if (int s = launch_w8_tiles<false>(which, x, M, K, wq, scales, N, y, out_f32, (hipStream_t)stream)) return s;
   return check_launch("ajq_w8a16_gemm");
+}
+
+int ajq_matmul_tile(int M, int N, int K, int w4) {
+  if (M <= kMaxGemvM || N < kTileN || N % kTileN || K < kGroup || K % kGroup) return 0;
+  switch (pick_matmul_kernel(M, N, K, w4 != 0)) {
+    case kStreaming: return 0;
+    case kTiles128: return kG1BM << 16 | kG1BN;
+    case kTurns256: return 256 << 16 | 256;
+    case kTurns192: return 192 << 16 | 256;
+    case kTurns128: return 128 << 16 | 256;
+    case kTurns192Narrow: return 192 << 16 | 128;
+    default: return w4 && takes_wide_tiles(M, N, false) ? kGWBM << 16 | kGWBN : kG2BM << 16 | kG2BN;
+  }
 }
 
 // ---- w1 | w3 GEMM with the SwiGLU gate formed in the epilogue (tile kernels only)

@@ -247,6 +247,8 @@ int ajq_matmul_workspace_set(void* workspace, size_t bytes);
  * ajq_matmul_scratch_bytes says how many bytes (0: none; w4: 1 for W4, 0 for W8).  With a smaller workspace (or none) the call
  * runs as ajq_*_gemm does. */
 size_t ajq_matmul_scratch_bytes(int M, int N, int K, int w4);
+/* The tiles that run a matmul in one piece, rows << 16 | columns; 0: the kernels without tiles. */
+int ajq_matmul_tile(int M, int N, int K, int w4);
 int ajq_w4a16_matmul(const uint16_t* x, int M, int K, const uint32_t* wq, const uint32_t* meta, int N, void* y, int out_dtype,
                      void* workspace, size_t workspace_bytes, void* stream);
 int ajq_w8a16_matmul(const uint16_t* x, int M, int K, const uint32_t* wq, const uint16_t* scales, int N, void* y, int out_dtype,

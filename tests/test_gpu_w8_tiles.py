@@ -8,9 +8,32 @@ import torch
 
 from ajllm_amd import _lib, asm_check, repack_w8
 
-# (rows, columns, K) by the tile they take: 192 x 128 (three), 128 x 256 (three), 192 x 256 (two), 256 x 256 (three)
-SIZES = [(2049, 5136, 128), (2305, 2064, 384), (3841, 4112, 384), (1537, 4112, 256), (600, 12304, 256), (257, 16400, 1024), (900, 9232, 384),
-         (520, 14352, 512), (3900, 3856, 640), (1000, 15888, 640), (3500, 4560, 512)]
+# (rows, columns, K) by the tile they take
+SIZES = {(192, 128): [(3841, 4112, 384), (1007, 10800, 128), (993, 10800, 256), (986, 10784, 384)],
+         (128, 256): [(1537, 4112, 256), (600, 12304, 256), (257, 16400, 1024)],
+         (192, 256): [(900, 9232, 384), (520, 14352, 512), (2049, 5136, 128)],
+         (256, 256): [(3900, 3856, 640), (1000, 15888, 640), (3500, 4560, 512)],
+         (256, 128): [(2305, 2064, 384)]}   # (their waves do not take turns: one more size of the int8 form)
+GATED = {(192, 128): [(998, 5440, 128), (978, 5440, 384)], (128, 256): [(1537, 2112, 256)], (192, 256): [(2049, 2624, 128), (900, 4672, 384)],
+         (256, 256): [(3900, 1984, 640)]}
+
+
+def test_sizes_take_the_tiles_they_are_listed_under():
+    lib = _lib.load()
+    for tile, sizes in SIZES.items():
+        for m, n, k in sizes:
+            assert divmod(lib.ajq_matmul_tile(m, n, k, 0), 1 << 16) == tile, (m, n, k)
+    for tile, sizes in GATED.items():
+        for m, f, k in sizes:
+            assert divmod(lib.ajq_matmul_tile(m, 2 * f, k, 0), 1 << 16) == tile, (m, f, k)
+
+
+def test_short_k_takes_the_tile_that_measured_faster():
+    """Below K = 1024 the 192 x 128 tile was chosen by times extrapolated from longer sums (fp32 out, us there / at the tile below: 17.9 / 15.8,
+    18.1 / 15.5, 17.8 / 16.0, 74.7 / 64.2, 169.5 / 147.6)."""
+    lib = _lib.load()
+    for m, n, k in ((2994, 4544, 128), (765, 17584, 128), (5888, 2336, 128), (1143, 23984, 896), (3109, 29472, 512)):
+        assert divmod(lib.ajq_matmul_tile(m, n, k, 0), 1 << 16) == (256, 256), (m, n, k)
 
 
 def _weights(n, k, cuda):
@@ -26,7 +49,7 @@ def _bound(x, w, k):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k", SIZES)
+@pytest.mark.parametrize("m,n,k", [s for sizes in SIZES.values() for s in sizes])
 def test_w8_tiles(cuda, m, n, k):
     lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
     wq, scales, w = _weights(n, k, cuda)
@@ -41,7 +64,7 @@ def test_w8_tiles(cuda, m, n, k):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,f,k", [(2049, 2624, 128), (1537, 2112, 256), (900, 4672, 384), (3900, 1984, 640)])
+@pytest.mark.parametrize("m,f,k", [s for sizes in GATED.values() for s in sizes])
 def test_w8_tiles_with_the_gate(cuda, m, f, k):
     lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
     wq, scales, w = _weights(2 * f, k, cuda)
