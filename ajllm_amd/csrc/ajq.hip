@@ -1035,9 +1035,9 @@ struct TileTimes {
   int bm, bn, least_rows;
   double launch, tile, step, least;
 };
-constexpr TileTimes kW8Tiles[] = {{kTurns256, 256, 256, 256, 1.91, 8.84, 1.441, 0.727}, {kTurns192, 192, 256, 17, 1.11, 7.51, 1.132, 0.811},
-                                  {kTurns128, 128, 256, 17, 1.00, 5.16, 0.861, 0.802},  {kTurns192Narrow, 192, 128, 17, 5.18, 2.00, 0.705, 0.894},
-                                  {kTiles256, 256, 128, 256, 0.25, 6.51, 0.776, 0.656}, {kTiles128, 128, 128, 128, 0.04, 4.31, 0.499, 0.694}};
+constexpr TileTimes kW8Tiles[] = {{kTurns256, 256, 256, 256, 1.91, 8.84, 1.441, 0.727}, {kTurns192, 192, 256, kG1BM, 1.11, 7.51, 1.132, 0.811},
+                                  {kTurns128, 128, 256, kG1BM, 1.00, 5.16, 0.861, 0.802},  {kTurns192Narrow, 192, 128, kG1BM, 5.18, 2.00, 0.705, 0.894},
+                                  {kTiles256, 256, 128, 256, 0.25, 6.51, 0.776, 0.656}, {kTiles128, 128, 128, kG1BM, 0.04, 4.31, 0.499, 0.694}};
 double w8_tiles_us(int M, int N, int K, MatmulKernel& which) {
   double least = 1e30;
   for (const TileTimes& t : kW8Tiles) {
@@ -1155,7 +1155,7 @@ SplitRoute pick_split(int M, int N, int K, bool w4) {
     other = std::min(other, (double)(((M + 255) / 256 * tn + 255) / 256) * G * (w4 ? 1.45 : 1.15) + 5.0);
   if (split >= 0.88 * other) return r;
   MatmulKernel which;
-  if (!w4 && w8_tiles_us(M, N, K, which) < 0.9 * split) return r;
+  if (!w4 && M >= kG1BM && w8_tiles_us(M, N, K, which) < 0.9 * split) return r;  // (fewer rows would go to the streaming kernel)
   r.kind = kRouteTiles;
   r.S = S;
   r.sums = w4 ? (group_sum_bytes(M, K) + 255) / 256 * 256 : 0;
