@@ -137,14 +137,14 @@ template <bool kW4, bool kGate = false>
 int launch_gemm256(const uint16_t* x, int M, int K, const uint32_t* wq, const uint32_t* meta, const uint16_t* scales8,
                    int N, void* y, int out_f32, hipStream_t stream) {
   const int tiles = ((M + kG2BM - 1) / kG2BM) * ((N + kG2BN - 1) / kG2BN);
-  if (kW4 && takes_wide_tiles(M, N, kGate)) {
-    const long long wide = (long long)((M + kGWBM - 1) / kGWBM) * ((N + kGWBN - 1) / kGWBN);
-    auto kernel = dequant_gemm256w_kernel<kW4, kGate>;
-    if (int s = allow_big_lds(kernel, kGWLdsBytes)) return s;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)wide), dim3(kGWThreads), kGWLdsBytes, stream, x, M, K,
-                       reinterpret_cast<const u32x4_t*>(wq), meta, scales8, N, y, out_f32);
-    return AJQ_OK;
-  }
+  if constexpr (kW4)
+    if (takes_wide_tiles(M, N, kGate)) {
+      auto kernel = dequant_gemm256w_kernel<kGate>;
+      if (int s = allow_big_lds(kernel, kGWLdsBytes)) return s;
+      hipLaunchKernelGGL(kernel, dim3(((M + kGWBM - 1) / kGWBM) * ((N + kGWBN - 1) / kGWBN)), dim3(kGWThreads), kGWLdsBytes, stream, x, M, K,
+                         reinterpret_cast<const u32x4_t*>(wq), meta, N, y, out_f32);
+      return AJQ_OK;
+    }
   if (!kW4 && K % 256 == 0) {
     auto ring = dequant_gemm256r_w8_kernel<kGate>;
     if (int s = allow_big_lds(ring, kGRLdsBytes)) return s;

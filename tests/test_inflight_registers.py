@@ -36,8 +36,9 @@ TILE_SOURCE = """
 #include "gemm_wide_kernels.h"
 namespace ajq {
 #define TILE const uint16_t*, int, int, const u32x4_t*, const uint32_t*, const uint16_t*, int, void*, int
-template __global__ void dequant_gemm256w_kernel<false, false>(TILE);
-template __global__ void dequant_gemm256w_kernel<true, true>(TILE);
+#define WIDE const uint16_t*, int, int, const u32x4_t*, const uint32_t*, int, void*, int
+template __global__ void dequant_gemm256w_kernel<false>(WIDE);
+template __global__ void dequant_gemm256w_kernel<true>(WIDE);
 template __global__ void dequant_gemm256s_kernel<true, false>(TILE);
 template __global__ void dequant_gemm256r_w8_kernel<false>(const uint16_t*, int, int, const u32x4_t*, const uint16_t*, int, void*, int);
 }
