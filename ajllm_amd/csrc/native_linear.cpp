@@ -34,7 +34,7 @@ const at::Tensor* plain(PyObject* object) {
   const at::Tensor& t = THPVariable_Unpack(object);
   const c10::DispatchKeySet special({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
                                      c10::DispatchKey::Functionalize, c10::DispatchKey::Conjugate, c10::DispatchKey::Negative,
-                                     c10::DispatchKey::ZeroTensor});
+                                     c10::DispatchKey::ZeroTensor, c10::DispatchKey::Named});
   return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(special) ? &t : nullptr;
 }
 

@@ -91,6 +91,8 @@ def test_anything_else_takes_the_general_path(cuda, calls):
         layer(x.cpu())
     with pytest.raises(RuntimeError):
         torch.func.vmap(layer)(x[:, None])
+    with pytest.raises(RuntimeError, match="named tensors"):
+        layer(x.rename("rows", "columns"))
 
 
 def test_without_the_module(cuda, calls, monkeypatch):
