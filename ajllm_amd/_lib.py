@@ -223,6 +223,7 @@ DENSE_SIGNATURES: dict[str, tuple] = {
     "ajqd_product_better": (c_int, [_I, _I, _I]),
     "ajqd_product": (c_int, [ctypes.POINTER(ProductArgs), _P]),
     "ajqd_product_parts": (c_int, [_I, _I, _I, _I]),
+    "ajqd_product_tile": (c_int, [_I, _I, _I, _I, _I, _I]),
     "ajqd_product_workspace": (c_size_t, [_I, _I, _I]),
     "ajqd_product_in_parts": (c_int, [ctypes.POINTER(ProductArgs), _I, _P, _P]),
     "ajqd_matvec": (c_int, [_P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P]),

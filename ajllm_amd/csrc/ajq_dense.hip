@@ -159,6 +159,7 @@ int pick_product_tile(int rows, int n, int k, int out_bytes, int parts, float* u
   if (us) *us = least;
   return best;
 }
+int product_out_bytes(int out_dtype, int pairs) { return out_dtype == AJQD_F32 ? 4 : pairs ? 1 : 2; }
 template <int QM, int QN, int EPI>
 int launch_product(const DenseGemm& a, hipStream_t stream) {
   constexpr int bytes = tile_lds_bytes(64 * QM, 128 * QN, EPI);
@@ -357,7 +358,7 @@ extern "C" {
 int ajqd_product(const ajqd_product_args* a, void* stream) {
   if (int e = check_product("ajqd_product", a)) return e;
   DenseGemm d{(const uint16_t*)a->x, (const uint16_t*)a->w, a->y, a->rows, a->n, a->k, a->ldx, a->ldy, a->act, a->k};
-  const int tile = pick_product_tile(a->rows, a->n, a->k, a->out_dtype == AJQD_F32 ? 4 : a->pairs ? 1 : 2, 1);
+  const int tile = pick_product_tile(a->rows, a->n, a->k, product_out_bytes(a->out_dtype, a->pairs), 1);
   if (a->out_dtype == AJQD_F32) return launch_product_tile<kTileF32>(tile, d, (hipStream_t)stream);
   if (a->act < 0) return launch_product_tile<kTileBf16>(tile, d, (hipStream_t)stream);
   return a->pairs ? launch_product_tile<kTilePairs>(tile, d, (hipStream_t)stream) : launch_product_tile<kTileAct>(tile, d, (hipStream_t)stream);
@@ -374,10 +375,16 @@ int ajqd_product_parts(int rows, int n, int k, int out_dtype) {
   for (int parts : kProductParts) {
     // (what the estimates were fitted to; 128 MiB of sums at most)
     if (parts > 1 && (k / parts < 256 || (long long)rows * n * parts > (1LL << 25))) continue;
-    pick_product_tile(rows, n, k, out_dtype == AJQD_F32 ? 4 : 2, parts, &us);
+    pick_product_tile(rows, n, k, product_out_bytes(out_dtype, 0), parts, &us);
     if (parts == 1 || us < least) { best = parts; least = us; }
   }
   return whole_parts(k, best);
+}
+int ajqd_product_tile(int rows, int n, int k, int out_dtype, int pairs, int parts) {
+  if (!product_made(rows, n, k) || !known(out_dtype)) return 0;
+  parts = whole_parts(k, std::max(1, std::min(parts, k / 64)));
+  const ProductTile& t = kProductTiles[pick_product_tile(rows, n, k, product_out_bytes(out_dtype, pairs), parts)];
+  return 64 * t.qm << 16 | 128 * t.qn;
 }
 size_t ajqd_product_workspace(int rows, int n, int parts) { return parts > 1 ? (size_t)parts * rows * n * sizeof(float) : 0; }
 int ajqd_product_in_parts(const ajqd_product_args* a, int parts, float* workspace, void* stream) {
@@ -389,7 +396,7 @@ int ajqd_product_in_parts(const ajqd_product_args* a, int parts, float* workspac
   if (!aligned16(workspace)) return fail(AJQ_ERR_ALIGN, "ajqd_product_in_parts: the workspace must start on a 16-byte boundary");
   const long long blocks = ((long long)a->rows * (a->n / 8) + 255) / 256;
   if (parts > 65535 || blocks > 0x7FFFFFFFll) return fail(AJQ_ERR_SHAPE, "ajqd_product_in_parts: too many workgroups");
-  const int out_bytes = a->out_dtype == AJQD_F32 ? 4 : 2, tile = pick_product_tile(a->rows, a->n, a->k, out_bytes, parts);
+  const int out_bytes = product_out_bytes(a->out_dtype, 0), tile = pick_product_tile(a->rows, a->n, a->k, out_bytes, parts);
   const DenseGemm d{(const uint16_t*)a->x, (const uint16_t*)a->w, workspace, a->rows, a->n, a->k, a->ldx, a->n, -1, 64 * part_steps(a->k, parts)};
   if (int e = launch_product_tile<kTileF32>(tile, d, (hipStream_t)stream)) return e;
   if (out_bytes == 4)

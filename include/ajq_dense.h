@@ -87,6 +87,8 @@ int ajqd_product(const ajqd_product_args* args, void* stream);
  * launch adds.  ajqd_product_parts: in how many parts it is made fastest; 0 where it is not made. */
 int ajqd_product_parts(int rows, int n, int k, int out_dtype);
 size_t ajqd_product_workspace(int rows, int n, int parts);
+/* the tile that makes it, rows << 16 | columns (0 where it is not made) */
+int ajqd_product_tile(int rows, int n, int k, int out_dtype, int pairs, int parts);
 int ajqd_product_in_parts(const ajqd_product_args* args, int parts, float* workspace, void* stream);
 
 typedef struct {

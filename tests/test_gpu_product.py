@@ -19,9 +19,33 @@ def _args(x, w, y, rows, n, k, ldx, ldy, out=_lib.AJQD_BF16, act=-1, pairs=0):
 
 
 # (rows, n, k): the smallest; a row and a tile's rows around 64; tiles of 64 x 128, 192 x 128, 128 x 128, 128 x 256, 192 x 256,
-# 256 x 256 with remainders on both sides; one, two, an odd and an even number of 64-k steps
+# 256 x 256 with remainders on both sides (asserted below); one, two, an odd and an even number of 64-k steps
 SIZES = [(1, 16, 64), (63, 144, 64), (65, 272, 192), (500, 1008, 320), (257, 16000, 192), (1025, 4112, 320), (4097, 4112, 64),
-         (1537, 4080, 64), (2040, 4080, 640), (2049, 5008, 128), (3000, 4048, 640), (3080, 8080, 64), (4000, 4016, 192)]
+         (1537, 4080, 64), (2040, 4080, 640), (2049, 5008, 128), (3000, 4048, 640), (3080, 8080, 64), (4000, 4016, 192),
+         (387, 4624, 192), (2307, 784, 256)]
+TILES = {(64, 128), (128, 128), (192, 128), (128, 256), (192, 256), (256, 256)}
+FORMS = {"fp32": (_lib.AJQD_F32, 0), "bf16": (_lib.AJQD_BF16, 0), "pairs": (_lib.AJQD_BF16, 1)}
+
+
+def _tiles(sizes, out, pairs):
+    """The tiles that sizes take with several of them and a remainder on both sides, and more steps of 64 k than the tile has buffers."""
+    lib, found = _lib.load_dense(), set()
+    for rows, n, k, *parts in sizes:
+        high, wide = divmod(lib.ajqd_product_tile(rows, n, k, out, pairs, *(parts or (1,))), 1 << 16)
+        if rows > high and rows % high and n > wide and n % wide and (parts or k >= 192):
+            found.add((high, wide))
+    return found
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_sizes_take_every_tile_in_every_form(form):
+    assert _tiles(SIZES, *FORMS[form]) == TILES
+
+
+@pytest.mark.parametrize("out", [_lib.AJQD_F32, _lib.AJQD_BF16])
+def test_sizes_in_parts_take_every_tile(out):
+    assert _tiles(PARTS, out, 0) == TILES
+    assert _lib.load_dense().ajqd_product_tile(64, 24, 64, out, 0, 1) == 0
 
 
 @pytest.mark.gpu
@@ -62,7 +86,8 @@ def test_product(cuda, rows, n, k, kind, out):
 
 
 # a part of one and of several 64-k steps, a last part that is shorter, more parts than steps, remainders of every tile's sides
-PARTS = [(1, 16, 128, 2), (65, 272, 192, 3), (130, 144, 448, 3), (500, 1008, 320, 4), (257, 4112, 640, 4), (1025, 1040, 832, 7), (33, 48, 320, 9)]
+PARTS = [(1, 16, 128, 2), (65, 272, 192, 3), (130, 144, 448, 3), (500, 1008, 320, 4), (257, 4112, 640, 4), (1025, 1040, 832, 7), (33, 48, 320, 9),
+         (129, 3616, 320, 4), (262, 3632, 320, 3), (770, 3120, 448, 4)]
 
 
 @pytest.mark.gpu
