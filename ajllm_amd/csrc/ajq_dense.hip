@@ -122,10 +122,14 @@ int launch_prefill_vt(int vt, const WindowedAttention& w, hipStream_t stream) {
 }
 
 // ---- products of many rows: tiles of 64 QM x 128 QN.  Microseconds of a tile that has a CU to itself, of its 64 k, and of its output's
-// bytes per element; and of the launch.  Fitted to the times of 345 random products (1 .. 9000 rows, 64 .. 22000 columns, k up to 18000;
-// every tile, k in one piece and in up to 24 parts) in a row of milliseconds with weights that are in no cache, as a model's are: the tile
-// and parts chosen with them take 1.3 % longer than the best ones on average.  (Fitted to short runs on weights that stay cached, 1500
+// bytes per element; and of the launch.  They settle the choice and are not the kernels' times: fitted to 345 random products (1 .. 9000
+// rows, 64 .. 22000 columns, k up to 18000; every tile, k in one piece and in up to 24 parts) in a row of milliseconds with weights that are
+// in no cache, as a model's are, each by how near the best of its size it is.  (Fitted to short runs on weights that stay cached, 1500
 // rows, 16384 -> 4096 came out as one piece: 162 us against 155 in two parts there, but 188 against 168 in a model.)
+// On 690 others (2 .. 9000 rows, 16 .. 116000 columns, k 64 .. 18432) they are 25 % off (rms), as a rule 17 % low and at large sizes, where
+// the clock falls, up to 40 % (8192 x 8192 x 8192: 551 us, measured 679).  What they choose takes 1.1 % longer than the best of the size
+// on average and more than 10 % at 26 of them (118 rows, 8192 -> 13936: 66.4 us, 55.9 in three parts).  Times with a power and a
+// memory limit, fitted without that weighting to 10 %, chose worse (3 %).
 struct ProductTile {
   int qm, qn;
   float launch, tile, step, out;
@@ -333,9 +337,11 @@ int ajqd_gated_activation(const void* y, int y_dtype, void* out, int out_ld, int
 
 int ajqd_product_better(int rows, int n, int k) {
   if (!product_made(rows, n, k)) return 0;
-  // A workgroup goes through all of k here: few tiles and a long k are made faster in parts (or by the vendor's kernels, which cut k as
-  // well) with the activation behind them (61 rows, 8576 -> 528: 37 us against 20; 919 rows, 15488 -> 640: 78 against 53).  Up to k = 2048
-  // (13 us in one wave of workgroups) or from a tile per CU on one piece is the faster.
+  // A workgroup goes through all of k here: few tiles and a long k are made faster in parts with the activation behind them (61 rows,
+  // 8576 -> 528: 37 us against 20; 919 rows, 15488 -> 640: 78 against 53).  Up to k = 2048 (13 us in one wave of workgroups) or from a tile
+  // per CU on one piece is the faster as a rule: over 433 such products 0.75 of the time of the other way.  24 of them are slower by more
+  // than 5 % (16 rows, 2048 -> 2048: 19.7 us against 10.6; 582 rows, 11264 -> 8656: 147 against 135) and stay, as their activation is taken
+  // of the fp32 sum here and of its bf16 rounding there.
   return k <= 2048 || product_tiles(1, 1, rows, n) >= kCus;
 }
 
@@ -368,8 +374,9 @@ int ajqd_product_parts(int rows, int n, int k, int out_dtype) {
   if (!product_made(rows, n, k) || !known(out_dtype)) return 0;
   // Few tiles leave the chip idle for all of k: then its parts are made side by side, as many as the estimates say.  Against the vendor's
   // products over the 345: 0.45 of their time (110 rows, 16960 -> 4544: 33 us, theirs 101, in one piece 83; 463 rows, 11392 -> 384: 15,
-  // 27, 56; 1500 rows, 8192 -> 288: 20, 22, 42); two are slower by more than 4 %, 4 rows against 11280 x 15872 most (75, 62).  Large
-  // outputs stay in one piece (4096 rows, 18432 -> 4096: 413 us, in two parts 447).
+  // 27, 56; 1500 rows, 8192 -> 288: 20, 22, 42); over 690 others 0.80 of it where a product takes 40 us or more, and nine are slower by 3 to
+  // 10 %, most of them heads of 17 to 250 rows (63 rows, 3008 -> 43408: 59.7 us, 54.5).  Large outputs stay in one piece (4096 rows,
+  // 18432 -> 4096: 413 us, in two parts 447).
   int best = 1;
   float least = 0.f, us;
   for (int parts : kProductParts) {
