@@ -82,8 +82,10 @@ def _stream() -> int:
 
 def _product_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether this library's product reads ``x`` and ``w``: bf16 rows of one length that start on 16-byte boundaries, at most 2^22 apart."""
-    return (x.dtype == w.dtype == torch.bfloat16 and x.shape[1] == w.shape[1] and x.device == w.device and w.is_contiguous()
-            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.shape[1] <= x.stride(0) <= 1 << 22 and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+    k = w.shape[1]
+    apart, unit = x.stride()
+    return (x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and x.shape[1] == k and unit == 1 and k <= apart <= 1 << 22 and apart % 8 == 0
+            and w.is_contiguous() and x.device == w.device and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def _own_product(x: torch.Tensor, w: torch.Tensor) -> bool:
