@@ -186,6 +186,59 @@ int launch_product_tile(int tile, const DenseGemm& a, hipStream_t stream) {
   }
 }
 
+// ---- products of one decode step
+constexpr int kTwoWaveColumns = 256;  // products of one or two blocks of columns run on two waves (stream_rows)
+// Batch rows go through LDS (stream_rows) where K is whole blocks and gives a wave some to stream; with less the trip costs more than it saves
+// (5 .. 16 sequences, K = 1000: 1.02 .. 1.09 of the time; more than 16, K = 600: 1.07).
+bool staged_rows(int batch, int k) { return k % kStreamBlock == 0 && k >= (batch > kGemvBatch ? 1024 : 2048); }
+constexpr int kLongRow = 8192;
+// How dense_out and dense_out_streams cut [width, k]: up to 128 tiles of 16 rows leave half the CUs idle, tiles of 8 rows on eight
+// waves use them all (2048 x 8192: 9.7 -> 7.5 us at 4 sequences, 15.4 -> 12.8 at 32), where K gives each of them a block (1024 x 512: 3.0 us
+// with them, 2.5 without).  More than 16 sequences: two row tiles per workgroup share the activations from 512 tiles on (35424 x 4096: 84 -> 65 us),
+// staged rows wherever one each would be more than a round of the CUs (5856 x 2048: 9.5 us, 7.9 with two; 4096 x 16384: 29.5, 38.0 with two); below
+// that, rows that are not staged have two blocks in flight instead (4096 x 18440: 44.2 -> 42.6) where K gives each wave several (5120 x 256,
+// 64 sequences: 9.1 us with two, 5.1 with one).  Up to 16, long staged rows: two blocks at a time (4096 x 16384: 26.6 -> 24.4).  K of one or two
+// blocks: two waves (32000 x 128, one sequence: 5.2 us on four, 4.4 on two).
+struct OutCut {
+  int rows, rt, bt;
+  dim3 grid;
+  int threads;
+};
+OutCut out_cut(int batch, int width, int k, bool sums) {
+  OutCut c;
+  c.bt = batch > kGemvBatch ? 2 : 1;
+  const int blocks = (batch + kGemvBatch * c.bt - 1) / (kGemvBatch * c.bt);
+  c.rows = (long long)(width / 16) * blocks <= 128 && (sums || k >= 1024) ? 8 : 16;
+  const bool few = c.rows == 16 && c.bt == 1 && k <= kTwoWaveColumns;
+  c.rt = c.bt == 2 && width % 32 == 0 && (staged_rows(batch, k) ? c.rows == 16 && (long long)(width / 16) * blocks > kCus : width >= 8192) ? 2 : 1;
+  c.grid = dim3(width / (c.rows * c.rt), blocks);
+  c.threads = c.rows == 8 ? 512 : few ? 128 : 256;
+  return c;
+}
+template <int N> using Int = std::integral_constant<int, N>;
+// go(waves, row tile, row tiles, batch tiles, blocks at a time, batch rows' instructions) of a cut
+template <typename Go>
+int with_out_cut(const OutCut& c, int batch, int k, Go&& go) {
+  if (c.threads == 128) return go(Int<2>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<1>{}, Int<kStreamDirect>{});
+  const bool staged = staged_rows(batch, k);
+  if (c.bt == 2) {
+    auto two_batch_tiles = [&](auto xq) {
+      if (c.rows == 8) return go(Int<8>{}, Int<8>{}, Int<1>{}, Int<2>{}, Int<1>{}, xq);
+      return c.rt == 2 ? go(Int<4>{}, Int<16>{}, Int<2>{}, Int<2>{}, Int<1>{}, xq) : go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<1>{}, xq);
+    };
+    if (staged) return two_batch_tiles(Int<4>{});
+    if (c.rows == 16 && c.rt == 1 && k >= 2048) return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<2>{}, Int<kStreamDirect>{});
+    return two_batch_tiles(Int<kStreamDirect>{});
+  }
+  if (!staged) return c.rows == 8 ? go(Int<8>{}, Int<8>{}, Int<1>{}, Int<1>{}, Int<1>{}, Int<kStreamDirect>{})
+                                  : go(Int<4>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<1>{}, Int<kStreamDirect>{});
+  auto by_batch = [&](auto xq) {
+    if (c.rows == 8) return go(Int<8>{}, Int<8>{}, Int<1>{}, Int<1>{}, Int<1>{}, xq);
+    return k >= kLongRow ? go(Int<4>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<2>{}, xq) : go(Int<4>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<1>{}, xq);
+  };
+  return batch <= 4 ? by_batch(Int<1>{}) : batch <= 8 ? by_batch(Int<2>{}) : by_batch(Int<4>{});
+}
+
 // ---- decode attention: (column steps, latent tiles per wave) that hold the widths
 int latent_tiles(int rankp) { const int t = (rankp + 63) / 64; return t <= 2 ? 2 : t <= 4 ? 4 : t <= 8 ? 8 : 0; }
 int latent_steps(int width) { const int s = (width + 31) / 32; return s <= 4 ? 4 : s <= 6 ? 6 : s <= 8 ? 8 : s <= 10 ? 10 : s <= 18 ? 18 : 0; }
@@ -465,7 +518,6 @@ int ajqd_windowed_prefill(const ajqd_windowed_attention_args* args, void* stream
   }
 }
 
-constexpr int kTwoWaveColumns = 256;  // products of one or two blocks of columns run on two waves (stream_rows)
 static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* sums, int parts, void* stream) {
   if (!a || (a->x ? (a->tiles1 && !a->gain1) || (a->tiles2 && !a->gain2) : (a->tiles1 && !a->n1) || (a->tiles2 && !a->n2)) ||
       (a->tiles1 && (!a->w1 || !a->y1)) || (a->tiles2 && (!a->w2 || !a->gated)))
@@ -482,11 +534,13 @@ static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* 
   d.batch = a->batch; d.D = a->true_width; d.Dp = a->width; d.tiles1 = a->tiles1; d.tiles2 = a->tiles2;
   d.gated_ld = a->gated_ld; d.act = a->act; d.center = a->center; d.pairs = a->pairs; d.eps = a->eps;
   d.sums = sums; d.parts = parts;
-  // more than 16 sequences: two batch tiles and (from two tiles of rows on) two row tiles per workgroup
-  const bool wide = a->batch > kGemvBatch;
+  // more than 16 sequences: two batch tiles and two row tiles per workgroup, or, where one each is no more than a round of the CUs, one on
+  // eight waves (2560 x 2048, 32 sequences: 8.7 -> 6.8 us; 4608 x 2048, 288 tiles: 9.2 with two, 11.6 so)
+  const bool wide = a->batch > kGemvBatch, few = a->width <= kTwoWaveColumns;
+  const bool staged = staged_rows(a->batch, a->width);
   const int block = wide ? 2 * kGemvBatch : kGemvBatch;
-  const bool few = a->width <= kTwoWaveColumns;
-  const int rt = wide && !few && a->tiles1 != 1 && a->tiles2 != 1 ? 2 : 1;
+  const bool short_of_tiles = staged && ((long long)a->tiles1 + a->tiles2) * ((a->batch + block - 1) / block) <= kCus;
+  const int rt = wide && !few && !short_of_tiles && a->tiles1 != 1 && a->tiles2 != 1 ? 2 : 1;
   const dim3 grid((a->tiles1 + rt - 1) / rt + (a->tiles2 + rt - 1) / rt, (a->batch + block - 1) / block);
   const int bytes = a->x ? 2 * a->batch * (a->width + 8) : 0;
   auto go = [&](auto kernel, int threads) {
@@ -498,12 +552,18 @@ static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* 
     // (rows so long that a workgroup's staging would not fit beside them run on two waves)
     // (and rows of more than 4096 columns on eight, whose registers hold them between the norm's passes: 8192 columns, 4 rows, 0 + 13648: 59.9
     // us on eight waves of the half-line form before, 96.7 on four of this one; 2016 + 6912: 43.7, 70.9, and 46.6 on eight)
-    if (bytes > 140 * 1024 || few) return go(dense_in_kernel<2, true, 1, 1>, 128);
-    if (a->width > 4096 && bytes <= 120 * 1024) return go(dense_in_kernel<8, true, 1, 1>, 512);
-    return go(dense_in_kernel<4, true, 1, 1>, 256);
+    if (bytes > 140 * 1024 || few) return go(dense_in_kernel<2, true, 1, 1, kStreamFrom, 1>, 128);
+    if (a->width > 4096 && bytes <= 120 * 1024) return go(dense_in_kernel<8, true, 1, 1, kStreamFrom, 1>, 512);
+    return go(dense_in_kernel<4, true, 1, 1, kStreamFrom, 1>, 256);
   }
-  if (few) return wide ? go(dense_in_kernel<2, false, 1, 2>, 128) : go(dense_in_kernel<2, false, 1, 1>, 128);
-  return rt == 2 ? go(dense_in_kernel<4, false, 2, 2>, 256) : wide ? go(dense_in_kernel<4, false, 1, 2>, 256) : go(dense_in_kernel<4, false, 1, 1>, 256);
+  if (few) return wide ? go(dense_in_kernel<2, false, 1, 2, kStreamDirect, 1>, 128) : go(dense_in_kernel<2, false, 1, 1, kStreamDirect, 1>, 128);
+  if (rt == 2) return staged ? go(dense_in_kernel<4, false, 2, 2, 4, 1>, 256) : go(dense_in_kernel<4, false, 2, 2, kStreamDirect, 1>, 256);
+  if (wide) return short_of_tiles ? go(dense_in_kernel<8, false, 1, 2, 4, 1>, 512) : go(dense_in_kernel<4, false, 1, 2, kStreamDirect, 1>, 256);
+  if (staged && a->batch > 8) return go(dense_in_kernel<4, false, 1, 1, 4, 1>, 256);
+  if (staged && a->batch > 4) return go(dense_in_kernel<4, false, 1, 1, 2, 1>, 256);
+  // up to four sequences: with few tiles, two blocks at a time where they come out even (4608 x 2048: 7.1 -> 6.8 us; 16384 x 4096: 21.2 -> 21.7)
+  if (staged && a->batch <= 4 && a->width % 1024 == 0 && a->tiles1 + a->tiles2 <= 384) return go(dense_in_kernel<4, false, 1, 1, 1, 2>, 256);
+  return go(dense_in_kernel<4, false, 1, 1, kStreamDirect, 1>, 256);
 }
 
 int ajqd_dense_in(const ajqd_dense_in_args* a, void* stream) { return dense_in("ajqd_dense_in", a, nullptr, 0, stream); }
@@ -514,29 +574,6 @@ int ajqd_dense_in_scaled(const ajqd_dense_in_args* a, const float* sums, int par
   return dense_in("ajqd_dense_in_scaled", a, sums, parts, stream);
 }
 
-// How dense_out and dense_out_streams cut [width, k]: up to 128 tiles of 16 rows leave half the CUs idle, tiles of 8 rows on eight
-// waves use them all (2048 x 8192: 9.4 -> 7.9 us at 4 sequences, 19.1 -> 17.9 at 32), where K gives each of them a block (1024 x 512: 3.0 us
-// with them, 2.5 without).  More than 16 sequences read each weight
-// fragment twice: from 512 tiles on two row tiles per workgroup share the activations (35424 x 4096: 84 -> 65 us), below that a
-// workgroup has two blocks in flight instead (4096 x 18432: 44.2 -> 42.6) where K gives each wave several (5120 x 256, 64 sequences: 9.1 us
-// with two, 5.1 with one).  K of one or two blocks: two waves (32000 x 128, one sequence: 5.2 us on four, 4.4 on two).
-struct OutCut {
-  int rows, rt, bt;
-  dim3 grid;
-  int threads;
-};
-OutCut out_cut(int batch, int width, int k, bool sums) {
-  OutCut c;
-  c.bt = batch > kGemvBatch ? 2 : 1;
-  const int blocks = (batch + kGemvBatch * c.bt - 1) / (kGemvBatch * c.bt);
-  c.rows = (long long)(width / 16) * blocks <= 128 && (sums || k >= 1024) ? 8 : 16;
-  const bool few = c.rows == 16 && c.bt == 1 && k <= kTwoWaveColumns;
-  c.rt = c.bt == 2 && width >= 8192 && width % 32 == 0 ? 2 : 1;
-  c.grid = dim3(width / (c.rows * c.rt), blocks);
-  c.threads = c.rows == 8 ? 512 : few ? 128 : 256;
-  return c;
-}
-
 int ajqd_dense_out(const void* in, const void* w, float* x, const float* again, const float* step, int batch, int k,
                    int width, void* stream) {
   if (!in || !w || !x) return fail(AJQ_ERR_NULL, "ajqd_dense_out: null pointer argument");
@@ -544,17 +581,11 @@ int ajqd_dense_out(const void* in, const void* w, float* x, const float* again, 
     return fail(AJQ_ERR_SHAPE, "ajqd_dense_out: unsupported shape (batch=%d k=%d width=%d)", batch, k, width);
   DenseOut d{(const uint16_t*)in, (const uint16_t*)w, x, again, step, batch, k, width};
   const OutCut c = out_cut(batch, width, k, false);
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, c.grid, dim3(c.threads), 0, (hipStream_t)stream, d);
+  return with_out_cut(c, batch, k, [&](auto waves, auto rows, auto rt, auto bt, auto uq, auto xq) {
+    hipLaunchKernelGGL((dense_out_kernel<waves(), rows(), rt(), bt(), uq(), xq()>), c.grid, dim3(c.threads), 0, (hipStream_t)stream, d);
     return check_launch("ajqd_dense_out");
-  };
-  if (c.rows == 8) return c.bt == 2 ? go(dense_out_kernel<8, 8, 1, 2, 1>) : go(dense_out_kernel<8, 8, 1, 1, 1>);
-  if (c.threads == 128) return go(dense_out_kernel<2, 16, 1, 1, 1>);
-  if (c.rt == 2) return go(dense_out_kernel<4, 16, 2, 2, 1>);
-  if (c.bt == 2) return k < 2048 ? go(dense_out_kernel<4, 16, 1, 2, 1>) : go(dense_out_kernel<4, 16, 1, 2, 2>);
-  return go(dense_out_kernel<4, 16, 1, 1, 1>);
+  });
 }
-
 int ajqd_latent_absorb(const float* y, int ldy, const ajqd_latent_shape* shape, const void* ukt, const float* latent_gain,
                        const float* cosine, const float* sine, int table_rows, const int64_t* pos, void* q, void* ring, int cap,
                        int batch, void* stream) {
@@ -697,17 +728,12 @@ static int dense_out_streams(const char* name, DenseOutStreams d, void* stream) 
   if (batch < 1 || k < 8 || k % 8 || width < 16 || width % 16)
     return fail(AJQ_ERR_SHAPE, "%s: unsupported shape (batch=%d k=%d width=%d)", name, batch, k, width);
   const OutCut c = out_cut(batch, width, k, !d.u);
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, c.grid, dim3(c.threads), 0, (hipStream_t)stream, d);
-    return check_launch(name);
-  };
   auto pick = [&](auto room) {
-    constexpr int M = decltype(room)::value;
-    if (c.rows == 8) return c.bt == 2 ? go(dense_out_streams_kernel<8, 8, 1, 2, 1, M>) : go(dense_out_streams_kernel<8, 8, 1, 1, 1, M>);
-    if (c.threads == 128) return go(dense_out_streams_kernel<2, 16, 1, 1, 1, M>);
-    if (c.rt == 2) return go(dense_out_streams_kernel<4, 16, 2, 2, 1, M>);
-    if (c.bt == 2) return k < 2048 ? go(dense_out_streams_kernel<4, 16, 1, 2, 1, M>) : go(dense_out_streams_kernel<4, 16, 1, 2, 2, M>);
-    return go(dense_out_streams_kernel<4, 16, 1, 1, 1, M>);
+    return with_out_cut(c, batch, k, [&](auto waves, auto rows, auto rt, auto bt, auto uq, auto xq) {
+      hipLaunchKernelGGL((dense_out_streams_kernel<waves(), rows(), rt(), bt(), uq(), xq(), decltype(room)::value>), c.grid, dim3(c.threads), 0,
+                         (hipStream_t)stream, d);
+      return check_launch(name);
+    });
   };
   switch (stream_room(streams)) {
     case 2: return pick(std::integral_constant<int, 2>{});

@@ -74,35 +74,54 @@ __device__ __forceinline__ void meet(f32x4_t (&acc)[RT][BT], float* red, int wav
 }
 
 // acc[n][t] += W[rows of tile n, :] x_t for RT tiles of ROWS (16 or 8) consecutive rows of a row-major W [.., K], K split over
-// kWaves waves in blocks of 128 columns.  `w`: the first row; `x(t, k)`: the B fragment of batch tile t at columns k + 8 g .. of
-// batch column r, asked for inside K only; `between` runs while the first blocks travel.  `lds`:
-// stream_lds() bytes; the tiles' sums of all waves are complete in wave n BT + t (as `meet` leaves them).
+// kWaves waves in blocks of 128 columns, UQ of them requested together.  `w`: the first row; `xrows`: the first of nb batch rows [.., K];
+// `between` runs while the first blocks travel.  `lds`: stream_lds() bytes; the tiles' sums of all waves are complete in wave n BT + t (as
+// `meet` leaves them).
 //
 // Bound: HBM.  What costs is how a row-major matrix is asked for: the product's own operand layout wants 64 bytes of each of 16
 // rows per instruction, half a line everywhere, and streams at 4.4 TB/s; four rows of 256 bytes per instruction stream at 5.9
 // (4096 x 18432, 8 sequences: 38.3 -> 25.7 us; 35424 x 4096: 63.0 -> 46.3; 2048 x 8192: 13.9 -> 7.9 with tiles of 8 rows on
 // twice as many CUs).  The block then takes the operand layout on its way through wave-private LDS (no barrier; chunk c of row
 // r lies in slot c ^ r, so that both the rows' writes and the operand reads meet all banks), while the next one travels.
+//
+// XQ: the batch rows go the same way, ahead of the weights, four rows per instruction: XQ = 1, 2 or 4 instructions per batch tile
+// and block hold up to 4, 8 or 16 of them.  In the operand layout they were four instructions of half lines whatever the batch, as many
+// as the weights' (twice as many for tiles of 8 rows).  us, before -> after: 2048 x 8192: 4 sequences 8.0 -> 7.5, 16 11.4 -> 9.7, 32 18.3 ->
+// 12.8; 4096 x 18432: 16 29.9 -> 27.5, 32 44.7 -> 35.0; 35424 x 4096: 16 55.6 -> 51.3, 32 68.5 -> 57.6.
+// XQ = kStreamDirect: `x(t, k)` gives the B fragment of batch tile t at columns k + 8 g .. of batch column r, from memory, asked for behind the
+// weights: short rows, and many tiles with up to four sequences (16384 x 4096: 21.2 us, 21.7 staged); kStreamFrom: from LDS, behind `between`.
 constexpr int kStreamBlock = 128;
-constexpr int stream_lds(int waves, int rows, int rt, int bt, int uq) {
-  return waves * uq * rt * rows * 256 > rt * bt * waves * 1024 ? waves * uq * rt * rows * 256 : rt * bt * waves * 1024;
+enum { kStreamFrom = 0, kStreamDirect = -1 };
+constexpr int stream_wave_lds(int rows, int rt, int bt, int uq, int xq) { return uq * (rt * rows + (xq > 0 ? bt * 4 * xq : 0)) * 256; }
+constexpr int stream_lds(int waves, int rows, int rt, int bt, int uq, int xq) {
+  const int blocks = waves * stream_wave_lds(rows, rt, bt, uq, xq), sums = rt * bt * waves * 1024;
+  return blocks > sums ? blocks : sums;
 }
-template <int kWaves, int ROWS, int RT, int BT, int UQ, bool kXFirst = true, typename Between, typename XFn>
+template <int kWaves, int ROWS, int RT, int BT, int UQ, int XQ, typename Between, typename XFn>
 __device__ __forceinline__ void stream_rows(const uint16_t* __restrict__ w, int K, int wave, int lane, unsigned char* lds,
-                                            f32x4_t (&acc)[RT][BT], Between&& between, XFn&& x) {
+                                            f32x4_t (&acc)[RT][BT], const uint16_t* __restrict__ xrows, int nb, Between&& between, XFn&& x) {
   static_assert(ROWS == 16 || ROWS == 8, "tiles of 16 or 8 rows");
   constexpr int kLoads = ROWS / 4;  // instructions of 1 KiB per tile and block
+  constexpr bool kStaged = XQ > 0, kAhead = XQ != kStreamFrom;
+  constexpr int kX = kStaged ? XQ : 4;
   const int r = lane & 15, g = lane >> 4, rr = ROWS == 16 ? r : r & 7;
   const int full = K / kStreamBlock, per = (full + kWaves - 1) / kWaves;
   const int begin = min(full, wave * per), count = min(full, begin + per) - begin;
-  unsigned char* mine = lds + wave * (UQ * RT * ROWS * 256);
+  unsigned char* mine = lds + wave * stream_wave_lds(ROWS, RT, BT, UQ, XQ);
+  unsigned char* mine_x = mine + UQ * RT * ROWS * 256;
   // row 4 j + lane / 16 of a tile, chunk (lane % 16) ^ row
-  uint32_t at[kLoads];
+  uint32_t at[kLoads], x_at[BT][kX];
 #pragma unroll
   for (int j = 0; j < kLoads; ++j) at[j] = (uint32_t)(4 * j + g) * (2u * K) + 16u * (r ^ (4 * j + g));
+  if (kStaged)
+#pragma unroll
+    for (int t = 0; t < BT; ++t)
+#pragma unroll
+      for (int j = 0; j < kX; ++j) x_at[t][j] = (uint32_t)min(16 * t + 4 * j + g, nb - 1) * (2u * K) + 16u * (r ^ (4 * j + g));
   const unsigned char* base = reinterpret_cast<const unsigned char*>(w);
+  const unsigned char* x_base = reinterpret_cast<const unsigned char*>(xrows);
   const size_t tile = (size_t)ROWS * 2 * K;
-  u32x4_t wr[2][UQ][RT][kLoads], xr[2][UQ][BT][4];
+  u32x4_t wr[2][UQ][RT][kLoads], xr[2][UQ][BT][kX];
   auto load_w = [&](int buf, int q) {
 #pragma unroll
     for (int i = 0; i < UQ; ++i)
@@ -118,53 +137,75 @@ __device__ __forceinline__ void stream_rows(const uint16_t* __restrict__ w, int 
 #pragma unroll
       for (int t = 0; t < BT; ++t)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) xr[buf][i][t][s] = x(t, kStreamBlock * (q + i) + 32 * s);
+        for (int s = 0; s < kX; ++s) {
+          if (kStaged) xr[buf][i][t][s] = *reinterpret_cast<const u32x4_t*>(x_base + (size_t)(q + i) * 256 + x_at[t][s]);
+          else xr[buf][i][t][s] = x(t, kStreamBlock * (q + i) + 32 * s);
+        }
   };
   auto put = [&](int i, int n, int j, const u32x4_t& v) {
     *reinterpret_cast<u32x4_t*>(mine + ((i * RT + n) * kLoads + j) * 1024 + lane * 16) = v;
   };
+  auto put_x = [&](int i, int t, int j, const u32x4_t& v) { *reinterpret_cast<u32x4_t*>(mine_x + ((i * BT + t) * kX + j) * 1024 + lane * 16) = v; };
   auto operand = [&](int i, int n, int s) {
     return *reinterpret_cast<const u32x4_t*>(mine + (i * RT + n) * kLoads * 1024 + rr * 256 + ((4 * s + g) ^ rr) * 16);
   };
+  const int rx = r & (4 * kX - 1);
+  auto operand_x = [&](int i, int t, int s) {
+    return *reinterpret_cast<const u32x4_t*>(mine_x + (i * BT + t) * kX * 1024 + rx * 256 + ((4 * s + g) ^ rx) * 16);
+  };
   auto use = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < UQ; ++i)
+    for (int i = 0; i < UQ; ++i) {
+      if (kStaged)
+#pragma unroll
+        for (int t = 0; t < BT; ++t)
+#pragma unroll
+          for (int j = 0; j < kX; ++j) put_x(i, t, j, xr[buf][i][t][j]);
 #pragma unroll
       for (int n = 0; n < RT; ++n)
 #pragma unroll
         for (int j = 0; j < kLoads; ++j) put(i, n, j, wr[buf][i][n][j]);
+    }
     wave_lds_order();
 #pragma unroll
     for (int i = 0; i < UQ; ++i)
 #pragma unroll
-      for (int n = 0; n < RT; ++n)
+      for (int s = 0; s < 4; ++s) {
+        u32x4_t v[BT];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
+        for (int t = 0; t < BT; ++t) v[t] = kStaged ? operand_x(i, t, s) : xr[buf][i][t][s & (kX - 1)];
+#pragma unroll
+        for (int n = 0; n < RT; ++n) {
           const u32x4_t f = operand(i, n, s);
 #pragma unroll
-          for (int t = 0; t < BT; ++t) acc[n][t] = mfma16(f, xr[buf][i][t][s], acc[n][t]);
+          for (int t = 0; t < BT; ++t) acc[n][t] = mfma16(f, v[t], acc[n][t]);
         }
+      }
     wave_lds_order();  // (the next block's puts overwrite what was read here)
   };
-  if (count >= UQ) load_w(0, begin);
-  if (kXFirst && count >= UQ) load_x(0, begin);
+  auto load = [&](int buf, int q) {
+    if (kStaged) load_x(buf, q);
+    load_w(buf, q);
+    if (!kStaged) load_x(buf, q);
+  };
+  if (count >= UQ) {
+    if (kAhead) load(0, begin);
+    else load_w(0, begin);
+  }
   between();
   int s = begin, left = count;
   if (left >= UQ) {
-    if (!kXFirst) load_x(0, s);
+    if (!kAhead) load_x(0, s);
     for (; left >= 3 * UQ; left -= 2 * UQ, s += 2 * UQ) {
-      load_w(1, s + UQ);
-      load_x(1, s + UQ);
+      load(1, s + UQ);
       __builtin_amdgcn_sched_barrier(0);
       use(0);
-      load_w(0, s + 2 * UQ);
-      load_x(0, s + 2 * UQ);
+      load(0, s + 2 * UQ);
       __builtin_amdgcn_sched_barrier(0);
       use(1);
     }
     if (left >= 2 * UQ) {
-      load_w(1, s + UQ);
-      load_x(1, s + UQ);
+      load(1, s + UQ);
       __builtin_amdgcn_sched_barrier(0);
       use(0);
       use(1);
@@ -182,40 +223,56 @@ __device__ __forceinline__ void stream_rows(const uint16_t* __restrict__ w, int 
   const bool cut = wave == kWaves - 1 && K % kStreamBlock != 0;
   for (; left > 0 || (left == 0 && cut); --left) {
     const int q = left == 0 ? full : s++;
-    u32x4_t wt[RT][kLoads], xt[BT][4];
-#pragma unroll
-    for (int n = 0; n < RT; ++n)
-#pragma unroll
-      for (int j = 0; j < kLoads; ++j) {
-        const int c = 8 * (r ^ (4 * j + g));  // (of which at[j] holds 2 c already)
-        const uint32_t to = at[j] + 2u * (uint32_t)(min(kStreamBlock * q + c, K - 8) - c);
-        wt[n][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(base + n * tile + to));
-      }
+    u32x4_t wt[RT][kLoads], xt[BT][kX];
+    auto inside = [&](int j) {  // this lane's column of row 4 j + g, held inside K: what to add to the row's offset
+      const int c = 8 * (r ^ (4 * j + g));  // (of which at[j] holds 2 c already)
+      return 2u * (uint32_t)(min(kStreamBlock * q + c, K - 8) - c);
+    };
+    auto live = [&](int j) { return kStreamBlock * q + 8 * (r ^ (4 * j + g)) < K; };
 #pragma unroll
     for (int t = 0; t < BT; ++t)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) xt[t][k] = x(t, min(kStreamBlock * q + 32 * k, K - 8 - 8 * g));
+      for (int k = 0; k < kX; ++k)
+        xt[t][k] = kStaged ? *reinterpret_cast<const u32x4_t*>(x_base + (x_at[t][k] + inside(k))) : x(t, min(kStreamBlock * q + 32 * k, K - 8 - 8 * g));
+#pragma unroll
+    for (int n = 0; n < RT; ++n)
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j)
+        wt[n][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(base + n * tile + (at[j] + inside(j))));
     const u32x4_t zero = {0u, 0u, 0u, 0u};
+    if (kStaged)
+#pragma unroll
+      for (int t = 0; t < BT; ++t)
+#pragma unroll
+        for (int j = 0; j < kX; ++j) {
+          asm volatile("" : "+v"(xt[t][j]));
+          put_x(0, t, j, live(j) ? xt[t][j] : zero);
+        }
 #pragma unroll
     for (int n = 0; n < RT; ++n)
 #pragma unroll
       for (int j = 0; j < kLoads; ++j) {
         asm volatile("" : "+v"(wt[n][j]));
-        put(0, n, j, kStreamBlock * q + 8 * (r ^ (4 * j + g)) < K ? wt[n][j] : zero);
+        put(0, n, j, live(j) ? wt[n][j] : zero);
       }
     wave_lds_order();
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
+      u32x4_t v[BT];
 #pragma unroll
       for (int t = 0; t < BT; ++t) {
-        asm volatile("" : "+v"(xt[t][k]));
-        xt[t][k] = kStreamBlock * q + 32 * k + 8 * g < K ? xt[t][k] : zero;
+        if (kStaged) {
+          v[t] = operand_x(0, t, k);
+        } else {
+          asm volatile("" : "+v"(xt[t][k & (kX - 1)]));
+          v[t] = kStreamBlock * q + 32 * k + 8 * g < K ? xt[t][k & (kX - 1)] : zero;
+        }
       }
 #pragma unroll
       for (int n = 0; n < RT; ++n) {
         const u32x4_t f = operand(0, n, k);
 #pragma unroll
-        for (int t = 0; t < BT; ++t) acc[n][t] = mfma16(f, xt[t][k], acc[n][t]);
+        for (int t = 0; t < BT; ++t) acc[n][t] = mfma16(f, v[t], acc[n][t]);
       }
     }
     wave_lds_order();
@@ -241,11 +298,11 @@ struct DenseIn {
 };
 
 // kNorm: the norm is formed here, for the rows of one batch block (dynamic LDS: rows x (Dp + 8) bf16).
-// RT: row tiles per workgroup (grid.x counts workgroups of the first matrix, then of the second), BT: batch tiles.
-template <int kWaves, bool kNorm, int RT, int BT>
+// RT: row tiles per workgroup (grid.x counts workgroups of the first matrix, then of the second), BT: batch tiles; XQ, UQ as in stream_rows.
+template <int kWaves, bool kNorm, int RT, int BT, int XQ, int UQ>
 __global__ __launch_bounds__(64 * kWaves) void dense_in_kernel(DenseIn a) {
   extern __shared__ __attribute__((aligned(16))) uint16_t normed[];
-  __shared__ __attribute__((aligned(16))) unsigned char lds[stream_lds(kWaves, 16, RT, BT, 1)];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[stream_lds(kWaves, 16, RT, BT, UQ, XQ)];
   __shared__ float stat[kNorm ? kWaves : kGemvBatch * BT];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int b0 = blockIdx.y * kGemvBatch * BT, nb = min(kGemvBatch * BT, a.batch - b0);
@@ -315,11 +372,12 @@ __global__ __launch_bounds__(64 * kWaves) void dense_in_kernel(DenseIn a) {
       }
       __syncthreads();
     };
-    stream_rows<kWaves, 16, RT, BT, 1, false>(wrow, a.Dp, wave, lane, lds, acc, norm, [&](int t, int k) {
+    static_assert(XQ == kStreamFrom, "formed rows lie in LDS");
+    stream_rows<kWaves, 16, RT, BT, UQ, XQ>(wrow, a.Dp, wave, lane, lds, acc, nullptr, nb, norm, [&](int t, int k) {
       return *reinterpret_cast<const u32x4_t*>(normed + min(16 * t + r, nb - 1) * stride + 8 * g + k);
     });
   } else {
-    const uint16_t* xr = (second ? a.n2 : a.n1) + (size_t)b0 * a.Dp + 8 * g;
+    const uint16_t *xr = (second ? a.n2 : a.n1) + (size_t)b0 * a.Dp, *xd = xr + 8 * g;
     // the rows' factors while the first weights travel: 16 lanes per row add its parts
     auto factors = [&]() {
       if (!a.sums) return;
@@ -338,8 +396,8 @@ __global__ __launch_bounds__(64 * kWaves) void dense_in_kernel(DenseIn a) {
         if (r == 0) stat[row] = 1.0f / sqrtf(ss / (float)a.D + a.eps);
       }
     };
-    stream_rows<kWaves, 16, RT, BT, 1>(wrow, a.Dp, wave, lane, lds, acc, factors, [&](int t, int k) {
-      return *reinterpret_cast<const u32x4_t*>(xr + (size_t)min(16 * t + r, nb - 1) * a.Dp + k);
+    stream_rows<kWaves, 16, RT, BT, UQ, XQ>(wrow, a.Dp, wave, lane, lds, acc, xr, nb, factors, [&](int t, int k) {
+      return *reinterpret_cast<const u32x4_t*>(xd + (size_t)min(16 * t + r, nb - 1) * a.Dp + k);
     });
   }
 #pragma unroll
@@ -374,14 +432,14 @@ struct DenseOut {
   const float* step;        // [Dp] or null, added too
   int batch, K, Dp;
 };
-// ROWS, kWaves: tiles of 16 rows on four waves, or of 8 on eight (few tiles); UQ as in stream_rows.
-template <int kWaves, int ROWS, int RT, int BT, int UQ>
+// ROWS, kWaves: tiles of 16 rows on four waves, or of 8 on eight (few tiles); UQ, XQ as in stream_rows.
+template <int kWaves, int ROWS, int RT, int BT, int UQ, int XQ>
 __global__ __launch_bounds__(64 * kWaves) void dense_out_kernel(DenseOut a) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[stream_lds(kWaves, ROWS, RT, BT, UQ)];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[stream_lds(kWaves, ROWS, RT, BT, UQ, XQ)];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int b0 = blockIdx.y * kGemvBatch * BT, nb = min(kGemvBatch * BT, a.batch - b0);
   const int first = blockIdx.x * RT * ROWS;  // (RT divides the row tiles: x is updated in place)
-  const uint16_t* xr = a.in + (size_t)b0 * a.K + 8 * g;
+  const uint16_t *xr = a.in + (size_t)b0 * a.K, *xd = xr + 8 * g;
   // what the product of tile wave = (row tile, batch tile) is added to, requested ahead of it by the wave that will write it
   const bool writes = wave < RT * BT && 4 * g < ROWS;
   const int row = 16 * (wave % BT) + r, column = first + ROWS * (wave / BT) + 4 * g;
@@ -392,8 +450,8 @@ __global__ __launch_bounds__(64 * kWaves) void dense_out_kernel(DenseOut a) {
   if (writes && a.again) again = load4(a.again + place);
   if (writes && a.step) step = load4(a.step + column);
   f32x4_t acc[RT][BT] = {};
-  stream_rows<kWaves, ROWS, RT, BT, UQ>(a.w + (size_t)first * a.K, a.K, wave, lane, lds, acc, [] {}, [&](int t, int k) {
-    return *reinterpret_cast<const u32x4_t*>(xr + (size_t)min(16 * t + r, nb - 1) * a.K + k);
+  stream_rows<kWaves, ROWS, RT, BT, UQ, XQ>(a.w + (size_t)first * a.K, a.K, wave, lane, lds, acc, xr, nb, [] {}, [&](int t, int k) {
+    return *reinterpret_cast<const u32x4_t*>(xd + (size_t)min(16 * t + r, nb - 1) * a.K + k);
   });
   if (a.again) { v.x += again.x; v.y += again.y; v.z += again.z; v.w += again.w; }
   if (a.step) { v.x += step.x; v.y += step.y; v.z += step.z; v.w += step.w; }
@@ -418,13 +476,13 @@ struct DenseOutStreams {
   float* sums;              // [B, Dp / ROWS] its sums of squares per tile
   int batch, K, Dp, streams;
 };
-template <int kWaves, int ROWS, int RT, int BT, int UQ, int MAXS>
+template <int kWaves, int ROWS, int RT, int BT, int UQ, int XQ, int MAXS>
 __global__ __launch_bounds__(64 * kWaves) void dense_out_streams_kernel(DenseOutStreams a) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[stream_lds(kWaves, ROWS, RT, BT, UQ)];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[stream_lds(kWaves, ROWS, RT, BT, UQ, XQ)];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int b0 = blockIdx.y * kGemvBatch * BT, nb = min(kGemvBatch * BT, a.batch - b0);
   const int first = blockIdx.x * RT * ROWS;
-  const uint16_t* xr = a.in + (size_t)b0 * a.K + 8 * g;
+  const uint16_t *xr = a.in + (size_t)b0 * a.K, *xd = xr + 8 * g;
   // the streams at this lane's place of tile wave = (row tile, batch tile), requested ahead of the product
   const bool writes = wave < RT * BT && 4 * g < ROWS;
   const int row = 16 * (wave % BT) + r, column = first + ROWS * (wave / BT) + 4 * g;
@@ -452,8 +510,8 @@ __global__ __launch_bounds__(64 * kWaves) void dense_out_streams_kernel(DenseOut
     }
   }
   f32x4_t acc[RT][BT] = {};
-  stream_rows<kWaves, ROWS, RT, BT, UQ>(a.w + (size_t)first * a.K, a.K, wave, lane, lds, acc, [] {}, [&](int t, int k) {
-    return *reinterpret_cast<const u32x4_t*>(xr + (size_t)min(16 * t + r, nb - 1) * a.K + k);
+  stream_rows<kWaves, ROWS, RT, BT, UQ, XQ>(a.w + (size_t)first * a.K, a.K, wave, lane, lds, acc, xr, nb, [] {}, [&](int t, int k) {
+    return *reinterpret_cast<const u32x4_t*>(xd + (size_t)min(16 * t + r, nb - 1) * a.K + k);
   });
 #pragma unroll
   for (int i = 0; i < RT * BT; ++i) {

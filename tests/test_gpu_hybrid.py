@@ -781,6 +781,17 @@ def test_streamed_products_of_short_rows(cuda, batch, k, width):
     test_streamed_products(cuda, batch, k, width)
 
 
+@pytest.mark.parametrize("batch,k,width", [
+    (4, 2048, 48), (3, 2176, 2064), (4, 3072, 6160),             # up to four sequences: two blocks at a time, one, from memory
+    (8, 1024, 48), (5, 2048, 2064), (8, 8320, 4112),             # up to eight, the last with blocks left over
+    (9, 2176, 2064), (16, 8192, 4112),
+    (32, 1024, 4096), (33, 1024, 4112), (64, 1152, 4128), (20, 1152, 6144)])
+def test_streamed_products_of_staged_rows(cuda, batch, k, width):
+    """The batch rows through LDS, four to an instruction, on either side of every rule that chooses the form."""
+    test_streamed_products(cuda, batch, k, width)
+    test_dense_out_streams(cuda, batch, (2, k, width))
+
+
 @pytest.mark.parametrize("batch,k", [(4, 256), (3, 264), (2, 4096), (4, 4104), (4, 8192), (3, 8200), (4, 15432), (4, 17928)])
 def test_norm_prologue_on_two_four_and_eight_waves(cuda, batch, k):
     """dense_in with the norm inside, at the row lengths where its workgroups change; an operand rounded the other way moves by 2^-8."""
