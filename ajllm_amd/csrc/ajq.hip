@@ -10,6 +10,7 @@
 #include "quantize_kernels.h"
 #include "gemv_kernels.h"
 #include "gemv_fused_kernels.h"
+#include "gemv_norm_kernels.h"
 #include "gemm_kernels.h"
 #include "gemm_ring_kernels.h"
 #include "gemm_split_kernels.h"
@@ -882,34 +883,34 @@ int launch_gemv_pro(int M, int K, const uint32_t* wq, const uint32_t* meta, cons
 #define AJQ_PRO(W, T, R)                                                                                              \
   return launch_gemv_pro_cfg<W, T, R, kW4, kPro, kOut>(M, K, wq, meta, scales8, N, y, out_f32, src0, src1, gain, eps, \
                                                        h_out, stream, S)
-  // One row with its norm from the sums: four waves of twice the groups.  Every wave forms the norm's divisor for itself, and with
-  // eight a launch of many workgroups is bounded by that arithmetic (int4, K = 2048, N = 6144 / 11264 / 32000: 3.87 / 4.93 / 9.24 us
-  // with eight waves, 3.67 / 4.57 / 8.19 with four; K = 1024, N = 11264: 4.18 / 3.59; int8, K = 2048, N = 11264: 6.25 / 6.12).
-  // K = 4096 has eight: a quarter of its columns is more than one load per lane, and that form is not built.
-  if constexpr (kPro == kProNormSums) {
-    if (M <= 1 && K == 1024) AJQ_PRO(4, 2, 1);
-    if (M <= 1 && K == 2048) AJQ_PRO(4, 4, 1);
+  // (norms from sums come here with three rows or more, of up to 4096 columns)
+#define AJQ_PRO_ROW(W, T)                     \
+  if constexpr (kPro != kProNormSums) {       \
+    if (M <= 1) AJQ_PRO(W, T, 1);             \
   }
   if (K == 1024) {
-    if (M <= 1) AJQ_PRO(8, 1, 1);
+    AJQ_PRO_ROW(8, 1)
     if (M <= 4) AJQ_PRO(8, 1, 4);
     if (M <= 8) AJQ_PRO(8, 1, 8);
     AJQ_PRO(8, 1, 16);
   }
   if (K == 2048) {
-    if (M <= 1) AJQ_PRO(8, 2, 1);
+    AJQ_PRO_ROW(8, 2)
     if (M <= 4) AJQ_PRO(8, 2, 4);
     if (M <= 8) AJQ_PRO(8, 2, 8);
     AJQ_PRO(8, 2, 16);
   }
-  if (K == 4096) {
-    if (M <= 1) AJQ_PRO(8, 4, 1);
+  if (K == 4096 || kPro == kProNormSums) {
+    AJQ_PRO_ROW(8, 4)
     if (M <= 4) AJQ_PRO(8, 4, 4);
     AJQ_PRO(8, 4, 8);
   }
-  if (M <= 1) AJQ_PRO(11, 4, 1);
-  if (M <= 4) AJQ_PRO(11, 4, 4);
-  AJQ_PRO(11, 4, 8);
+  if constexpr (kPro != kProNormSums) {
+    if (M <= 1) AJQ_PRO(11, 4, 1);
+    if (M <= 4) AJQ_PRO(11, 4, 4);
+    AJQ_PRO(11, 4, 8);
+  }
+#undef AJQ_PRO_ROW
 #undef AJQ_PRO
 }
 
@@ -974,6 +975,62 @@ int gemv_merge_residual(const char* name, const float* partial, int S, int M, in
   return check_launch(name);
 }
 
+template <int N> using Int = std::integral_constant<int, N>;
+// The norm from its sums on up to four rows: T tiles per workgroup (gemv_norm_kernels.h).
+template <int kWaves, int TPW, int MROWS, int T, bool kW4, bool kGate>
+int launch_gemv_norm_cfg(int M, int K, const uint32_t* wq, const uint32_t* meta, const uint16_t* scales8, int N, void* y, int out_f32, const float* h,
+                         const float* ssq, const float* gain, float eps, int parts, hipStream_t stream) {
+  constexpr size_t lds = gemv_norm_lds_bytes(kWaves, TPW, MROWS, T);
+  auto kernel = dequant_gemv_norm_kernel<kWaves, TPW, MROWS, T, kW4, kGate>;
+  if (int s = allow_big_lds(kernel, lds)) return s;
+  hipLaunchKernelGGL(kernel, dim3((N / kTileN + T - 1) / T), dim3(kWaves * 64), lds, stream, reinterpret_cast<const u32x4_t*>(wq), meta, K,
+                     M | (out_f32 << 8), N, y, scales8, h, ssq, gain, eps, parts);
+  return AJQ_OK;
+}
+// Tiles per workgroup: up to three rounds of the CUs in one; beyond, several workgroups share a CU and their number counts, the more the more rows there
+// are to norm.  Rows of 4096 int8 weights fill the registers (28672 columns, 1 row: 19.2 us with one tile, 22.0 with two).
+template <bool kW4>
+int gemv_norm_tiles(int M, int K, int tiles) {
+  const int rounds = (tiles + 255) / 256;
+  if (rounds <= 3) return rounds;
+  if (K == 4096) return kW4 ? 2 : 1;
+  return M == 1 ? 2 : 4;
+}
+// One tile of three or four rows: without holding the sums (gemv_fused_kernels.h; 2048 x 2048, 4 rows: 3.6 us, 3.9 here), but for long int8 rows (4096
+// columns: 5.6 us there, 5.2 here).
+template <bool kW4>
+bool gemv_norm_few_rows(int M, int K, int N) {
+  return M <= 4 && (M <= 2 || gemv_norm_tiles<kW4>(M, K, N / kTileN) > 1 || (!kW4 && K == 4096));
+}
+template <bool kW4, bool kGate>
+int launch_gemv_norm(int M, int K, const uint32_t* wq, const uint32_t* meta, const uint16_t* scales8, int N, void* y, int out_f32, const float* h,
+                     const float* ssq, const float* gain, float eps, int parts, hipStream_t stream) {
+  const int tiles = gemv_norm_tiles<kW4>(M, K, N / kTileN);
+  auto go = [&](auto waves, auto tpw, auto rows, auto t) {
+    return launch_gemv_norm_cfg<waves(), tpw(), rows(), t(), kW4, kGate>(M, K, wq, meta, scales8, N, y, out_f32, h, ssq, gain, eps, parts, stream);
+  };
+  auto by_tiles = [&](auto waves, auto tpw, auto rows) {
+    switch (tiles) {
+      case 1: return go(waves, tpw, rows, Int<1>{});
+      case 2: return go(waves, tpw, rows, Int<2>{});
+      case 3: return go(waves, tpw, rows, Int<3>{});
+      default: return go(waves, tpw, rows, Int<4>{});
+    }
+  };
+  auto by_rows = [&](auto tpw) {
+    if (M == 1) {
+      // One tile of one row: four waves of twice the groups.  Every wave forms the norm's divisor for itself (int4, K = 2048, N = 2048: 2.87 us with
+      // eight, 2.75 with four); a quarter of K = 4096 would be more than one load per lane.
+      if constexpr (tpw() < 4) {
+        if (tiles == 1) return go(Int<4>{}, Int<2 * tpw()>{}, Int<1>{}, Int<1>{});
+      }
+      return by_tiles(Int<8>{}, tpw, Int<1>{});
+    }
+    return M == 2 ? by_tiles(Int<8>{}, tpw, Int<2>{}) : by_tiles(Int<8>{}, tpw, Int<4>{});
+  };
+  return K == 1024 ? by_rows(Int<1>{}) : K == 2048 ? by_rows(Int<2>{}) : by_rows(Int<4>{});
+}
+
 template <bool kW4>
 int gemv_norm_sums(const char* name, const float* h, const float* ssq, int parts, const float* gain, float eps, int M, int K,
                    const uint32_t* wq, const void* aux, int N, void* y, int out_dtype, int gate, void* stream) {
@@ -987,10 +1044,15 @@ int gemv_norm_sums(const char* name, const float* h, const float* ssq, int parts
   if (gate && out_dtype != AJQ_OUT_BF16) return fail(AJQ_ERR_UNSUPPORTED, "%s: the gated output is bf16", name);
   const uint32_t* meta = kW4 ? static_cast<const uint32_t*>(aux) : nullptr;
   const uint16_t* scales = kW4 ? nullptr : static_cast<const uint16_t*>(aux);
-  const int s = gate ? launch_gemv_pro<kW4, kProNormSums, kOutGate>(M, K, wq, meta, scales, N, y, 0, h, ssq, gain, eps, nullptr,
-                                                                    (hipStream_t)stream, parts)
-                     : launch_gemv_pro<kW4, kProNormSums>(M, K, wq, meta, scales, N, y, out_dtype == AJQ_OUT_F32, h, ssq, gain,
-                                                          eps, nullptr, (hipStream_t)stream, parts);
+  hipStream_t st = (hipStream_t)stream;
+  const int f32 = out_dtype == AJQ_OUT_F32;
+  int s;
+  if (gemv_norm_few_rows<kW4>(M, K, N))
+    s = gate ? launch_gemv_norm<kW4, true>(M, K, wq, meta, scales, N, y, 0, h, ssq, gain, eps, parts, st)
+             : launch_gemv_norm<kW4, false>(M, K, wq, meta, scales, N, y, f32, h, ssq, gain, eps, parts, st);
+  else
+    s = gate ? launch_gemv_pro<kW4, kProNormSums, kOutGate>(M, K, wq, meta, scales, N, y, 0, h, ssq, gain, eps, nullptr, st, parts)
+             : launch_gemv_pro<kW4, kProNormSums>(M, K, wq, meta, scales, N, y, f32, h, ssq, gain, eps, nullptr, st, parts);
   if (s) return s;
   return check_launch(name);
 }

@@ -18,10 +18,10 @@
 // LDS behind one barrier (the weight loads are in flight meanwhile).  Workgroup 0 writes the
 // updated residual stream, to a buffer other than the one being read.
 // What bounds these launches is the chain of round trips to memory, so no load may wait for another's value: the activations'
-// way into LDS has no branch and no select that would draw a load into itself (kProNormSums used to fetch h and the gain only
+// way into LDS has no branch and no select that would draw a load into itself (a norm from its sums used to fetch h and the gain only
 // after the row sums had arrived: a 12-layer int4 step of width 2048 at batch 1 took 0.326 ms with that, 0.313 without).  Several
 // rows with their sums are the exception: up to sixteen vectors of sums, the rows and the gains held at once cost more registers than the
-// trip is worth (int8, K = 1024, N = 11264, 12 rows: 12.2 us so, 9.0 with the sums dropped at the load; K = 2048, 4 rows: 7.7 / 7.2).
+// trip is worth (int8, K = 1024, N = 11264, 12 rows: 12.2 us so, 9.0 with the sums dropped at the load).
 #pragma once
 #include "gemv_kernels.h"
 #include "decode_kernels.h"
@@ -139,9 +139,6 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   constexpr int kLanesPerRow = 64 / MROWS;
   constexpr int kPartLoads = kPro == kProNormSums ? (64 + kLanesPerRow - 1) / kLanesPerRow : 1;  // up to 256 parts
   float4 sums[kPartLoads];
-  // what the activations need is held from its request on; several rows and their sums only where that was the faster
-  // (int8, K = 4096, N = 11264, 4 rows: 12.4 us, 14.3 without; int4 gains nothing from it)
-  constexpr bool kHeld = kPro != kProNormSums || MROWS == 1 || (!kW4 && MROWS <= 4 && kWaves * kSlice == 4096);
   if (kPro == kProNormSums) {
     const int row = lane / kLanesPerRow, piece = lane % kLanesPerRow;
 #pragma unroll
@@ -149,7 +146,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
       const int j = piece + u * kLanesPerRow;
       const bool live = 4 * j < S && row < M;  // (idle lanes re-read the first 16 bytes)
       sums[u] = *reinterpret_cast<const float4*>(src1 + (live ? (size_t)row * S + 4 * j : 0));
-      if (!kHeld) sums[u] = live ? sums[u] : float4{0.f, 0.f, 0.f, 0.f};
+      sums[u] = live ? sums[u] : float4{0.f, 0.f, 0.f, 0.f};
     }
   }
   if (kW4) {  // before the weights: scales and zero-points are there when the first tile lands
@@ -169,7 +166,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   constexpr int kLiveRows = MROWS < 4 ? MROWS : 4;
   float h_old[kLiveRows], gain_n = 0.f;
   uint32_t scale_bits = 0;  // (what is used at the very end goes behind the weights in issue order)
-  constexpr bool kScaleAhead = !kW4 && kHeld && (kPro != kProMerge || MROWS == 1);
+  constexpr bool kScaleAhead = !kW4 && kPro != kProNormSums && (kPro != kProMerge || MROWS == 1);
   if (kScaleAhead) scale_bits = scales8[nt * kTileN + nl];
   if (kResid) {
     gain_n = gain[nt * kTileN + nl];
@@ -219,12 +216,8 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
     // a row's total in its first lane, then through the wave's own LDS words to whoever holds a piece of the row
     float total = 0.f;
 #pragma unroll
-    for (int u = 0; u < kPartLoads; ++u) {
-      // (the idle lanes' words are dropped here and not at the load, which would become a branch of its own)
-      if (kHeld) asm volatile("" : "+v"(sums[u].x), "+v"(sums[u].y), "+v"(sums[u].z), "+v"(sums[u].w));
-      const bool live = !kHeld || (4 * (lane % kLanesPerRow + u * kLanesPerRow) < S && lane / kLanesPerRow < M);
-      total += live ? (sums[u].x + sums[u].y) + (sums[u].z + sums[u].w) : 0.f;
-    }
+    for (int u = 0; u < kPartLoads; ++u)
+      total += (sums[u].x + sums[u].y) + (sums[u].z + sums[u].w);
     if (kLanesPerRow >= 16) {
       total = team_sum16(total);  // DPP row rotates inside each 16 lanes, then lane swaps for whole rows of 16
       if (kLanesPerRow == 64) total = quad_sum(total);
@@ -233,12 +226,11 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
 #pragma unroll
       for (int off = kLanesPerRow / 2; off > 0; off >>= 1) total += __shfl_xor(total, off);
     }
-    if (MROWS > 1 && lane % kLanesPerRow == 0) ssq[(lane / kLanesPerRow) * kWaves + wave] = total;
+    if (lane % kLanesPerRow == 0) ssq[(lane / kLanesPerRow) * kWaves + wave] = total;
 #pragma unroll
     for (int i = 0; i < kXLoads; ++i) {
       const int v = min(lane + 64 * i, kVecs - 1);
-      // one row: every lane already holds its total
-      const Divisor by_rms(sqrtf((MROWS > 1 ? ssq[(v / kVecPerRow) * kWaves + wave] : total) / (float)(kWaves * kSlice) + eps));  // (K, so a product where it is a power of two)
+      const Divisor by_rms(sqrtf(ssq[(v / kVecPerRow) * kWaves + wave] / (float)(kWaves * kSlice) + eps));  // (K, so a product where it is a power of two)
       const float4 h0 = a0[i][0], h1 = a0[i][1], g0v = a2[i][0], g1v = a2[i][1];
       xv[i][0] = by_rms.divide(h0.x) * g0v.x; xv[i][1] = by_rms.divide(h0.y) * g0v.y;
       xv[i][2] = by_rms.divide(h0.z) * g0v.z; xv[i][3] = by_rms.divide(h0.w) * g0v.w;
@@ -303,7 +295,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   }
   // bf16, into the wave's own LDS rows.  Lanes past the slice write its last vector once more (the same value): a branch here
   // would draw the loads of h and gain into itself, behind the wait for the row sums.
-  constexpr bool kAllStore = kHeld;
+  constexpr bool kAllStore = kPro != kProNormSums;
 #pragma unroll
   for (int i = 0; i < (kPro == kProMerge ? 0 : kXLoads); ++i) {
     const int v = kAllStore ? min(lane + 64 * i, kVecs - 1) : lane + 64 * i;
@@ -335,12 +327,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
   }
   const W4Consts w4c = w4_consts();
   const u32x4_t ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
-  // Four waves of twice the groups keep the sums of their two halves apart: added up like those of eight waves, the outputs are
-  // the same bit for bit.
-  constexpr int kHalves = kWaves == 4 ? 2 : 1;
-  static_assert(TPW % kHalves == 0, "whole groups per half");
-  f32x4_t acc[kHalves] = {};
-  auto half = [](int p) { return p * kHalves / TPW; };
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   if constexpr (kValuSums) {  // the same arithmetic as dequant_gemv_body, bit for bit
 #pragma unroll
     for (int p = 0; p < TPW; ++p) {
@@ -348,7 +335,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) part = mfma16(fragment(p, j), w4_unpack(w[p][0][j], w4c), part);
 #pragma unroll
-      for (int i = 0; i < MROWS; ++i) acc[half(p)][i] += sc[p] * (part[i] - zc[p] * gs[i][p]);
+      for (int i = 0; i < MROWS; ++i) acc[i] += sc[p] * (part[i] - zc[p] * gs[i][p]);
     }
   } else if (kW4) {
 #pragma unroll
@@ -361,7 +348,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
         asum = mfma16(a, ones, asum);
       }
 #pragma unroll
-      for (int i = 0; i < (MROWS < 4 ? MROWS : 4); ++i) acc[half(p)][i] += sc[p] * (part[i] - zc[p] * asum[i]);
+      for (int i = 0; i < (MROWS < 4 ? MROWS : 4); ++i) acc[i] += sc[p] * (part[i] - zc[p] * asum[i]);
     }
   } else {
 #pragma unroll
@@ -371,34 +358,28 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
         const u32x4_t a = fragment(p, j);
         const u32x2_t lo = w8_to_bf16(w[p][j >> 1][2 * (j & 1)]);
         const u32x2_t hi = w8_to_bf16(w[p][j >> 1][2 * (j & 1) + 1]);
-        acc[half(p)] = mfma16(a, u32x4_t{lo.x, lo.y, hi.x, hi.y}, acc[half(p)]);
+        acc = mfma16(a, u32x4_t{lo.x, lo.y, hi.x, hi.y}, acc);
       }
   }
 
   // ---- the waves' partial sums meet in LDS; wave 0 adds them in wave order
-#pragma unroll
-  for (int u = 0; u < kHalves; ++u) asm volatile("" : "+v"(acc[u]));
+  asm volatile("" : "+v"(acc));
   if (kScaleAhead) asm volatile("" : "+v"(scale_bits));
   constexpr int kLive = MROWS < 4 ? MROWS : 4;
   typedef float live_t __attribute__((ext_vector_type(kLive == 3 ? 4 : kLive)));
   live_t* redv = reinterpret_cast<live_t*>(red);
+  live_t mine;
 #pragma unroll
-  for (int u = 0; u < kHalves; ++u) {
-    live_t mine;
-#pragma unroll
-    for (int i = 0; i < kLive; ++i) mine[i] = acc[u][i];
-    if (kc < kRowQuads) redv[(wave * kHalves + u) * (16 * kRowQuads) + lane] = mine;
-  }
+  for (int i = 0; i < kLive; ++i) mine[i] = acc[i];
+  if (kc < kRowQuads) redv[wave * (16 * kRowQuads) + lane] = mine;
   __syncthreads();
   if (wave != 0 || kc >= kRowQuads) return;
-  constexpr int kParts = kWaves * kHalves;
-  static_assert(16 * kRowQuads * kLive * kHalves <= 256, "a wave's words of the reduction");
-  live_t part[kParts];
+  live_t part[kWaves];
 #pragma unroll
-  for (int u = 0; u < kParts; ++u) part[u] = redv[u * (16 * kRowQuads) + lane];
+  for (int u = 0; u < kWaves; ++u) part[u] = redv[u * (16 * kRowQuads) + lane];
   live_t sum = part[0];
 #pragma unroll
-  for (int u = 1; u < kParts; ++u) sum += part[u];
+  for (int u = 1; u < kWaves; ++u) sum += part[u];
   const int n = nt * kTileN + nl;
   float cs = 1.0f;
   if (!kW4) cs = f16_bits_to_f32(kScaleAhead ? scale_bits : (uint32_t)scales8[n]);

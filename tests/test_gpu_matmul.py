@@ -634,6 +634,14 @@ def test_norm_from_sums_on_one_row(cuda, scheme, m, k1, d, n2):
 
 
 @pytest.mark.parametrize("scheme", ["w4", "w8"])
+@pytest.mark.parametrize("m,d,n2", [(1, 2048, 4096), (2, 2048, 4112), (4, 1024, 8192), (1, 1024, 8208), (3, 2048, 12288), (4, 2048, 12304),
+                                    (1, 2048, 12336), (2, 4096, 4112), (3, 4096, 32), (1, 4096, 12304)])
+def test_norm_from_sums_of_neighbouring_tiles(cuda, scheme, m, d, n2):
+    """One to four row tiles per workgroup, on either side of every line, with a last workgroup that has fewer."""
+    test_gemv_residual_then_rowscale_against_the_oracle(cuda, scheme, m, 1024, d, n2)
+
+
+@pytest.mark.parametrize("scheme", ["w4", "w8"])
 @pytest.mark.parametrize("k,n", [(1024, 48), (2048, 48), (2048, 8208)])
 def test_norm_from_sums_adds_in_one_order(cuda, scheme, k, n):
     """One row's four waves add up in the order of two rows' eight: the same bits (the rows' sums of squares are whole numbers, so
