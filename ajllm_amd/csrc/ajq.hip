@@ -1870,22 +1870,18 @@ int ajq_attn_prefill(const float* q, const void* kcache, const void* vcache, int
   if (!aligned16(q) || !aligned16(kcache) || !aligned16(vcache) || !aligned16(out))
     return fail(AJQ_ERR_ALIGN, "ajq_attn_prefill: q, the caches and out must be 16-byte aligned");
   const dim3 grid((unsigned)(((T + kPfBQ - 1) / kPfBQ) * B * H));  // (the kernel orders the work by cost)
-  const bool f32 = cache_dtype == AJQ_KV_F32;
-  auto launch = [&](auto kernel, auto* cache_element) {
-    using CacheT = std::remove_pointer_t<decltype(cache_element)>;
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, q, reinterpret_cast<const CacheT*>(kcache),
-                       reinterpret_cast<const CacheT*>(vcache), H, Hkv, T, start, max_len, out, out_bf16);
+  auto launch = [&](auto dim) {
+    constexpr int HD = decltype(dim)::value;
+    if (cache_dtype == AJQ_KV_F32)
+      hipLaunchKernelGGL(attn_prefill_kernel<HD>, grid, dim3(256), 0, (hipStream_t)stream, q, reinterpret_cast<const float*>(kcache),
+                         reinterpret_cast<const float*>(vcache), H, Hkv, T, start, max_len, out, out_bf16);
+    else
+      hipLaunchKernelGGL(attn_prefill_steps_kernel<HD>, grid, dim3(256), 0, (hipStream_t)stream, q, reinterpret_cast<const uint16_t*>(kcache),
+                         reinterpret_cast<const uint16_t*>(vcache), H, Hkv, T, start, max_len, out, out_bf16);
   };
-  if (head_dim == 128) {
-    if (f32) launch(attn_prefill_kernel<float, 128>, (float*)nullptr);
-    else launch(attn_prefill_kernel<uint16_t, 128>, (uint16_t*)nullptr);
-  } else if (head_dim == 64) {
-    if (f32) launch(attn_prefill_kernel<float, 64>, (float*)nullptr);
-    else launch(attn_prefill_kernel<uint16_t, 64>, (uint16_t*)nullptr);
-  } else {
-    if (f32) launch(attn_prefill_kernel<float, 32>, (float*)nullptr);
-    else launch(attn_prefill_kernel<uint16_t, 32>, (uint16_t*)nullptr);
-  }
+  if (head_dim == 128) launch(std::integral_constant<int, 128>{});
+  else if (head_dim == 64) launch(std::integral_constant<int, 64>{});
+  else launch(std::integral_constant<int, 32>{});
   return check_launch("ajq_attn_prefill");
 }
 

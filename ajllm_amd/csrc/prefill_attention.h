@@ -27,13 +27,18 @@
 // the row index so that the fragment reads spread over all banks.
 //
 // Softmax bookkeeping is kept off the common path.  A row's reference point only moves when an
-// exponent would exceed 2^kPfSlack (always on the first block): the test is one compare of the
+// exponent would exceed 2^kPfSlack (always on the first keys): the test is one compare of the
 // lane's sum of new probabilities (a sum of positives bounds each of them; inf passes it too),
 // and only then are the maxima taken (across the four lanes of a row with two lane swaps), the
 // probabilities recomputed and the accumulators rescaled.  Row sums stay per lane and meet once,
 // at the end.  bf16 inputs, fp32 scores, probabilities rounded to bf16 for the second product,
 // fp32 accumulators: the usual flash-attention arithmetic, not the eager fp32 one.
+//
+// Two kernels: bf16 caches (attn_prefill_steps_kernel) interleave both products and the softmax of three neighbouring half blocks;
+// fp32 caches pass through registers that are converted on the way, which leaves none for that (attn_prefill_kernel).
 #pragma once
+#include <type_traits>
+
 #include "ajq_common.h"
 #include "gemm_kernels.h"  // dma16: global -> LDS without registers
 
@@ -54,12 +59,10 @@ struct Raw8F32 {
 __device__ __forceinline__ Raw8F32 load8_raw(const float* p) {
   return Raw8F32{reinterpret_cast<const float4*>(p)[0], reinterpret_cast<const float4*>(p)[1]};
 }
-__device__ __forceinline__ u32x4_t load8_raw(const uint16_t* p) { return *reinterpret_cast<const u32x4_t*>(p); }
 __device__ __forceinline__ u32x4_t to_bf16x8(const Raw8F32& r) {
   const float v[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
   return pack8_bf16(v);
 }
-__device__ __forceinline__ u32x4_t to_bf16x8(const u32x4_t& r) { return r; }
 
 typedef short pf_i16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) pf_i16x4_t pf_lds_i16x4_t;
@@ -75,15 +78,15 @@ __device__ __forceinline__ u32x2_t pf_read_tr(uint32_t address) {
 __device__ __forceinline__ u32x4_t pf_read128(uint32_t address) { return *(pf_lds_u32x4_t*)address; }
 #pragma clang diagnostic pop
 
-template <typename CacheT, int HD>
-__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __restrict__ q, const CacheT* __restrict__ kcache,
-                                                           const CacheT* __restrict__ vcache, int H, int Hkv, int T,
+template <int HD>
+__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __restrict__ q, const float* __restrict__ kcache,
+                                                           const float* __restrict__ vcache, int H, int Hkv, int T,
                                                            int start, int max_len, void* __restrict__ out, int out_bf16) {
   static_assert(HD == 128 || HD == 64 || HD == 32, "head_dim 128, 64 or 32");
   constexpr int kPfHD = HD;
   constexpr int RB = 2 * HD;          // bytes of a key (value) row as bf16
   constexpr int C = HD / 8;           // 16-byte chunks per row
-  constexpr int KS = HD / 32;         // k-steps of the first product; also the parts a block's DMA is issued in
+  constexpr int KS = HD / 32;         // k-steps of the first product
   constexpr int TT = HD / 16;         // 32-byte segments per row = 16-dim output tiles
   constexpr int kPfTileBytes = kPfBK * RB;  // one block of keys (or values) as bf16: 16 KiB at HD = 128
   // LDS map (byte addresses relative to lds0, the array's LDS address, which is 0 because the kernel
@@ -118,8 +121,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
   const float qscale =  // log2(e) / sqrt(HD)
       1.4426950408889634f * (HD == 128 ? 0.08838834764831845f : HD == 64 ? 0.125f : 0.17677669529663687f);
 
-  const CacheT* kbase = kcache + ((size_t)b * Hkv + hk) * max_len * kPfHD;
-  const CacheT* vbase = vcache + ((size_t)b * Hkv + hk) * max_len * kPfHD;
+  const float* kbase = kcache + ((size_t)b * Hkv + hk) * max_len * kPfHD;
+  const float* vbase = vcache + ((size_t)b * Hkv + hk) * max_len * kPfHD;
   const int kv_len = start + T;                               // rows the caches hold for this call
   const int kv_end = min(kv_len, start + q0 + kPfBQ);         // keys any row of this workgroup may see
   const int nblk = (kv_end + kPfBK - 1) / kPfBK;
@@ -137,37 +140,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
     for (int t = 0; t < TT; ++t) o[u][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 
-  // ---- Keys and values on their way into LDS.
-  // bf16 caches: global -> LDS directly, one block ahead.  A wave-wide request fills 1 KiB = 4 key
-  // rows (8 rows at HD = 64); wave w takes rows 4 w .. 4 w + 3 of every group of 16, so (row & 15) = 4 w + lane / 16 is
-  // fixed per lane and the chunk it must fetch for its slot is too.
-  // fp32 caches: through registers (converted on the way), one block in registers while the
+  // ---- Keys and values on their way into LDS: through registers (converted on the way), one block in registers while the
   // previous one is being read: chunk ci = tid + 256 i (i < 4) is (key ci / 16, dims 8 (ci % 16) ..).
   // Rows past the filled part of the cache repeat its last row (finite values; those keys are masked).
-  constexpr bool kDma = sizeof(CacheT) == 2;
-  constexpr int kReqRows = 1024 / RB;  // key rows of one wave-wide request: 4 (HD = 128) or 8
-  const int krow = kReqRows * wave + lane / C, slot = lane % C;
-  const uint32_t k_chunk = (uint32_t)(slot ^ (krow & (C - 1)));
-  const uint32_t v_chunk = (uint32_t)((((slot >> 1) ^ (krow & (TT - 1))) << 1) | (slot & 1));
-  // part i (0 .. KS - 1) of block jblk: this wave's kReqRows key rows and value rows of the i-th group of 4 * kReqRows
-  auto issue_dma = [&](int jblk, int i) {
-    const int kb0 = jblk * kPfBK;
-    const uint32_t stage = lds0 + (uint32_t)((jblk & 1) * 2 * kPfTileBytes);
-    const uint32_t k_to = stage + (uint32_t)((wave + 4 * i) * 1024), v_to = k_to + (uint32_t)kPfTileBytes;
-    if (kb0 + kPfBK <= kv_len) {
-      const size_t row0 = (size_t)(kb0 + 4 * kReqRows * i) * RB;
-      dma16(reinterpret_cast<const char*>(kbase) + row0, (uint32_t)(krow * RB) + k_chunk * 16u, k_to);
-      dma16(reinterpret_cast<const char*>(vbase) + row0, (uint32_t)(krow * RB) + v_chunk * 16u, v_to);
-    } else {
-      const uint32_t row = (uint32_t)min(kb0 + 4 * kReqRows * i + krow, kv_len - 1) * (uint32_t)RB;
-      dma16(kbase, row + k_chunk * 16u, k_to);
-      dma16(vbase, row + v_chunk * 16u, v_to);
-    }
-  };
-  typedef decltype(load8_raw(kbase)) raw8_t;
-  constexpr int kRegParts = kDma ? 0 : kPfBK * C / 256;  // 16-byte chunks of a block per thread: 4 (HD = 128) or 2
-  raw8_t kraw[kDma ? 1 : kRegParts], vraw[kDma ? 1 : kRegParts];
-  uint32_t k_st[kDma ? 1 : kRegParts], v_st[kDma ? 1 : kRegParts];
+  constexpr int kRegParts = kPfBK * C / 256;  // 16-byte chunks of a block per thread: 4 (HD = 128) or 2
+  Raw8F32 kraw[kRegParts], vraw[kRegParts];
+  uint32_t k_st[kRegParts], v_st[kRegParts];
   auto fetch = [&](int kb0) {
 #pragma unroll
     for (int i = 0; i < kRegParts; ++i) {
@@ -203,14 +181,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
   for (int t = 0; t < TT; ++t)
     v_rd[t] = lds0 + (uint32_t)(kPfTileBytes + vkey * RB + 32 * (t ^ (vkey & (TT - 1))) + 8 * (r & 3));
 
-  if (kDma) {
-#pragma unroll
-    for (int i = 0; i < KS; ++i) issue_dma(0, i);
-  } else {
-    fetch(0);
-    lay_down(0);
-    if (nblk > 1) fetch(kPfBK);
-  }
+  fetch(0);
+  lay_down(0);
+  if (nblk > 1) fetch(kPfBK);
   // ---- (after the first block's requests, so that both round trips to memory overlap)
   // Q fragments of the wave's two groups of 16 rows: Q[qrow][32 s + 8 g .. + 8), scaled, bf16.
   // Group u of wave w holds rows q0 + 32 w + 16 u .. + 15; this lane's row of it is qrow[u].
@@ -229,26 +202,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
       qf[u][s] = pack8_bf16(v);
     }
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   for (int j = 0; j < nblk; ++j) {
-    // One barrier per block: block j is complete in stage j & 1 (it landed before the previous
-    // barrier); block j + 1 goes into the other stage, which was last read before that barrier
-    // too (fp32 caches: from registers, while block j + 2 starts its flight from memory).
+    // One barrier per block: block j is complete in stage j & 1 (it was laid down before the previous barrier); block j + 1 goes into
+    // the other stage, which was last read before that barrier too, while block j + 2 starts its flight from memory.
     const int kb0 = j * kPfBK;
-    // bf16 caches: the requests for block j + 1 are issued between the products below (one part
-    // per k-step), or here by a wave that has no products to form
-    const bool more = j + 1 < nblk;
-    if (more) {
-      if (kDma) {
-        if (kb0 > wave_last_pos) {
-#pragma unroll
-          for (int i = 0; i < KS; ++i) issue_dma(j + 1, i);
-        }
-      } else {
-        lay_down((j + 1) & 1);
-        if (j + 2 < nblk) fetch(kb0 + 2 * kPfBK);
-      }
+    if (j + 1 < nblk) {
+      lay_down((j + 1) & 1);
+      if (j + 2 < nblk) fetch(kb0 + 2 * kPfBK);
     }
     // a wave whose last query lies before the block has nothing to add
     if (kb0 <= wave_last_pos) {
@@ -261,19 +222,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
       for (int jb = 0; jb < 4; ++jb) ka[jb] = pf_read128(k_rd[0] + (uint32_t)(jb * 16 * RB));
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        u32x4_t kn[4];
-        if (kDma && s < KS - 1) {  // (the fp32 path has no registers to spare for a second set)
-#pragma unroll
-          for (int jb = 0; jb < 4; ++jb) kn[jb] = pf_read128(k_rd[s + 1] + (uint32_t)(jb * 16 * RB));
-        }
 #pragma unroll
         for (int jb = 0; jb < 4; ++jb)
 #pragma unroll
           for (int u = 0; u < 2; ++u) sc[u][jb] = mfma16(ka[jb], qf[u][s], s == 0 ? negm[u] : sc[u][jb]);
-        if (kDma && more) issue_dma(j + 1, s);
         if (s < KS - 1) {
 #pragma unroll
-          for (int jb = 0; jb < 4; ++jb) ka[jb] = kDma ? kn[jb] : pf_read128(k_rd[s + 1] + (uint32_t)(jb * 16 * RB));
+          for (int jb = 0; jb < 4; ++jb) ka[jb] = pf_read128(k_rd[s + 1] + (uint32_t)(jb * 16 * RB));
         }
       }
       // only blocks that reach past the wave's first query position need the causal mask
@@ -326,7 +281,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
       // ---- O^T[hd 16 t + 4 g + i][qrow] += sum over the keys of each 32-key half; a value fragment
       // (two transposing reads: the half's first and second 16-key tile) meets both query groups.
       // The second half's fragments are requested as the first half's are consumed.
-      constexpr int kRing = kDma ? (TT < 8 ? TT : 8) : 4;  // fragments in flight (the fp32 path has fewer registers to spare)
+      constexpr int kRing = 4;  // fragments in flight
       auto v_lo = [&](int i) { return pf_read_tr(v_rd[i % TT] + (uint32_t)((i / TT) * 32 * RB)); };
       auto v_hi = [&](int i) { return pf_read_tr(v_rd[i % TT] + (uint32_t)((i / TT) * 32 * RB + 16 * RB)); };
       u32x2_t vlo[kRing], vhi[kRing];
@@ -351,9 +306,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
     for (int s = 0; s < KS; ++s) k_rd[s] ^= (uint32_t)(2 * kPfTileBytes);
 #pragma unroll
     for (int t = 0; t < TT; ++t) v_rd[t] ^= (uint32_t)(2 * kPfTileBytes);
-    // the next block must have landed and every wave must be done with this one
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    __syncthreads();  // every wave is done with this block
   }
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
@@ -372,6 +325,284 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
       for (int t = 0; t < TT; ++t)
         *reinterpret_cast<float4*>(dst + 16 * t) =
             float4{o[u][t][0] * inv, o[u][t][1] * inv, o[u][t][2] * inv, o[u][t][3] * inv};
+    }
+  }
+}
+
+// bf16 caches.  The keys are walked in steps of 32.  Step t holds three things that need nothing of each other: the exponents of step t + 1, the
+// softmax of step t, and the values of step t - 1 times their probabilities; they are laid out in HD / 16 pieces of two MFMAs of either product, their
+// share of the exponentials and sums, and the fragments three pieces ahead, in that order for good (sched_barrier): a wave has MFMAs and
+// vector work to issue side by side instead of one after the other, and two waves per SIMD fill what is left.  Before, each wave went through
+// product, softmax and product in turn and a CU's two workgroups overlapped by chance: 3440 cycles per 64 keys and two waves, 2730 now (64 MFMAs a
+// wave are 2048).  What bounds it is the clock (2.19 -> 1.95 GHz as the matrix pipes fill).  B = 4, 32 / 8 heads, T = 2048: 164 -> 152 us alone, 171 -> 155
+// in a row; a few short grids, where a wave's own length counts: 0.79 .. 0.9 of the time; heads of 64: 0.92, of 32: 0.98.
+//
+// Keys run a step ahead of the values, so key block j + 2 and value block j + 1 are asked for in the second step of block j, behind the one
+// barrier per block: every wave has consumed what lay there (keys of block j, values of block j - 1), and what it
+// reads next (keys j + 1, values j) was asked for a block before and waited for in front of that barrier.
+// Four steps at places known to the compiler make the body; a wave's last ones (masked, or with blocks cut short) go one by one.
+template <int HD>
+__global__ __launch_bounds__(256, 2) void attn_prefill_steps_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kcache,
+                                                                 const uint16_t* __restrict__ vcache, int H, int Hkv, int T,
+                                                                 int start, int max_len, void* __restrict__ out, int out_bf16) {
+  static_assert(HD == 128 || HD == 64 || HD == 32, "head_dim 128, 64 or 32");
+  // bytes of a row, 16-byte chunks of it, k-steps of the first product (and a wave's requests per tile), 16-dim output tiles
+  constexpr int RB = 2 * HD, C = HD / 8, KS = HD / 32, TT = HD / 16, U = 2, kAhead = 3;
+  constexpr int kTile = kPfBK * RB;  // LDS: two stages of a key tile and a value tile, laid out as below
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[4 * kTile];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(pf_lds_char_t*)lds;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  // (work order: see attn_prefill_kernel)
+  const int qblocks = (T + kPfBQ - 1) / kPfBQ;
+  const int BH = (int)(gridDim.x / (unsigned)qblocks);
+  int qb, bh;
+  if ((BH & 7) == 0) {
+    const int per_xcd = BH >> 3, m = (int)(blockIdx.x >> 3);
+    qb = qblocks - 1 - m / per_xcd;
+    bh = (int)(blockIdx.x & 7) * per_xcd + m % per_xcd;
+  } else {
+    qb = qblocks - 1 - (int)blockIdx.x / BH;
+    bh = (int)blockIdx.x % BH;
+  }
+  const int b = bh / H, h = bh % H, hk = h / (H / Hkv);
+  const int q0 = qb * kPfBQ;
+  const float qscale = 1.4426950408889634f * (HD == 128 ? 0.08838834764831845f : HD == 64 ? 0.125f : 0.17677669529663687f);
+  const uint16_t* kbase = kcache + ((size_t)b * Hkv + hk) * max_len * HD;
+  const uint16_t* vbase = vcache + ((size_t)b * Hkv + hk) * max_len * HD;
+  const int kv_len = start + T;
+  const int kv_end = min(kv_len, start + q0 + kPfBQ);
+  const int nblk = (kv_end + kPfBK - 1) / kPfBK;
+  const int wave_first = q0 + 16 * U * wave;
+  const int first_pos = start + wave_first;                                   // of this wave's queries
+  const int steps = wave_first < T ? (min(first_pos + 16 * U - 1, kv_len - 1) >> 5) + 1 : 0;  // of 32 keys each
+  float m_run[U] = {}, l_run[U] = {};
+  f32x4_t negm[U] = {};
+  f32x4_t o[U][TT];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int t = 0; t < TT; ++t) o[u][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // ---- requests: 1 KiB of rows each, global -> LDS; wave w takes rows kReqRows w .. of every group of 4 kReqRows, so the chunk that belongs in a lane's
+  // slot is the same for all of them.  Rows past the filled part of the cache repeat its last row (finite values; those keys are masked).
+  constexpr int kReqRows = 1024 / RB;
+  const int krow = kReqRows * wave + lane / C, slot = lane % C;
+  const uint32_t k_chunk = (uint32_t)(slot ^ (krow & (C - 1))) * 16u;
+  const uint32_t v_chunk = (uint32_t)((((slot >> 1) ^ (krow & (TT - 1))) << 1) | (slot & 1)) * 16u;
+  const uint32_t k_lane = (uint32_t)(krow * RB) + k_chunk, v_lane = (uint32_t)(krow * RB) + v_chunk;
+  auto place = [&](bool values, int i, int stage) __attribute__((always_inline)) {
+    return lds0 + (uint32_t)(stage * 2 * kTile + (values ? kTile : 0) + (wave + 4 * i) * 1024);
+  };
+  auto request = [&](int j, bool values) __attribute__((always_inline)) {  // of block j < nblk
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      const uint32_t row = (uint32_t)min(4 * kReqRows * i + krow, kv_len - 1 - j * kPfBK) * (uint32_t)RB;
+      dma16(reinterpret_cast<const char*>(values ? vbase : kbase) + (size_t)j * kPfBK * RB, row + (values ? v_chunk : k_chunk), place(values, i, j & 1));
+    }
+  };
+  // ---- LDS read addresses within stage 0 (fragments and their places: see attn_prefill_kernel)
+  uint32_t k_rd[KS], v_rd[TT];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) k_rd[s] = lds0 + (uint32_t)(r * RB + 16 * ((4 * s + g) ^ (r & (C - 1))));
+  const int vkey = 4 * g + (r >> 2);
+#pragma unroll
+  for (int t = 0; t < TT; ++t) v_rd[t] = lds0 + (uint32_t)(kTile + vkey * RB + 32 * (t ^ (vkey & (TT - 1))) + 8 * (r & 3));
+
+  request(0, false);
+  request(0, true);
+  int q_pos[U];
+  u32x4_t qf[U][KS];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int row = wave_first + 16 * u + r;
+    q_pos[u] = start + row;
+    const float* qp = q + ((size_t)bh * T + min(row, T - 1)) * HD + 8 * g;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const float4 a = reinterpret_cast<const float4*>(qp + 32 * s)[0], c = reinterpret_cast<const float4*>(qp + 32 * s)[1];
+      const float v[8] = {a.x * qscale, a.y * qscale, a.z * qscale, a.w * qscale, c.x * qscale, c.y * qscale, c.z * qscale, c.w * qscale};
+      qf[u][s] = pack8_bf16(v);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[u][s]));
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (nblk > 1) request(1, false);
+  turn_barrier();
+  f32x4_t sn[U][2];  // exponents of the step ahead
+  u32x4_t pf[U];     // probabilities of the step behind
+  auto key_frag = [&](int at, int i) __attribute__((always_inline)) { return pf_read128(k_rd[i >> 1] + (uint32_t)(at + (i & 1) * 16 * RB)); };
+  auto score = [&](const u32x4_t& kf, int i) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) sn[u][i & 1] = mfma16(kf, qf[u][i >> 1], i < 2 ? negm[u] : sn[u][i & 1]);
+  };
+  // Step t: exponents from the keys at k_at, values at v_at (kV: not in the very first, which takes its reference points instead), and req(piece)
+  auto step = [&](int t, auto values, auto masked, int k_at, int v_at, auto req) __attribute__((always_inline)) {
+    constexpr bool kV = decltype(values)::value;
+    f32x4_t sc[U][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb) sc[u][jb] = sn[u][jb];
+    u32x4_t kf[TT];
+    u32x2_t vl[TT], vh[TT];
+    auto fetch = [&](int i) __attribute__((always_inline)) {
+      kf[i] = key_frag(k_at, i);
+      if (kV) {
+        vl[i] = pf_read_tr(v_rd[i] + (uint32_t)v_at);
+        vh[i] = pf_read_tr(v_rd[i] + (uint32_t)(v_at + 16 * RB));
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < (kAhead < TT ? kAhead : TT); ++i) fetch(i);
+    if (decltype(masked)::value && 32 * t + 31 > first_pos) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (32 * t + 16 * jb + 4 * g + i > q_pos[u]) sc[u][jb][i] = -INFINITY;
+    }
+    u32x4_t pn[U];
+    float p[U][8], psum[U] = {};
+    constexpr int kPer = 8 * U / TT;  // exponentials of a piece
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+      if (i + kAhead < TT) fetch(i + kAhead);
+      req(i);
+      score(kf[i], i);
+#pragma unroll
+      for (int x = 0; x < kPer; ++x) {
+        const int u = (i * kPer + x) >> 3, e = (i * kPer + x) & 7;
+        p[u][e] = __builtin_amdgcn_exp2f(sc[u][e >> 2][e & 3]);
+        psum[u] += p[u][e];
+      }
+      if (U * (i + 1) % TT == 0) {  // a group of rows is through (pinned: the compiler would sink it behind the branches below)
+        const int u = U * i / TT;
+        pn[u] = pack8_bf16(p[u]);
+        asm volatile("" : "+v"(pn[u]), "+v"(psum[u]));
+      }
+      if (kV) {
+        const u32x4_t vf = {vl[i].x, vl[i].y, vh[i].x, vh[i].y};
+#pragma unroll
+        for (int u = 0; u < U; ++u) o[u][i] = mfma16(vf, pf[u], o[u][i]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool revisit = !kV || psum[u] > kPfTrigger;
+      if (!kV || __builtin_amdgcn_ballot_w64(revisit) != 0) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) mx = fmaxf(mx, sc[u][e >> 2][e & 3]);
+        if (!kV)  // the first reference point is that of the whole first block
+#pragma unroll
+          for (int e = 0; e < 8; ++e) mx = fmaxf(mx, 32 + 16 * (e >> 2) + 4 * g + (e & 3) > q_pos[u] ? -INFINITY : sn[u][e >> 2][e & 3]);
+        mx = quad_max(mx);
+        const bool move = !kV || mx > kPfSlack;
+        const float shift = move ? mx : 0.f;
+        const float corr = (move && kV) ? __builtin_amdgcn_exp2f(-shift) : 1.0f;
+        psum[u] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          p[u][e] = __builtin_amdgcn_exp2f(sc[u][e >> 2][e & 3] - shift);
+          psum[u] += p[u][e];
+        }
+        pn[u] = pack8_bf16(p[u]);
+        m_run[u] += shift;
+        negm[u] = f32x4_t{-m_run[u], -m_run[u], -m_run[u], -m_run[u]};
+#pragma unroll
+        for (int jb = 0; jb < 2; ++jb) sn[u][jb] -= shift;  // (began at the old reference point)
+        if (kV) {
+          l_run[u] *= corr;
+#pragma unroll
+          for (int tt = 0; tt < TT; ++tt) o[u][tt] *= corr;
+        }
+      }
+      l_run[u] += psum[u];
+      pf[u] = pn[u];
+    }
+  };
+  auto last_values = [&](int v_at) __attribute__((always_inline)) {
+    u32x2_t vl[TT], vh[TT];
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+      vl[i] = pf_read_tr(v_rd[i] + (uint32_t)v_at);
+      vh[i] = pf_read_tr(v_rd[i] + (uint32_t)(v_at + 16 * RB));
+    }
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+      const u32x4_t vf = {vl[i].x, vl[i].y, vh[i].x, vh[i].y};
+#pragma unroll
+      for (int u = 0; u < U; ++u) o[u][i] = mfma16(vf, pf[u], o[u][i]);
+    }
+  };
+  constexpr std::integral_constant<bool, true> yes{};
+  constexpr std::integral_constant<bool, false> no{};
+  auto none = [](int) {};
+  if (steps > 0) {
+    u32x4_t kf[TT];
+#pragma unroll
+    for (int i = 0; i < TT; ++i) kf[i] = key_frag(0, i);
+#pragma unroll
+    for (int i = 0; i < TT; ++i) score(kf[i], i);
+    step(0, no, yes, 32 * RB, 0, none);
+  }
+  // blocks j (even) and j + 1: the second step of j, both of j + 1, the first of j + 2
+  int j = 0;
+  const char* k_from = reinterpret_cast<const char*>(kbase) + 2 * kPfBK * RB;
+  const char* v_from = reinterpret_cast<const char*>(vbase) + kPfBK * RB;
+  for (; 2 * j + 5 < steps && 64 * j + 159 <= first_pos && (j + 4) * kPfBK <= kv_end; j += 2) {
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      turn_barrier();
+      step(2 * j + 2 * x + 1, yes, no, (x ^ 1) * 2 * kTile, x * 2 * kTile, [&](int i) __attribute__((always_inline)) {
+        if (i < KS) dma16(k_from + i * 4096, k_lane, place(false, i, x));
+        else dma16(v_from + (i - KS) * 4096, v_lane, place(true, i - KS, x ^ 1));
+      });
+      k_from += kPfBK * RB;
+      v_from += kPfBK * RB;
+      step(2 * j + 2 * x + 2, yes, no, (x ^ 1) * 2 * kTile + 32 * RB, x * 2 * kTile + 32 * RB, none);
+    }
+  }
+  for (int t = 2 * j + 1; t < 2 * nblk; ++t) {
+    const int block = t >> 1;
+    if (t & 1) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      turn_barrier();
+      if (block + 2 < nblk) request(block + 2, false);
+      if (block + 1 < nblk) request(block + 1, true);
+    }
+    auto half = [&](int n) { return ((n >> 1) & 1) * 2 * kTile + (n & 1) * 32 * RB; };  // where step n's keys (values) lie
+    // (the last step's exponents of the one behind it are of no use, whatever lies there)
+    if (t < steps) step(t, yes, yes, half(t + 1), half(t - 1), none);
+    else if (t == steps) last_values(half(t - 1));
+  }
+  if (steps == 2 * nblk) last_values(((nblk - 1) & 1) * 2 * kTile + 32 * RB);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float inv = 1.0f / quad_sum(l_run[u]);
+    const int row = wave_first + 16 * u + r;
+    if (row >= T) continue;
+    const size_t at = ((size_t)b * T + row) * ((size_t)H * HD) + (size_t)h * HD + 4 * g;
+    if (out_bf16) {
+      uint16_t* dst = reinterpret_cast<uint16_t*>(out) + at;
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+        *reinterpret_cast<u32x2_t*>(dst + 16 * t) =
+            u32x2_t{pack2_bf16(o[u][t][0] * inv, o[u][t][1] * inv), pack2_bf16(o[u][t][2] * inv, o[u][t][3] * inv)};
+    } else {
+      float* dst = reinterpret_cast<float*>(out) + at;
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+        *reinterpret_cast<float4*>(dst + 16 * t) = float4{o[u][t][0] * inv, o[u][t][1] * inv, o[u][t][2] * inv, o[u][t][3] * inv};
     }
   }
 }

@@ -632,6 +632,26 @@ def test_flash_prefill_attention(cuda, b, heads, kv_heads, t, start, cache_dtype
     assert errors(got, want.cpu())[1] <= 1e-2, errors(got, want.cpu())
 
 
+@pytest.mark.parametrize("hd", [128, 64, 32])
+@pytest.mark.parametrize("t,start", [(31, 0), (32, 1), (33, 31), (64, 0), (65, 32), (96, 63), (127, 64), (129, 0), (160, 95), (191, 129), (256, 33), (289, 287)])
+def test_flash_prefill_on_bf16_caches_at_the_edges_of_its_steps(cuda, t, start, hd):
+    """Last steps, blocks and query groups cut short, rows past the fill never read (NaN), and scores that grow along the keys, so that
+    reference points move in either half of a block while the step ahead has begun at the old ones; tolerance as above."""
+    from ajllm_amd.attention import flash_prefill
+    g, total, heads = torch.Generator().manual_seed(t + start + hd), start + t, 4
+    q = 3 * torch.randn((2, heads, t, hd), generator=g)
+    keys, values = (torch.randn((2, 2, total + 5, hd), generator=g) for _ in range(2))
+    keys *= torch.linspace(0.2, 4, total + 5)[:, None]
+    keys[:, :, total:] = values[:, :, total:] = float("nan")
+    q, keys, values = q.to(cuda), keys.to(cuda).bfloat16(), values.to(cuda).bfloat16()
+    got = flash_prefill(q, keys, values, start)
+    k32, v32 = (x[:, :, :total].float().repeat_interleave(heads // 2, dim=1) for x in (keys, values))
+    mask = torch.ones(t, total, dtype=torch.bool, device=cuda).tril_(diagonal=start)
+    scaled = (q * (1.4426950408889634 * hd ** -0.5)).bfloat16().float() / (1.4426950408889634 * hd ** -0.5)   # (as the kernel rounds them)
+    want = modeling.scaled_dot_product_attention(scaled, k32, v32, mask).transpose(1, 2).reshape(2, t, heads * hd)
+    assert errors(got, want.cpu())[1] <= 4e-3
+
+
 def test_model_with_flash_attention_flag(cuda):
     """use_flash_attention on every attention layer: prefill logits stay within flash-attention noise of
     the eager model, with and without a KV cache, and a following cached step agrees as well."""
