@@ -7,7 +7,7 @@
 // Prompts (any number of tokens, from any position; also one token on any operand type):
 //   conv_silu_kernel, conv_silu_run_kernel (prompts with usual widths), scan_kernel
 // One token in bf16:
-//   scan_project_kernel, scan_step_kernel
+//   scan_project_kernel, scan_step_kernel, scan_step_narrow_kernel
 //
 // States and a2 = A log2(e) (decays are taken in base 2) are stored in planes of four: [states / 4][channels][4], so that threads
 // of neighbouring channels load whole lines; `states` is a multiple of 4 (states past a model's own are zero).
@@ -337,9 +337,14 @@ __device__ __forceinline__ int column_slot(int slot, int back, int reach) {
 }
 
 // The projection of the convolved columns to (dt rank | B | C): `rows` weight rows (a multiple of 16), K = inner cut into
-// `splits` parts whose sums scan_step_kernel adds.  A workgroup takes RT row tiles and a part of K in blocks of kScanBlock
-// channels: a wave requests its weights, all threads convolve the block's channels into LDS (a thread 8 channels of every
-// second sequence, its weights in registers), then the product.  Grid (row groups, splits, batch blocks).
+// `splits` parts whose sums the step's kernel adds.  A workgroup takes RT row tiles and a part of K in blocks of 128 kSteps
+// channels: a wave requests its weights, all threads convolve the block's channels into LDS (a thread 8 channels of some
+// sequences, the weights in registers), then the product.  Grid (row groups, splits, batch blocks).  What a CU can pull bounds
+// it: every row group convolves the channels again, so a block of 1024 leaves most CUs idle while the others read weights, taps
+// and columns of four times as many channels.  With 256 (4096 channels, 160 rows; 1 / 4 / 16 / 32 sequences): 4.2 / 5.1 / 9.7
+// / 9.8 -> 3.2 / 3.3 / 4.2 / 4.6 us.  Held against requests of the ring's rows ahead of the position (5.1 -> 6.4: the
+// position is a scalar load and early enough, the choice among the rows is not free) and more waves on 1024 channels (8.4).
+__host__ __device__ constexpr int scan_block(int steps) { return 4 * 32 * steps; }
 struct ScanProject {
   const float* y;           // [B, ldy]: convolved columns, then z
   const uint16_t* ring;     // [B, taps - 1, inner]
@@ -350,11 +355,10 @@ struct ScanProject {
   float* partial;           // [splits, B, rows]
   int batch, ldy, inner, taps, rows, splits;
 };
-constexpr int kScanBlock = 1024;
-// TAPS: the convolution's width, or 0 for any
-template <int RT, int TAPS>
+// TAPS: the convolution's width, or 0 for any; kSteps: of 32 channels, a wave's share of a block
+template <int RT, int TAPS, int kSteps>
 __global__ __launch_bounds__(256) void scan_project_kernel(ScanProject a) {
-  constexpr int kSteps = kScanBlock / 32 / 4, kLd = kScanBlock + 8;
+  constexpr int kBlock = scan_block(kSteps), kLd = kBlock + 8, kLanes = kBlock / 8;
   __shared__ __attribute__((aligned(16))) uint16_t conv[kGemvBatch * kLd];
   __shared__ __attribute__((aligned(16))) float red[RT * 4 * 256];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
@@ -364,9 +368,9 @@ __global__ __launch_bounds__(256) void scan_project_kernel(ScanProject a) {
   const int steps = (a.inner + 31) >> 5, per = (steps + a.splits - 1) / a.splits;
   const int lo = min(steps, (int)blockIdx.y * per), hi = min(steps, lo + per);
   const uint16_t* wrow = a.w + (size_t)(16 * tile0 + r) * a.inner;
-  const int vl = 8 * (tid & 127);
+  const int vl = 8 * (tid % kLanes);
   f32x4_t acc[RT][1] = {};
-  for (int s0 = lo; s0 < hi; s0 += kScanBlock / 32) {
+  for (int s0 = lo; s0 < hi; s0 += kBlock / 32) {
     const int mine = s0 + kSteps * wave;
     u32x4_t w[kSteps][RT];
 #pragma unroll
@@ -385,7 +389,7 @@ __global__ __launch_bounds__(256) void scan_project_kernel(ScanProject a) {
       for (int j = 0; j < TAPS; ++j) f[j] = load8(a.weight + (size_t)(reach - j) * a.inner + c);
       // (a sequence's rows as they lie, so that none is waited for before all are requested)
       constexpr int kHeld = TAPS > 1 ? TAPS - 1 : 1;
-      for (int b = tid >> 7; b < nb; b += 2) {
+      for (int b = tid / kLanes; b < nb; b += 256 / kLanes) {
         const uint16_t* ring = a.ring + (size_t)(b0 + b) * reach * a.inner + c;
         u32x4_t held[kHeld];
         if (TAPS > 1)
@@ -578,6 +582,120 @@ __global__ __launch_bounds__(256) void scan_step_kernel(ScanStep a) {
       move(n, p > 0 ? load4(state + (size_t)n * a.inner * 4) : float4{0.f, 0.f, 0.f, 0.f}, load4(a.a2 + ((size_t)n * a.inner + c) * 4));
     a.out[(size_t)(b0 + b) * a.out_ld + c] = f32_to_bf16_rne(out * silu_for<uint16_t>(z[t]));
   }
+}
+
+// The same for 16 channels of four sequences, a wave per sequence, a lane per channel and plane of four states (planes past the
+// fourth in turns): four times as many workgroups, a quarter of the exponentials in a lane's chain, and no second barrier, as
+// every wave makes the tile of step sizes itself (its operand repeats the four sequences in each group of rows, so that lane
+// (channel, plane) finds its sequence's among its own four).  Up to kNarrowRank columns of w_dt.  Launch and latency bound; at
+// more than a workgroup per CU the parts, which every workgroup adds again, cost more than the rest saves.  4096 channels, 16
+// states, rank 128, 16 parts, 1 / 4 / 8 sequences: 5.8 -> 4.6 / 6.0 -> 5.2 / 6.6 -> 7.1 us.
+constexpr int kNarrowBatch = 4, kNarrowRank = 128;
+__global__ __launch_bounds__(256) void scan_step_narrow_kernel(ScanStep a) {
+  constexpr int kSteps = kNarrowRank / 32, kAhead = 16, kHeld = 3;
+  extern __shared__ __attribute__((aligned(16))) unsigned char scan_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
+  // (an XCD takes a contiguous eighth of the channels: neighbours share lines)
+  const int block = (gridDim.x & 7) == 0 ? (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+  const int b0 = blockIdx.y * kNarrowBatch, nb = min(kNarrowBatch, a.batch - b0), c = 16 * block + r;
+  const int ld = a.rank + 8, used = a.rank + 2 * a.states, quads = used >> 2, planes = a.states >> 2, reach = a.taps - 1;
+  float* bc = reinterpret_cast<float*>(scan_lds);                                 // [kNarrowBatch][2 states]
+  uint16_t* low = reinterpret_cast<uint16_t*>(bc + kNarrowBatch * 2 * a.states);  // [kNarrowBatch][rank + 8]
+  float4 ahead[kAhead];
+  auto request = [&](int i, int s0) {  // (in fours: a branch per part took 0.4 us of the launch)
+    const float* src = a.partial + (size_t)(b0 + i / quads) * a.rows + 4 * (i % quads);
+#pragma unroll
+    for (int q = 0; q < kAhead; q += 4)
+      if (s0 + q < a.splits)
+#pragma unroll
+        for (int k = q; k < q + 4; ++k) ahead[k] = load4(src + (size_t)min(s0 + k, a.splits - 1) * a.batch * a.rows);
+  };
+  if (tid < nb * quads) request(tid, 0);
+  u32x4_t w[kSteps];
+  const uint16_t* wrow = a.w_dt + (size_t)c * a.rank;
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s) w[s] = *reinterpret_cast<const u32x4_t*>(wrow + min(32 * s + 8 * g, a.rank - 8));
+  const float dt_bias = a.dt_bias[c], skip = a.d[c], conv_bias = a.bias[c], own_weight = a.weight[(size_t)reach * a.inner + c];
+  const float4 f = load4(a.a2 + ((size_t)min(g, planes - 1) * a.inner + c) * 4);
+  float tap[kHeld];
+#pragma unroll
+  for (int j = 0; j < kHeld; ++j) tap[j] = a.weight[(size_t)max(reach - 1 - j, 0) * a.inner + c];
+  const int own_b = b0 + min(wave, nb - 1);  // (a wave without a sequence leaves behind the barrier)
+  const float* y = a.y + (size_t)own_b * a.ldy + c;
+  float* state = a.state + (size_t)own_b * a.states * a.inner + 4 * c;
+  uint16_t* ring = a.ring + (size_t)own_b * reach * a.inner + c;
+  const float4 st = load4(state + (size_t)min(g, planes - 1) * a.inner * 4);
+  const float y_in = y[0], z = y[a.inner];
+  uint16_t held[kHeld];  // the ring's rows as they lie
+  if (reach > 0)
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) held[j] = ring[(size_t)min(j, reach - 1) * a.inner];
+  const int p = clamped_position(a.pos, 0, 0x7FFFFFFF), slot = reach > 0 ? p % reach : 0;
+  for (int i = tid; i < nb * quads; i += 256) {
+    float4 v = float4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < a.splits; s0 += kAhead) {
+      if (i != tid || s0 > 0) request(i, s0);
+#pragma unroll
+      for (int q = 0; q < kAhead; q += 4)
+        if (s0 + q < a.splits)
+#pragma unroll
+          for (int k = q; k < q + 4; ++k) {
+            const bool live = s0 + k < a.splits;
+            v.x += live ? ahead[k].x : 0.f; v.y += live ? ahead[k].y : 0.f; v.z += live ? ahead[k].z : 0.f; v.w += live ? ahead[k].w : 0.f;
+          }
+    }
+    const int b = i / quads, n = 4 * (i % quads);
+    if (n < a.rank) store4(low + b * ld + n, v);
+    else store4(bc + b * 2 * a.states + n - a.rank, v);
+  }
+  __syncthreads();
+  if (wave >= nb) return;
+  // step sizes: rows 4 g + i of the product are sequence i, columns the channels
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  const uint16_t* lrow = low + min(r & 3, nb - 1) * ld + 8 * g;
+  const u32x4_t none = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int s = 0; s < kSteps; ++s)
+    if (32 * s < a.rank) {
+      const bool live = 32 * s + 8 * g < a.rank;
+      acc = mfma16(live ? *reinterpret_cast<const u32x4_t*>(lrow + 32 * s) : none, live ? w[s] : none, acc);
+    }
+  const float dt = softplus_f32((wave == 0 ? acc[0] : wave == 1 ? acc[1] : wave == 2 ? acc[2] : acc[3]) + dt_bias);
+  const uint16_t own = f32_to_bf16_rne(y_in);
+  float x = conv_bias;
+  if (reach <= kHeld) {
+#pragma unroll
+    for (int j = kHeld; j > 0; --j)
+      if (j <= min(reach, p)) {
+        const int at = column_slot(slot, j, reach);
+        x = fmaf(tap[j - 1], to_f32(at == 0 ? held[0] : at == 1 ? held[1] : held[2]), x);
+      }
+  } else {
+#pragma unroll 4
+    for (int j = min(reach, p); j > 0; --j)
+      x = fmaf(a.weight[(size_t)(reach - j) * a.inner + c], to_f32(ring[(size_t)column_slot(slot, j, reach) * a.inner]), x);
+  }
+  x = fmaf(own_weight, to_f32(own), x);
+  if (reach > 0 && g == 0) ring[(size_t)slot * a.inner] = own;
+  const float v = silu_for<uint16_t>(x), dx = dt * v;
+  const float* bs = bc + wave * 2 * a.states;
+  float out = g == 0 ? skip * v : 0.f;
+  auto move = [&](int n, float4 s, const float4& k) {
+    const float4 bn = load4(bs + 4 * n), cn = load4(bs + a.states + 4 * n);
+    s.x = fmaf(__builtin_amdgcn_exp2f(dt * k.x), s.x, dx * bn.x);
+    s.y = fmaf(__builtin_amdgcn_exp2f(dt * k.y), s.y, dx * bn.y);
+    s.z = fmaf(__builtin_amdgcn_exp2f(dt * k.z), s.z, dx * bn.z);
+    s.w = fmaf(__builtin_amdgcn_exp2f(dt * k.w), s.w, dx * bn.w);
+    store4(state + (size_t)n * a.inner * 4, s);
+    out = fmaf(s.x, cn.x, fmaf(s.y, cn.y, fmaf(s.z, cn.z, fmaf(s.w, cn.w, out))));
+  };
+  const float4 zero = {0.f, 0.f, 0.f, 0.f};
+  if (g < planes) move(g, p > 0 ? st : zero, f);
+  for (int n = 4 + g; n < planes; n += 4)
+    move(n, p > 0 ? load4(state + (size_t)n * a.inner * 4) : zero, load4(a.a2 + ((size_t)n * a.inner + c) * 4));
+  out += __shfl_xor(out, 16);
+  out += __shfl_xor(out, 32);
+  if (g == 0) a.out[(size_t)own_b * a.out_ld + c] = f32_to_bf16_rne(out * silu_for<uint16_t>(z));
 }
 
 }  // namespace ajq
