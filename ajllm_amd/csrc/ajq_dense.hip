@@ -817,6 +817,42 @@ int ajqd_key_value_split(const ajqd_key_value_split_args* a, int y_dtype, int dt
   return status != AJQ_OK ? status : check_launch("ajqd_key_value_split");
 }
 
+int ajqd_group_decode_built(int share, int dimp, int rot) {
+  return share >= 1 && share <= kGroupShare && dimp >= 16 && dimp % 16 == 0 && latent_steps(2 * dimp) > 0 && latent_steps(2 * dimp) <= 10 && rot >= 0 && rot % 8 == 0;
+}
+
+int ajqd_group_decode(const ajqd_key_value_split_args* a, float* partial, int chunks, float scale, void* stream) {
+  if (!a || !partial || !a->y || !a->q_gain || !a->k_gain || (a->rot && !a->half_turns) || !a->rows || !a->pos)
+    return fail(AJQ_ERR_NULL, "ajqd_group_decode: null pointer argument");
+  if (a->tokens < 1 || a->seq != 1 || a->groups < 1 || a->heads < 1 || a->heads % a->groups || a->dim < 1 || a->dimp < a->dim || a->rot > a->dim ||
+      a->ldy < (a->heads + a->groups) * a->dimp || a->ldy % 4 || a->cap < 1 || a->kept < 0 || a->kept >= a->cap || a->prior != 0 ||
+      a->rows_head != (int64_t)a->cap * 2 * a->dimp || a->rows_batch != a->groups * a->rows_head || chunks < 1 || chunks > kLatentMaxChunks || !(scale > 0.f))
+    return fail(AJQ_ERR_SHAPE, "ajqd_group_decode: unsupported shape (tokens=%d heads=%d groups=%d dim=%d/%d rot=%d cap=%d kept=%d chunks=%d)", a->tokens,
+                a->heads, a->groups, a->dim, a->dimp, a->rot, a->cap, a->kept, chunks);
+  const int share = a->heads / a->groups;
+  if (!ajqd_group_decode_built(share, a->dimp, a->rot))
+    return fail(AJQ_ERR_UNSUPPORTED, "ajqd_group_decode: %d heads of %d columns, %d of them turned, are not built", share, a->dimp, a->rot);
+  if (!aligned16(a->y) || !aligned16(a->rows) || !aligned16(a->q_gain) || !aligned16(a->k_gain))
+    return fail(AJQ_ERR_ALIGN, "ajqd_group_decode: rows must be 16-byte aligned");
+  const long long units = (long long)a->tokens * a->groups;
+  if (units * chunks > 0x7FFFFFFFll) return fail(AJQ_ERR_SHAPE, "ajqd_group_decode: too many workgroups");
+  LatentDecode d{nullptr, (const uint16_t*)a->rows, positions64(a->pos), partial, heads_at(partial, (int)units, share, chunks, a->dimp), (int)units, share,
+                 a->dimp, 2 * a->dimp, a->cap, chunks, a->dimp / 32, scale * kLog2eF};
+  GroupRow k{(const float*)a->y, a->q_gain, a->k_gain, a->half_turns, a->ldy, a->groups, a->dim, a->rot, a->kept, a->eps};
+  auto go = [&](auto kernel, int ks) {
+    const int bytes = latent_decode_lds(ks, 1);
+    if (int e = allow_lds(kernel, bytes, "ajqd_group_decode")) return e;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(units * chunks)), dim3(256), bytes, (hipStream_t)stream, d, k);
+    return check_launch("ajqd_group_decode");
+  };
+  switch (latent_steps(2 * a->dimp)) {
+    case 4: return go(group_decode_kernel<4>, 4);
+    case 6: return go(group_decode_kernel<6>, 6);
+    case 8: return go(group_decode_kernel<8>, 8);
+    default: return go(group_decode_kernel<10>, 10);
+  }
+}
+
 int ajqd_group_merge(const float* partial, const float* gate, int gate_ld, void* out, int out_ld, int batch, int groups, int share,
                      int chunks, int dimp, void* stream) {
   if (!partial || !out) return fail(AJQ_ERR_NULL, "ajqd_group_merge: null pointer argument");

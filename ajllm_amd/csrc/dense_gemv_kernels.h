@@ -669,8 +669,33 @@ constexpr int kLatentRows = 64;
 constexpr int kBufferWord3 = 0x00020000;  // last word of a raw buffer descriptor: 32-bit elements, no swizzle
 constexpr int kLatentPBytes = (kLatentRows + 8) * 2;
 constexpr int latent_decode_lds(int ks, int ht) { return ks * 8192 + ht * 16 * kLatentPBytes; }  // two stages of ks / 2 panels
-template <int KS, int RT, int HT>
-__global__ __launch_bounds__(256 * HT) void latent_decode_kernel(LatentDecode a) {
+// Where the queries come from, and which row of the ring the launch itself makes: rows of `q`, and none.
+template <int KS>
+struct LatentQueries {
+  static constexpr bool kMakesRow = false;
+  // Requested before the position is known and in one go, through a buffer descriptor of the sequence's queries: chunks past the
+  // width are addressed past its end, which reads as zeros (left out by a branch, each was waited for before the next was
+  // requested; cleared by selects, 18 of them cost a microsecond of arithmetic).
+  __device__ __forceinline__ void request(const LatentDecode& a, int b, int h0, u32x4_t (&qf)[KS]) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4, cw = a.width >> 3;
+    const uint32_t q_bytes = 2u * (uint32_t)(a.heads * a.width);  // (a launch's queries of one sequence stay far below 2 GiB)
+    const __amdgpu_buffer_rsrc_t q_rows =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.q) + (size_t)b * a.heads * a.width, 0, (int)q_bytes, kBufferWord3);
+    const uint32_t q_at = 2u * (uint32_t)(min(h0 + r, a.heads - 1) * a.width);
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+      qf[s] = __builtin_amdgcn_raw_buffer_load_b128(q_rows, (int)(4 * s + g < cw ? q_at + 16u * (uint32_t)(4 * s + g) : q_bytes), 0, 0);
+  }
+  // (the queries are waited for behind the first block's requests and not in the loop, where the wait would be for the block ahead as well)
+  template <typename Fetch>
+  __device__ __forceinline__ void ready(const LatentDecode&, int, int, int, u32x4_t (&qf)[KS], Fetch&& fetch) {
+    fetch();
+#pragma unroll
+    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));
+  }
+};
+template <int KS, int RT, int HT, typename Front>
+__device__ __forceinline__ void latent_decode(const LatentDecode& a, Front& front) {
   constexpr int NP = KS / 2, kPanel = kLatentRows * 128, kStage = NP * kPanel, kWaves = 4 * HT;
   static_assert(KS % 2 == 0, "whole panels");
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -690,18 +715,9 @@ __global__ __launch_bounds__(256 * HT) void latent_decode_kernel(LatentDecode a)
   }
   const int b = unit / a.chunks, chunk = unit % a.chunks, h0 = 16 * (HT * group + ht);
   const int cw = a.width >> 3;
-  // Requested before the position is known and in one go, through a buffer descriptor of the sequence's queries: chunks past the
-  // width are addressed past its end, which reads as zeros (left out by a branch, each was waited for before the next was
-  // requested; cleared by selects, 18 of them cost a microsecond of arithmetic).
   u32x4_t qf[KS];
-  const uint32_t q_bytes = 2u * (uint32_t)(a.heads * a.width);  // (a launch's queries of one sequence stay far below 2 GiB)
-  const __amdgpu_buffer_rsrc_t q_rows =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.q) + (size_t)b * a.heads * a.width, 0, (int)q_bytes, kBufferWord3);
-  const uint32_t q_at = 2u * (uint32_t)(min(h0 + r, a.heads - 1) * a.width);
-#pragma unroll
-  for (int s = 0; s < KS; ++s)
-    qf[s] = __builtin_amdgcn_raw_buffer_load_b128(q_rows, (int)(4 * s + g < cw ? q_at + 16u * (uint32_t)(4 * s + g) : q_bytes), 0, 0);
-  const int valid = (int)min(max(*a.pos, 0ll), (long long)a.cap - 1) + 1;  // rows the ring holds
+  front.request(a, b, h0, qf);
+  const int position = (int)min(max(*a.pos, 0ll), 0x7FFFFFFEll), valid = min(position, a.cap - 1) + 1;  // (rows the ring holds)
   const int per = (((valid + a.chunks - 1) / a.chunks) + kLatentRows - 1) & ~(kLatentRows - 1);
   const int begin = chunk * per, end = min(valid, begin + per);
   float m = -INFINITY, l = 0.f;
@@ -722,11 +738,7 @@ __global__ __launch_bounds__(256 * HT) void latent_decode_kernel(LatentDecode a)
         dma16_gather(ring + (size_t)row * (uint32_t)(2 * a.width) + 16u * c, to + (uint32_t)(req * 1024));
       }
     };
-    fetch(begin);
-    // (the queries are waited for here, where the first block is on its way, and not in the loop, where the wait would be for the
-    // block ahead as well)
-#pragma unroll
-    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));
+    front.ready(a, position, begin, end, qf, [&]() __attribute__((always_inline)) { fetch(begin); });
     // keys: row 16 part + r, chunk 4 (s & 1) + g of panel s / 2
     const uint32_t k_rd[2] = {lds0 + (uint32_t)((16 * part + r) * 128 + 16 * (g ^ (r & 6 | r >> 3))),
                               lds0 + (uint32_t)((16 * part + r) * 128 + 16 * ((4 + g) ^ (r & 6 | r >> 3)))};
@@ -738,6 +750,7 @@ __global__ __launch_bounds__(256 * HT) void latent_decode_kernel(LatentDecode a)
       // this block has landed; every wave is done with the one before, whose stage the next block goes to
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
+      if constexpr (Front::kMakesRow) front.place(a, lds, (((j0 - begin) / kLatentRows) & 1) * kStage, j0, end);
       if (j0 + kLatentRows < end) fetch(j0 + kLatentRows);
       const uint32_t stage = (uint32_t)((((j0 - begin) / kLatentRows) & 1) * kStage);
       f32x4_t sc[2] = {};
@@ -823,6 +836,12 @@ __global__ __launch_bounds__(256 * HT) void latent_decode_kernel(LatentDecode a)
     const int tile = part + 4 * t;
     if (16 * tile < a.rankp) store4(out + 256 * tile, float4{u[t][0], u[t][1], u[t][2], u[t][3]});
   }
+}
+
+template <int KS, int RT, int HT>
+__global__ __launch_bounds__(256 * HT) void latent_decode_kernel(LatentDecode a) {
+  LatentQueries<KS> front;
+  latent_decode<KS, RT, HT>(a, front);
 }
 
 struct LatentExpand {

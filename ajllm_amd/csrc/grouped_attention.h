@@ -46,6 +46,13 @@ __device__ __forceinline__ void norm_rotate(const Y* __restrict__ src, const Key
   for (int i = 4 * lane; i < s.dimp; i += 4 * LPH) put(i, float4{turned(i), turned(i + 1), turned(i + 2), turned(i + 3)});
 }
 
+// four normed columns, turned against those half the rotated width away: v, w over the norm, times gains and (cos, -+ sin)
+__device__ __forceinline__ float4 turned_quad(const float4& v, const float4& w, const Divisor& by, const float4& g, const float4& h, const float4& c,
+                                              const float4& d) {
+  return float4{by.divide(v.x) * g.x * c.x + by.divide(w.x) * h.x * d.x, by.divide(v.y) * g.y * c.y + by.divide(w.y) * h.y * d.y,
+                by.divide(v.z) * g.z * c.z + by.divide(w.z) * h.z * d.z, by.divide(v.w) * g.w * c.w + by.divide(w.w) * h.w * d.w};
+}
+
 struct KeyValueSplit {
   const void* y;            // [M, ldy]: queries (heads x dimp), keys (groups x dimp), then whatever else
   int ldy;
@@ -106,9 +113,7 @@ __global__ __launch_bounds__(256) void key_value_split_kernel(KeyValueSplit a) {
       for (int off = LPH / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
       const Divisor by(sqrtf(ss / (float)s.dim + s.eps));
       const bool is_query = n < s.heads;
-      const float4 g = is_query ? gq : gk, h = is_query ? hq : hk;
-      const float4 out = float4{by.divide(v.x) * g.x * c.x + by.divide(w.x) * h.x * d.x, by.divide(v.y) * g.y * c.y + by.divide(w.y) * h.y * d.y,
-                                by.divide(v.z) * g.z * c.z + by.divide(w.z) * h.z * d.z, by.divide(v.w) * g.w * c.w + by.divide(w.w) * h.w * d.w};
+      const float4 out = turned_quad(v, w, by, is_query ? gq : gk, is_query ? hq : hk, c, d);
       if (is_query) {
         T* dst = query(n);
         for (int k = i; k < a.q_at; k += 4 * LPH) store4(dst + k, zero);
@@ -137,6 +142,134 @@ __global__ __launch_bounds__(256) void key_value_split_kernel(KeyValueSplit a) {
       }
     }
   }
+}
+
+// key_value_split_kernel's one token per sequence at the front of the decode attention: every chunk's workgroup makes its key/value
+// head's queries from the projection row (as four columns per lane, so half the rotated width is a multiple of 4), and the one whose
+// rows hold the token's slot makes the new row too, writes it to the ring and lays it over what its block brought from there.
+// The rows and gains are requested ahead of the position, waited for, then the block's requests go out and the norms, the angles
+// and the turns run beside them.  A workgroup holds the 16 heads of one key/value head at most.  Launch and latency bound: what
+// it replaces is a launch of 20 rows of arithmetic.  16 heads of 128 on 4 rings of 1028 rows, both launches -> this one: 1
+// sequence 7.0 -> 5.2 us, 4: 9.0 -> 6.6, 16: 13.9 -> 10.8, 64: 28.2 -> 25.5; 98 shapes: 0.78, the most 0.93.
+__device__ __forceinline__ void pin(float4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+struct GroupRow {
+  const float* y;           // [B, ldy]: queries (groups x share x dimp), keys (groups x dimp), ..
+  const float *q_gain, *k_gain;
+  const double* half_turns;
+  int ldy, groups, dim, rot, kept;
+  float eps;
+};
+constexpr int kGroupShare = 16;
+template <int KS>
+struct GroupFront {
+  static constexpr bool kMakesRow = true;
+  static constexpr int kDim = 16 * KS, kLanes = kDim <= 64 ? 16 : kDim <= 128 ? 32 : 64, kTeams = 256 / kLanes;  // lanes a head, heads at once
+  static constexpr int kTurns = (kGroupShare + kTeams) / kTeams, kLd = kDim + 8;
+  struct Lds {
+    float trig[2][kDim / 2];
+    __attribute__((aligned(16))) uint16_t q[kGroupShare][kLd], row[2 * kDim];
+  };
+  const GroupRow k;
+  Lds& lds;
+  float4 v[kTurns], w[kTurns], gq, hq, gk, hk;
+  double half_turn;
+  int slot, unit;
+  __device__ __forceinline__ GroupFront(const GroupRow& k, Lds& lds) : k(k), lds(lds) {}
+  __device__ __forceinline__ void request(const LatentDecode& a, int of, int, u32x4_t (&)[KS]) {
+    unit = of;
+    const int dimp = a.rankp, half = k.rot >> 1, i = 4 * (threadIdx.x % kLanes), team = threadIdx.x / kLanes;
+    const int at = min(i, dimp - 4), other = i >= k.rot ? at : i < half ? i + half : i - half;
+    const float* row = k.y + (size_t)(unit / k.groups) * k.ldy;
+    const int group = unit % k.groups;
+#pragma unroll
+    for (int t = 0; t < kTurns; ++t)
+      if (kTeams * t <= a.heads) {
+        const int n = min(team + kTeams * t, a.heads);
+        const float* src = row + (n < a.heads ? group * a.heads + n : k.groups * a.heads + group) * dimp;
+        v[t] = load4(src + at);
+        w[t] = load4(src + other);
+      }
+    gq = load4(k.q_gain + at); hq = load4(k.q_gain + other);
+    gk = load4(k.k_gain + at); hk = load4(k.k_gain + other);
+    half_turn = k.rot ? k.half_turns[min((int)threadIdx.x, half - 1)] : 0.0;
+  }
+  template <typename Fetch>
+  __device__ __forceinline__ void ready(const LatentDecode& a, int position, int begin, int end, u32x4_t (&qf)[KS], Fetch&& fetch) {
+    const int dimp = a.rankp, half = k.rot >> 1, lane = threadIdx.x % kLanes, i = 4 * lane, team = threadIdx.x / kLanes;
+    const bool mine = i < dimp, pairs = i < k.rot;
+    slot = ring_slot(position, a.cap, k.kept);
+#pragma unroll
+    for (int t = 0; t < kTurns; ++t) {
+      pin(v[t]);
+      pin(w[t]);
+    }
+    pin(gq); pin(hq); pin(gk); pin(hk);
+    asm volatile("" : "+v"(half_turn));
+    fetch();
+    if ((int)threadIdx.x < half) {  // as `angles`
+      const double x = (double)position * half_turn;
+      sincospif((float)(x - 2.0 * rint(0.5 * x)), &lds.trig[1][threadIdx.x], &lds.trig[0][threadIdx.x]);
+    }
+    __syncthreads();
+    const float4 zero = float4{0.f, 0.f, 0.f, 0.f};
+    float4 c = float4{1.f, 1.f, 1.f, 1.f}, d = zero;
+    if (pairs) {
+      const int e = i < half ? i : i - half;
+      c = load4(&lds.trig[0][e]);
+      d = load4(&lds.trig[1][e]);
+      if (i < half) d = float4{-d.x, -d.y, -d.z, -d.w};
+    }
+#pragma unroll
+    for (int t = 0; t < kTurns; ++t) {
+      const int n = team + kTeams * t;
+      if (kTeams * t > a.heads) continue;
+      const float4 own = mine ? v[t] : zero, far = pairs ? w[t] : zero;
+      float ss = (own.x * own.x + own.y * own.y) + (own.z * own.z + own.w * own.w);
+#pragma unroll
+      for (int off = kLanes / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+      const Divisor by(sqrtf(ss / (float)k.dim + k.eps));
+      const bool is_query = n < a.heads;
+      const float4 out = turned_quad(own, far, by, is_query ? gq : gk, is_query ? hq : hk, c, d);
+      if (mine && is_query) store4(&lds.q[n][i], out);
+      if (mine && n == a.heads) {
+        store4(lds.row + i, own);
+        store4(lds.row + dimp + i, out);
+      }
+    }
+    __syncthreads();
+    const int r = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4, first = dimp >> 3;  // (zeros ahead of the key's columns and past them)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int at = 4 * s + g;
+      qf[s] = u32x4_t{0u, 0u, 0u, 0u};
+      if (at >= first && at < 2 * first) qf[s] = *reinterpret_cast<const u32x4_t*>(&lds.q[min(r, a.heads - 1)][8 * (at - first)]);
+    }
+  }
+  // the new row, in the block that brought its slot: over what lay there, and into the ring
+  __device__ __forceinline__ void place(const LatentDecode& a, unsigned char* stages, int stage, int j0, int end) {
+    if (slot < j0 || slot >= min(j0 + kLatentRows, end)) return;
+    const int at = slot - j0, c = threadIdx.x;
+    auto put = [&](int row, int c, const u32x4_t& piece) {
+      *reinterpret_cast<u32x4_t*>(stages + stage + (c >> 3) * (kLatentRows * 128) + row * 128 + 16 * ((c & 7) ^ ((row & 6) | ((row >> 3) & 1)))) = piece;
+    };
+    // What lay in the slot may be no number, which a weight of zero does not silence: neither in the chunks past the width, which repeat
+    // the row's last one, nor in the values of the rows past the end, which repeat the last row.
+    if (c < 4 * KS) {
+      const bool live = c < (a.width >> 3);
+      const u32x4_t piece = live ? *reinterpret_cast<const u32x4_t*>(lds.row + 8 * c) : u32x4_t{0u, 0u, 0u, 0u};
+      put(at, c, piece);
+      if (live) *reinterpret_cast<u32x4_t*>(const_cast<uint16_t*>(a.ring) + ((size_t)unit * a.cap + slot) * a.width + 8 * c) = piece;
+    }
+    if (slot == end - 1 && (c & 63) < (a.rankp >> 3))
+      for (int row = at + 1 + (c >> 6); row < kLatentRows; row += 4) put(row, c & 63, u32x4_t{0u, 0u, 0u, 0u});
+    __syncthreads();
+  }
+};
+template <int KS>
+__global__ __launch_bounds__(256) void group_decode_kernel(LatentDecode a, GroupRow k) {
+  __shared__ typename GroupFront<KS>::Lds lds;
+  GroupFront<KS> front(k, lds);
+  latent_decode<KS, (KS + 3) / 4, 1>(a, front);
 }
 
 // Merge of latent_decode_kernel's row chunks (a sequence there is a (b, key/value head) here) and the output gate:

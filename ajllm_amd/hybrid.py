@@ -322,13 +322,19 @@ class HybridLM(DenseLM):
         _lib.check_dense(_lib.load_dense().ajqd_activation(_ptr(y), _ptr(y), y.numel(), act, _flag(y.dtype), _stream()), "activation")
         return y
 
+    @staticmethod
+    def _split_args(y: torch.Tensor, w: PackedAttention, q: torch.Tensor | None, q_at: int, rows: torch.Tensor, seq: int, start: int,
+                    pos: torch.Tensor | None, prior: int, kept: int) -> _lib.KeyValueSplitArgs:
+        return _lib.KeyValueSplitArgs(
+            y=_ptr(y), q_gain=_ptr(w.q_gain), k_gain=_ptr(w.k_gain), half_turns=_ptr(w.half_turns), pos=_ptr(pos), q=_ptr(q), rows=_ptr(rows),
+            rows_batch=rows.stride(0), rows_head=rows.stride(1), tokens=y.shape[0], seq=seq, start=start, ldy=y.shape[1], heads=w.heads,
+            groups=w.groups, dim=w.dim, dimp=w.dimp, rot=w.rot, q_ld=0 if q is None else q.shape[-1], q_at=q_at, prior=prior, cap=rows.shape[2],
+            kept=kept, eps=w.eps)
+
     def _split(self, y: torch.Tensor, w: PackedAttention, q: torch.Tensor, q_at: int, rows: torch.Tensor, seq: int, start: int,
                pos: torch.Tensor | None, prior: int, kept: int) -> None:
         """Queries into ``q [.., heads, columns]``; keys and values into ``rows [B, groups, slots, row]``."""
-        args = _lib.KeyValueSplitArgs(
-            y=_ptr(y), q_gain=_ptr(w.q_gain), k_gain=_ptr(w.k_gain), half_turns=_ptr(w.half_turns), pos=_ptr(pos), q=_ptr(q), rows=_ptr(rows),
-            rows_batch=rows.stride(0), rows_head=rows.stride(1), tokens=y.shape[0], seq=seq, start=start, ldy=y.shape[1], heads=w.heads,
-            groups=w.groups, dim=w.dim, dimp=w.dimp, rot=w.rot, q_ld=q.shape[-1], q_at=q_at, prior=prior, cap=rows.shape[2], kept=kept, eps=w.eps)
+        args = self._split_args(y, w, q, q_at, rows, seq, start, pos, prior, kept)
         _lib.check_dense(_lib.load_dense().ajqd_key_value_split(ctypes.byref(args), _flag(y.dtype), _flag(q.dtype), _stream()), "key_value_split")
 
     def _windowed(self, w: PackedAttention, q: torch.Tensor, rows: torch.Tensor, y: torch.Tensor, seq: int, prior: int,
@@ -489,12 +495,16 @@ class HybridLM(DenseLM):
         chunks = lib.ajqd_latent_decode_chunks(batch * w.groups, w.share, w.dimp, w.dimp, cap)
         if chunks == 0:   # heads wider than the kernel takes
             return self._attend_token(y.to(torch.bfloat16), w, cache, run)
-        q = torch.empty((batch, w.heads, w.row), dtype=torch.bfloat16, device=y.device)
-        self._split(y, w, q, w.dimp, ring, 1, 0, cache.position, 0, cache.kept[run])
         units = batch * w.groups
         partial = torch.empty(lib.ajqd_latent_decode_workspace(units, w.share, w.dimp, chunks), dtype=torch.uint8, device=y.device)
-        _lib.check_dense(lib.ajqd_latent_decode(_ptr(q), _ptr(ring), _ptr(cache.position), _ptr(partial), units, w.share, w.dimp, w.dimp, cap,
-                                                chunks, w.dimp, w.scale, st), "latent_decode")
+        if lib.ajqd_group_decode_built(w.share, w.dimp, w.rot):
+            args = self._split_args(y, w, None, 0, ring, 1, 0, cache.position, 0, cache.kept[run])
+            _lib.check_dense(lib.ajqd_group_decode(ctypes.byref(args), _ptr(partial), chunks, w.scale, st), "group_decode")
+        else:
+            q = torch.empty((batch, w.heads, w.row), dtype=torch.bfloat16, device=y.device)
+            self._split(y, w, q, w.dimp, ring, 1, 0, cache.position, 0, cache.kept[run])
+            _lib.check_dense(lib.ajqd_latent_decode(_ptr(q), _ptr(ring), _ptr(cache.position), _ptr(partial), units, w.share, w.dimp, w.dimp, cap,
+                                                    chunks, w.dimp, w.scale, st), "latent_decode")
         out = torch.empty((batch, w.heads * w.dimp), dtype=torch.bfloat16, device=y.device)
         _lib.check_dense(lib.ajqd_group_merge(_ptr(partial), y.data_ptr() + 4 * w.gate_column, y.shape[1], _ptr(out), out.shape[1], batch,
                                               w.groups, w.share, chunks, w.dimp, st), "group_merge")

@@ -147,26 +147,24 @@ def bench_kernels(name: str, device, log=print, batches=(1, 8, 32)) -> list[dict
         # ---- attention of one token
         rings = [bf(batch, groups, window + size["keep"], a0.row) for _ in range(max(2, min(32, int(4e8 / (2 * batch * groups * window * a0.row)))))]
         cap, units = rings[0].shape[2], batch * groups
-        q = torch.empty((batch, heads, a0.row), dtype=torch.bfloat16, device=device)
-        split = lambda r: model._split(y, a0, q, a0.dimp, r, 1, 0, pos, 0, size["keep"])
         latents = [bf(batch, near_size["window"], b0.width) for _ in range(max(2, min(32, int(4e8 / (2 * batch * near_size["window"] * b0.width)))))]
         near_q = torch.empty((batch, heads, b0.width), dtype=torch.bfloat16, device=device)
         absorb = lambda w: _lib.check_dense(lib.ajqd_latent_absorb(
             near_y.data_ptr(), near_y.shape[1], ctypes.byref(w.shape), w.ukt.data_ptr(), w.latent_gain.data_ptr(), w.cosine.data_ptr(),
             w.sine.data_ptr(), CONTEXT + 512, pos.data_ptr(), near_q.data_ptr(), latents[0].data_ptr(), near_size["window"], batch, _st()), "latent_absorb")
-        add("key_value_split: norms, rotation, cache rows", batch,
-            _hbm(batch * (4 * (heads + groups) * a0.dimp + 2 * heads * a0.row + 2 * groups * a0.row), _graph_us([lambda r=r: split(r) for r in rings])),
-            "latent_absorb", _hbm(_bytes(b0.ukt) + batch * (4 * near_y.shape[1] + 2 * heads * b0.width), _graph_us([lambda w=w: absorb(w) for w in blocks])))
         chunks = lib.ajqd_latent_decode_chunks(units, a0.share, a0.dimp, a0.dimp, cap)
         partial = torch.empty(lib.ajqd_latent_decode_workspace(units, a0.share, a0.dimp, chunks), dtype=torch.uint8, device=device)
-        attend = lambda r: _lib.check_dense(lib.ajqd_latent_decode(q.data_ptr(), r.data_ptr(), pos.data_ptr(), partial.data_ptr(), units, a0.share, a0.dimp,
-                                                                   a0.dimp, cap, chunks, a0.dimp, a0.scale, _st()), "latent_decode")
+        attend = lambda r: _lib.check_dense(lib.ajqd_group_decode(ctypes.byref(model._split_args(y, a0, None, 0, r, 1, 0, pos, 0, size["keep"])),
+                                                                  partial.data_ptr(), chunks, a0.scale, _st()), "group_decode")
         near_chunks = lib.ajqd_latent_decode_chunks(batch, heads, b0.rankp, b0.rotp, near_size["window"])
         near_partial = torch.empty(lib.ajqd_latent_decode_workspace(batch, heads, b0.rankp, near_chunks), dtype=torch.uint8, device=device)
         near_attend = lambda r: _lib.check_dense(lib.ajqd_latent_decode(near_q.data_ptr(), r.data_ptr(), pos.data_ptr(), near_partial.data_ptr(), batch, heads,
                                                                         b0.rankp, b0.rotp, near_size["window"], near_chunks, 0, b0.scale, _st()), "latent_decode")
-        add(f"latent_decode on (value | key) rows, {cap} per head", batch, _hbm(_bytes(rings[0]), _graph_us([lambda r=r: attend(r) for r in rings])),
-            f"latent_decode on {near_size['window']} latents", _hbm(_bytes(latents[0]), _graph_us([lambda r=r: near_attend(r) for r in latents])))
+        add(f"group_decode: norms, rotation, new row, attention over {cap} (value | key) rows per head", batch,
+            _hbm(_bytes(rings[0]) + 4 * batch * (heads + groups) * a0.dimp, _graph_us([lambda r=r: attend(r) for r in rings])),
+            f"latent_absorb and latent_decode on {near_size['window']} latents",
+            _hbm(_bytes(b0.ukt, latents[0]) + batch * (4 * near_y.shape[1] + 2 * heads * b0.width),
+                 _graph_us([lambda w=w: absorb(w) for w in blocks]) + _graph_us([lambda r=r: near_attend(r) for r in latents])))
         merge = lambda: _lib.check_dense(lib.ajqd_group_merge(partial.data_ptr(), y.data_ptr() + 4 * a0.gate_column, y.shape[1], joined.data_ptr(),
                                                               joined.shape[1], batch, groups, a0.share, chunks, a0.dimp, _st()), "group_merge")
         expand = lambda w: _lib.check_dense(lib.ajqd_latent_expand(near_partial.data_ptr(), w.sink.data_ptr(), near_y.data_ptr() + 4 * b0.gate_column,

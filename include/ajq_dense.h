@@ -198,6 +198,11 @@ typedef struct {
  * makes a row (key as projected | normed and rotated key) of 2 dimp elements at rows[b * rows_batch + group * rows_head + slot *
  * 2 dimp].  slot = prior + t at position start + t, or (pos) the position's slot in a ring of cap rows, `kept` of which stay. */
 int ajqd_key_value_split(const ajqd_key_value_split_args* args, int y_dtype, int dtype, void* stream);
+/* ajqd_key_value_split of one token per sequence (q, q_ld and q_at are not used; rows is a whole ring [tokens, groups, cap, 2 dimp], y fp32)
+ * and ajqd_latent_decode of its queries, share = heads / groups heads a (sequence, key / value head), in one launch.  Built where
+ * ajqd_group_decode_built says so; chunks and workspace as ajqd_latent_decode's. */
+int ajqd_group_decode_built(int share, int dimp, int rot);
+int ajqd_group_decode(const ajqd_key_value_split_args* args, float* partial, int chunks, float scale, void* stream);
 /* merge of ajqd_latent_decode's chunks where a (sequence, key / value head) was a sequence of `share` heads and dimp the
  * latent's width; output gate sigmoid(gate[b * gate_ld + head * dimp + c]) (or NULL) -> out bf16 [batch, out_ld] */
 int ajqd_group_merge(const float* partial, const float* gate, int gate_ld, void* out, int out_ld, int batch, int groups, int share,

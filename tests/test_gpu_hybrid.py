@@ -310,6 +310,47 @@ def test_decode_attention_and_merge(cuda, shape):
             assert (out[:, heads * d:] == 5.0).all()
 
 
+@pytest.mark.parametrize("shape", [  # batch, groups, share, dim, rot, rows of the ring, rows that stay
+    (1, 1, 1, 16, 16, 45, 0), (2, 3, 4, 64, 16, 64, 4), (1, 2, 16, 72, 0, 65, 3), (3, 1, 7, 96, 96, 130, 129), (2, 2, 8, 120, 40, 128, 4), (1, 2, 4, 128, 32, 1028, 4),
+    (1, 1, 9, 136, 8, 70, 1), (2, 1, 16, 160, 152, 200, 0),
+])
+def test_decode_attention_that_makes_its_row(cuda, shape):
+    """group_decode against key_value_split and latent_decode: the same queries, row, arithmetic and order, so the same bits; slots in the
+    first, an inner and the last block, kept ones, and around the ring; rows that were never written, the slot's own among them."""
+    batch, groups, share, dim, rot, cap, kept = shape
+    lib, g, dimp, heads, units = _lib.load_dense(), torch.Generator().manual_seed(sum(shape)), _up(dim, 16), groups * share, batch * groups
+    assert lib.ajqd_group_decode_built(share, dimp, rot) and not lib.ajqd_group_decode_built(17, dimp, rot) and not lib.ajqd_group_decode_built(share, 176, rot)
+    assert not lib.ajqd_group_decode_built(share, dimp, rot + 2)
+    ld = (heads + groups) * dimp + 8
+    y = torch.randn((batch, ld), generator=g)
+    y[:, : (heads + groups) * dimp].view(batch, heads + groups, dimp)[:, :, dim:] = 0
+    y, qg, kg = y.to(cuda), _padded(torch.randn(dim, generator=g), dimp).to(cuda), _padded(torch.randn(dim, generator=g), dimp).to(cuda)
+    turns = (dense.rotary_frequencies(700.0, rot, None) / math.pi).to(cuda) if rot else torch.zeros(1, dtype=torch.float64, device=cuda)
+    for position in sorted({0, 1, kept, 63 % cap, 64 % cap, cap - 1, cap, cap + (cap - kept) // 2, 5 * cap + 3}):
+        ring = _bf(g, batch, groups, cap, 2 * dimp)
+        ring[:, :, min(position, cap):] = float("nan")
+        ring, pos = ring.to(cuda), torch.tensor([position], device=cuda)
+        q = torch.zeros((batch, heads, 2 * dimp), dtype=torch.bfloat16, device=cuda)
+        for chunks in sorted({1, 3, lib.ajqd_latent_decode_chunks(units, share, dimp, dimp, cap)}):
+            got = []
+            for whole in (False, True):
+                rows = ring.clone()
+                args = _lib.KeyValueSplitArgs(
+                    y=_p(y), q_gain=_p(qg), k_gain=_p(kg), half_turns=_p(turns), pos=_p(pos), q=None if whole else _p(q), rows=_p(rows),
+                    rows_batch=rows.stride(0), rows_head=rows.stride(1), tokens=batch, seq=1, start=0, ldy=ld, heads=heads, groups=groups, dim=dim,
+                    dimp=dimp, rot=rot, q_ld=0 if whole else 2 * dimp, q_at=0 if whole else dimp, prior=0, cap=cap, kept=kept, eps=1e-4)
+                partial = torch.zeros(lib.ajqd_latent_decode_workspace(units, share, dimp, chunks), dtype=torch.uint8, device=cuda)
+                if whole:
+                    _ok(lib.ajqd_group_decode(ctypes.byref(args), _p(partial), chunks, dim ** -0.5, _st()))
+                else:
+                    _ok(lib.ajqd_key_value_split(ctypes.byref(args), dense._flag(y.dtype), dense._flag(q.dtype), _st()))
+                    _ok(lib.ajqd_latent_decode(_p(q), _p(rows), _p(pos), _p(partial), units, share, dimp, dimp, cap, chunks, dimp, dim ** -0.5, _st()))
+                out = torch.empty((batch, heads * dimp), dtype=torch.bfloat16, device=cuda)
+                _ok(lib.ajqd_group_merge(_p(partial), None, 0, _p(out), heads * dimp, batch, groups, share, chunks, dimp, _st()))
+                got.append((rows.view(torch.int16), out))
+            assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and not got[1][1].isnan().any(), (position, chunks)
+
+
 def test_ring_copy_keeps_the_first_rows(cuda):
     lib, kept, cap = _lib.load_dense(), 3, 8
     line = torch.arange(20 * 4, dtype=torch.float32, device=cuda).view(1, 20, 4)

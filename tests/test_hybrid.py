@@ -289,3 +289,21 @@ def test_dense_library_refuses_bad_arguments_before_any_launch():
     step = _lib.ScanStepArgs(y=p, ring=p, weight=p, bias=p, pos=p, partial=p, w_dt=p, dt_bias=p, a2=p, d=p, state=p, out=p, batch=1, ldy=32, inner=16,
                              taps=4, rows=16, splits=1, rank=8, states=8, out_ld=16)
     assert lib.ajqd_scan_step(ctypes.byref(step), None) == -2                                            # 8 + 16 rows in 16
+
+
+def test_decode_attention_that_makes_its_row_refuses_bad_arguments():
+    lib = _lib.load_dense()
+    buf = ctypes.create_string_buffer(4096)
+    p = ctypes.c_void_p((ctypes.addressof(buf) + 15) & ~15)
+    args = _lib.KeyValueSplitArgs(y=p, q_gain=p, k_gain=p, half_turns=p, pos=p, rows=p, tokens=1, seq=1, ldy=64, heads=2, groups=2, dim=16, dimp=16, rot=8,
+                                  cap=4, kept=0, rows_head=128, rows_batch=256)
+    run = lambda chunks=1: lib.ajqd_group_decode(ctypes.byref(args), p, chunks, 1.0, None)
+    assert run(0) == -2 and run(33) == -2
+    for name, value, code in (("pos", None, -1), ("half_turns", None, -1), ("seq", 2, -2), ("heads", 3, -2), ("kept", 4, -2), ("rows_head", 160, -2), ("prior", 1, -2),
+                              ("rows_batch", 288, -2), ("ldy", 60, -2), ("rot", 6, -4), ("rot", 18, -2)):
+        before = getattr(args, name)
+        setattr(args, name, value)
+        assert run() == code, name
+        setattr(args, name, before)
+    args.y = ctypes.c_void_p(p.value + 4)
+    assert run() == -3
