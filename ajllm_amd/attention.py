@@ -8,9 +8,14 @@ online softmax), not bit-for-bit the eager fp32 one, so it is opt-in.
 
 from __future__ import annotations
 
+from contextlib import nullcontext
+
 import torch
 
 from . import _lib
+
+_HERE = nullcontext()
+COPIED_WORK = 3.6e9   # half the FLOP below which ajq_attn_prefill_workspace says 0: short calls are not asked
 
 
 def flash_prefill(q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, start: int,
@@ -35,10 +40,27 @@ def flash_prefill(q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, sta
     q = q.float().contiguous()
     out = torch.empty((batch, seq, heads * hd), dtype=out_dtype, device=q.device)
     flag = _lib.AJQ_KV_F32 if keys.dtype == torch.float32 else _lib.AJQ_KV_BF16
-    with torch.cuda.device(q.device):
-        status = _lib.load().ajq_attn_prefill(q.data_ptr(), keys.data_ptr(), values.data_ptr(), flag, batch, heads,
-                                              kv_heads, seq, start, max_len, hd, out.data_ptr(),
-                                              _lib.AJQ_OUT_F32 if out_dtype == torch.float32 else _lib.AJQ_OUT_BF16,
-                                              torch.cuda.current_stream().cuda_stream)
+    # (entering and leaving a device that is the current one anyway: 1.1 of 12.2 us, what a small call takes)
+    with _HERE if q.get_device() == torch.cuda.current_device() else torch.cuda.device(q.device):
+        status = prefill_attention(q, keys, values, flag, batch, heads, kv_heads, seq, start, max_len, hd, out,
+                                   _lib.AJQ_OUT_F32 if out_dtype == torch.float32 else _lib.AJQ_OUT_BF16,
+                                   torch.cuda.current_stream().cuda_stream)
     _lib.check(status, "attn_prefill")
     return out
+
+
+def prefill_attention(q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, flag: int, batch: int, heads: int, kv_heads: int, seq: int,
+                      start: int, max_len: int, hd: int, out: torch.Tensor, out_flag: int, stream: int) -> int:
+    """``ajq_attn_prefill`` on the current device, with a bf16 copy of fp32 caches where that is faster; its status."""
+    lib = _lib.load()
+    if flag == _lib.AJQ_KV_F32 and batch * heads * seq * (2 * start + seq) * hd > COPIED_WORK:
+        size = lib.ajq_attn_prefill_workspace(flag, batch, heads, kv_heads, seq, start, hd)
+        try:
+            room = torch.empty(size, dtype=torch.uint8, device=q.device) if size else None
+        except torch.OutOfMemoryError:  # (the kernel that needs no copy)
+            room = None
+        if room is not None:
+            return lib.ajq_attn_prefill_in(q.data_ptr(), keys.data_ptr(), values.data_ptr(), flag, batch, heads, kv_heads, seq, start, max_len,
+                                           hd, out.data_ptr(), out_flag, room.data_ptr(), size, stream)
+    return lib.ajq_attn_prefill(q.data_ptr(), keys.data_ptr(), values.data_ptr(), flag, batch, heads, kv_heads, seq, start, max_len, hd,
+                                out.data_ptr(), out_flag, stream)

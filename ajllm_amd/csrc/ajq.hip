@@ -1654,6 +1654,7 @@ auto pick_attn(int R, int cache_dtype, int head_dim) {
   return head_dim == 32 ? pick_attn_hd<kStep, 32>(R, cache_dtype)
                         : head_dim == 64 ? pick_attn_hd<kStep, 64>(R, cache_dtype) : pick_attn_hd<kStep, 128>(R, cache_dtype);
 }
+constexpr double kCopiedBytes = 512e6;  // prefill attention: the most bytes a bf16 copy of fp32 caches takes
 }  // namespace
 
 extern "C" {
@@ -1853,8 +1854,24 @@ int ajq_sample_pick(const float* logits, int B, int V, int ld, float temperature
   return check_launch("ajq_sample_pick");
 }
 
+// fp32 caches: a bf16 copy of the rows pays where attention on it saves more than the copy takes.  The kernel on the copy saves a third (heads
+// of 128; a fifth with 64, nothing with 32) of a time of 4 FLOP a score and column at 520 TFLOP/s; the copy is a launch and 12 bytes an
+// element at 6.7 TB/s.  Heads of 128: 4 x 32 / 8 x 2048 positions 212 -> 169 us, 1 x 32 / 8 x 4096 197 -> 147; not made for 1 x 16 / 16 x 2048 (62).
+size_t ajq_attn_prefill_workspace(int cache_dtype, int B, int H, int Hkv, int T, int start, int head_dim) {
+  if (cache_dtype != AJQ_KV_F32 || B < 1 || H < 1 || Hkv < 1 || T < 1 || start < 0 || head_dim < 64) return 0;
+  const double elements = (double)B * Hkv * ((double)start + T) * head_dim, bytes = 4 * elements;
+  const double flops = 4.0 * B * H * head_dim * (double)T * (start + 0.5 * T);
+  if (bytes > kCopiedBytes || (head_dim < 128 ? 0.2 : 0.33) * flops / 5.2e14 < 1.15 * (4e-6 + 12 * elements / 6.7e12)) return 0;
+  return (size_t)bytes;
+}
+
 int ajq_attn_prefill(const float* q, const void* kcache, const void* vcache, int cache_dtype, int B, int H, int Hkv,
                      int T, int start, int max_len, int head_dim, void* out, int out_dtype, void* stream) {
+  return ajq_attn_prefill_in(q, kcache, vcache, cache_dtype, B, H, Hkv, T, start, max_len, head_dim, out, out_dtype, nullptr, 0, stream);
+}
+
+int ajq_attn_prefill_in(const float* q, const void* kcache, const void* vcache, int cache_dtype, int B, int H, int Hkv, int T, int start,
+                        int max_len, int head_dim, void* out, int out_dtype, void* workspace, size_t workspace_bytes, void* stream) {
   if (!q || !kcache || !vcache || !out) return fail(AJQ_ERR_NULL, "ajq_attn_prefill: null pointer argument");
   if (head_dim != 128 && head_dim != 64 && head_dim != 32)
     return fail(AJQ_ERR_UNSUPPORTED, "ajq_attn_prefill: head_dim %d (128, 64 and 32 are built)", head_dim);
@@ -1869,6 +1886,19 @@ int ajq_attn_prefill(const float* q, const void* kcache, const void* vcache, int
   const int out_bf16 = out_dtype == AJQ_OUT_BF16;
   if (!aligned16(q) || !aligned16(kcache) || !aligned16(vcache) || !aligned16(out))
     return fail(AJQ_ERR_ALIGN, "ajq_attn_prefill: q, the caches and out must be 16-byte aligned");
+  const size_t need = workspace ? ajq_attn_prefill_workspace(cache_dtype, B, H, Hkv, T, start, head_dim) : 0;
+  if (need > 0 && workspace_bytes >= need) {
+    if (!aligned16(workspace)) return fail(AJQ_ERR_ALIGN, "ajq_attn_prefill: the workspace must be 16-byte aligned");
+    const long long rows8 = (long long)(start + T) * (head_dim / 8), groups8 = rows8 * B * Hkv;
+    uint16_t *keys = static_cast<uint16_t*>(workspace), *values = keys + 8 * groups8;
+    hipLaunchKernelGGL(caches_to_bf16_kernel, dim3((unsigned)((groups8 + 255) / 256), 2), dim3(256), 0, (hipStream_t)stream,
+                       static_cast<const float*>(kcache), static_cast<const float*>(vcache), keys, values, rows8, (long long)max_len * head_dim, groups8);
+    if (int e = check_launch("ajq_attn_prefill")) return e;
+    kcache = keys;
+    vcache = values;
+    cache_dtype = AJQ_KV_BF16;
+    max_len = start + T;
+  }
   const dim3 grid((unsigned)(((T + kPfBQ - 1) / kPfBQ) * B * H));  // (the kernel orders the work by cost)
   auto launch = [&](auto dim) {
     constexpr int HD = decltype(dim)::value;

@@ -35,7 +35,8 @@
 // fp32 accumulators: the usual flash-attention arithmetic, not the eager fp32 one.
 //
 // Two kernels: bf16 caches (attn_prefill_steps_kernel) interleave both products and the softmax of three neighbouring half blocks;
-// fp32 caches pass through registers that are converted on the way, which leaves none for that (attn_prefill_kernel).
+// fp32 caches pass through registers that are converted on the way, which leaves none for that (attn_prefill_kernel), unless
+// there is work enough to make a bf16 copy of the rows first (caches_to_bf16_kernel).
 #pragma once
 #include <type_traits>
 
@@ -327,6 +328,16 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
             float4{o[u][t][0] * inv, o[u][t][1] * inv, o[u][t][2] * inv, o[u][t][3] * inv};
     }
   }
+}
+
+// The first `rows8` groups of eight elements of every (b, hk) of both fp32 caches (pitch `stride` elements), rounded to bf16 as the kernel
+// above does it and packed.  A thread eight elements, the caches in blockIdx.y; bounded by HBM (4 x 8 heads x 2048 rows of 128: 101 MB).
+__global__ __launch_bounds__(256) void caches_to_bf16_kernel(const float* __restrict__ k, const float* __restrict__ v, uint16_t* __restrict__ kb,
+                                                             uint16_t* __restrict__ vb, long long rows8, long long stride, long long groups8) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= groups8) return;
+  const float* from = (blockIdx.y ? v : k) + i / rows8 * stride + i % rows8 * 8;
+  *reinterpret_cast<u32x4_t*>((blockIdx.y ? vb : kb) + 8 * i) = to_bf16x8(load8_raw(from));
 }
 
 // bf16 caches.  The keys are walked in steps of 32.  Step t holds three things that need nothing of each other: the exponents of step t + 1, the

@@ -15,6 +15,7 @@ import ctypes
 import torch
 
 from . import _lib, dense, modeling
+from .attention import prefill_attention
 from .quant import QuantLinear, repack_w4, repack_w8, w4a16_matmul, w8a16_matmul
 
 
@@ -559,9 +560,8 @@ class FusedDecoder(GraphDecoder):
                                             self.kv_heads, self.head_dim, 0, self.max_len, st), "rope_prefill")
             del qkv
             attended = torch.empty((m, d), dtype=torch.bfloat16, device=self.device)
-            _lib.check(lib.ajq_attn_prefill(q_rot.data_ptr(), keys.data_ptr(), values.data_ptr(), self.kv_flag, rows,
-                                            self.heads, self.kv_heads, seq, 0, self.max_len, self.head_dim, attended.data_ptr(),
-                                            _lib.AJQ_OUT_BF16, st), "attn_prefill")
+            _lib.check(prefill_attention(q_rot, keys, values, self.kv_flag, rows, self.heads, self.kv_heads, seq, 0, self.max_len, self.head_dim,
+                                         attended, _lib.AJQ_OUT_BF16, st), "attn_prefill")
             delta = w["o"](attended)
             del attended
             _lib.check(lib.ajq_add_rmsnorm(hidden.data_ptr(), delta.data_ptr(), w["g2"].data_ptr(), w["eps2"],

@@ -7,7 +7,7 @@ import copy
 import pytest
 import torch
 
-from ajllm_amd import QuantLinear, decoding, modeling, quantize_model_
+from ajllm_amd import QuantLinear, _lib, decoding, modeling, quantize_model_
 from oracle import qspec
 from tests.helpers import MAX_ABS_TOL, REL_FRO_TOL, compare_greedy, errors, make_activations, make_weight
 
@@ -650,6 +650,33 @@ def test_flash_prefill_on_bf16_caches_at_the_edges_of_its_steps(cuda, t, start, 
     scaled = (q * (1.4426950408889634 * hd ** -0.5)).bfloat16().float() / (1.4426950408889634 * hd ** -0.5)   # (as the kernel rounds them)
     want = modeling.scaled_dot_product_attention(scaled, k32, v32, mask).transpose(1, 2).reshape(2, t, heads * hd)
     assert errors(got, want.cpu())[1] <= 4e-3
+
+
+@pytest.mark.parametrize("hd", [128, 64])
+@pytest.mark.parametrize("b,heads,kv_heads,t,start", [(16, 64, 1, 128, 901), (2, 32, 2, 2047, 0), (1, 64, 4, 1500, 1), (3, 96, 3, 513, 700)])
+def test_flash_prefill_on_a_copy_of_fp32_caches(cuda, b, heads, kv_heads, t, start, hd):
+    """fp32 caches of much work against the same rows as a bf16 cache, which the copy is bit for bit, and against no copy; rows past
+    the fill are NaN."""
+    from ajllm_amd.attention import flash_prefill
+    lib, g, total = _lib.load(), torch.Generator().manual_seed(t + hd), start + t
+    size = lib.ajq_attn_prefill_workspace(_lib.AJQ_KV_F32, b, heads, kv_heads, t, start, hd)
+    assert size == 4 * b * kv_heads * total * hd and lib.ajq_attn_prefill_workspace(_lib.AJQ_KV_BF16, b, heads, kv_heads, t, start, hd) == 0
+    assert lib.ajq_attn_prefill_workspace(_lib.AJQ_KV_F32, b, heads, kv_heads, t, start, 32) == 0
+    assert lib.ajq_attn_prefill_workspace(_lib.AJQ_KV_F32, 1, heads, heads, 256, 0, hd) == 0
+    q = torch.randn((b, heads, t, hd), generator=g).to(cuda)
+    keys, values = (torch.randn((b, kv_heads, total + 3, hd), generator=g) for _ in range(2))
+    keys[:, :, total:] = values[:, :, total:] = float("nan")
+    keys, values = keys.to(cuda), values.to(cuda)
+    got = flash_prefill(q, keys, values, start)
+    assert torch.equal(got, flash_prefill(q, keys.bfloat16(), values.bfloat16(), start))
+    plain, room = torch.empty_like(got), torch.empty(size, dtype=torch.uint8, device=cuda)
+    for bytes_, near in ((size - 1, 0.0), (size, 4e-3)):   # too small a workspace is none
+        out = torch.empty_like(got)
+        _lib.check(lib.ajq_attn_prefill(q.data_ptr(), keys.data_ptr(), values.data_ptr(), _lib.AJQ_KV_F32, b, heads, kv_heads, t, start, total + 3, hd,
+                                        plain.data_ptr(), _lib.AJQ_OUT_F32, torch.cuda.current_stream().cuda_stream), "attn_prefill")
+        _lib.check(lib.ajq_attn_prefill_in(q.data_ptr(), keys.data_ptr(), values.data_ptr(), _lib.AJQ_KV_F32, b, heads, kv_heads, t, start, total + 3, hd,
+                                           out.data_ptr(), _lib.AJQ_OUT_F32, room.data_ptr(), bytes_, torch.cuda.current_stream().cuda_stream), "attn_prefill")
+        assert errors(out, plain.cpu())[1] <= near
 
 
 def test_model_with_flash_attention_flag(cuda):
