@@ -951,9 +951,9 @@ int ajqd_scan_in_parts(const ajqd_scan_args* a, int parts, float* workspace, int
 // Parts of the projection: what smaller blocks save in scan_project_kernel, the step's kernel pays in parts (0.04 us a part at
 // 4 sequences, 0.15 at 16 of 8192 channels, 0.13 at 64 of 4096).  Both launches with blocks of 1024 / 512 / 256: 4 sequences
 // of 4096 channels 9.6 / 8.5 / 8.3 us, 16: 15.2 / 12.2 / 11.2, 64: 22.5 / 20.1 / 21.0; 5120, 12: 14.1 / 12.0 / 11.6; 8192, 1: 10.6 / 10.9 / 11.5,
-// 8: 14.3 / 14.3 / 15.7, 16: 19.1 / 18.2 / 19.5, 64: 40.0 / 42.6 / 48.6.
+// 8: 14.3 / 14.3 / 15.7, 16: 19.1 / 18.2 / 19.5, 24: 22.4 / 21.9 / 24.5, 32: 24.5 / 24.8 (512), 64: 40.0 / 42.6 / 48.6.
 int ajqd_scan_splits(int batch, int inner) {
-  const int block = inner <= 5120 ? scan_block(batch <= 32 ? 2 : 4) : scan_block(batch > 8 && batch <= 32 ? 4 : 8);
+  const int block = inner <= 5120 ? scan_block(batch <= 32 ? 2 : 4) : scan_block(batch > 8 && batch <= 24 ? 4 : 8);
   const int s = (inner + block - 1) / block;
   return s < 1 ? 1 : s > 20 ? 20 : s;
 }
@@ -964,10 +964,10 @@ int ajqd_scan_project(const float* y, int ldy, const void* ring, const float* we
   if (batch < 1 || inner < 8 || inner % 8 || taps < 1 || rows < 16 || rows % 16 || splits < 1 || splits > 65535 || ldy < 2 * inner || ldy % 4)
     return fail(AJQ_ERR_SHAPE, "ajqd_scan_project: unsupported shape (batch=%d inner=%d taps=%d rows=%d splits=%d)", batch, inner, taps, rows, splits);
   ScanProject p{y, (const uint16_t*)ring, weight, bias, positions64(pos), (const uint16_t*)w, partial, batch, ldy, inner, taps, rows, splits};
-  // the smallest block that holds a part; two row tiles where single ones are more than the CUs take at once (a block of 1024: two each)
+  // the smallest block that holds a part; two row tiles, which share the convolution, where single ones are more than one a CU
   const int part = 32 * (((inner + 31) / 32 + splits - 1) / splits), kb = part <= scan_block(2) ? 2 : part <= scan_block(4) ? 4 : 8;
   const long long tiles = (long long)(rows / 16) * splits * ((batch + kGemvBatch - 1) / kGemvBatch);
-  const int rt = tiles > (kb == 8 ? 512 : 256) && rows >= 32 ? 2 : 1;
+  const int rt = tiles > 256 && rows >= 32 ? 2 : 1;
   const dim3 grid((rows / 16 + rt - 1) / rt, splits, (batch + kGemvBatch - 1) / kGemvBatch);
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, p); };
   auto with = [&](auto steps) {
@@ -997,9 +997,9 @@ int ajqd_scan_step(const ajqd_scan_step_args* a, void* stream) {
   };
   if (a->rank <= kNarrowRank && (long long)(a->inner / 16) * ((a->batch + kNarrowBatch - 1) / kNarrowBatch) <= 256)  // (a workgroup per CU)
     return go(scan_step_narrow_kernel, 16, kNarrowBatch);
-  // eight sequences a workgroup read the weights and decays less often, four fill the chip: 24 of 8192 channels 12.7 (four) / 13.8, 32 of 4096 9.3 /
-  // 11.0, 64 of either 33.3 / 30.4 and 16.1 / 15.3 us
-  return a->batch > 32 ? go(scan_step_kernel<8>, 64, 8) : go(scan_step_kernel<4>, 64, 4);
+  // four sequences a workgroup fill the chip, eight read the weights and decays less often: four while every workgroup finds room at once,
+  // three to a CU (four / eight: 24 of 8192 channels 12.7 / 13.8 us, 32 of 4096 9.3 / 11.0; 32 of 8192 19.2 / 16.7, 64 of 4096 16.1 / 15.3)
+  return (long long)((a->inner + 63) / 64) * ((a->batch + 3) / 4) > 3 * 256 ? go(scan_step_kernel<8>, 64, 8) : go(scan_step_kernel<4>, 64, 4);
 }
 
 }  // extern "C"
