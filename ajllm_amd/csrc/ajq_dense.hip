@@ -953,9 +953,9 @@ int ajqd_scan_in_parts(const ajqd_scan_args* a, int parts, float* workspace, int
 // of 4096 channels 9.6 / 8.5 / 8.3 us, 16: 15.2 / 12.2 / 11.2, 64: 22.5 / 20.1 / 21.0; 5120, 12: 14.1 / 12.0 / 11.6; 8192, 1: 10.6 / 10.9 / 11.5,
 // 8: 14.3 / 14.3 / 15.7, 16: 19.1 / 18.2 / 19.5, 24: 22.4 / 21.9 / 24.5, 32: 24.5 / 24.8 (512), 64: 40.0 / 42.6 / 48.6.
 int ajqd_scan_splits(int batch, int inner) {
-  const int block = inner <= 5120 ? scan_block(batch <= 32 ? 2 : 4) : scan_block(batch > 8 && batch <= 24 ? 4 : 8);
-  const int s = (inner + block - 1) / block;
-  return s < 1 ? 1 : s > 20 ? 20 : s;
+  const int block = inner <= 5120 ? scan_block(batch <= 32 ? 2 : 4) : scan_block(batch > 8 && batch <= 24 && inner <= 10240 ? 4 : 8);
+  const int s = (inner + block - 1) / block, most = inner <= 10240 ? 20 : 8;  // (not timed past 10240 channels: as it was)
+  return s < 1 ? 1 : s > most ? most : s;
 }
 
 int ajqd_scan_project(const float* y, int ldy, const void* ring, const float* weight, const float* bias, const int64_t* pos, const void* w,
