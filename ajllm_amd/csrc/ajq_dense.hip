@@ -199,44 +199,53 @@ constexpr int kLongRow = 8192;
 // that, rows that are not staged have two blocks in flight instead (4096 x 18440: 44.2 -> 42.6) where K gives each wave several (5120 x 256,
 // 64 sequences: 9.1 us with two, 5.1 with one).  Up to 16, long staged rows: two blocks at a time (4096 x 16384: 26.6 -> 24.4).  K of one or two
 // blocks: two waves (32000 x 128, one sequence: 5.2 us on four, 4.4 on two).
+// More than four streams leave a wave of 16-row tiles and two batch tiles no registers for more than the plainest form: rows from memory, one row
+// tile, one block at a time takes 240, every other form 280 and more, and then a CU holds one workgroup instead of two (12 streams of 2064
+// columns, 33 sequences, K = 1152: 17.0 us, 34.1 with staged rows; 16 of 2560, 48 sequences, K = 2048: 28.7, 39.5).  Rows of 8192 columns make up
+// for that (8 of 4096, 64 sequences: 44.4 us staged, 50.4 from memory) but where the last batch block is nearly empty (5 of 2560, 33: 34.5, 33.6).
 struct OutCut {
-  int rows, rt, bt;
+  int rows, rt, bt, uq, xq;  // row tile, row tiles, batch tiles, blocks at a time, batch rows' instructions
   dim3 grid;
   int threads;
 };
-OutCut out_cut(int batch, int width, int k, bool sums) {
+OutCut out_cut(int batch, int width, int k, bool sums, int streams) {
   OutCut c;
   c.bt = batch > kGemvBatch ? 2 : 1;
   const int blocks = (batch + kGemvBatch * c.bt - 1) / (kGemvBatch * c.bt);
-  c.rows = (long long)(width / 16) * blocks <= 128 && (sums || k >= 1024) ? 8 : 16;
-  const bool few = c.rows == 16 && c.bt == 1 && k <= kTwoWaveColumns;
-  c.rt = c.bt == 2 && width % 32 == 0 && (staged_rows(batch, k) ? c.rows == 16 && (long long)(width / 16) * blocks > kCus : width >= 8192) ? 2 : 1;
+  const long long tiles = (long long)(width / 16) * blocks;
+  c.rows = tiles <= 128 && (sums || k >= 1024) ? 8 : 16;
+  const bool few = c.rows == 16 && c.bt == 1 && k <= kTwoWaveColumns, plain = c.rows == 16 && c.bt == 2 && streams > 4;
+  const bool staged = staged_rows(batch, k) && (!plain || k >= kLongRow);
+  c.xq = few || !staged ? kStreamDirect : batch <= 4 ? 1 : batch <= 8 ? 2 : 4;
+  c.rt = c.bt == 2 && width % 32 == 0 && (staged ? c.rows == 16 && tiles > kCus : !plain && width >= 8192) ? 2 : 1;
+  c.uq = c.rows == 8 || c.rt == 2 || few ? 1 : c.bt == 1 ? (staged && k >= kLongRow ? 2 : 1) : !staged && !plain && k >= 2048 ? 2 : 1;
   c.grid = dim3(width / (c.rows * c.rt), blocks);
   c.threads = c.rows == 8 ? 512 : few ? 128 : 256;
   return c;
 }
 template <int N> using Int = std::integral_constant<int, N>;
-// go(waves, row tile, row tiles, batch tiles, blocks at a time, batch rows' instructions) of a cut
-template <typename Go>
-int with_out_cut(const OutCut& c, int batch, int k, Go&& go) {
+// go(waves, row tile, row tiles, batch tiles, blocks at a time, batch rows' instructions) of a cut; kMany: more than four streams
+template <bool kMany, typename Go>
+int with_out_cut(const OutCut& c, Go&& go) {
   if (c.threads == 128) return go(Int<2>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<1>{}, Int<kStreamDirect>{});
-  const bool staged = staged_rows(batch, k);
   if (c.bt == 2) {
-    auto two_batch_tiles = [&](auto xq) {
-      if (c.rows == 8) return go(Int<8>{}, Int<8>{}, Int<1>{}, Int<2>{}, Int<1>{}, xq);
-      return c.rt == 2 ? go(Int<4>{}, Int<16>{}, Int<2>{}, Int<2>{}, Int<1>{}, xq) : go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<1>{}, xq);
-    };
-    if (staged) return two_batch_tiles(Int<4>{});
-    if (c.rows == 16 && c.rt == 1 && k >= 2048) return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<2>{}, Int<kStreamDirect>{});
-    return two_batch_tiles(Int<kStreamDirect>{});
+    if (c.rows == 8) return c.xq == 4 ? go(Int<8>{}, Int<8>{}, Int<1>{}, Int<2>{}, Int<1>{}, Int<4>{})
+                                      : go(Int<8>{}, Int<8>{}, Int<1>{}, Int<2>{}, Int<1>{}, Int<kStreamDirect>{});
+    if (c.xq == 4) return c.rt == 2 ? go(Int<4>{}, Int<16>{}, Int<2>{}, Int<2>{}, Int<1>{}, Int<4>{}) : go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<1>{}, Int<4>{});
+    if constexpr (!kMany) {
+      if (c.uq == 2) return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<2>{}, Int<kStreamDirect>{});
+      if (c.rt == 2) return go(Int<4>{}, Int<16>{}, Int<2>{}, Int<2>{}, Int<1>{}, Int<kStreamDirect>{});
+    }
+    return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<1>{}, Int<kStreamDirect>{});
   }
-  if (!staged) return c.rows == 8 ? go(Int<8>{}, Int<8>{}, Int<1>{}, Int<1>{}, Int<1>{}, Int<kStreamDirect>{})
-                                  : go(Int<4>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<1>{}, Int<kStreamDirect>{});
-  auto by_batch = [&](auto xq) {
+  auto with = [&](auto xq) {
     if (c.rows == 8) return go(Int<8>{}, Int<8>{}, Int<1>{}, Int<1>{}, Int<1>{}, xq);
-    return k >= kLongRow ? go(Int<4>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<2>{}, xq) : go(Int<4>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<1>{}, xq);
+    if constexpr (xq() != kStreamDirect) {
+      if (c.uq == 2) return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<2>{}, xq);
+    }
+    return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<1>{}, xq);
   };
-  return batch <= 4 ? by_batch(Int<1>{}) : batch <= 8 ? by_batch(Int<2>{}) : by_batch(Int<4>{});
+  return c.xq == 1 ? with(Int<1>{}) : c.xq == 2 ? with(Int<2>{}) : c.xq == 4 ? with(Int<4>{}) : with(Int<kStreamDirect>{});
 }
 
 // ---- decode attention: (column steps, latent tiles per wave) that hold the widths
@@ -580,8 +589,8 @@ int ajqd_dense_out(const void* in, const void* w, float* x, const float* again, 
   if (batch < 1 || k < 8 || k % 8 || width < 16 || width % 16)
     return fail(AJQ_ERR_SHAPE, "ajqd_dense_out: unsupported shape (batch=%d k=%d width=%d)", batch, k, width);
   DenseOut d{(const uint16_t*)in, (const uint16_t*)w, x, again, step, batch, k, width};
-  const OutCut c = out_cut(batch, width, k, false);
-  return with_out_cut(c, batch, k, [&](auto waves, auto rows, auto rt, auto bt, auto uq, auto xq) {
+  const OutCut c = out_cut(batch, width, k, false, 1);
+  return with_out_cut<false>(c, [&](auto waves, auto rows, auto rt, auto bt, auto uq, auto xq) {
     hipLaunchKernelGGL((dense_out_kernel<waves(), rows(), rt(), bt(), uq(), xq()>), c.grid, dim3(c.threads), 0, (hipStream_t)stream, d);
     return check_launch("ajqd_dense_out");
   });
@@ -727,9 +736,9 @@ static int dense_out_streams(const char* name, DenseOutStreams d, void* stream) 
   if (int e = check_streams(streams, name)) return e;
   if (batch < 1 || k < 8 || k % 8 || width < 16 || width % 16)
     return fail(AJQ_ERR_SHAPE, "%s: unsupported shape (batch=%d k=%d width=%d)", name, batch, k, width);
-  const OutCut c = out_cut(batch, width, k, !d.u);
+  const OutCut c = out_cut(batch, width, k, !d.u, streams);
   auto pick = [&](auto room) {
-    return with_out_cut(c, batch, k, [&](auto waves, auto rows, auto rt, auto bt, auto uq, auto xq) {
+    return with_out_cut<(room() > 4)>(c, [&](auto waves, auto rows, auto rt, auto bt, auto uq, auto xq) {
       hipLaunchKernelGGL((dense_out_streams_kernel<waves(), rows(), rt(), bt(), uq(), xq(), decltype(room)::value>), c.grid, dim3(c.threads), 0,
                          (hipStream_t)stream, d);
       return check_launch(name);
@@ -749,7 +758,13 @@ int ajqd_dense_out_streams(const void* in, const void* w, float* x, const float*
                                                                      nullptr, nullptr, batch, k, width, streams}, stream);
 }
 
-int ajqd_dense_out_parts(int batch, int width) { return batch < 1 || width < 16 || width % 16 ? 0 : width / out_cut(batch, width, kTwoWaveColumns, true).rows; }
+int ajqd_dense_out_parts(int batch, int width) { return batch < 1 || width < 16 || width % 16 ? 0 : width / out_cut(batch, width, kTwoWaveColumns, true, 1).rows; }
+
+int ajqd_dense_out_form(int batch, int k, int width, int streams, int scaled) {
+  if (batch < 1 || k < 8 || k % 8 || width < 16 || width % 16 || streams < 0 || streams > kMaxStreams) return 0;
+  const OutCut c = out_cut(batch, width, k, scaled != 0, streams < 1 ? 1 : streams);
+  return 100000 * (c.threads / 64) + 10000 * (c.rows / 8) + 1000 * c.rt + 100 * c.bt + 10 * c.uq + (c.xq > 0 ? c.xq : 0);
+}
 
 int ajqd_dense_out_streams_scaled(const void* in, const void* w, float* x, const float* scale, const float* out, const float* mix,
                                   const float* next, const float* gain, void* scaled, float* sums, int streams, int batch, int k, int width,

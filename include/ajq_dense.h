@@ -177,6 +177,9 @@ int ajqd_dense_out_streams_scaled(const void* in, const void* w, float* x, const
                                   const float* next, const float* gain, void* scaled, float* sums, int streams, int batch, int k, int width,
                                   void* stream);
 int ajqd_dense_out_parts(int batch, int width);
+/* the form that ajqd_dense_out (streams = 0), ajqd_dense_out_streams and (scaled) ajqd_dense_out_streams_scaled take, in decimal digits: waves,
+ * row tile / 8, row tiles, batch tiles, blocks of columns at a time, batch rows per load instruction / 4 (0: rows not staged); 0 if refused */
+int ajqd_dense_out_form(int batch, int k, int width, int streams, int scaled);
 
 /* out = act(y), `count` (a multiple of 8) elements of dtype; may be in place */
 int ajqd_activation(const void* y, void* out, int64_t count, int act, int dtype, void* stream);

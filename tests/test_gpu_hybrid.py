@@ -129,6 +129,13 @@ def test_dense_out_streams(cuda, batch, shape):
         assert _rel(u, (weights[:, None, None] * want).sum(0)) < 4e-6
 
 
+@pytest.mark.parametrize("streams,batch,k,width", [(12, 33, 1152, 2064), (5, 40, 2048, 4128), (16, 17, 1024, 4128), (8, 33, 2056, 2560), (16, 48, 8192, 2080),
+                                                   (6, 20, 8320, 2064)])
+def test_dense_out_streams_of_many_streams_and_sequences(cuda, streams, batch, k, width):
+    """Tiles of 16 rows with more than four streams: from memory below rows of 8192 columns, staged from there on one and on two row tiles."""
+    test_dense_out_streams(cuda, batch, (streams, k, width))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_squared_relu(cuda, dtype):
     y = torch.randn(7, 40).to(dtype)

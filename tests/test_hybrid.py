@@ -291,6 +291,17 @@ def test_dense_library_refuses_bad_arguments_before_any_launch():
     assert lib.ajqd_scan_step(ctypes.byref(step), None) == -2                                            # 8 + 16 rows in 16
 
 
+@pytest.mark.parametrize("streams,batch,k,width,scaled,form", [
+    # more than four streams and 16 sequences on 16-row tiles: from memory, one tile, one block, up to rows of 8192 columns
+    (12, 33, 1152, 2064, 1, 421210), (5, 17, 1024, 8192, 1, 421210), (16, 64, 8064, 4096, 0, 421210),
+    (8, 64, 8192, 4096, 1, 422214), (16, 17, 8192, 2064, 1, 421214), (8, 64, 8200, 8192, 1, 421210),
+    # and the forms beside it: 8-row tiles, up to four streams, up to 16 sequences
+    (12, 64, 1024, 512, 1, 811214), (4, 33, 1152, 2064, 1, 421214), (4, 33, 1152, 4096, 1, 422214), (4, 17, 2056, 4096, 1, 421220), (16, 16, 4096, 4096, 1, 421114),
+])
+def test_form_of_a_decode_product_with_streams(streams, batch, k, width, scaled, form):
+    assert _lib.load_dense().ajqd_dense_out_form(batch, k, width, streams, scaled) == form
+
+
 def test_decode_attention_that_makes_its_row_refuses_bad_arguments():
     lib = _lib.load_dense()
     buf = ctypes.create_string_buffer(4096)
