@@ -188,16 +188,30 @@ int launch_product_tile(int tile, const DenseGemm& a, hipStream_t stream) {
 
 // ---- products of one decode step
 constexpr int kTwoWaveColumns = 256;  // products of one or two blocks of columns run on two waves (stream_rows)
-// Batch rows go through LDS (stream_rows) where K is whole blocks and gives a wave some to stream; with less the trip costs more than it saves
-// (5 .. 16 sequences, K = 1000: 1.02 .. 1.09 of the time; more than 16, K = 600: 1.07).
-bool staged_rows(int batch, int k) { return k % kStreamBlock == 0 && k >= (batch > kGemvBatch ? 1024 : 2048); }
 constexpr int kLongRow = 8192;
+// Batch rows go through LDS (stream_rows) where K is whole blocks and the trip gains something (figures: the time over that from memory).  From 1024
+// columns on with more than 16 sequences, 2048 with fewer (half of that would still gain, 512 columns 0.92 .. 0.98 at 32 sequences and 0.95 .. 0.98 at
+// 16, but not at eight and fewer: 0.98 .. 1.03).  With five to eight a wave whose share is a block short waits for the others, until K hides that (5
+// sequences, 96 tiles of dense_in: K = 2048 1.00, 2176 1.03, 2560 1.00, 3200 1.025, 4096 0.995; 7: 1.02 at 2176, 0.98 from 2560 on) or there is more
+// than a round of workgroups (0.95 .. 0.98).  Up to four, an instruction brings few bytes either way: eight waves gain with even shares or 3072
+// columns (width 1024, one sequence: K = 2048 0.955, 2176 1.01, 3584 0.95, 8192 0.89; width 2048 at 2176 and 2560: 1.04), four waves in the first
+// half of a second round (320 tiles: 0.96 .. 1.00) and with long rows (K = 9216: 0.93 at 129 tiles, 0.96 at 320).  A round that is nearly full keeps the
+// memory busy by itself, but where rows lie 16 KiB apart (256 tiles: K = 4096 1.01, 8192 0.94, 9216 1.02, 11136 1.02).
+bool staged_rows(int batch, int k, int waves, long long tiles) {
+  if (k % kStreamBlock != 0 || k < (batch > kGemvBatch ? 1024 : 2048)) return false;
+  if (batch > 8) return true;
+  const bool even = k % (kStreamBlock * waves) == 0;
+  if (batch > 4) return waves == 8 || even || tiles > kCus || k >= (batch <= 6 ? 3584 : 2560);
+  if (waves == 8) return even || k >= 3072;
+  return (tiles > kCus && tiles <= 384) || (k >= kLongRow && (tiles <= 192 || tiles > kCus || k % kLongRow == 0));
+}
 // How dense_out and dense_out_streams cut [width, k]: up to 128 tiles of 16 rows leave half the CUs idle, tiles of 8 rows on eight
 // waves use them all (2048 x 8192: 9.7 -> 7.5 us at 4 sequences, 15.4 -> 12.8 at 32), where K gives each of them a block (1024 x 512: 3.0 us
 // with them, 2.5 without).  More than 16 sequences: two row tiles per workgroup share the activations from 512 tiles on (35424 x 4096: 84 -> 65 us),
 // staged rows wherever one each would be more than a round of the CUs (5856 x 2048: 9.5 us, 7.9 with two; 4096 x 16384: 29.5, 38.0 with two); below
 // that, rows that are not staged have two blocks in flight instead (4096 x 18440: 44.2 -> 42.6) where K gives each wave several (5120 x 256,
-// 64 sequences: 9.1 us with two, 5.1 with one).  Up to 16, long staged rows: two blocks at a time (4096 x 16384: 26.6 -> 24.4).  K of one or two
+// 64 sequences: 9.1 us with two, 5.1 with one).  Up to 16, long staged rows that come out even: two blocks at a time (4096 x 16384: 26.6 -> 24.4;
+// 4096 x 8448, 5 sequences: 12.7, 12.3 with one).  K of one or two
 // blocks: two waves (32000 x 128, one sequence: 5.2 us on four, 4.4 on two).
 // More than four streams leave a wave of 16-row tiles and two batch tiles no registers for more than the plainest form: rows from memory, one row
 // tile, one block at a time takes 240, every other form 280 and more, and then a CU holds one workgroup instead of two (12 streams of 2064
@@ -215,10 +229,10 @@ OutCut out_cut(int batch, int width, int k, bool sums, int streams) {
   const long long tiles = (long long)(width / 16) * blocks;
   c.rows = tiles <= 128 && (sums || k >= 1024) ? 8 : 16;
   const bool few = c.rows == 16 && c.bt == 1 && k <= kTwoWaveColumns, plain = c.rows == 16 && c.bt == 2 && streams > 4;
-  const bool staged = staged_rows(batch, k) && (!plain || k >= kLongRow);
+  const bool staged = staged_rows(batch, k, c.rows == 8 ? 8 : 4, tiles) && (!plain || k >= kLongRow);
   c.xq = few || !staged ? kStreamDirect : batch <= 4 ? 1 : batch <= 8 ? 2 : 4;
   c.rt = c.bt == 2 && width % 32 == 0 && (staged ? c.rows == 16 && tiles > kCus : !plain && width >= 8192) ? 2 : 1;
-  c.uq = c.rows == 8 || c.rt == 2 || few ? 1 : c.bt == 1 ? (staged && k >= kLongRow ? 2 : 1) : !staged && !plain && k >= 2048 ? 2 : 1;
+  c.uq = c.rows == 8 || c.rt == 2 || few ? 1 : c.bt == 1 ? (staged && k >= kLongRow && k % 1024 == 0 ? 2 : 1) : !staged && !plain && k >= 2048 ? 2 : 1;
   c.grid = dim3(width / (c.rows * c.rt), blocks);
   c.threads = c.rows == 8 ? 512 : few ? 128 : 256;
   return c;
@@ -546,9 +560,9 @@ static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* 
   // more than 16 sequences: two batch tiles and two row tiles per workgroup, or, where one each is no more than a round of the CUs, one on
   // eight waves (2560 x 2048, 32 sequences: 8.7 -> 6.8 us; 4608 x 2048, 288 tiles: 9.2 with two, 11.6 so)
   const bool wide = a->batch > kGemvBatch, few = a->width <= kTwoWaveColumns;
-  const bool staged = staged_rows(a->batch, a->width);
   const int block = wide ? 2 * kGemvBatch : kGemvBatch;
-  const bool short_of_tiles = staged && ((long long)a->tiles1 + a->tiles2) * ((a->batch + block - 1) / block) <= kCus;
+  const long long tiles = ((long long)a->tiles1 + a->tiles2) * ((a->batch + block - 1) / block);
+  const bool staged = staged_rows(a->batch, a->width, 4, tiles), short_of_tiles = staged && tiles <= kCus;
   const int rt = wide && !few && !short_of_tiles && a->tiles1 != 1 && a->tiles2 != 1 ? 2 : 1;
   const dim3 grid((a->tiles1 + rt - 1) / rt + (a->tiles2 + rt - 1) / rt, (a->batch + block - 1) / block);
   const int bytes = a->x ? 2 * a->batch * (a->width + 8) : 0;
@@ -571,7 +585,7 @@ static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* 
   if (staged && a->batch > 8) return go(dense_in_kernel<4, false, 1, 1, 4, 1>, 256);
   if (staged && a->batch > 4) return go(dense_in_kernel<4, false, 1, 1, 2, 1>, 256);
   // up to four sequences: with few tiles, two blocks at a time where they come out even (4608 x 2048: 7.1 -> 6.8 us; 16384 x 4096: 21.2 -> 21.7)
-  if (staged && a->batch <= 4 && a->width % 1024 == 0 && a->tiles1 + a->tiles2 <= 384) return go(dense_in_kernel<4, false, 1, 1, 1, 2>, 256);
+  if (a->batch <= 4 && a->width % 1024 == 0 && a->width >= 2048 && a->tiles1 + a->tiles2 <= 384) return go(dense_in_kernel<4, false, 1, 1, 1, 2>, 256);
   return go(dense_in_kernel<4, false, 1, 1, kStreamDirect, 1>, 256);
 }
 

@@ -850,6 +850,21 @@ def test_streamed_products_of_staged_rows(cuda, batch, k, width):
     test_dense_out_streams(cuda, batch, (2, k, width))
 
 
+FORMS = [  # batch, k, width: together every form of dense_out and dense_in (tests/test_hybrid.py counts them)
+    (3, 256, 2064),                                                                             # two waves
+    (4, 2056, 48), (4, 2048, 48), (3, 3200, 2048), (8, 2048, 48), (5, 8192, 2048), (16, 2048, 2048),   # tiles of 8 rows on eight waves
+    (2, 4096, 4096), (4, 2560, 5120), (4, 8320, 2064), (3, 16384, 2064),                        # up to four sequences on 16: from memory, staged, two blocks
+    (5, 2176, 2064), (6, 3584, 2064), (7, 2560, 2064), (8, 8192, 4112), (16, 2176, 2064), (12, 8192, 2064),
+    (32, 1032, 48), (20, 1024, 2048), (32, 1024, 4096), (33, 1024, 4128), (24, 1024, 4112), (20, 2056, 2064), (17, 136, 8192), (33, 136, 2064),
+]
+
+
+@pytest.mark.parametrize("batch,k,width", FORMS)
+def test_every_form_of_a_decode_product(cuda, batch, k, width):
+    test_streamed_products(cuda, batch, k, width)
+    test_dense_out_streams(cuda, batch, (2, k, width))
+
+
 @pytest.mark.parametrize("batch,k", [(4, 256), (3, 264), (2, 4096), (4, 4104), (4, 8192), (3, 8200), (4, 15432), (4, 17928)])
 def test_norm_prologue_on_two_four_and_eight_waves(cuda, batch, k):
     """dense_in with the norm inside, at the row lengths where its workgroups change; an operand rounded the other way moves by 2^-8."""
@@ -864,9 +879,20 @@ def test_norm_prologue_on_two_four_and_eight_waves(cuda, batch, k):
 @pytest.mark.parametrize("batch", [1, 5, 16, 17, 33])
 @pytest.mark.parametrize("width,streams", [(48, 1), (2048, 2), (2064, 3)])
 def test_norm_carried_to_the_outputs(cuda, batch, width, streams):
+    _norm_carried_to_the_outputs(cuda, batch, width, streams, 264, 96)
+
+
+@pytest.mark.parametrize("batch,width,streams,k,n", [(4, 2048, 2, 2048, 96), (3, 2064, 2, 8192, 4128), (8, 2048, 3, 8192, 96), (8, 2560, 2, 2048, 5120), (16, 2048, 2, 2048, 96),
+                                                     (33, 2048, 2, 1024, 4128), (24, 1024, 2, 2048, 2064), (32, 2064, 4, 1152, 4112)])
+def test_norm_carried_to_the_outputs_by_staged_rows(cuda, batch, width, streams, k, n):
+    """The same where batch rows go through LDS, in front of dense_in and in it, with one and two row tiles."""
+    _norm_carried_to_the_outputs(cuda, batch, width, streams, k, n)
+
+
+def _norm_carried_to_the_outputs(cuda, batch, width, streams, k, n):
     """dense_out_streams_scaled and the dense_in behind it against the norm as a launch of its own: the scaled rows are the rounding of
     u gain, the sums are u's, and the two products agree as far as one rounding of an operand each (2^-9 a value, independent) lets them."""
-    g, k, n = torch.Generator().manual_seed(width + batch), 264, 96
+    g = torch.Generator().manual_seed(width + batch)
     a, w, w2 = _bf(g, batch, k), _bf(g, width, k, std=k ** -0.5), _bf(g, n, width, std=width ** -0.5)
     x, scale, gain, hc, reads = torch.randn((batch, streams, width), generator=g), torch.randn(width, generator=g), torch.randn(width, generator=g), _coefficients(g, streams), torch.randn(streams, generator=g)
     d = {m: v.to(cuda) for m, v in dict(a=a, w=w, w2=w2, x=x, scale=scale, gain=gain, reads=reads, **hc).items()}

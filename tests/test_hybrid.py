@@ -291,6 +291,26 @@ def test_dense_library_refuses_bad_arguments_before_any_launch():
     assert lib.ajqd_scan_step(ctypes.byref(step), None) == -2                                            # 8 + 16 rows in 16
 
 
+def test_every_form_of_a_decode_product_is_run():
+    """The shapes that the GPU test runs reach every form of a product without many streams that the library holds."""
+    from tests.test_gpu_hybrid import FORMS
+    lib = _lib.load_dense()
+    forms = {lib.ajqd_dense_out_form(batch, k, width, 2, 0) for batch, k, width in FORMS}
+    assert forms == {221110, 811110, 811111, 811112, 811114, 811210, 811214, 421110, 421111, 421121, 421112, 421122, 421114, 421124, 421210, 421214, 421220,
+                     422210, 422214}
+    assert forms >= {lib.ajqd_dense_out_form(b, k, 16 * n, s, 0) for b in (1, 3, 5, 8, 9, 17, 33, 64) for k in (8, 128, 264, 1000, 1024, 2048, 2176, 4096, 8192, 8200, 8320)
+                     for n in (1, 64, 128, 129, 256, 257, 258, 320, 512, 513, 1000) for s in (1, 4)}
+
+
+@pytest.mark.parametrize("batch,k,width,form", [  # few sequences: staged rows on both sides of each line
+    (1, 2048, 1024, 811111), (1, 2176, 1024, 811110), (4, 3072, 2048, 811111), (4, 2560, 2048, 811110), (1, 4096, 4096, 421110), (1, 4096, 4112, 421111),
+    (1, 4096, 6144, 421111), (1, 4096, 6160, 421110), (4, 8192, 4096, 421121), (4, 9216, 4096, 421110), (4, 9216, 3072, 421121), (1, 8320, 3072, 421111),
+    (5, 2176, 4096, 421110), (5, 2560, 4096, 421112), (5, 2176, 4112, 421112), (6, 3200, 4096, 421110), (7, 3200, 4096, 421112), (6, 3584, 4096, 421112), (9, 2176, 4096, 421114),
+])
+def test_form_of_a_decode_product_of_few_sequences(batch, k, width, form):
+    assert _lib.load_dense().ajqd_dense_out_form(batch, k, width, 0, 0) == form
+
+
 @pytest.mark.parametrize("streams,batch,k,width,scaled,form", [
     # more than four streams and 16 sequences on 16-row tiles: from memory, one tile, one block, up to rows of 8192 columns
     (12, 33, 1152, 2064, 1, 421210), (5, 17, 1024, 8192, 1, 421210), (16, 64, 8064, 4096, 0, 421210),
