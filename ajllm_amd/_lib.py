@@ -248,6 +248,7 @@ DENSE_SIGNATURES: dict[str, tuple] = {
     "ajqd_streams_norm": (c_int, [_P, _P, _P, _P, _P, _P, _P, _F, _P, _P, _I, _I, _I, _I, _I, _P]),
     "ajqd_dense_out_streams_scaled": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "ajqd_dense_out_parts": (c_int, [_I, _I]),
+    "ajqd_dense_in_form": (c_int, [_I, _I, _I, _I]),
     "ajqd_dense_out_form": (c_int, [_I, _I, _I, _I, _I]),
     "ajqd_dense_out_streams": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "ajqd_activation": (c_int, [_P, _P, _L, _I, _I, _P]),

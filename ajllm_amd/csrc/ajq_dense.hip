@@ -237,6 +237,33 @@ OutCut out_cut(int batch, int width, int k, bool sums, int streams) {
   c.threads = c.rows == 8 ? 512 : few ? 128 : 256;
   return c;
 }
+// How dense_in cuts [16 (tiles1 + tiles2), k] without the norm.  More than 16 sequences: two batch tiles and two row tiles per workgroup, or, where one each is
+// no more than a round of the CUs, one on eight waves (2560 x 2048, 32 sequences: 8.7 -> 6.8 us; 4608 x 2048, 288 tiles: 9.2 with two, 11.6 so).  Up to
+// four: two blocks at a time where they come out even and the last round of workgroups is up to three quarters full, and not beyond 384, from where
+// the rows' trip is for nothing (one sequence, K = 4096: 96 tiles 0.93 of the time, 192 0.99, 256 1.03, 288 0.96, 384 0.97, 480 1.03, 1024 1.03; K =
+// 2048: 0.97, 0.97, 1.03, 0.96, 0.98, 1.00, 1.02).
+struct InCut {
+  int waves, rt, bt, uq, xq;
+};
+InCut in_cut(int batch, int k, int tiles1, int tiles2) {
+  InCut c{4, 1, batch > kGemvBatch ? 2 : 1, 1, kStreamDirect};
+  const int blocks = (batch + kGemvBatch * c.bt - 1) / (kGemvBatch * c.bt);
+  const long long tiles = ((long long)tiles1 + tiles2) * blocks;
+  if (k <= kTwoWaveColumns) {
+    c.waves = 2;
+    return c;
+  }
+  const bool staged = staged_rows(batch, k, 4, tiles);
+  if (c.bt == 2) {
+    if (staged && tiles <= kCus) c.waves = 8, c.xq = 4;
+    else if (tiles1 != 1 && tiles2 != 1) c.rt = 2, c.xq = staged ? 4 : kStreamDirect;
+  } else if (batch > 4) {
+    if (staged) c.xq = batch > 8 ? 4 : 2;
+  } else if (k % 1024 == 0 && k >= 2048 && (tiles <= 192 || (tiles > kCus && tiles <= 384))) {
+    c.uq = 2, c.xq = 1;
+  }
+  return c;
+}
 template <int N> using Int = std::integral_constant<int, N>;
 // go(waves, row tile, row tiles, batch tiles, blocks at a time, batch rows' instructions) of a cut; kMany: more than four streams
 template <bool kMany, typename Go>
@@ -557,14 +584,9 @@ static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* 
   d.batch = a->batch; d.D = a->true_width; d.Dp = a->width; d.tiles1 = a->tiles1; d.tiles2 = a->tiles2;
   d.gated_ld = a->gated_ld; d.act = a->act; d.center = a->center; d.pairs = a->pairs; d.eps = a->eps;
   d.sums = sums; d.parts = parts;
-  // more than 16 sequences: two batch tiles and two row tiles per workgroup, or, where one each is no more than a round of the CUs, one on
-  // eight waves (2560 x 2048, 32 sequences: 8.7 -> 6.8 us; 4608 x 2048, 288 tiles: 9.2 with two, 11.6 so)
-  const bool wide = a->batch > kGemvBatch, few = a->width <= kTwoWaveColumns;
-  const int block = wide ? 2 * kGemvBatch : kGemvBatch;
-  const long long tiles = ((long long)a->tiles1 + a->tiles2) * ((a->batch + block - 1) / block);
-  const bool staged = staged_rows(a->batch, a->width, 4, tiles), short_of_tiles = staged && tiles <= kCus;
-  const int rt = wide && !few && !short_of_tiles && a->tiles1 != 1 && a->tiles2 != 1 ? 2 : 1;
-  const dim3 grid((a->tiles1 + rt - 1) / rt + (a->tiles2 + rt - 1) / rt, (a->batch + block - 1) / block);
+  const InCut c = in_cut(a->batch, a->width, a->tiles1, a->tiles2);
+  const int block = kGemvBatch * c.bt;
+  const dim3 grid((a->tiles1 + c.rt - 1) / c.rt + (a->tiles2 + c.rt - 1) / c.rt, (a->batch + block - 1) / block);
   const int bytes = a->x ? 2 * a->batch * (a->width + 8) : 0;
   auto go = [&](auto kernel, int threads) {
     if (int e = allow_lds(kernel, bytes, name)) return e;
@@ -575,18 +597,26 @@ static int dense_in(const char* name, const ajqd_dense_in_args* a, const float* 
     // (rows so long that a workgroup's staging would not fit beside them run on two waves)
     // (and rows of more than 4096 columns on eight, whose registers hold them between the norm's passes: 8192 columns, 4 rows, 0 + 13648: 59.9
     // us on eight waves of the half-line form before, 96.7 on four of this one; 2016 + 6912: 43.7, 70.9, and 46.6 on eight)
-    if (bytes > 140 * 1024 || few) return go(dense_in_kernel<2, true, 1, 1, kStreamFrom, 1>, 128);
+    if (bytes > 140 * 1024 || c.waves == 2) return go(dense_in_kernel<2, true, 1, 1, kStreamFrom, 1>, 128);
     if (a->width > 4096 && bytes <= 120 * 1024) return go(dense_in_kernel<8, true, 1, 1, kStreamFrom, 1>, 512);
     return go(dense_in_kernel<4, true, 1, 1, kStreamFrom, 1>, 256);
   }
-  if (few) return wide ? go(dense_in_kernel<2, false, 1, 2, kStreamDirect, 1>, 128) : go(dense_in_kernel<2, false, 1, 1, kStreamDirect, 1>, 128);
-  if (rt == 2) return staged ? go(dense_in_kernel<4, false, 2, 2, 4, 1>, 256) : go(dense_in_kernel<4, false, 2, 2, kStreamDirect, 1>, 256);
-  if (wide) return short_of_tiles ? go(dense_in_kernel<8, false, 1, 2, 4, 1>, 512) : go(dense_in_kernel<4, false, 1, 2, kStreamDirect, 1>, 256);
-  if (staged && a->batch > 8) return go(dense_in_kernel<4, false, 1, 1, 4, 1>, 256);
-  if (staged && a->batch > 4) return go(dense_in_kernel<4, false, 1, 1, 2, 1>, 256);
-  // up to four sequences: with few tiles, two blocks at a time where they come out even (4608 x 2048: 7.1 -> 6.8 us; 16384 x 4096: 21.2 -> 21.7)
-  if (a->batch <= 4 && a->width % 1024 == 0 && a->width >= 2048 && a->tiles1 + a->tiles2 <= 384) return go(dense_in_kernel<4, false, 1, 1, 1, 2>, 256);
-  return go(dense_in_kernel<4, false, 1, 1, kStreamDirect, 1>, 256);
+  if (c.waves == 2) return c.bt == 2 ? go(dense_in_kernel<2, false, 1, 2, kStreamDirect, 1>, 128) : go(dense_in_kernel<2, false, 1, 1, kStreamDirect, 1>, 128);
+  if (c.waves == 8) return go(dense_in_kernel<8, false, 1, 2, 4, 1>, 512);
+  if (c.rt == 2) return c.xq == 4 ? go(dense_in_kernel<4, false, 2, 2, 4, 1>, 256) : go(dense_in_kernel<4, false, 2, 2, kStreamDirect, 1>, 256);
+  if (c.bt == 2) return go(dense_in_kernel<4, false, 1, 2, kStreamDirect, 1>, 256);
+  switch (c.xq) {
+    case 1: return go(dense_in_kernel<4, false, 1, 1, 1, 2>, 256);
+    case 2: return go(dense_in_kernel<4, false, 1, 1, 2, 1>, 256);
+    case 4: return go(dense_in_kernel<4, false, 1, 1, 4, 1>, 256);
+    default: return go(dense_in_kernel<4, false, 1, 1, kStreamDirect, 1>, 256);
+  }
+}
+
+int ajqd_dense_in_form(int batch, int k, int tiles1, int tiles2) {
+  if (batch < 1 || k < 8 || k % 8 || tiles1 < 0 || tiles2 < 0 || tiles1 + tiles2 < 1) return 0;
+  const InCut c = in_cut(batch, k, tiles1, tiles2);
+  return 100000 * c.waves + 20000 + 1000 * c.rt + 100 * c.bt + 10 * c.uq + (c.xq > 0 ? c.xq : 0);
 }
 
 int ajqd_dense_in(const ajqd_dense_in_args* a, void* stream) { return dense_in("ajqd_dense_in", a, nullptr, 0, stream); }

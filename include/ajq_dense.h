@@ -180,6 +180,8 @@ int ajqd_dense_out_parts(int batch, int width);
 /* the form that ajqd_dense_out (streams = 0), ajqd_dense_out_streams and (scaled) ajqd_dense_out_streams_scaled take, in decimal digits: waves,
  * row tile / 8, row tiles, batch tiles, blocks of columns at a time, batch rows per load instruction / 4 (0: rows not staged); 0 if refused */
 int ajqd_dense_out_form(int batch, int k, int width, int streams, int scaled);
+/* the same of ajqd_dense_in without its norm and of ajqd_dense_in_scaled */
+int ajqd_dense_in_form(int batch, int k, int tiles1, int tiles2);
 
 /* out = act(y), `count` (a multiple of 8) elements of dtype; may be in place */
 int ajqd_activation(const void* y, void* out, int64_t count, int act, int dtype, void* stream);

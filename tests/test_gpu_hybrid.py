@@ -855,7 +855,7 @@ FORMS = [  # batch, k, width: together every form of dense_out and dense_in (tes
     (4, 2056, 48), (4, 2048, 48), (3, 3200, 2048), (8, 2048, 48), (5, 8192, 2048), (16, 2048, 2048),   # tiles of 8 rows on eight waves
     (2, 4096, 4096), (4, 2560, 5120), (4, 8320, 2064), (3, 16384, 2064),                        # up to four sequences on 16: from memory, staged, two blocks
     (5, 2176, 2064), (6, 3584, 2064), (7, 2560, 2064), (8, 8192, 4112), (16, 2176, 2064), (12, 8192, 2064),
-    (32, 1032, 48), (20, 1024, 2048), (32, 1024, 4096), (33, 1024, 4128), (24, 1024, 4112), (20, 2056, 2064), (17, 136, 8192), (33, 136, 2064),
+    (17, 128, 48), (32, 1032, 48), (20, 1024, 2048), (32, 1024, 4096), (33, 1024, 4128), (24, 1024, 4112), (20, 2056, 2064), (17, 136, 8192), (33, 136, 2064),
 ]
 
 

@@ -302,6 +302,23 @@ def test_every_form_of_a_decode_product_is_run():
                      for n in (1, 64, 128, 129, 256, 257, 258, 320, 512, 513, 1000) for s in (1, 4)}
 
 
+def test_every_form_of_a_decode_product_of_the_inputs_is_run():
+    from tests.test_gpu_hybrid import FORMS
+    lib = _lib.load_dense()
+    forms = {lib.ajqd_dense_in_form(batch, k, width // 16, 0) for batch, k, width in FORMS}
+    assert forms == {221110, 221210, 821214, 422214, 422210, 421110, 421121, 421112, 421114}
+    assert forms | {421210} == {lib.ajqd_dense_in_form(b, k, n, m) for b in (1, 3, 5, 8, 9, 17, 33, 64) for k in (8, 128, 264, 1000, 1024, 2048, 2176, 4096, 8192, 8200)
+                                for n in (0, 1, 64, 129, 256, 320, 1000) for m in (0, 2, 128, 400) if n + m}
+
+
+@pytest.mark.parametrize("batch,k,tiles1,tiles2,form", [  # two blocks of columns at a time, and not in a round that is nearly full or past 384 tiles
+    (1, 2048, 192, 0, 421121), (1, 2048, 0, 194, 421110), (4, 4096, 256, 0, 421110), (2, 2048, 129, 128, 421121), (4, 2048, 384, 0, 421121), (4, 2048, 385, 0, 421110),
+    (4, 1024, 64, 0, 421110), (4, 2176, 64, 0, 421110), (5, 2048, 64, 0, 421112), (33, 2048, 128, 0, 821214), (33, 2048, 129, 0, 422214),
+])
+def test_form_of_a_decode_product_of_the_inputs(batch, k, tiles1, tiles2, form):
+    assert _lib.load_dense().ajqd_dense_in_form(batch, k, tiles1, tiles2) == form
+
+
 @pytest.mark.parametrize("batch,k,width,form", [  # few sequences: staged rows on both sides of each line
     (1, 2048, 1024, 811111), (1, 2176, 1024, 811110), (4, 3072, 2048, 811111), (4, 2560, 2048, 811110), (1, 4096, 4096, 421110), (1, 4096, 4112, 421111),
     (1, 4096, 6144, 421111), (1, 4096, 6160, 421110), (4, 8192, 4096, 421121), (4, 9216, 4096, 421110), (4, 9216, 3072, 421121), (1, 8320, 3072, 421111),
