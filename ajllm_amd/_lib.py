@@ -254,6 +254,7 @@ DENSE_SIGNATURES: dict[str, tuple] = {
     "ajqd_activation": (c_int, [_P, _P, _L, _I, _I, _P]),
     "ajqd_key_value_split": (c_int, [ctypes.POINTER(KeyValueSplitArgs), _I, _I, _P]),
     "ajqd_group_decode_built": (c_int, [_I, _I, _I]),
+    "ajqd_group_decode_better": (c_int, [_I, _I, _I, _I, _I]),
     "ajqd_group_decode": (c_int, [ctypes.POINTER(KeyValueSplitArgs), _P, _I, _F, _P]),
     "ajqd_group_merge": (c_int, [_P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P]),
     "ajqd_conv_silu": (c_int, [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P, _I, _P]),

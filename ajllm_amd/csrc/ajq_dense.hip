@@ -880,6 +880,16 @@ int ajqd_group_decode_built(int share, int dimp, int rot) {
   return share >= 1 && share <= kGroupShare && dimp >= 16 && dimp % 16 == 0 && latent_steps(2 * dimp) > 0 && latent_steps(2 * dimp) <= 10 && rot >= 0 && rot % 8 == 0;
 }
 
+// Heads of up to 128 columns: two workgroups share a CU and one's front runs beside the other's rows (160 shapes: 0.84 of the time of two launches, the
+// most 1.02).  Wider ones have a CU each, so the front is paid once a round and only one round may be; it takes a turn per four heads (up to 7 heads: 160
+// shapes 0.70 .. 1.02), and with a third turn pays where the rings are long enough to fill the chip (8 heads, 256 workgroups: 0.82 .. 0.96, 1.07 at the
+// first positions; 2 to 128: 0.88 .. 1.10; 16 heads: 0.93 .. 1.25; 26 x 10 workgroups, two rounds: 1.08 .. 1.39).
+int ajqd_group_decode_better(int units, int share, int dimp, int rot, int chunks) {
+  if (!ajqd_group_decode_built(share, dimp, rot) || units < 1 || chunks < 1) return 0;
+  const long long workgroups = (long long)units * chunks;
+  return dimp <= 128 || (workgroups <= kCus && (share <= 7 || (share <= 11 && workgroups > 128)));
+}
+
 int ajqd_group_decode(const ajqd_key_value_split_args* a, float* partial, int chunks, float scale, void* stream) {
   if (!a || !partial || !a->y || !a->q_gain || !a->k_gain || (a->rot && !a->half_turns) || !a->rows || !a->pos)
     return fail(AJQ_ERR_NULL, "ajqd_group_decode: null pointer argument");

@@ -497,7 +497,7 @@ class HybridLM(DenseLM):
             return self._attend_token(y.to(torch.bfloat16), w, cache, run)
         units = batch * w.groups
         partial = torch.empty(lib.ajqd_latent_decode_workspace(units, w.share, w.dimp, chunks), dtype=torch.uint8, device=y.device)
-        if lib.ajqd_group_decode_built(w.share, w.dimp, w.rot):
+        if lib.ajqd_group_decode_better(units, w.share, w.dimp, w.rot, chunks):
             args = self._split_args(y, w, None, 0, ring, 1, 0, cache.position, 0, cache.kept[run])
             _lib.check_dense(lib.ajqd_group_decode(ctypes.byref(args), _ptr(partial), chunks, w.scale, st), "group_decode")
         else:

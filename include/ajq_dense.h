@@ -207,6 +207,8 @@ int ajqd_key_value_split(const ajqd_key_value_split_args* args, int y_dtype, int
  * and ajqd_latent_decode of its queries, share = heads / groups heads a (sequence, key / value head), in one launch.  Built where
  * ajqd_group_decode_built says so; chunks and workspace as ajqd_latent_decode's. */
 int ajqd_group_decode_built(int share, int dimp, int rot);
+/* 1 where that is faster than the two launches, for units = sequences x groups */
+int ajqd_group_decode_better(int units, int share, int dimp, int rot, int chunks);
 int ajqd_group_decode(const ajqd_key_value_split_args* args, float* partial, int chunks, float scale, void* stream);
 /* merge of ajqd_latent_decode's chunks where a (sequence, key / value head) was a sequence of `share` heads and dimp the
  * latent's width; output gate sigmoid(gate[b * gate_ld + head * dimp + c]) (or NULL) -> out bf16 [batch, out_ld] */

@@ -533,6 +533,9 @@ SHAPES = {
     # sizes of a larger model's heads and channels
     "wide": dict(layers=[attention(heads=4, kv_heads=2, dim=128, rot=32, scaling=SCALING, window=70, keep=4, ff=520), scan(inner=640, state=24, rank=20, ff=264)],
                  width=320, streams=2, loop={"start": 0, "stop": 1, "times": 2}),
+    # heads of which a CU holds one workgroup: few of them on a key head in one launch, many in two
+    "broad": dict(layers=[attention(heads=6, kv_heads=2, dim=144, rot=40, window=70, keep=4), attention(heads=12, kv_heads=1, dim=136, rot=24, window=70, keep=4)],
+                  loop=None),
     # heads wider than the MFMA kernels take, many states per channel
     "beyond": dict(layers=[attention(heads=2, kv_heads=1, dim=304, rot=60, window=20, keep=3), scan(inner=32, state=70, rank=12)], loop=None),
 }

@@ -339,6 +339,14 @@ def test_form_of_a_decode_product_with_streams(streams, batch, k, width, scaled,
     assert _lib.load_dense().ajqd_dense_out_form(batch, k, width, streams, scaled) == form
 
 
+@pytest.mark.parametrize("units,share,dimp,chunks,better", [
+    (512, 16, 128, 32, 1), (26, 16, 128, 10, 1), (128, 7, 144, 2, 1), (128, 1, 160, 2, 1), (129, 4, 160, 2, 0), (26, 16, 160, 10, 0), (4, 8, 144, 32, 0), (65, 8, 144, 2, 1),
+    (64, 11, 160, 4, 1), (64, 12, 160, 4, 0), (4, 17, 128, 4, 0), (4, 4, 176, 4, 0),
+])
+def test_one_launch_for_the_decode_attention_where_it_is_the_faster(units, share, dimp, chunks, better):
+    assert _lib.load_dense().ajqd_group_decode_better(units, share, dimp, 64, chunks) == better
+
+
 def test_decode_attention_that_makes_its_row_refuses_bad_arguments():
     lib = _lib.load_dense()
     buf = ctypes.create_string_buffer(4096)
