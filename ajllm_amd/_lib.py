@@ -71,6 +71,7 @@ SIGNATURES: dict[str, tuple] = {
         c_int,
         [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p],
     ),
+    "ajq_attn_prefill_steps": (c_int, [c_int, c_int, c_int, c_int, c_int]),
     "ajq_attn_prefill_workspace": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "ajq_attn_prefill_in": (
         c_int,

@@ -1865,6 +1865,11 @@ size_t ajq_attn_prefill_workspace(int cache_dtype, int B, int H, int Hkv, int T,
   return (size_t)bytes;
 }
 
+int ajq_attn_prefill_steps(int B, int H, int T, int start, int head_dim) {
+  if (B < 1 || H < 1 || T < 1 || start < 0 || (head_dim != 128 && head_dim != 64 && head_dim != 32)) return -1;
+  return prefill_in_steps((long long)B * H, T, start, head_dim);
+}
+
 int ajq_attn_prefill(const float* q, const void* kcache, const void* vcache, int cache_dtype, int B, int H, int Hkv,
                      int T, int start, int max_len, int head_dim, void* out, int out_dtype, void* stream) {
   return ajq_attn_prefill_in(q, kcache, vcache, cache_dtype, B, H, Hkv, T, start, max_len, head_dim, out, out_dtype, nullptr, 0, stream);
@@ -1902,12 +1907,16 @@ int ajq_attn_prefill_in(const float* q, const void* kcache, const void* vcache, 
   const dim3 grid((unsigned)(((T + kPfBQ - 1) / kPfBQ) * B * H));  // (the kernel orders the work by cost)
   auto launch = [&](auto dim) {
     constexpr int HD = decltype(dim)::value;
-    if (cache_dtype == AJQ_KV_F32)
-      hipLaunchKernelGGL(attn_prefill_kernel<HD>, grid, dim3(256), 0, (hipStream_t)stream, q, reinterpret_cast<const float*>(kcache),
-                         reinterpret_cast<const float*>(vcache), H, Hkv, T, start, max_len, out, out_bf16);
-    else
-      hipLaunchKernelGGL(attn_prefill_steps_kernel<HD>, grid, dim3(256), 0, (hipStream_t)stream, q, reinterpret_cast<const uint16_t*>(kcache),
-                         reinterpret_cast<const uint16_t*>(vcache), H, Hkv, T, start, max_len, out, out_bf16);
+    auto go = [&](auto kernel, auto* cache_element) {
+      using CacheT = std::remove_pointer_t<decltype(cache_element)>;
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, q, reinterpret_cast<const CacheT*>(kcache),
+                         reinterpret_cast<const CacheT*>(vcache), H, Hkv, T, start, max_len, out, out_bf16);
+    };
+    if (cache_dtype == AJQ_KV_F32) return go(attn_prefill_kernel<float, HD>, (float*)nullptr);
+    if constexpr (HD < 128) {
+      if (!prefill_in_steps((long long)B * H, T, start, HD)) return go(attn_prefill_kernel<uint16_t, HD>, (uint16_t*)nullptr);
+    }
+    go(attn_prefill_steps_kernel<HD>, (uint16_t*)nullptr);
   };
   if (head_dim == 128) launch(std::integral_constant<int, 128>{});
   else if (head_dim == 64) launch(std::integral_constant<int, 64>{});

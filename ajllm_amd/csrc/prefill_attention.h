@@ -34,9 +34,10 @@
 // at the end.  bf16 inputs, fp32 scores, probabilities rounded to bf16 for the second product,
 // fp32 accumulators: the usual flash-attention arithmetic, not the eager fp32 one.
 //
-// Two kernels: bf16 caches (attn_prefill_steps_kernel) interleave both products and the softmax of three neighbouring half blocks;
-// fp32 caches pass through registers that are converted on the way, which leaves none for that (attn_prefill_kernel), unless
-// there is work enough to make a bf16 copy of the rows first (caches_to_bf16_kernel).
+// Two kernels: attn_prefill_steps_kernel on bf16 caches interleaves both products and the softmax of three neighbouring half blocks;
+// attn_prefill_kernel goes block by block, for narrow heads where that is the faster (prefill_in_steps) and for fp32 caches, which pass through
+// registers that are converted on the way and leave none for the other, unless there is work enough to make a bf16 copy of the rows first
+// (caches_to_bf16_kernel).
 #pragma once
 #include <type_traits>
 
@@ -60,10 +61,12 @@ struct Raw8F32 {
 __device__ __forceinline__ Raw8F32 load8_raw(const float* p) {
   return Raw8F32{reinterpret_cast<const float4*>(p)[0], reinterpret_cast<const float4*>(p)[1]};
 }
+__device__ __forceinline__ u32x4_t load8_raw(const uint16_t* p) { return *reinterpret_cast<const u32x4_t*>(p); }
 __device__ __forceinline__ u32x4_t to_bf16x8(const Raw8F32& r) {
   const float v[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
   return pack8_bf16(v);
 }
+__device__ __forceinline__ u32x4_t to_bf16x8(const u32x4_t& r) { return r; }
 
 typedef short pf_i16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) pf_i16x4_t pf_lds_i16x4_t;
@@ -79,15 +82,15 @@ __device__ __forceinline__ u32x2_t pf_read_tr(uint32_t address) {
 __device__ __forceinline__ u32x4_t pf_read128(uint32_t address) { return *(pf_lds_u32x4_t*)address; }
 #pragma clang diagnostic pop
 
-template <int HD>
-__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __restrict__ q, const float* __restrict__ kcache,
-                                                           const float* __restrict__ vcache, int H, int Hkv, int T,
+template <typename CacheT, int HD>
+__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __restrict__ q, const CacheT* __restrict__ kcache,
+                                                           const CacheT* __restrict__ vcache, int H, int Hkv, int T,
                                                            int start, int max_len, void* __restrict__ out, int out_bf16) {
   static_assert(HD == 128 || HD == 64 || HD == 32, "head_dim 128, 64 or 32");
   constexpr int kPfHD = HD;
   constexpr int RB = 2 * HD;          // bytes of a key (value) row as bf16
   constexpr int C = HD / 8;           // 16-byte chunks per row
-  constexpr int KS = HD / 32;         // k-steps of the first product
+  constexpr int KS = HD / 32;         // k-steps of the first product; also the parts a block's DMA is issued in
   constexpr int TT = HD / 16;         // 32-byte segments per row = 16-dim output tiles
   constexpr int kPfTileBytes = kPfBK * RB;  // one block of keys (or values) as bf16: 16 KiB at HD = 128
   // LDS map (byte addresses relative to lds0, the array's LDS address, which is 0 because the kernel
@@ -122,8 +125,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
   const float qscale =  // log2(e) / sqrt(HD)
       1.4426950408889634f * (HD == 128 ? 0.08838834764831845f : HD == 64 ? 0.125f : 0.17677669529663687f);
 
-  const float* kbase = kcache + ((size_t)b * Hkv + hk) * max_len * kPfHD;
-  const float* vbase = vcache + ((size_t)b * Hkv + hk) * max_len * kPfHD;
+  const CacheT* kbase = kcache + ((size_t)b * Hkv + hk) * max_len * kPfHD;
+  const CacheT* vbase = vcache + ((size_t)b * Hkv + hk) * max_len * kPfHD;
   const int kv_len = start + T;                               // rows the caches hold for this call
   const int kv_end = min(kv_len, start + q0 + kPfBQ);         // keys any row of this workgroup may see
   const int nblk = (kv_end + kPfBK - 1) / kPfBK;
@@ -141,12 +144,37 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
     for (int t = 0; t < TT; ++t) o[u][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
 
-  // ---- Keys and values on their way into LDS: through registers (converted on the way), one block in registers while the
+  // ---- Keys and values on their way into LDS.
+  // bf16 caches: global -> LDS directly, one block ahead.  A wave-wide request fills 1 KiB = 4 key
+  // rows (8 rows at HD = 64); wave w takes rows 4 w .. 4 w + 3 of every group of 16, so (row & 15) = 4 w + lane / 16 is
+  // fixed per lane and the chunk it must fetch for its slot is too.
+  // fp32 caches: through registers (converted on the way), one block in registers while the
   // previous one is being read: chunk ci = tid + 256 i (i < 4) is (key ci / 16, dims 8 (ci % 16) ..).
   // Rows past the filled part of the cache repeat its last row (finite values; those keys are masked).
-  constexpr int kRegParts = kPfBK * C / 256;  // 16-byte chunks of a block per thread: 4 (HD = 128) or 2
-  Raw8F32 kraw[kRegParts], vraw[kRegParts];
-  uint32_t k_st[kRegParts], v_st[kRegParts];
+  constexpr bool kDma = sizeof(CacheT) == 2;
+  constexpr int kReqRows = 1024 / RB;  // key rows of one wave-wide request: 4 (HD = 128) or 8
+  const int krow = kReqRows * wave + lane / C, slot = lane % C;
+  const uint32_t k_chunk = (uint32_t)(slot ^ (krow & (C - 1)));
+  const uint32_t v_chunk = (uint32_t)((((slot >> 1) ^ (krow & (TT - 1))) << 1) | (slot & 1));
+  // part i (0 .. KS - 1) of block jblk: this wave's kReqRows key rows and value rows of the i-th group of 4 * kReqRows
+  auto issue_dma = [&](int jblk, int i) {
+    const int kb0 = jblk * kPfBK;
+    const uint32_t stage = lds0 + (uint32_t)((jblk & 1) * 2 * kPfTileBytes);
+    const uint32_t k_to = stage + (uint32_t)((wave + 4 * i) * 1024), v_to = k_to + (uint32_t)kPfTileBytes;
+    if (kb0 + kPfBK <= kv_len) {
+      const size_t row0 = (size_t)(kb0 + 4 * kReqRows * i) * RB;
+      dma16(reinterpret_cast<const char*>(kbase) + row0, (uint32_t)(krow * RB) + k_chunk * 16u, k_to);
+      dma16(reinterpret_cast<const char*>(vbase) + row0, (uint32_t)(krow * RB) + v_chunk * 16u, v_to);
+    } else {
+      const uint32_t row = (uint32_t)min(kb0 + 4 * kReqRows * i + krow, kv_len - 1) * (uint32_t)RB;
+      dma16(kbase, row + k_chunk * 16u, k_to);
+      dma16(vbase, row + v_chunk * 16u, v_to);
+    }
+  };
+  typedef decltype(load8_raw(kbase)) raw8_t;
+  constexpr int kRegParts = kDma ? 0 : kPfBK * C / 256;  // 16-byte chunks of a block per thread: 4 (HD = 128) or 2
+  raw8_t kraw[kDma ? 1 : kRegParts], vraw[kDma ? 1 : kRegParts];
+  uint32_t k_st[kDma ? 1 : kRegParts], v_st[kDma ? 1 : kRegParts];
   auto fetch = [&](int kb0) {
 #pragma unroll
     for (int i = 0; i < kRegParts; ++i) {
@@ -182,9 +210,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
   for (int t = 0; t < TT; ++t)
     v_rd[t] = lds0 + (uint32_t)(kPfTileBytes + vkey * RB + 32 * (t ^ (vkey & (TT - 1))) + 8 * (r & 3));
 
-  fetch(0);
-  lay_down(0);
-  if (nblk > 1) fetch(kPfBK);
+  if (kDma) {
+#pragma unroll
+    for (int i = 0; i < KS; ++i) issue_dma(0, i);
+  } else {
+    fetch(0);
+    lay_down(0);
+    if (nblk > 1) fetch(kPfBK);
+  }
   // ---- (after the first block's requests, so that both round trips to memory overlap)
   // Q fragments of the wave's two groups of 16 rows: Q[qrow][32 s + 8 g .. + 8), scaled, bf16.
   // Group u of wave w holds rows q0 + 32 w + 16 u .. + 15; this lane's row of it is qrow[u].
@@ -203,14 +236,26 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
       qf[u][s] = pack8_bf16(v);
     }
   }
+  if (kDma) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   for (int j = 0; j < nblk; ++j) {
-    // One barrier per block: block j is complete in stage j & 1 (it was laid down before the previous barrier); block j + 1 goes into
-    // the other stage, which was last read before that barrier too, while block j + 2 starts its flight from memory.
+    // One barrier per block: block j is complete in stage j & 1 (it landed before the previous
+    // barrier); block j + 1 goes into the other stage, which was last read before that barrier
+    // too (fp32 caches: from registers, while block j + 2 starts its flight from memory).
     const int kb0 = j * kPfBK;
-    if (j + 1 < nblk) {
-      lay_down((j + 1) & 1);
-      if (j + 2 < nblk) fetch(kb0 + 2 * kPfBK);
+    // bf16 caches: the requests for block j + 1 are issued between the products below (one part
+    // per k-step), or here by a wave that has no products to form
+    const bool more = j + 1 < nblk;
+    if (more) {
+      if (kDma) {
+        if (kb0 > wave_last_pos) {
+#pragma unroll
+          for (int i = 0; i < KS; ++i) issue_dma(j + 1, i);
+        }
+      } else {
+        lay_down((j + 1) & 1);
+        if (j + 2 < nblk) fetch(kb0 + 2 * kPfBK);
+      }
     }
     // a wave whose last query lies before the block has nothing to add
     if (kb0 <= wave_last_pos) {
@@ -223,13 +268,19 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
       for (int jb = 0; jb < 4; ++jb) ka[jb] = pf_read128(k_rd[0] + (uint32_t)(jb * 16 * RB));
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
+        u32x4_t kn[4];
+        if (kDma && s < KS - 1) {  // (the fp32 path has no registers to spare for a second set)
+#pragma unroll
+          for (int jb = 0; jb < 4; ++jb) kn[jb] = pf_read128(k_rd[s + 1] + (uint32_t)(jb * 16 * RB));
+        }
 #pragma unroll
         for (int jb = 0; jb < 4; ++jb)
 #pragma unroll
           for (int u = 0; u < 2; ++u) sc[u][jb] = mfma16(ka[jb], qf[u][s], s == 0 ? negm[u] : sc[u][jb]);
+        if (kDma && more) issue_dma(j + 1, s);
         if (s < KS - 1) {
 #pragma unroll
-          for (int jb = 0; jb < 4; ++jb) ka[jb] = pf_read128(k_rd[s + 1] + (uint32_t)(jb * 16 * RB));
+          for (int jb = 0; jb < 4; ++jb) ka[jb] = kDma ? kn[jb] : pf_read128(k_rd[s + 1] + (uint32_t)(jb * 16 * RB));
         }
       }
       // only blocks that reach past the wave's first query position need the causal mask
@@ -282,7 +333,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
       // ---- O^T[hd 16 t + 4 g + i][qrow] += sum over the keys of each 32-key half; a value fragment
       // (two transposing reads: the half's first and second 16-key tile) meets both query groups.
       // The second half's fragments are requested as the first half's are consumed.
-      constexpr int kRing = 4;  // fragments in flight
+      constexpr int kRing = kDma ? (TT < 8 ? TT : 8) : 4;  // fragments in flight (the fp32 path has fewer registers to spare)
       auto v_lo = [&](int i) { return pf_read_tr(v_rd[i % TT] + (uint32_t)((i / TT) * 32 * RB)); };
       auto v_hi = [&](int i) { return pf_read_tr(v_rd[i % TT] + (uint32_t)((i / TT) * 32 * RB + 16 * RB)); };
       u32x2_t vlo[kRing], vhi[kRing];
@@ -307,7 +358,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const float* __res
     for (int s = 0; s < KS; ++s) k_rd[s] ^= (uint32_t)(2 * kPfTileBytes);
 #pragma unroll
     for (int t = 0; t < TT; ++t) v_rd[t] ^= (uint32_t)(2 * kPfTileBytes);
-    __syncthreads();  // every wave is done with this block
+    // the next block must have landed and every wave must be done with this one (fp32 caches: the block in registers may still be on its way)
+    if (kDma) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
   }
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
@@ -346,12 +399,25 @@ __global__ __launch_bounds__(256) void caches_to_bf16_kernel(const float* __rest
 // vector work to issue side by side instead of one after the other, and two waves per SIMD fill what is left.  Before, each wave went through
 // product, softmax and product in turn and a CU's two workgroups overlapped by chance: 3440 cycles per 64 keys and two waves, 2730 now (64 MFMAs a
 // wave are 2048).  What bounds it is the clock (2.19 -> 1.95 GHz as the matrix pipes fill).  B = 4, 32 / 8 heads, T = 2048: 164 -> 152 us alone, 171 -> 155
-// in a row; a few short grids, where a wave's own length counts: 0.79 .. 0.9 of the time; heads of 64: 0.92, of 32: 0.98.
+// in a row; a few short grids, where a wave's own length counts: 0.79 .. 0.9 of the time.
 //
 // Keys run a step ahead of the values, so key block j + 2 and value block j + 1 are asked for in the second step of block j, behind the one
 // barrier per block: every wave has consumed what lay there (keys of block j, values of block j - 1), and what it
 // reads next (keys j + 1, values j) was asked for a block before and waited for in front of that barrier.
 // Four steps at places known to the compiler make the body; a wave's last ones (masked, or with blocks cut short) go one by one.
+//
+// prefill_in_steps: which bf16 calls it takes (figures: its time over attn_prefill_kernel's).  Heads of 128 all (78 shapes: 0.83 .. 1.03).  Narrower ones have
+// few MFMAs in a step beside its latency, so short prompts are faster in whole blocks: 64 columns 1.03 .. 1.09 at 40 .. 64 keys, 0.99 / 1.09 at 100, 1.03 at
+// 192, 1.00 at 256, 0.93 at 512, 0.79 at 4096 with few workgroups; with more than a round of them from 128 on (200 keys: 0.98), over 194 shapes 0.93 (left: 1.05 where rounds come
+// out even, 1024 workgroups of 4096 queries).  32 columns: 1.04 ..
+// 1.10 up to 256, 0.985 at 333, 0.96 at 512 and 0.83 at 4096 while two workgroups a CU hold the launch; beyond, the exponentials bound both and the
+// steps' share of vector work is the larger (768 workgroups and more: 1.01 .. 1.05; 384 of 312 queries 1.04, 512 of 900 0.91).
+__host__ __device__ inline bool prefill_in_steps(long long heads, int T, int start, int head_dim) {
+  const long long workgroups = heads * ((T + kPfBQ - 1) / kPfBQ), keys = (long long)start + T;
+  if (head_dim == 128) return true;
+  if (head_dim == 64) return keys >= 256 || (keys > 128 && workgroups > 256);
+  return keys > 320 && (workgroups <= 256 || (workgroups <= 512 && T >= 600));
+}
 template <int HD>
 __global__ __launch_bounds__(256, 2) void attn_prefill_steps_kernel(const float* __restrict__ q, const uint16_t* __restrict__ kcache,
                                                                  const uint16_t* __restrict__ vcache, int H, int Hkv, int T,

@@ -341,6 +341,8 @@ int ajq_swiglu(const float* ab, uint16_t* out, int B, int F, void* stream);
  * the benchmark models and of the reference's configs/models/transformer_medium.yaml and transformer_baseline.yaml). */
 int ajq_attn_prefill(const float* q, const void* kcache, const void* vcache, int cache_dtype, int B, int H,
                      int Hkv, int T, int start, int max_len, int head_dim, void* out, int out_dtype, void* stream);
+/* 1 where bf16 caches (or a bf16 copy) are walked in half blocks, 0 block by block, -1 if no such call is built */
+int ajq_attn_prefill_steps(int B, int H, int T, int start, int head_dim);
 /* The same with a workspace for a bf16 copy of fp32 caches (the same roundings): ajq_attn_prefill_workspace says how many bytes make
  * it faster, 0 for none.  Less than that, or NULL, is ajq_attn_prefill. */
 size_t ajq_attn_prefill_workspace(int cache_dtype, int B, int H, int Hkv, int T, int start, int head_dim);

@@ -281,3 +281,12 @@ def test_a_layer_does_without_the_extension_module(monkeypatch):
     assert first() is None and quant._linear is first
     with pytest.raises(RuntimeError, match="ajllm_amd.build"):
         _lib.load_native()
+
+
+@pytest.mark.parametrize("b,heads,t,start,hd,steps", [
+    (1, 8, 1, 0, 128, 1), (64, 64, 4096, 0, 128, 1), (1, 8, 255, 0, 64, 0), (1, 8, 1, 255, 64, 1), (16, 16, 129, 0, 64, 1), (16, 16, 128, 0, 64, 0), (8, 16, 200, 0, 64, 0),
+    (8, 32, 200, 0, 64, 1), (1, 8, 320, 0, 32, 0), (1, 8, 321, 0, 32, 1), (8, 32, 128, 300, 32, 1), (9, 32, 128, 300, 32, 0), (1, 32, 2048, 0, 32, 1), (1, 32, 2049, 0, 32, 0),
+    (4, 64, 200, 0, 32, 0), (1, 8, 8, 0, 48, -1), (0, 8, 8, 0, 64, -1),
+])
+def test_which_prompts_are_walked_in_half_blocks(b, heads, t, start, hd, steps):
+    assert _lib.load().ajq_attn_prefill_steps(b, heads, t, start, hd) == steps

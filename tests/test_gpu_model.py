@@ -652,6 +652,14 @@ def test_flash_prefill_on_bf16_caches_at_the_edges_of_its_steps(cuda, t, start, 
     assert errors(got, want.cpu())[1] <= 4e-3
 
 
+@pytest.mark.parametrize("hd", [64, 32])
+@pytest.mark.parametrize("t,start", [(1, 320), (31, 225), (31, 321), (33, 289), (64, 257), (95, 161), (97, 520), (129, 255), (191, 321), (256, 65), (321, 0), (384, 2), (449, 319)])
+def test_flash_prefill_of_narrow_heads_in_half_blocks(cuda, t, start, hd):
+    """The same from where narrow heads are walked in steps (257 keys here and fewer with 32 columns are not)."""
+    assert _lib.load().ajq_attn_prefill_steps(2, 4, t, start, hd) == (start + t > 320 or hd == 64)
+    test_flash_prefill_on_bf16_caches_at_the_edges_of_its_steps(cuda, t, start, hd)
+
+
 @pytest.mark.parametrize("hd", [128, 64])
 @pytest.mark.parametrize("b,heads,kv_heads,t,start", [(16, 64, 1, 128, 901), (2, 32, 2, 2047, 0), (1, 64, 4, 1500, 1), (3, 96, 3, 513, 700)])
 def test_flash_prefill_on_a_copy_of_fp32_caches(cuda, b, heads, kv_heads, t, start, hd):
