@@ -987,14 +987,21 @@ int launch_gemv_norm_cfg(int M, int K, const uint32_t* wq, const uint32_t* meta,
                      M | (out_f32 << 8), N, y, scales8, h, ssq, gain, eps, parts);
   return AJQ_OK;
 }
-// Tiles per workgroup: up to three rounds of the CUs in one; beyond, several workgroups share a CU and their number counts, the more the more rows there
-// are to norm.  Rows of 4096 int8 weights fill the registers (28672 columns, 1 row: 19.2 us with one tile, 22.0 with two).
+// Tiles per workgroup.  Up to three rounds of the CUs in one; beyond, several workgroups share a CU and their rounds count: four tiles, and three where
+// that takes no more rounds (K = 2048, 4 rows, three / four: 1212 tiles int8 9.5 / 11.0 us, int4 7.4 / 8.45; 1700 tiles int8 12.8 / 11.7;
+// 2300 int4 10.4 / 11.2).  One row asks for little norm: two (int4 1700 tiles 0.96 of the time with one, with three 1.01), three in those cases (int8 K =
+// 2048, 1400 tiles: 8.8 us, 9.5 with two), and with int8 rows of 2048 one past 1024 tiles (0.99, with two 1.02 .. 1.05).  int8 rows of 4096 fill the
+// registers and gain from sharing the norm only while the last round of single tiles is up to two thirds full (one row, two tiles over one: 320
+// tiles 0.91, 384 0.96, 448 1.00, 512 1.02; three: 576 0.94, 640 0.99, 752 1.04); past three rounds never (1400 tiles: 1.08), int4 ones by two.
 template <bool kW4>
 int gemv_norm_tiles(int M, int K, int tiles) {
   const int rounds = (tiles + 255) / 256;
+  if (!kW4 && K == 4096 && M == 1 && tiles - 256 * (rounds - 1) > 170) return 1;
   if (rounds <= 3) return rounds;
   if (K == 4096) return kW4 ? 2 : 1;
-  return M == 1 ? 2 : 4;
+  if ((tiles + 767) / 768 == (tiles + 1023) / 1024) return 3;
+  if (M > 1) return 4;
+  return kW4 || K == 1024 || tiles <= 1024 ? 2 : 1;
 }
 // One tile of three or four rows: without holding the sums (gemv_fused_kernels.h; 2048 x 2048, 4 rows: 3.6 us, 3.9 here), but for long int8 rows (4096
 // columns: 5.6 us there, 5.2 here).
@@ -1307,6 +1314,12 @@ int ajq_w4a16_gemv_gated(const uint16_t* x, int M, int K, const uint32_t* wq, co
 int ajq_w8a16_gemv_gated(const uint16_t* x, int M, int K, const uint32_t* wq, const uint16_t* scales, int N, void* y,
                          void* stream) {
   return gemv_gated<false>("ajq_w8a16_gemv_gated", x, M, K, wq, scales, N, y, stream);
+}
+
+int ajq_gemv_norm_sums_tiles(int M, int K, int N, int w4) {
+  if (!gemv_pro_supported(M, K) || K > 4096 || N < kTileN || N % kTileN != 0) return -1;
+  if (w4 ? !gemv_norm_few_rows<true>(M, K, N) : !gemv_norm_few_rows<false>(M, K, N)) return 0;
+  return w4 ? gemv_norm_tiles<true>(M, K, N / kTileN) : gemv_norm_tiles<false>(M, K, N / kTileN);
 }
 
 int ajq_w4a16_gemv_norm_sums(const float* h, const float* ssq, int parts, const float* gain, float eps, int M, int K,

@@ -190,6 +190,8 @@ int ajq_w4a16_gemv_norm_sums(const float* h, const float* ssq, int parts, const 
 int ajq_w8a16_gemv_norm_sums(const float* h, const float* ssq, int parts, const float* gain, float eps, int M, int K,
                              const uint32_t* wq, const uint16_t* scales, int N, void* y, int out_dtype, int gate,
                              void* stream);
+/* row tiles per workgroup that these take; 0: the kernel without tiles, -1: not built */
+int ajq_gemv_norm_sums_tiles(int M, int K, int N, int w4);
 /*   _merge_residual: _residual whose x is the single-query attention output merged from the S partial results
  *              per (row, head) in ajq_attn_step_partial's workspace, as in _merge below (same limits:
  *              ajq_gemv_merge_max_splits): the output projection of a decode step at small batch, with the

@@ -290,3 +290,14 @@ def test_a_layer_does_without_the_extension_module(monkeypatch):
 ])
 def test_which_prompts_are_walked_in_half_blocks(b, heads, t, start, hd, steps):
     assert _lib.load().ajq_attn_prefill_steps(b, heads, t, start, hd) == steps
+
+
+@pytest.mark.parametrize("m,k,tiles,w4,want", [  # rows, columns, row tiles: tiles a workgroup takes in int4 and in int8
+    (1, 2048, 256, 1, 1), (1, 2048, 257, 2, 2), (4, 1024, 768, 3, 3), (4, 1024, 769, 4, 4), (2, 2048, 1024, 4, 4), (2, 2048, 1025, 3, 3), (4, 2048, 1536, 3, 3),
+    (3, 1024, 1537, 4, 4), (4, 2048, 2049, 3, 3), (1, 2048, 1024, 2, 2), (1, 2048, 1025, 3, 3), (1, 2048, 1537, 2, 1), (1, 1024, 1537, 2, 2), (1, 4096, 426, 2, 2),
+    (1, 4096, 427, 2, 1), (1, 4096, 170, 1, 1), (1, 4096, 256, 1, 1), (1, 4096, 682, 3, 3), (1, 4096, 683, 3, 1), (2, 4096, 768, 3, 3), (2, 4096, 769, 2, 1), (3, 2048, 256, 0, 0), (4, 4096, 100, 0, 1),
+    (5, 2048, 400, 0, 0), (1, 5632, 100, -1, -1), (17, 1024, 100, -1, -1),
+])
+def test_row_tiles_of_a_norm_from_its_sums(m, k, tiles, w4, want):
+    lib = _lib.load()
+    assert (lib.ajq_gemv_norm_sums_tiles(m, k, 16 * tiles, 1), lib.ajq_gemv_norm_sums_tiles(m, k, 16 * tiles, 0)) == (w4, want)

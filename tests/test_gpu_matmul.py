@@ -642,6 +642,13 @@ def test_norm_from_sums_of_neighbouring_tiles(cuda, scheme, m, d, n2):
 
 
 @pytest.mark.parametrize("scheme", ["w4", "w8"])
+@pytest.mark.parametrize("m,d,n2", [(1, 2048, 16400), (4, 1024, 16400), (2, 2048, 24592), (1, 2048, 24592), (3, 2048, 32800), (1, 4096, 6816), (1, 4096, 6832), (1, 4096, 10928)])
+def test_norm_from_sums_past_a_round_of_shared_tiles(cuda, scheme, m, d, n2):
+    """Where three tiles take no more rounds than four, and where one row of long or many int8 tiles shares none."""
+    test_gemv_residual_then_rowscale_against_the_oracle(cuda, scheme, m, 1024, d, n2)
+
+
+@pytest.mark.parametrize("scheme", ["w4", "w8"])
 @pytest.mark.parametrize("k,n", [(1024, 48), (2048, 48), (2048, 8208)])
 def test_norm_from_sums_adds_in_one_order(cuda, scheme, k, n):
     """One row's four waves add up in the order of two rows' eight: the same bits (the rows' sums of squares are whole numbers, so
