@@ -54,7 +54,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_norm_kernel(
   }
 #pragma unroll
   for (int t = 0; t < T; ++t) {
-    const size_t at = (size_t)min(nt0 + t, tiles - 1) * G + g0;
+    const size_t at = (size_t)(T > 1 ? min(nt0 + t, tiles - 1) : nt0) * G + g0;
     if (kW4) {
 #pragma unroll
       for (int p = 0; p < TPW; ++p) mw[t][p] = meta[(at + p) * 16 + nl];
@@ -66,7 +66,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_norm_kernel(
       for (int q = 0; q < kLoadsPerGroup; ++q) w[t][p][q] = __builtin_nontemporal_load(wtile + (p * kLoadsPerGroup + q) * 64);
   }
   uint32_t scale_bits = 0;
-  if (!kW4) scale_bits = scales8[min(nt0 + min(wave, T - 1), tiles - 1) * kTileN + nl];
+  if (!kW4) scale_bits = scales8[(T > 1 ? min(nt0 + min(wave, T - 1), tiles - 1) : nt0) * kTileN + nl];
   __builtin_amdgcn_sched_barrier(0);
   // ---- a row's total in all of its lanes: the kLanesPerRow lanes of a row share the parts
   float total = 0.f;
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_norm_kernel(
   if (!kW4) asm volatile("" : "+v"(scale_bits));
   __syncthreads();
   const int nt = nt0 + wave;
-  if (wave >= T || nt >= tiles || kc >= kRowQuads) return;
+  if (wave >= T || (T > 1 && nt >= tiles) || kc >= kRowQuads) return;
   live_t sum = redv[wave * kParts * (16 * kRowQuads) + lane];
 #pragma unroll
   for (int u = 1; u < kParts; ++u) sum += redv[(wave * kParts + u) * (16 * kRowQuads) + lane];
