@@ -902,7 +902,9 @@ int launch_gemv_pro(int M, int K, const uint32_t* wq, const uint32_t* meta, cons
   }
   if (K == 4096 || kPro == kProNormSums) {
     AJQ_PRO_ROW(8, 4)
-    if (M <= 4) AJQ_PRO(8, 4, 4);
+    if constexpr (kW4 || kPro != kProNormSums) {  // (up to four int8 rows: gemv_norm_few_rows)
+      if (M <= 4) AJQ_PRO(8, 4, 4);
+    }
     AJQ_PRO(8, 4, 8);
   }
   if constexpr (kPro != kProNormSums) {
@@ -1016,13 +1018,15 @@ int launch_gemv_norm(int M, int K, const uint32_t* wq, const uint32_t* meta, con
   auto go = [&](auto waves, auto tpw, auto rows, auto t) {
     return launch_gemv_norm_cfg<waves(), tpw(), rows(), t(), kW4, kGate>(M, K, wq, meta, scales8, N, y, out_f32, h, ssq, gain, eps, parts, stream);
   };
-  auto by_tiles = [&](auto waves, auto tpw, auto rows) {
-    switch (tiles) {
-      case 1: return go(waves, tpw, rows, Int<1>{});
-      case 2: return go(waves, tpw, rows, Int<2>{});
-      case 3: return go(waves, tpw, rows, Int<3>{});
-      default: return go(waves, tpw, rows, Int<4>{});
+  auto by_tiles = [&](auto tpw, auto rows) {  // (what gemv_norm_tiles and gemv_norm_few_rows say, and no more)
+    constexpr bool kOne = rows() < 4 ? rows() == 2 || tpw() == 4 : !kW4 && tpw() == 4, kFour = rows() > 1 && tpw() < 4;
+    if constexpr (kOne) {
+      if (tiles == 1) return go(Int<8>{}, tpw, rows, Int<1>{});
     }
+    if constexpr (kFour) {
+      if (tiles == 4) return go(Int<8>{}, tpw, rows, Int<4>{});
+    }
+    return tiles == 2 ? go(Int<8>{}, tpw, rows, Int<2>{}) : go(Int<8>{}, tpw, rows, Int<3>{});
   };
   auto by_rows = [&](auto tpw) {
     if (M == 1) {
@@ -1031,9 +1035,9 @@ int launch_gemv_norm(int M, int K, const uint32_t* wq, const uint32_t* meta, con
       if constexpr (tpw() < 4) {
         if (tiles == 1) return go(Int<4>{}, Int<2 * tpw()>{}, Int<1>{}, Int<1>{});
       }
-      return by_tiles(Int<8>{}, tpw, Int<1>{});
+      return by_tiles(tpw, Int<1>{});
     }
-    return M == 2 ? by_tiles(Int<8>{}, tpw, Int<2>{}) : by_tiles(Int<8>{}, tpw, Int<4>{});
+    return M == 2 ? by_tiles(tpw, Int<2>{}) : by_tiles(tpw, Int<4>{});
   };
   return K == 1024 ? by_rows(Int<1>{}) : K == 2048 ? by_rows(Int<2>{}) : by_rows(Int<4>{});
 }

@@ -136,6 +136,7 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
     }
   }
   // kProNormSums: the 64 / MROWS lanes of a row share the parts of its sum of squares
+  static_assert(kPro != kProNormSums || MROWS >= 4, "fewer rows: gemv_norm_kernels.h");
   constexpr int kLanesPerRow = 64 / MROWS;
   constexpr int kPartLoads = kPro == kProNormSums ? (64 + kLanesPerRow - 1) / kLanesPerRow : 1;  // up to 256 parts
   float4 sums[kPartLoads];
@@ -218,10 +219,8 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
 #pragma unroll
     for (int u = 0; u < kPartLoads; ++u)
       total += (sums[u].x + sums[u].y) + (sums[u].z + sums[u].w);
-    if (kLanesPerRow >= 16) {
-      total = team_sum16(total);  // DPP row rotates inside each 16 lanes, then lane swaps for whole rows of 16
-      if (kLanesPerRow == 64) total = quad_sum(total);
-      else if (kLanesPerRow == 32) total += __shfl_xor(total, 16);
+    if (kLanesPerRow == 16) {
+      total = team_sum16(total);  // DPP row rotates inside each 16 lanes
     } else {
 #pragma unroll
       for (int off = kLanesPerRow / 2; off > 0; off >>= 1) total += __shfl_xor(total, off);
