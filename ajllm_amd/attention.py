@@ -15,7 +15,7 @@ import torch
 from . import _lib
 
 _HERE = nullcontext()
-COPIED_WORK = 3.6e9   # half the FLOP below which ajq_attn_prefill_workspace says 0: short calls are not asked
+COPIED_WORK = 3.6e9   # half the FLOP below which ajq_attn_prefill_workspace says 0 (tests/test_modeling.py): short calls are not asked
 
 
 def flash_prefill(q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, start: int,

@@ -275,3 +275,43 @@ def test_token_file_windows_and_evaluation(tmp_path):
     assert abs(got["perplexity"] - math.exp(got["loss"])) < 1e-9
     with pytest.raises(ValueError):
         evaluation.evaluate_model(model, data, 0, 2, 8, "cpu", 9)
+
+
+# ------------------------------------------------------------------ a bf16 copy of fp32 caches for prompt attention
+def test_calls_that_are_not_asked_for_a_copy_take_none():
+    """Below COPIED_WORK (batch x heads x queries x (2 start + queries) x columns) the library never says that a copy pays."""
+    from ajllm_amd import _lib
+    from ajllm_amd.attention import COPIED_WORK
+    lib, took = _lib.load(), 0
+    for hd in (128, 64, 32):
+        for heads in (1, 2, 7, 16, 33, 64, 128):
+            for start in (0, 1, 100, 3000):
+                t = int(((start * start + COPIED_WORK / (heads * hd)) ** 0.5) - start)   # the most queries that stay below
+                while t > 0 and heads * t * (2 * start + t) * hd > COPIED_WORK:
+                    t -= 1
+                for kv_heads in {1, heads}:
+                    if t > 0:
+                        assert lib.ajq_attn_prefill_workspace(_lib.AJQ_KV_F32, 1, heads, kv_heads, t, start, hd) == 0, (heads, kv_heads, t, start, hd)
+                    took += lib.ajq_attn_prefill_workspace(_lib.AJQ_KV_F32, 1, heads, 1, t + t // 8 + 8, start, hd) > 0
+    assert took > 0
+
+
+def test_prompt_attention_without_memory_for_a_copy(monkeypatch):
+    """No memory for the copy: the kernel that needs none, with the same arguments; a copy's room otherwise."""
+    from types import SimpleNamespace
+
+    from ajllm_amd import _lib, attention
+    calls = []
+    lib = SimpleNamespace(ajq_attn_prefill=lambda *a: calls.append(("plain", a)) or 0, ajq_attn_prefill_in=lambda *a: calls.append(("copy", a)) or 0,
+                          ajq_attn_prefill_workspace=lambda *a: 4096)
+    monkeypatch.setattr(_lib, "load", lambda: lib)
+    q, keys, values, out = (torch.zeros(16) for _ in range(4))
+    run = lambda flag, seq: attention.prefill_attention(q, keys, values, flag, 4, 32, 8, seq, 0, seq, 128, out, 0, 7)
+    assert run(_lib.AJQ_KV_F32, 2048) == 0 and calls[-1][0] == "copy" and calls[-1][1][-2:] == (4096, 7)
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: (_ for _ in ()).throw(torch.OutOfMemoryError()) if k.get("dtype") == torch.uint8 else empty(*a, **k))
+    assert run(_lib.AJQ_KV_F32, 2048) == 0 and calls[-1][0] == "plain" and calls[-1][1][:3] == (q.data_ptr(), keys.data_ptr(), values.data_ptr())
+    monkeypatch.undo()
+    monkeypatch.setattr(_lib, "load", lambda: lib)
+    assert run(_lib.AJQ_KV_BF16, 2048) == 0 and calls[-1][0] == "plain"
+    assert run(_lib.AJQ_KV_F32, 64) == 0 and calls[-1][0] == "plain"
