@@ -1017,6 +1017,29 @@ int ajqd_scan_in_parts(const ajqd_scan_args* a, int parts, float* workspace, int
                             : launch_scan_parts<float, 4>(s, a->batch, count, cut, (hipStream_t)stream);
 }
 
+// scan_project: the smallest block that holds a part; two row tiles, which share the convolution, where single ones are more than one a CU
+struct ScanCut {
+  int kb, rt;
+};
+static ScanCut scan_cut(int batch, int inner, int rows, int splits) {
+  const int part = 32 * (((inner + 31) / 32 + splits - 1) / splits);
+  const long long tiles = (long long)(rows / 16) * splits * ((batch + kGemvBatch - 1) / kGemvBatch);
+  return ScanCut{part <= scan_block(2) ? 2 : part <= scan_block(4) ? 4 : 8, tiles > kCus && rows >= 32 ? 2 : 1};
+}
+// scan_step: sequences a workgroup of the wide kernel, 0 for the narrow one (a workgroup per CU).  Four sequences a workgroup fill the chip, eight read
+// the weights and decays less often: four while every workgroup finds room at once, three to a CU (four / eight: 24 of 8192 channels 12.7 / 13.8
+// us, 32 of 4096 9.3 / 11.0; 32 of 8192 19.2 / 16.7, 64 of 4096 16.1 / 15.3)
+static int scan_step_batch(int batch, int inner, int rank) {
+  if (rank <= kNarrowRank && (long long)(inner / 16) * ((batch + kNarrowBatch - 1) / kNarrowBatch) <= kCus) return 0;
+  return (long long)((inner + 63) / 64) * ((batch + 3) / 4) > 3 * kCus ? 8 : 4;
+}
+
+int ajqd_scan_form(int batch, int inner, int rows, int splits, int rank) {
+  if (batch < 1 || inner < 16 || inner % 16 || rows < 16 || rows % 16 || splits < 1 || rank < 8) return 0;
+  const ScanCut c = scan_cut(batch, inner, rows, splits);
+  return 1000 * c.kb + 100 * c.rt + 10 * (rows / 16 % 2) + scan_step_batch(batch, inner, rank);
+}
+
 // Parts of the projection: what smaller blocks save in scan_project_kernel, the step's kernel pays in parts (0.04 us a part at
 // 4 sequences, 0.15 at 16 of 8192 channels, 0.13 at 64 of 4096).  Both launches with blocks of 1024 / 512 / 256: 4 sequences
 // of 4096 channels 9.6 / 8.5 / 8.3 us, 16: 15.2 / 12.2 / 11.2, 64: 22.5 / 20.1 / 21.0; 5120, 12: 14.1 / 12.0 / 11.6; 8192, 1: 10.6 / 10.9 / 11.5,
@@ -1033,10 +1056,8 @@ int ajqd_scan_project(const float* y, int ldy, const void* ring, const float* we
   if (batch < 1 || inner < 8 || inner % 8 || taps < 1 || rows < 16 || rows % 16 || splits < 1 || splits > 65535 || ldy < 2 * inner || ldy % 4)
     return fail(AJQ_ERR_SHAPE, "ajqd_scan_project: unsupported shape (batch=%d inner=%d taps=%d rows=%d splits=%d)", batch, inner, taps, rows, splits);
   ScanProject p{y, (const uint16_t*)ring, weight, bias, positions64(pos), (const uint16_t*)w, partial, batch, ldy, inner, taps, rows, splits};
-  // the smallest block that holds a part; two row tiles, which share the convolution, where single ones are more than one a CU
-  const int part = 32 * (((inner + 31) / 32 + splits - 1) / splits), kb = part <= scan_block(2) ? 2 : part <= scan_block(4) ? 4 : 8;
-  const long long tiles = (long long)(rows / 16) * splits * ((batch + kGemvBatch - 1) / kGemvBatch);
-  const int rt = tiles > 256 && rows >= 32 ? 2 : 1;
+  const ScanCut c = scan_cut(batch, inner, rows, splits);
+  const int kb = c.kb, rt = c.rt;
   const dim3 grid((rows / 16 + rt - 1) / rt, splits, (batch + kGemvBatch - 1) / kGemvBatch);
   auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, p); };
   auto with = [&](auto steps) {
@@ -1064,11 +1085,11 @@ int ajqd_scan_step(const ajqd_scan_step_args* a, void* stream) {
     hipLaunchKernelGGL(kernel, dim3((a->inner + channels - 1) / channels, (a->batch + bb - 1) / bb), dim3(256), bytes, (hipStream_t)stream, s);
     return check_launch("ajqd_scan_step");
   };
-  if (a->rank <= kNarrowRank && (long long)(a->inner / 16) * ((a->batch + kNarrowBatch - 1) / kNarrowBatch) <= 256)  // (a workgroup per CU)
-    return go(scan_step_narrow_kernel, 16, kNarrowBatch);
-  // four sequences a workgroup fill the chip, eight read the weights and decays less often: four while every workgroup finds room at once,
-  // three to a CU (four / eight: 24 of 8192 channels 12.7 / 13.8 us, 32 of 4096 9.3 / 11.0; 32 of 8192 19.2 / 16.7, 64 of 4096 16.1 / 15.3)
-  return (long long)((a->inner + 63) / 64) * ((a->batch + 3) / 4) > 3 * 256 ? go(scan_step_kernel<8>, 64, 8) : go(scan_step_kernel<4>, 64, 4);
+  switch (scan_step_batch(a->batch, a->inner, a->rank)) {
+    case 0: return go(scan_step_narrow_kernel, 16, kNarrowBatch);
+    case 4: return go(scan_step_kernel<4>, 64, 4);
+    default: return go(scan_step_kernel<8>, 64, 8);
+  }
 }
 
 }  // extern "C"

@@ -504,12 +504,26 @@ def test_decode_step_of_the_scan(cuda, shape):
         assert _rel(torch.stack([o[b] for o in got]), want) < 2e-2 and _rel(state[b], hybrid.state_planes(end)) < 2e-2
 
 
-@pytest.mark.parametrize("shape", [  # batch, inner, states, rank, taps
+SCAN_FORMS = [  # batch, inner, states, rank, taps: with STEPS and SCAN_LINES every form of both kernels (tests/test_hybrid.py counts them)
+    # two row tiles on blocks of 256, 512 and 1024 channels, an odd and an even number of them, four taps and others, eight sequences a workgroup
+    (32, 4096, 16, 128, 4), (29, 4096, 16, 112, 3), (16, 8192, 16, 256, 4), (17, 8192, 4, 256, 5), (27, 8192, 16, 256, 4), (25, 8192, 8, 256, 2), (51, 4096, 4, 128, 4),
+]
+
+
+@pytest.mark.parametrize("shape", SCAN_FORMS)
+def test_decode_step_of_the_scan_on_many_row_tiles(cuda, shape):
+    test_decode_step_of_the_scan(cuda, shape)
+
+
+SCAN_LINES = [  # batch, inner, states, rank, taps
     # 16 channels a workgroup: a workgroup per CU and one too many, ranks at and past its last, one plane of states, five, seven taps, none kept
     (4, 4096, 16, 128, 4), (5, 4096, 16, 128, 4), (2, 1024, 16, 128, 3), (2, 1024, 16, 136, 4), (2, 272, 4, 8, 4), (3, 144, 20, 24, 7), (6, 96, 12, 16, 1),
-    # blocks of 256, 512 and 1024 channels, parts that end inside one, one and two row tiles, four and eight sequences
+    # blocks of 256, 512 and 1024 channels, parts that end inside one, one row tile, four sequences
     (2, 5120, 16, 8, 4), (1, 5136, 16, 8, 4), (9, 5136, 8, 8, 4), (33, 1040, 16, 32, 4), (33, 272, 8, 120, 2), (2, 16400, 4, 8, 3),
-])
+]
+
+
+@pytest.mark.parametrize("shape", SCAN_LINES)
 def test_decode_step_of_the_scan_at_the_lines_of_its_kernels(cuda, shape):
     test_decode_step_of_the_scan(cuda, shape)
 

@@ -291,6 +291,15 @@ def test_dense_library_refuses_bad_arguments_before_any_launch():
     assert lib.ajqd_scan_step(ctypes.byref(step), None) == -2                                            # 8 + 16 rows in 16
 
 
+def test_every_form_of_a_decode_step_of_the_scan_is_run():
+    from tests.test_gpu_hybrid import SCAN_FORMS, SCAN_LINES, STEPS
+    lib, up = _lib.load_dense(), lambda n: -(-n // 16) * 16
+    form = lambda batch, inner, states, rank, taps: (lib.ajqd_scan_form(batch, inner, up(rank + 2 * states), lib.ajqd_scan_splits(batch, inner), rank), taps == 4)
+    got = {form(*s) for s in STEPS + SCAN_LINES + SCAN_FORMS}
+    assert {(f // 100, four) for f, four in got} == {(10 * kb + rt, four) for kb in (2, 4, 8) for rt in (1, 2) for four in (True, False)}
+    assert {f % 10 for f, _ in got} == {0, 4, 8} and {f // 10 % 10 for f, _ in got if f // 100 % 10 == 2} == {0, 1}
+
+
 def test_every_form_of_a_decode_product_is_run():
     """The shapes that the GPU test runs reach every form of a product without many streams that the library holds."""
     from tests.test_gpu_hybrid import FORMS
