@@ -47,7 +47,9 @@
 namespace ajq {
 
 constexpr float kPfSlack = 8.0f;          // log2 of how far a row's exponents may exceed its reference point
-constexpr float kPfTrigger = 4096.0f;     // lane sum of 16 probabilities above which the reference point is revisited
+// A lane's sum of new probabilities above which the reference point is revisited.  Up to there none of them passes 2^12; above, the largest of
+// a block's 16 passes 2^8, of a step's 8 (attn_prefill_steps_kernel) 2^9, so that the revisit always finds one past the slack.
+constexpr float kPfTrigger = 4096.0f;
 constexpr int kPfBQ = 128, kPfBK = 64;
 
 __device__ __forceinline__ u32x4_t pack8_bf16(const float* v) {
