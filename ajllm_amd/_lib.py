@@ -266,7 +266,7 @@ DENSE_SIGNATURES: dict[str, tuple] = {
     "ajqd_scan_in_parts": (c_int, [ctypes.POINTER(ScanArgs), _I, _P, _I, _P]),
     "ajqd_scan_splits": (c_int, [_I, _I]),
     "ajqd_scan_project": (c_int, [_P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
-    "ajqd_scan_form": (c_int, [_I, _I, _I, _I, _I]),
+    "ajqd_scan_form": (c_int, [_I, _I, _I, _I, _I, _I]),
     "ajqd_scan_step": (c_int, [ctypes.POINTER(ScanStepArgs), _P]),
 }
 

@@ -1026,26 +1026,30 @@ static ScanCut scan_cut(int batch, int inner, int rows, int splits) {
   const long long tiles = (long long)(rows / 16) * splits * ((batch + kGemvBatch - 1) / kGemvBatch);
   return ScanCut{part <= scan_block(2) ? 2 : part <= scan_block(4) ? 4 : 8, tiles > kCus && rows >= 32 ? 2 : 1};
 }
-// scan_step: sequences a workgroup of the wide kernel, 0 for the narrow one (a workgroup per CU).  Four sequences a workgroup fill the chip, eight read
-// the weights and decays less often: four while every workgroup finds room at once, three to a CU (four / eight: 24 of 8192 channels 12.7 / 13.8
-// us, 32 of 4096 9.3 / 11.0; 32 of 8192 19.2 / 16.7, 64 of 4096 16.1 / 15.3)
-static int scan_step_batch(int batch, int inner, int rank) {
+// scan_step: sequences a workgroup of the wide kernel, 0 for the narrow one (a workgroup per CU).  Eight read the weights and decays less often, four
+// carry half a lane's chain.  Three workgroups of four find room on a CU, two of eight: eight where they take one round instead of two (us with four /
+// eight: 24 of 8192 channels 12.7 / 13.8; 13 of 13440 13.3 / 11.6, 33 of 6672 with 64 states 28.3 / 25.4; 16 of 17360 18.2 / 20.5, 13 of
+// 18576 with 64 states 48.4 / 61.9) and past two rounds of four (31 of 13440 33.6 / 30.3, 33 of 13744 33.6 / 30.1), unless there are many states, which lie
+// in a lane's chain (64 states, 64 of 9664: 89 / 100; 48 of 6992: 48 / 63).
+static int scan_step_batch(int batch, int inner, int rank, int states) {
   if (rank <= kNarrowRank && (long long)(inner / 16) * ((batch + kNarrowBatch - 1) / kNarrowBatch) <= kCus) return 0;
-  return (long long)((inner + 63) / 64) * ((batch + 3) / 4) > 3 * kCus ? 8 : 4;
+  const long long fours = (long long)((inner + 63) / 64) * ((batch + 3) / 4);
+  return (fours > 3 * kCus && fours <= 4 * kCus) || (fours > 6 * kCus && states <= 32) ? 8 : 4;
 }
 
-int ajqd_scan_form(int batch, int inner, int rows, int splits, int rank) {
-  if (batch < 1 || inner < 16 || inner % 16 || rows < 16 || rows % 16 || splits < 1 || rank < 8) return 0;
+int ajqd_scan_form(int batch, int inner, int rows, int splits, int rank, int states) {
+  if (batch < 1 || inner < 16 || inner % 16 || rows < 16 || rows % 16 || splits < 1 || rank < 8 || states < 4) return 0;
   const ScanCut c = scan_cut(batch, inner, rows, splits);
-  return 1000 * c.kb + 100 * c.rt + 10 * (rows / 16 % 2) + scan_step_batch(batch, inner, rank);
+  return 1000 * c.kb + 100 * c.rt + 10 * (rows / 16 % 2) + scan_step_batch(batch, inner, rank, states);
 }
 
 // Parts of the projection: what smaller blocks save in scan_project_kernel, the step's kernel pays in parts (0.04 us a part at
 // 4 sequences, 0.15 at 16 of 8192 channels, 0.13 at 64 of 4096).  Both launches with blocks of 1024 / 512 / 256: 4 sequences
 // of 4096 channels 9.6 / 8.5 / 8.3 us, 16: 15.2 / 12.2 / 11.2, 64: 22.5 / 20.1 / 21.0; 5120, 12: 14.1 / 12.0 / 11.6; 8192, 1: 10.6 / 10.9 / 11.5,
-// 8: 14.3 / 14.3 / 15.7, 16: 19.1 / 18.2 / 19.5, 24: 22.4 / 21.9 / 24.5, 32: 24.5 / 24.8 (512), 64: 40.0 / 42.6 / 48.6.
+// 8: 14.3 / 14.3 / 15.7, 16: 19.1 / 18.2 / 19.5, 24: 22.4 / 21.9 / 24.5, 32: 24.5 / 24.8 (512), 64: 40.0 / 42.6 / 48.6.  Few sequences of more than 4096
+// channels pay the parts and have little to convolve: 2 of 4640, rank 288, 9.4 / 9.4 / 9.8; 3 of 4960, 128 states, 22.0 / 22.1 / 23.2.
 int ajqd_scan_splits(int batch, int inner) {
-  const int block = inner <= 5120 ? scan_block(batch <= 32 ? 2 : 4) : scan_block(batch > 8 && batch <= 24 && inner <= 10240 ? 4 : 8);
+  const int block = inner <= 5120 ? scan_block(batch > 32 || (batch <= 4 && inner > 4096) ? 4 : 2) : scan_block(batch > 8 && batch <= 24 && inner <= 10240 ? 4 : 8);
   const int s = (inner + block - 1) / block, most = inner <= 10240 ? 20 : 8;  // (not timed past 10240 channels: as it was)
   return s < 1 ? 1 : s > most ? most : s;
 }
@@ -1085,7 +1089,7 @@ int ajqd_scan_step(const ajqd_scan_step_args* a, void* stream) {
     hipLaunchKernelGGL(kernel, dim3((a->inner + channels - 1) / channels, (a->batch + bb - 1) / bb), dim3(256), bytes, (hipStream_t)stream, s);
     return check_launch("ajqd_scan_step");
   };
-  switch (scan_step_batch(a->batch, a->inner, a->rank)) {
+  switch (scan_step_batch(a->batch, a->inner, a->rank, a->states)) {
     case 0: return go(scan_step_narrow_kernel, 16, kNarrowBatch);
     case 4: return go(scan_step_kernel<4>, 64, 4);
     default: return go(scan_step_kernel<8>, 64, 8);

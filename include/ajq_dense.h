@@ -243,7 +243,7 @@ int ajqd_scan_in_parts(const ajqd_scan_args* args, int parts, float* workspace, 
 int ajqd_scan_splits(int batch, int inner);
 /* in decimal digits: steps of 32 channels a wave of ajqd_scan_project takes of a block, its row tiles, 1 if their number is odd, and the sequences a
  * workgroup of ajqd_scan_step takes (0: 16 channels of four sequences); 0 if refused */
-int ajqd_scan_form(int batch, int inner, int rows, int splits, int rank);
+int ajqd_scan_form(int batch, int inner, int rows, int splits, int rank, int states);
 int ajqd_scan_project(const float* y, int ldy, const void* ring, const float* weight, const float* bias, const int64_t* pos, const void* w,
                       float* partial, int batch, int inner, int taps, int rows, int splits, void* stream);
 typedef struct {

@@ -294,10 +294,23 @@ def test_dense_library_refuses_bad_arguments_before_any_launch():
 def test_every_form_of_a_decode_step_of_the_scan_is_run():
     from tests.test_gpu_hybrid import SCAN_FORMS, SCAN_LINES, STEPS
     lib, up = _lib.load_dense(), lambda n: -(-n // 16) * 16
-    form = lambda batch, inner, states, rank, taps: (lib.ajqd_scan_form(batch, inner, up(rank + 2 * states), lib.ajqd_scan_splits(batch, inner), rank), taps == 4)
+    form = lambda batch, inner, states, rank, taps: (lib.ajqd_scan_form(batch, inner, up(rank + 2 * states), lib.ajqd_scan_splits(batch, inner), rank, states), taps == 4)
     got = {form(*s) for s in STEPS + SCAN_LINES + SCAN_FORMS}
     assert {(f // 100, four) for f, four in got} == {(10 * kb + rt, four) for kb in (2, 4, 8) for rt in (1, 2) for four in (True, False)}
     assert {f % 10 for f, _ in got} == {0, 4, 8} and {f // 10 % 10 for f, _ in got if f // 100 % 10 == 2} == {0, 1}
+
+
+@pytest.mark.parametrize("batch,inner,rank,states,splits,sequences", [
+    # the step: 16 channels, four sequences, eight in one round where four take two, and past two rounds of fours with up to 32 states
+    (4, 4096, 128, 16, 16, 0), (5, 4096, 128, 16, 16, 4), (24, 8192, 256, 16, 16, 4), (13, 13440, 208, 16, 8, 8), (32, 8192, 256, 64, 8, 8), (16, 17360, 272, 16, 8, 4),
+    (13, 18576, 512, 64, 8, 4), (31, 13440, 512, 16, 8, 8), (31, 13440, 512, 32, 8, 8), (48, 9712, 304, 36, 10, 4), (64, 12288, 384, 64, 8, 4),
+    # parts of the projection, few sequences past 4096 channels
+    (4, 4112, 256, 16, 9, 4), (5, 4112, 256, 16, 17, 4), (1, 5120, 160, 16, 10, 4), (1, 5136, 160, 16, 6, 4), (33, 4096, 128, 16, 8, 4),
+])
+def test_forms_of_a_decode_step_of_the_scan(batch, inner, rank, states, splits, sequences):
+    lib = _lib.load_dense()
+    assert lib.ajqd_scan_splits(batch, inner) == splits
+    assert lib.ajqd_scan_form(batch, inner, -(-(rank + 2 * states) // 16) * 16, splits, rank, states) % 10 == sequences
 
 
 def test_every_form_of_a_decode_product_is_run():
