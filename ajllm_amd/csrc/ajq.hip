@@ -1873,12 +1873,13 @@ int ajq_sample_pick(const float* logits, int B, int V, int ld, float temperature
 
 // fp32 caches: a bf16 copy of the rows pays where attention on it saves more than the copy takes.  The kernel on the copy saves a third (heads
 // of 128; a fifth with 64, nothing with 32) of a time of 4 FLOP a score and column at 520 TFLOP/s; the copy is a launch and 12 bytes an
-// element at 6.7 TB/s.  Heads of 128: 4 x 32 / 8 x 2048 positions 212 -> 169 us, 1 x 32 / 8 x 4096 197 -> 147; not made for 1 x 16 / 16 x 2048 (62).
+// element at 6.7 TB/s.  Heads of 128: 4 x 32 / 8 x 2048 positions 212 -> 169 us, 1 x 32 / 8 x 4096 197 -> 147; not made for 1 x 16 / 16 x 2048 (62), nor,
+// with 64 columns, for 16 x 2 / 2 x 3846 (86.0 us, 88.6 with it).
 size_t ajq_attn_prefill_workspace(int cache_dtype, int B, int H, int Hkv, int T, int start, int head_dim) {
   if (cache_dtype != AJQ_KV_F32 || B < 1 || H < 1 || Hkv < 1 || T < 1 || start < 0 || head_dim < 64) return 0;
   const double elements = (double)B * Hkv * ((double)start + T) * head_dim, bytes = 4 * elements;
   const double flops = 4.0 * B * H * head_dim * (double)T * (start + 0.5 * T);
-  if (bytes > kCopiedBytes || (head_dim < 128 ? 0.2 : 0.33) * flops / 5.2e14 < 1.15 * (4e-6 + 12 * elements / 6.7e12)) return 0;
+  if (bytes > kCopiedBytes || (head_dim < 128 ? 0.2 / 1.3 : 0.33 / 1.15) * flops / 5.2e14 < 4e-6 + 12 * elements / 6.7e12) return 0;
   return (size_t)bytes;
 }
 
@@ -1929,6 +1930,9 @@ int ajq_attn_prefill_in(const float* q, const void* kcache, const void* vcache, 
       hipLaunchKernelGGL(kernel, grid, dim3(256), 0, (hipStream_t)stream, q, reinterpret_cast<const CacheT*>(kcache),
                          reinterpret_cast<const CacheT*>(vcache), H, Hkv, T, start, max_len, out, out_bf16);
     };
+    if constexpr (HD == 64) {
+      if (cache_dtype == AJQ_KV_F32 && prefill_waits(B, H, Hkv, HD)) return go(attn_prefill_kernel<float, HD, true>, (float*)nullptr);
+    }
     if (cache_dtype == AJQ_KV_F32) return go(attn_prefill_kernel<float, HD>, (float*)nullptr);
     if constexpr (HD < 128) {
       if (!prefill_in_steps((long long)B * H, T, start, HD)) return go(attn_prefill_kernel<uint16_t, HD>, (uint16_t*)nullptr);

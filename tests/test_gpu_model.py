@@ -687,6 +687,21 @@ def test_flash_prefill_on_a_copy_of_fp32_caches(cuda, b, heads, kv_heads, t, sta
         assert errors(out, plain.cpu())[1] <= near
 
 
+@pytest.mark.parametrize("t,start", [(1, 0), (2, 63), (64, 0), (65, 1), (127, 66), (130, 257), (192, 0), (200, 3)])
+def test_flash_prefill_of_many_fp32_heads(cuda, t, start):
+    """More than 192 heads of 64 columns that share no keys wait for every block: the same bits as eight sequences at a time, which do not."""
+    from ajllm_amd.attention import flash_prefill
+    g, total = torch.Generator().manual_seed(t + start), start + t
+    q, keys, values = (torch.randn((16, 16, n, 64), generator=g) for n in (t, total + 2, total + 2))
+    keys[:, :, total:] = values[:, :, total:] = float("nan")
+    q, keys, values = q.to(cuda), keys.to(cuda), values.to(cuda)
+    got = flash_prefill(q, keys, values, start)
+    assert torch.equal(got, torch.cat([flash_prefill(q[b:b + 8], keys[b:b + 8], values[b:b + 8], start) for b in (0, 8)]))
+    mask = torch.ones(t, total, dtype=torch.bool, device=cuda).tril_(diagonal=start)
+    want = modeling.scaled_dot_product_attention(q, keys[:, :, :total], values[:, :, :total], mask).transpose(1, 2).reshape(16, t, 1024)
+    assert errors(got, want.cpu())[1] <= 8e-3   # bf16 operands: 2^-9 each of queries, keys, probabilities and values
+
+
 def test_model_with_flash_attention_flag(cuda):
     """use_flash_attention on every attention layer: prefill logits stay within flash-attention noise of
     the eager model, with and without a KV cache, and a following cached step agrees as well."""
