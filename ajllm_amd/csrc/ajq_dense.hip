@@ -211,12 +211,16 @@ bool staged_rows(int batch, int k, int waves, long long tiles) {
 // staged rows wherever one each would be more than a round of the CUs (5856 x 2048: 9.5 us, 7.9 with two; 4096 x 16384: 29.5, 38.0 with two); below
 // that, rows that are not staged have two blocks in flight instead (4096 x 18440: 44.2 -> 42.6) where K gives each wave several (5120 x 256,
 // 64 sequences: 9.1 us with two, 5.1 with one).  Up to 16, long staged rows that come out even: two blocks at a time (4096 x 16384: 26.6 -> 24.4;
-// 4096 x 8448, 5 sequences: 12.7, 12.3 with one).  K of one or two
+// 4096 x 8448, 5 sequences: 12.7, 12.3 with one), with more than eight sequences, whose rows are half of what is asked for, only where rows lie whole
+// multiples of 16 KiB apart (0.977 of the time with one) or, past twelve, of 4 KiB (9 sequences: 4032 x 11264 17.45 us, 16.2 with one).  K of one or two
 // blocks: two waves (32000 x 128, one sequence: 5.2 us on four, 4.4 on two).
 // More than four streams leave a wave of 16-row tiles and two batch tiles no registers for more than the plainest form: rows from memory, one row
 // tile, one block at a time takes 240, every other form 280 and more, and then a CU holds one workgroup instead of two (12 streams of 2064
 // columns, 33 sequences, K = 1152: 17.0 us, 34.1 with staged rows; 16 of 2560, 48 sequences, K = 2048: 28.7, 39.5).  Rows of 8192 columns make up
-// for that (8 of 4096, 64 sequences: 44.4 us staged, 50.4 from memory) but where the last batch block is nearly empty (5 of 2560, 33: 34.5, 33.6).
+// for that (8 of 4096, 64 sequences: 44.4 us staged, 50.4 from memory) but where the last batch block is nearly empty (5 of 2560, 33: 34.5, 33.6).  Rows off the 128-column
+// grid that are long beside what the streams take have two blocks in flight where there is a workgroup per CU anyway (6 of 2976, 31 sequences, K =
+// 16024: 49.3 -> 44.6; 15 of 2336, K = 13576: 1.085).  Up to 16 sequences two blocks of more than eight's staged rows take 273 registers
+// (13 of 11168, 12 sequences, K = 10240: 80.9 us, 55.1 with one; 140 shapes: 1.087 of the time from memory, 0.922 with one).
 struct OutCut {
   int rows, rt, bt, uq, xq;  // row tile, row tiles, batch tiles, blocks at a time, batch rows' instructions
   dim3 grid;
@@ -232,7 +236,9 @@ OutCut out_cut(int batch, int width, int k, bool sums, int streams) {
   const bool staged = staged_rows(batch, k, c.rows == 8 ? 8 : 4, tiles) && (!plain || k >= kLongRow);
   c.xq = few || !staged ? kStreamDirect : batch <= 4 ? 1 : batch <= 8 ? 2 : 4;
   c.rt = c.bt == 2 && width % 32 == 0 && (staged ? c.rows == 16 && tiles > kCus : !plain && width >= 8192) ? 2 : 1;
-  c.uq = c.rows == 8 || c.rt == 2 || few ? 1 : c.bt == 1 ? (staged && k >= kLongRow && k % 1024 == 0 ? 2 : 1) : !staged && !plain && k >= 2048 ? 2 : 1;
+  const bool pays = c.xq < 4 ? k % 1024 == 0 : streams <= 4 && (k % 8192 == 0 || (batch > 12 && k % 2048 == 0));
+  const bool room = plain ? tiles <= kCus && k >= kLongRow && k >= 1100 * streams : k >= 2048;
+  c.uq = c.rows == 16 && c.rt == 1 && !few && (c.bt == 1 ? staged && k >= kLongRow && pays : !staged && room) ? 2 : 1;
   c.grid = dim3(width / (c.rows * c.rt), blocks);
   c.threads = c.rows == 8 ? 512 : few ? 128 : 256;
   return c;
@@ -273,15 +279,15 @@ int with_out_cut(const OutCut& c, Go&& go) {
     if (c.rows == 8) return c.xq == 4 ? go(Int<8>{}, Int<8>{}, Int<1>{}, Int<2>{}, Int<1>{}, Int<4>{})
                                       : go(Int<8>{}, Int<8>{}, Int<1>{}, Int<2>{}, Int<1>{}, Int<kStreamDirect>{});
     if (c.xq == 4) return c.rt == 2 ? go(Int<4>{}, Int<16>{}, Int<2>{}, Int<2>{}, Int<1>{}, Int<4>{}) : go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<1>{}, Int<4>{});
+    if (c.uq == 2) return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<2>{}, Int<kStreamDirect>{});
     if constexpr (!kMany) {
-      if (c.uq == 2) return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<2>{}, Int<kStreamDirect>{});
       if (c.rt == 2) return go(Int<4>{}, Int<16>{}, Int<2>{}, Int<2>{}, Int<1>{}, Int<kStreamDirect>{});
     }
     return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<2>{}, Int<1>{}, Int<kStreamDirect>{});
   }
   auto with = [&](auto xq) {
     if (c.rows == 8) return go(Int<8>{}, Int<8>{}, Int<1>{}, Int<1>{}, Int<1>{}, xq);
-    if constexpr (xq() != kStreamDirect) {
+    if constexpr (xq() != kStreamDirect && !(kMany && xq() == 4)) {
       if (c.uq == 2) return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<2>{}, xq);
     }
     return go(Int<4>{}, Int<16>{}, Int<1>{}, Int<1>{}, Int<1>{}, xq);

@@ -130,9 +130,10 @@ def test_dense_out_streams(cuda, batch, shape):
 
 
 @pytest.mark.parametrize("streams,batch,k,width", [(12, 33, 1152, 2064), (5, 40, 2048, 4128), (16, 17, 1024, 4128), (8, 33, 2056, 2560), (16, 48, 8192, 2080),
-                                                   (6, 20, 8320, 2064)])
+                                                   (6, 20, 8320, 2064), (5, 17, 8200, 2064), (6, 33, 9224, 2064), (13, 12, 10240, 2064), (5, 9, 8192, 2080)])
 def test_dense_out_streams_of_many_streams_and_sequences(cuda, streams, batch, k, width):
-    """Tiles of 16 rows with more than four streams: from memory below rows of 8192 columns, staged from there on one and on two row tiles."""
+    """Tiles of 16 rows with more than four streams: from memory below rows of 8192 columns, one block or two at a time, staged from there on
+    one and on two row tiles; up to 16 sequences one block of long rows."""
     test_dense_out_streams(cuda, batch, (streams, k, width))
 
 

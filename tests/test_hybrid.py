@@ -356,6 +356,10 @@ def test_form_of_a_decode_product_of_few_sequences(batch, k, width, form):
     (8, 64, 8192, 4096, 1, 422214), (16, 17, 8192, 2064, 1, 421214), (8, 64, 8200, 8192, 1, 421210),
     # and the forms beside it: 8-row tiles, up to four streams, up to 16 sequences
     (12, 64, 1024, 512, 1, 811214), (4, 33, 1152, 2064, 1, 421214), (4, 33, 1152, 4096, 1, 422214), (4, 17, 2056, 4096, 1, 421220), (16, 16, 4096, 4096, 1, 421114),
+    # two blocks at a time: rows off the grid that are long for their streams, and up to 16 sequences
+    (6, 31, 16024, 2976, 0, 421220), (6, 33, 16024, 2976, 0, 421210), (16, 31, 16024, 2976, 0, 421210), (5, 17, 8184, 2976, 0, 421210), (5, 17, 8200, 2976, 0, 421220),
+    (5, 12, 16384, 4096, 0, 421114), (5, 8, 16384, 4096, 1, 421122), (4, 9, 16384, 4096, 1, 421124), (1, 12, 11264, 4096, 0, 421114), (1, 16, 10240, 4096, 0, 421124),
+    (1, 16, 9216, 4096, 0, 421114),
 ])
 def test_form_of_a_decode_product_with_streams(streams, batch, k, width, scaled, form):
     assert _lib.load_dense().ajqd_dense_out_form(batch, k, width, streams, scaled) == form
