@@ -1934,9 +1934,7 @@ int ajq_attn_prefill_in(const float* q, const void* kcache, const void* vcache, 
       if (cache_dtype == AJQ_KV_F32 && prefill_waits(B, H, Hkv, HD)) return go(attn_prefill_kernel<float, HD, true>, (float*)nullptr);
     }
     if (cache_dtype == AJQ_KV_F32) return go(attn_prefill_kernel<float, HD>, (float*)nullptr);
-    if constexpr (HD < 128) {
-      if (!prefill_in_steps((long long)B * H, T, start, HD)) return go(attn_prefill_kernel<uint16_t, HD>, (uint16_t*)nullptr);
-    }
+    if (!prefill_in_steps((long long)B * H, T, start, HD)) return go(attn_prefill_kernel<uint16_t, HD>, (uint16_t*)nullptr);
     go(attn_prefill_steps_kernel<HD>, (uint16_t*)nullptr);
   };
   if (head_dim == 128) launch(std::integral_constant<int, 128>{});

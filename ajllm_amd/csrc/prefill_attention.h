@@ -35,7 +35,7 @@
 // fp32 accumulators: the usual flash-attention arithmetic, not the eager fp32 one.
 //
 // Two kernels: attn_prefill_steps_kernel on bf16 caches interleaves both products and the softmax of three neighbouring half blocks;
-// attn_prefill_kernel goes block by block, for narrow heads where that is the faster (prefill_in_steps) and for fp32 caches, which pass through
+// attn_prefill_kernel goes block by block, where that is the faster (prefill_in_steps) and for fp32 caches, which pass through
 // registers that are converted on the way and leave none for the other, unless there is work enough to make a bf16 copy of the rows first
 // (caches_to_bf16_kernel).
 #pragma once
@@ -415,7 +415,9 @@ __global__ __launch_bounds__(256) void caches_to_bf16_kernel(const float* __rest
 // reads next (keys j + 1, values j) was asked for a block before and waited for in front of that barrier.
 // Four steps at places known to the compiler make the body; a wave's last ones (masked, or with blocks cut short) go one by one.
 //
-// prefill_in_steps: which bf16 calls it takes (figures: its time over attn_prefill_kernel's).  Heads of 128 all (78 shapes: 0.83 .. 1.03).  Narrower ones have
+// prefill_in_steps: which bf16 calls it takes (figures: its time over attn_prefill_kernel's).  Heads of 128 but for a few of up to 256 keys: a last block
+// that is more than half full is two masked steps there, which counts while a few rows behind others are all there is to do (1.04 .. 1.08; less than
+// half full 0.98) and while a CU's two workgroups finish together (257 .. 512 of 33 .. 128 keys: 1.03 .. 1.10); 9300 other shapes 0.975, the most 1.07.  Narrower ones have
 // few MFMAs in a step beside its latency, so short prompts are faster in whole blocks: 64 columns 1.03 .. 1.09 at 40 .. 64 keys, 0.99 / 1.09 at 100, 1.03 at
 // 192, 1.00 at 256, 0.93 at 512, 0.79 at 4096 with few workgroups; with more than a round of them from 128 on (200 keys: 0.98), over 194 shapes 0.93 (left: 1.05 where rounds come
 // out even, 1024 workgroups of 4096 queries).  32 columns: 1.04 ..
@@ -423,7 +425,11 @@ __global__ __launch_bounds__(256) void caches_to_bf16_kernel(const float* __rest
 // steps' share of vector work is the larger (768 workgroups and more: 1.01 .. 1.05; 384 of 312 queries 1.04, 512 of 900 0.91).
 __host__ __device__ inline bool prefill_in_steps(long long heads, int T, int start, int head_dim) {
   const long long workgroups = heads * ((T + kPfBQ - 1) / kPfBQ), keys = (long long)start + T;
-  if (head_dim == 128) return true;
+  if (head_dim == 128) {
+    if (keys <= 32 || keys > 256) return true;
+    if (workgroups <= 256) return T > 64 || start == 0 || ((keys - 1) & 32) == 0;
+    return workgroups > 512 || T <= 32 || keys > 128;
+  }
   if (head_dim == 64) return keys >= 256 || (keys > 128 && workgroups > 256);
   return keys > 320 && (workgroups <= 256 || (workgroups <= 512 && T >= 600));
 }

@@ -284,7 +284,8 @@ def test_a_layer_does_without_the_extension_module(monkeypatch):
 
 
 @pytest.mark.parametrize("b,heads,t,start,hd,steps", [
-    (1, 8, 1, 0, 128, 1), (64, 64, 4096, 0, 128, 1), (1, 8, 255, 0, 64, 0), (1, 8, 1, 255, 64, 1), (16, 16, 129, 0, 64, 1), (16, 16, 128, 0, 64, 0), (8, 16, 200, 0, 64, 0),
+    (1, 8, 1, 0, 128, 1), (64, 64, 4096, 0, 128, 1), (1, 8, 24, 8, 128, 1), (1, 8, 25, 8, 128, 0), (1, 8, 33, 0, 128, 1), (8, 32, 64, 0, 128, 1), (8, 32, 64, 64, 128, 0),
+    (8, 32, 65, 60, 128, 1), (9, 32, 64, 0, 128, 0), (9, 32, 32, 8, 128, 1), (9, 32, 65, 64, 128, 1), (17, 32, 64, 0, 128, 1), (1, 8, 20, 236, 128, 0), (1, 8, 20, 237, 128, 1), (1, 8, 255, 0, 64, 0), (1, 8, 1, 255, 64, 1), (16, 16, 129, 0, 64, 1), (16, 16, 128, 0, 64, 0), (8, 16, 200, 0, 64, 0),
     (8, 32, 200, 0, 64, 1), (1, 8, 320, 0, 32, 0), (1, 8, 321, 0, 32, 1), (8, 32, 128, 300, 32, 1), (9, 32, 128, 300, 32, 0), (1, 32, 2048, 0, 32, 1), (1, 32, 2049, 0, 32, 0),
     (4, 64, 200, 0, 32, 0), (1, 8, 8, 0, 48, -1), (0, 8, 8, 0, 64, -1),
 ])

@@ -660,6 +660,13 @@ def test_flash_prefill_of_narrow_heads_in_half_blocks(cuda, t, start, hd):
     test_flash_prefill_on_bf16_caches_at_the_edges_of_its_steps(cuda, t, start, hd)
 
 
+@pytest.mark.parametrize("t,start", [(1, 32), (1, 63), (2, 95), (31, 2), (32, 96), (33, 31), (64, 33), (63, 65), (17, 160), (64, 192), (40, 210)])
+def test_flash_prefill_of_wide_heads_in_whole_blocks(cuda, t, start):
+    """The same for the few rows behind others that heads of 128 columns take block by block."""
+    assert _lib.load().ajq_attn_prefill_steps(2, 4, t, start, 128) == 0
+    test_flash_prefill_on_bf16_caches_at_the_edges_of_its_steps(cuda, t, start, 128)
+
+
 @pytest.mark.parametrize("hd", [128, 64])
 @pytest.mark.parametrize("b,heads,kv_heads,t,start", [(16, 64, 1, 128, 901), (2, 32, 2, 2047, 0), (1, 64, 4, 1500, 1), (3, 96, 3, 513, 700)])
 def test_flash_prefill_on_a_copy_of_fp32_caches(cuda, b, heads, kv_heads, t, start, hd):
