@@ -20,8 +20,7 @@
 // What bounds these launches is the chain of round trips to memory, so no load may wait for another's value: the activations'
 // way into LDS has no branch and no select that would draw a load into itself (a norm from its sums used to fetch h and the gain only
 // after the row sums had arrived: a 12-layer int4 step of width 2048 at batch 1 took 0.326 ms with that, 0.313 without).  Several
-// rows with their sums are the exception: up to sixteen vectors of sums, the rows and the gains held at once cost more registers than the
-// trip is worth (int8, K = 1024, N = 11264, 12 rows: 12.2 us so, 9.0 with the sums dropped at the load).
+// rows with their sums are the exception: the sums, the rows and the gains held at once cost more registers than the trip is worth.
 #pragma once
 #include "gemv_kernels.h"
 #include "decode_kernels.h"
@@ -135,19 +134,26 @@ __global__ __launch_bounds__(kWaves * 64) void dequant_gemv_pro_kernel(
       a1[i][1] = pu[1];
     }
   }
-  // kProNormSums: the 64 / MROWS lanes of a row share the parts of its sum of squares
+  // kProNormSums: the 64 / MROWS lanes of a row share the parts of its sum of squares.  16 rows: no more loads than there are parts, all of them live
+  // (rows past the last repeat it and are never read).  Fewer rows keep a branch around each load: without, the compiler requests less ahead of
+  // it (8 rows of 4096 int4 columns: 1.15 .. 1.34 of the time; int8, 4 rows of 2048: 1.12).
   static_assert(kPro != kProNormSums || MROWS >= 4, "fewer rows: gemv_norm_kernels.h");
   constexpr int kLanesPerRow = 64 / MROWS;
-  constexpr int kPartLoads = kPro == kProNormSums ? (64 + kLanesPerRow - 1) / kLanesPerRow : 1;  // up to 256 parts
+  constexpr bool kExact = MROWS == 16;
+  constexpr int kPartLoads = kPro != kProNormSums ? 1 : kExact ? kWaves * kSlice / 64 / kLanesPerRow : (64 + kLanesPerRow - 1) / kLanesPerRow;  // (256 parts)
   float4 sums[kPartLoads];
   if (kPro == kProNormSums) {
     const int row = lane / kLanesPerRow, piece = lane % kLanesPerRow;
 #pragma unroll
     for (int u = 0; u < kPartLoads; ++u) {
       const int j = piece + u * kLanesPerRow;
-      const bool live = 4 * j < S && row < M;  // (idle lanes re-read the first 16 bytes)
-      sums[u] = *reinterpret_cast<const float4*>(src1 + (live ? (size_t)row * S + 4 * j : 0));
-      sums[u] = live ? sums[u] : float4{0.f, 0.f, 0.f, 0.f};
+      if (kExact) {
+        sums[u] = *reinterpret_cast<const float4*>(src1 + (size_t)min(row, M - 1) * S + 4 * j);
+      } else {
+        const bool live = 4 * j < S && row < M;  // (idle lanes re-read the first 16 bytes)
+        sums[u] = *reinterpret_cast<const float4*>(src1 + (live ? (size_t)row * S + 4 * j : 0));
+        sums[u] = live ? sums[u] : float4{0.f, 0.f, 0.f, 0.f};
+      }
     }
   }
   if (kW4) {  // before the weights: scales and zero-points are there when the first tile lands
